@@ -92,7 +92,10 @@ int jc_jaccard(const jc_csr *g, const float *vertex_weights, float *result, int 
 
 /* jc_jaccard with flags (JC_FLAG_*) and an optional caller workspace of at
  * least jc_jaccard_workspace_size() bytes (NULL: allocate per call). With a
- * workspace the call allocates nothing. No reference counterpart: the
+ * workspace the call allocates nothing. From 2^22 stored edges on that size
+ * includes the oriented engine's arrays (about 37 bytes per edge); a smaller
+ * workspace that still holds the owner engine's is accepted, and the call
+ * then uses that engine alone, with the same bits. No reference counterpart: the
  * reference allocates temporaries inside the call (jaccard.cpp:931-934). */
 int jc_jaccard_ex(const jc_csr *g, const float *vertex_weights, float *result, int edge_centric,
                   unsigned flags, void *workspace, size_t workspace_bytes, jc_stream_t stream);
@@ -124,15 +127,19 @@ typedef struct jc_tuning {
                                   home bucket; a task whose table then does not build is
                                   redone with the 32-bit table (1 forces that for every
                                   chunk with a full bucket) */
-  int32_t reserved[2];
+  int32_t engine;              /* 0 (default), JC_ENGINE_OWNER or JC_ENGINE_ORIENTED (then
+                                  the owner engine for what that one cannot do) */
+  int32_t reserved[1];
 } jc_tuning;
+#define JC_ENGINE_OWNER 1    /* each pair by streaming its shorter row */
+#define JC_ENGINE_ORIENTED 2 /* from the triangles, where that applies */
 
 /* jc_jaccard_ex that allocates nothing, for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops, hosts
  * that forbid allocation). No reference counterpart. Its workspace is a
  * fixed array of JC_NOALLOC_SCRATCH_BYTES that the library holds on every
- * device it runs on until the process ends; a graph whose
- * jc_jaccard_workspace_size() exceeds it gives JC_ERR_SCRATCH_LIMIT (32 MiB:
+ * device it runs on until the process ends; a graph whose owner-engine
+ * workspace exceeds it gives JC_ERR_SCRATCH_LIMIT (32 MiB:
  * about 1.18M vertices edge-centric weighted, 2.05M unweighted, at 16 to 30
  * stored edges per vertex; vertex-centric also needs 8 or 16 bytes per
  * stored edge). Inputs and the result are the

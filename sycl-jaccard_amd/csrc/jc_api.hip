@@ -74,6 +74,17 @@ Layout layout(int32_t n, int32_t m, bool weighted, bool ec) {
   return L;
 }
 
+// Oriented engine (jc_tri.hip) before the owner engine: from kTriMinEdges
+// stored edges on, where no tuning is given. Measured: RMAT-16 (1.8M entries)
+// 0.27 ms by the owner engine, 0.40 by this one, whose two dozen dependent
+// launches are then most of it; RMAT of 200003 vertices (5.7M) 1.58 and 1.12.
+constexpr int32_t kTriMinEdges = 1 << 22;
+
+bool tri_wanted(const jc_csr* g, const jc_tuning* t) {
+  if (t && (t->engine == JC_ENGINE_OWNER || t->wide_index || t->hash_table == 1 || t->quot_max_disp > 0)) return false;
+  return (t && t->engine == JC_ENGINE_ORIENTED) || (!t && g->m >= kTriMinEdges);
+}
+
 // RAII for a stream-ordered allocation.
 struct AsyncBuf {
   void* p = nullptr;
@@ -83,8 +94,10 @@ struct AsyncBuf {
   }
 };
 
+// ws: layout(...).total bytes; tri_ws: tri_workspace_bytes(...) bytes, or
+// nullptr to run the owner engine alone.
 int run_jaccard(const jc_csr* g, const float* vw, float* result, bool ec, unsigned flags,
-                unsigned char* ws, const jc_tuning* tuning, hipStream_t s) {
+                unsigned char* ws, unsigned char* tri_ws, const jc_tuning* tuning, hipStream_t s) {
   const bool weighted = vw != nullptr;
   const bool fixup = (flags & JC_FLAG_ASSUME_SYMMETRIC) == 0;
   const Layout L = layout(g->n, g->m, weighted, ec);
@@ -100,17 +113,27 @@ int run_jaccard(const jc_csr* g, const float* vw, float* result, bool ec, unsign
   a.bitmap_blocks_per_cu = tuning ? tuning->bitmap_blocks_per_cu : 0;
   a.hash_table = tuning ? tuning->hash_table : 0;
   a.quot_max_disp = tuning ? tuning->quot_max_disp : 0;
+  if (tri_ws) {
+    // both algorithms: the oriented engine's row sums, intersections and
+    // quotients are the vertex-centric pipeline's values
+    jc::EngineArgs t = a;
+    t.out32 = result;
+    JC_TRY(jc::run_tri(weighted ? jc::kModeEcW : jc::kModeEcU, t, tri_ws, &a.skip, s));
+  }
   double* S64 = weighted ? reinterpret_cast<double*>(ws + L.s64) : nullptr;
   if (weighted) {
     jc::ExactInfo* ex = reinterpret_cast<jc::ExactInfo*>(ws + L.exact);
-    JC_TRY(jc::launch_rowsum_f64(g->n, g->offsets, g->indices, vw, S64, ws + L.rows, s));
-    JC_TRY(jc::launch_exact_info(g->n, vw, S64, ex, s));
+    JC_TRY(jc::launch_rowsum_f64(g->n, g->offsets, g->indices, vw, S64, ws + L.rows, s, a.skip));
+    JC_TRY(jc::launch_exact_info(g->n, vw, S64, ex, s, a.skip));
     a.exact = ex;
   }
   a.S64 = S64;
-  if (ec) {
+  if (ec || tri_ws) {
+    // (vertex-centric after the oriented engine: what that left is computed
+    // by the fused pass, with the same bits)
     a.out32 = result;
-    if (fixup) JC_TRY(jc::launch_fill_u32(reinterpret_cast<uint32_t*>(result), g->m, jc::kSentinel32, s));
+    if (fixup)
+      JC_TRY(jc::launch_fill_u32(reinterpret_cast<uint32_t*>(result), g->m, jc::kSentinel32, s, a.skip));
     JC_TRY(jc::run_engine(weighted ? jc::kModeEcW : jc::kModeEcU, weighted, a, ws + L.engine, fixup, s));
     return JC_OK;
   }
@@ -178,7 +201,9 @@ extern "C" {
 
 size_t jc_jaccard_workspace_size(int32_t n, int32_t m, int weighted, int edge_centric) {
   if (n < 0 || m < 0) return 0;
-  return layout(n, m, weighted != 0, edge_centric != 0).total;
+  size_t b = layout(n, m, weighted != 0, edge_centric != 0).total;
+  if (m >= kTriMinEdges) b += al(jc::tri_workspace_bytes(n, m, weighted != 0));
+  return b;
 }
 
 int jc_jaccard_tuned(const jc_csr* g, const float* vertex_weights, float* result, int edge_centric,
@@ -187,16 +212,27 @@ int jc_jaccard_tuned(const jc_csr* g, const float* vertex_weights, float* result
   if (!csr_args_ok(g) || (g->m > 0 && !result) || (flags & ~JC_FLAG_ASSUME_SYMMETRIC)) return JC_ERR_INVALID_ARG;
   if (g->n == 0 || g->m == 0) return JC_OK;
   const bool ec = edge_centric != 0;
-  const size_t need = layout(g->n, g->m, vertex_weights != nullptr, ec).total;
+  const bool weighted = vertex_weights != nullptr;
+  const size_t need = layout(g->n, g->m, weighted, ec).total;
+  const size_t full = need + al(jc::tri_workspace_bytes(g->n, g->m, weighted));
   hipStream_t s = hs(stream);
+  bool tri = tri_wanted(g, tuning);
   if (workspace) {
     if (workspace_bytes < need) return JC_ERR_WORKSPACE;
-    return run_jaccard(g, vertex_weights, result, ec, flags, static_cast<unsigned char*>(workspace), tuning, s);
+    unsigned char* ws = static_cast<unsigned char*>(workspace);
+    return run_jaccard(g, vertex_weights, result, ec, flags, ws,
+                       tri && workspace_bytes >= full ? ws + need : nullptr, tuning, s);
   }
   AsyncBuf buf;
   buf.s = s;
-  JC_TRY(hipMallocAsync(&buf.p, need, s));
-  return run_jaccard(g, vertex_weights, result, ec, flags, static_cast<unsigned char*>(buf.p), tuning, s);
+  if (tri && hipMallocAsync(&buf.p, full, s) != hipSuccess) {
+    (void)hipGetLastError();
+    buf.p = nullptr;
+    tri = false;  // the owner engine needs a small part of it
+  }
+  if (!tri) JC_TRY(hipMallocAsync(&buf.p, need, s));
+  unsigned char* ws = static_cast<unsigned char*>(buf.p);
+  return run_jaccard(g, vertex_weights, result, ec, flags, ws, tri ? ws + need : nullptr, tuning, s);
 }
 
 int jc_jaccard_ex(const jc_csr* g, const float* vertex_weights, float* result, int edge_centric,
@@ -221,7 +257,8 @@ int jc_jaccard_noalloc(const jc_csr* g, const float* vertex_weights, float* resu
   JC_TRY(scratch_address(&ws));
   // Every part of the workspace that must start at zero (schedule counters,
   // range facts, row-sum queue) is cleared by the kernels of the call itself.
-  return run_jaccard(g, vertex_weights, result, ec, flags, static_cast<unsigned char*>(ws), nullptr, hs(stream));
+  return run_jaccard(g, vertex_weights, result, ec, flags, static_cast<unsigned char*>(ws), nullptr, nullptr,
+                     hs(stream));
 }
 
 int jc_jaccard_list(const jc_csr* g, const float* vertex_weights, int32_t num_pairs,

@@ -57,7 +57,8 @@ int grid_rows(int64_t rows, int waves_per_block, int cap_per_cu) {
 }  // namespace
 
 template <typename T>
-__global__ void k_fill(T* __restrict__ x, int64_t n, T v) {
+__global__ void k_fill(T* __restrict__ x, int64_t n, T v, const int* skip) {
+  if (skip && *skip) return;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     x[i] = v;
 }
@@ -65,19 +66,20 @@ __global__ void k_fill(T* __restrict__ x, int64_t n, T v) {
 hipError_t launch_fill_f32(float* x, int64_t n, float v, hipStream_t s) {
   ProfScope ps_("fill", s);
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fill<float>, dim3(grid_for(n, 256 * 4, 32)), dim3(256), 0, s, x, n, v);
+  hipLaunchKernelGGL(k_fill<float>, dim3(grid_for(n, 256 * 4, 32)), dim3(256), 0, s, x, n, v,
+                     (const int*)nullptr);
   return hipGetLastError();
 }
-hipError_t launch_fill_u32(uint32_t* x, int64_t n, uint32_t v, hipStream_t s) {
+hipError_t launch_fill_u32(uint32_t* x, int64_t n, uint32_t v, hipStream_t s, const int* skip) {
   ProfScope ps_("fill", s);
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fill<uint32_t>, dim3(grid_for(n, 256 * 4, 32)), dim3(256), 0, s, x, n, v);
+  hipLaunchKernelGGL(k_fill<uint32_t>, dim3(grid_for(n, 256 * 4, 32)), dim3(256), 0, s, x, n, v, skip);
   return hipGetLastError();
 }
-hipError_t launch_fill_u64(uint64_t* x, int64_t n, uint64_t v, hipStream_t s) {
+hipError_t launch_fill_u64(uint64_t* x, int64_t n, uint64_t v, hipStream_t s, const int* skip) {
   ProfScope ps_("fill", s);
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fill<uint64_t>, dim3(grid_for(n, 256 * 4, 32)), dim3(256), 0, s, x, n, v);
+  hipLaunchKernelGGL(k_fill<uint64_t>, dim3(grid_for(n, 256 * 4, 32)), dim3(256), 0, s, x, n, v, skip);
   return hipGetLastError();
 }
 
@@ -138,7 +140,8 @@ constexpr int kRowGroup = JC_ROW_GROUP;
 
 template <typename OutT, bool IDX>
 __global__ void k_rowsum_w(int32_t n, const int32_t* __restrict__ off, const int32_t* __restrict__ ind,
-                           const float* __restrict__ v, OutT* __restrict__ out) {
+                           const float* __restrict__ v, OutT* __restrict__ out, const int* skip) {
+  if (skip && *skip) return;
   constexpr int R = kWave / kRowGroup;  // rows per wave and iteration
   const int lane = lane_id();
   const int gl = lane % kRowGroup;
@@ -215,7 +218,9 @@ __global__ void k_rowsum_w_med(int32_t n, const int32_t* __restrict__ off, const
 // one counter serialised: 0.22 ms on RMAT-22).
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_collect_rows(int32_t n, const int32_t* __restrict__ off,
-                                                        int* __restrict__ list, int* __restrict__ counters) {
+                                                        int* __restrict__ list, int* __restrict__ counters,
+                                                        const int* skip) {
+  if (skip && *skip) return;  // empty lists: the kernels over them end at once
   constexpr int NW = BLOCK / kWave;
   __shared__ int s_w[2][NW];
   __shared__ int s_base[2];
@@ -312,7 +317,7 @@ size_t rowsum_scratch_bytes(int32_t n) { return ((size_t)std::max(n, 1) + 4) * s
 // allocation for the call.
 template <typename OutT>
 static hipError_t rowsum_both(int32_t n, const int32_t* off, const int32_t* ind, const float* v, OutT* out,
-                              void* scratch, hipStream_t s) {
+                              void* scratch, hipStream_t s, const int* skip = nullptr) {
   void* own = nullptr;
   hipError_t err;
   if (!scratch) {
@@ -322,18 +327,20 @@ static hipError_t rowsum_both(int32_t n, const int32_t* off, const int32_t* ind,
   int* counters = static_cast<int*>(scratch);
   int* list = counters + 4;
   const int cus = device_cu_count();
-  hipLaunchKernelGGL(k_fill<uint32_t>, dim3(1), dim3(64), 0, s, reinterpret_cast<uint32_t*>(counters), (int64_t)4, 0u);
-  hipLaunchKernelGGL(k_collect_rows<256>, dim3(grid_for(n, 256 * 4, 4)), dim3(256), 0, s, n, off, list, counters);
+  hipLaunchKernelGGL(k_fill<uint32_t>, dim3(1), dim3(64), 0, s, reinterpret_cast<uint32_t*>(counters), (int64_t)4, 0u,
+                     (const int*)nullptr);
+  hipLaunchKernelGGL(k_collect_rows<256>, dim3(grid_for(n, 256 * 4, 4)), dim3(256), 0, s, n, off, list, counters,
+                     skip);
   const int gs = grid_rows((n + kWave / kRowGroup - 1) / (kWave / kRowGroup), 4, 64);
   const int gm = grid_rows(n, 4, 64);  // at most n listed rows, one per wave
   if (ind) {
-    hipLaunchKernelGGL((k_rowsum_w<OutT, true>), dim3(gs), dim3(256), 0, s, n, off, ind, v, out);
+    hipLaunchKernelGGL((k_rowsum_w<OutT, true>), dim3(gs), dim3(256), 0, s, n, off, ind, v, out, skip);
     hipLaunchKernelGGL((k_rowsum_w_med<OutT, true>), dim3(gm), dim3(256), 0, s, n, off, ind, v, out, list,
                        counters);
     hipLaunchKernelGGL((k_rowsum_w_long<OutT, true, 1024>), dim3(cus * 2), dim3(1024), 0, s, off, ind, v, out,
                        list, counters);
   } else {
-    hipLaunchKernelGGL((k_rowsum_w<OutT, false>), dim3(gs), dim3(256), 0, s, n, off, ind, v, out);
+    hipLaunchKernelGGL((k_rowsum_w<OutT, false>), dim3(gs), dim3(256), 0, s, n, off, ind, v, out, skip);
     hipLaunchKernelGGL((k_rowsum_w_med<OutT, false>), dim3(gm), dim3(256), 0, s, n, off, ind, v, out, list,
                        counters);
     hipLaunchKernelGGL((k_rowsum_w_long<OutT, false, 1024>), dim3(cus * 2), dim3(1024), 0, s, off, ind, v, out,
@@ -359,10 +366,10 @@ hipError_t launch_rowsum_f32(int32_t n, const int32_t* off, const int32_t* ind, 
 }
 
 hipError_t launch_rowsum_f64(int32_t n, const int32_t* off, const int32_t* ind, const float* v,
-                             double* S, void* scratch, hipStream_t s) {
+                             double* S, void* scratch, hipStream_t s, const int* skip) {
   ProfScope ps_("rowsum", s);
   if (n <= 0) return hipSuccess;
-  return rowsum_both<double>(n, off, ind, v, S, scratch, s);
+  return rowsum_both<double>(n, off, ind, v, S, scratch, s, skip);
 }
 
 hipError_t launch_vertex_weights(int32_t n, const int32_t* off, const float* edge_w, float* W,
@@ -521,7 +528,9 @@ __global__ void k_exact_init(ExactInfo* e) {
 }
 
 __global__ __launch_bounds__(256) void k_exact_scan(int32_t n, const float* __restrict__ vw,
-                                                    const double* __restrict__ S, ExactInfo* info) {
+                                                    const double* __restrict__ S, ExactInfo* info,
+                                                    const int* skip) {
+  if (skip && *skip) return;
   int lsb = INT32_MAX, mx = INT32_MIN, bad = 0;
   for (int32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const uint32_t b = __float_as_uint(vw[i]);
@@ -566,9 +575,11 @@ __global__ __launch_bounds__(256) void k_exact_scan(int32_t n, const float* __re
   }
 }
 
-hipError_t launch_exact_info(int32_t n, const float* vw, const double* S, ExactInfo* info, hipStream_t s) {
+hipError_t launch_exact_info(int32_t n, const float* vw, const double* S, ExactInfo* info, hipStream_t s,
+                             const int* skip) {
   hipLaunchKernelGGL(k_exact_init, dim3(1), dim3(64), 0, s, info);
-  if (n > 0) hipLaunchKernelGGL(k_exact_scan, dim3(grid_for(n, 256 * 4, 4)), dim3(256), 0, s, n, vw, S, info);
+  if (n > 0) hipLaunchKernelGGL(k_exact_scan, dim3(grid_for(n, 256 * 4, 4)), dim3(256), 0, s, n, vw, S, info,
+                                skip);
   return hipGetLastError();
 }
 

@@ -30,6 +30,9 @@ constexpr uint64_t kSentinel64 = 0xFFFFFFFFFFFFFFFFull;
 
 __device__ __forceinline__ int lane_id() { return (int)__lane_id(); }
 
+// Orders one wave's LDS accesses before and after it (LDS private to the wave).
+__device__ __forceinline__ void lds_fence_wave() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront"); }
+
 __device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
 
 __device__ __forceinline__ int popc64(uint64_t x) { return __popcll(x); }

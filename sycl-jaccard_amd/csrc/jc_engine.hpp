@@ -1922,6 +1922,7 @@ __device__ __forceinline__ bool is_sentinel(const void* arr, int64_t k) {
 // Fix-up: recompute positions still holding the sentinel.
 template <int MODE, bool W, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_fixup(EngineArgs a) {
+  if (a.skip && *a.skip) return;
   constexpr bool F64 = MODE == kModeIsF64;
   const void* flag_arr = MODE == kModeEcU || MODE == kModeEcW ? (const void*)a.out32
                          : MODE == kModeIsF32                ? (const void*)a.ws32
@@ -2025,7 +2026,8 @@ template <bool W, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_sched_count(int32_t rows, const int32_t* __restrict__ off,
                                                        const int32_t* __restrict__ ind, Sched* sc, int small_max,
                                                        size_t bm_budget, int whole_max, const int2* segs,
-                                                       int nseg) {
+                                                       int nseg, const int* skip) {
+  if (skip && *skip) return;  // empty task lists: the kernels over them end at once
   __shared__ int hist[2 * kBuckets + 1];
   for (int i = threadIdx.x; i < 2 * kBuckets + 1; i += BLOCK) hist[i] = 0;
   __syncthreads();
@@ -2075,7 +2077,9 @@ template <bool W, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_sched_emit(int32_t rows, const int32_t* __restrict__ off,
                                                       const int32_t* __restrict__ ind, Sched* sc, int2* tasks,
                                                       int32_t* small_rows, int small_max, size_t bm_budget,
-                                                      int whole_max, const int2* segs, int nseg) {
+                                                      int whole_max, const int2* segs, int nseg,
+                                                      const int* skip) {
+  if (skip && *skip) return;
   constexpr int kSmallBin = 2 * kBuckets;
   __shared__ int hist[kSmallBin + 1];
   __shared__ int basep[kSmallBin + 1];
@@ -2191,10 +2195,10 @@ hipError_t run_engine_t(const EngineArgs& base, void* ws, bool fixup, hipStream_
     {
       ProfScope ps("sched", stream);
       hipLaunchKernelGGL((k_sched_count<W, PB>), dim3(g), dim3(PB), 0, stream, rows, a.off, a.ind, sc, a.small_max,
-                         bm_budget, whole_max, a.segs, a.nseg);
+                         bm_budget, whole_max, a.segs, a.nseg, a.skip);
       hipLaunchKernelGGL(k_sched_scan, dim3(1), dim3(64), 0, stream, sc);
       hipLaunchKernelGGL((k_sched_emit<W, PB>), dim3(g), dim3(PB), 0, stream, rows, a.off, a.ind, sc, tasks, small,
-                         a.small_max, bm_budget, whole_max, a.segs, a.nseg);
+                         a.small_max, bm_budget, whole_max, a.segs, a.nseg, a.skip);
       if ((err = hipGetLastError()) != hipSuccess) return err;
     }
 

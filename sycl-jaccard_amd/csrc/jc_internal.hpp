@@ -96,7 +96,18 @@ struct EngineArgs {
   int* redo;
   int* num_redo;
   int redo_pass;
+  // Device flag, or nullptr: when it is not 0 the results are already there
+  // (the oriented engine delivered them) and the pass does nothing.
+  const int* skip;
 };
+
+// Oriented engine (jc_tri.hip): kModeEcU / kModeEcW (out32 the result) and
+// kModeIsF32. It delivers only where its conditions hold, which the device
+// decides; *done then receives the address (in ws) of a flag that is set when
+// the results were written, for EngineArgs::skip of the owner engine that
+// must follow. ws holds tri_workspace_bytes(n, m, weighted) bytes.
+size_t tri_workspace_bytes(int32_t n, int64_t m, bool weighted);
+hipError_t run_tri(int mode, const EngineArgs& base, void* ws, const int** done, hipStream_t s);
 
 // Workspace needed by an owner-engine pass over a graph with n vertices and m
 // stored edges (task list, small-row list, counters). With row segments, n and
@@ -117,22 +128,24 @@ hipError_t run_pairs(int mode, bool weighted, int32_t n, const int32_t* off, con
                      hipStream_t stream);
 
 // Fills *info (device memory) for vertex weights vw[n] and their row sums S[n].
-hipError_t launch_exact_info(int32_t n, const float* vw, const double* S, ExactInfo* info, hipStream_t s);
+hipError_t launch_exact_info(int32_t n, const float* vw, const double* S, ExactInfo* info, hipStream_t s,
+                             const int* skip = nullptr);
 
 // Records a failing HIP call for jc_last_hip_error(); returns the JC_ERR_* code.
 int note_hip_error(hipError_t e);
 
 // Streaming kernels.
 hipError_t launch_fill_f32(float* x, int64_t n, float v, hipStream_t s);
-hipError_t launch_fill_u32(uint32_t* x, int64_t n, uint32_t v, hipStream_t s);
-hipError_t launch_fill_u64(uint64_t* x, int64_t n, uint64_t v, hipStream_t s);
+// (skip: as EngineArgs::skip)
+hipError_t launch_fill_u32(uint32_t* x, int64_t n, uint32_t v, hipStream_t s, const int* skip = nullptr);
+hipError_t launch_fill_u64(uint64_t* x, int64_t n, uint64_t v, hipStream_t s, const int* skip = nullptr);
 // Row sums take a scratch area of rowsum_scratch_bytes(n) (long-row list),
 // or nullptr to allocate one on the stream for the call.
 size_t rowsum_scratch_bytes(int32_t n);
 hipError_t launch_rowsum_f32(int32_t n, const int32_t* off, const int32_t* ind, const float* v,
                              float* work, void* scratch, hipStream_t s);
 hipError_t launch_rowsum_f64(int32_t n, const int32_t* off, const int32_t* ind, const float* v,
-                             double* S, void* scratch, hipStream_t s);
+                             double* S, void* scratch, hipStream_t s, const int* skip = nullptr);
 hipError_t launch_vertex_weights(int32_t n, const int32_t* off, const float* edge_w, float* W,
                                  void* scratch, hipStream_t s);
 hipError_t launch_jw_f32(int64_t m, const float* wi, const float* ws, float* out, hipStream_t s);

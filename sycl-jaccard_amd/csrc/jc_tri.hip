@@ -1,0 +1,1235 @@
+// Oriented engine: every intersection of a symmetric graph from its triangles.
+//
+// The owner engine (jc_engine.hpp) streams, for each pair {u, x}, the whole
+// shorter row: sum over pairs of min(d_u, d_x) entries (4.3e10 on RMAT-22).
+// I(u, v) is also the weight of the triangles over the edge {u, v}, and one
+// triangle serves three edges. Ranking the vertices by degree (rank 0 the
+// largest) and keeping of each row only the neighbours of lower rank,
+// R(u), leaves rows of at most sqrt(2m) entries, and every triangle
+// {w < v < u by rank} once: v, w in R(u), w in R(v). That is
+// sum |R(u)|^2 / 2 tests (7.2e9 on RMAT-22, a sixth), each against a bitmap
+// over the ranks below v, which for the vertices that matter is a few KiB.
+//
+//   rank     degree-bucket counting sort of the vertices
+//   orient   per row: R(u) sorted by rank (32-bit and, saturated, 16-bit
+//            copies, at the row's own offset), the row sum of the weights,
+//            and emap[k], the oriented slot of a stored entry (u, v in R(u))
+//   plan     places in the bit matrix, task lists
+//   wedge    per v: the bitmap of R(v) in LDS; for every u with v in R(u) (the
+//            entries of v's own row that are not in R(v); the position p of v
+//            in R(u) by binary search, which also fills emap for the entry
+//            and proves the entry has its mirror) the p entries before v are
+//            tested. Hits go two ways: into the LDS sum of the pair (v, w),
+//            weight W[u], and as one bit each into row p of u's bit matrix
+//   reduce   per u: the symmetric bit matrix M over R(u) times the weights
+//            gives the parts of the pairs (u, v) that have the third vertex
+//            in R(u); with the LDS sums of wedge that is the whole
+//            intersection, and the quotient is formed
+//   deliver  result[k] = value[emap[k]]
+//
+// No part depends on the order of the sums: counts are integers, and weights
+// are added in fp64 only when ExactInfo shows that every sum is exact. What
+// the engine cannot do it refuses before anything is written to the result
+// (TriCtl::bad): a graph that is not symmetric, has self loops or rows out of
+// order, weights
+// whose fp64 sums may round, a bit matrix larger than its budget, an |R(u)|
+// above kTriMaxOut. The owner engine, launched after it, then runs; when the
+// oriented engine has delivered, the owner engine's kernels return at once.
+//
+// Measured against the owner engine (whole calls): RMAT-22 weighted 58.3 ->
+// 26.6 ms, RMAT of 200003 vertices weighted vertex-centric 1.58 -> 1.12 ms,
+// Chung-Lu 2^20 4.01 -> 3.63 ms.
+#include <type_traits>
+
+#include "jc_device.hpp"
+#include "jc_internal.hpp"
+#include "jc_profile.hpp"
+
+namespace jc {
+
+namespace {
+
+constexpr int kTriBuckets = 1024;
+constexpr int kTriMaxOut = 4096;   // largest |R(u)|: the sort and reduce buffers in LDS
+constexpr int kTriRowWave = 1024;  // rows up to this many entries are oriented by one wave
+constexpr int kSat16 = 65535;      // 16-bit ranks saturate here
+constexpr int kWgMinDeg = 192;     // rows of at least this many entries get a workgroup in wedge
+constexpr int kWedgeB = 512;       // threads of a wedge workgroup, entries of a wedge task
+constexpr int kTabA = 2048;        // bitmap words of the 16-bit wedge kernel (65536 ranks)
+constexpr int kAccA = 1536;        // largest |R(v)| of the 16-bit wedge kernel
+constexpr int kTabB = 8192;        // the same for the 32-bit wedge kernel (262144 ranks)
+constexpr int kAccB = kTriMaxOut;
+constexpr int kWaveTab = 256;      // |R(v)| held in LDS by the one-wave wedge kernel
+
+// Monotone in the degree: exact below 512, 16 steps per octave above.
+__device__ __forceinline__ int deg_bucket(int d) {
+  if (d < 512) return d;
+  const int e = 31 - __clz(d);  // >= 9
+  return 512 + (e - 9) * 16 + ((d >> (e - 4)) & 15);
+}
+
+// Words of the bit matrix rows of 0 .. L-1 columns: sum of ceil(l / 32).
+__device__ __forceinline__ uint32_t tri_words(int L) {
+  const uint32_t t = (uint32_t)max(L - 1, 0), k = t >> 5;
+  return 16u * k * (k + 1u) + (t - 32u * k) * (k + 1u);
+}
+
+struct TriTask {
+  int32_t r;      // rank of v
+  int32_t piece;  // entries [piece * kWedgeB, ...) of v's row
+};
+
+}  // namespace
+
+struct TriCtl {
+  int bad;
+  int done;
+  int lsb, maxexp;               // exactness of the weights (see ExactInfo)
+  unsigned long long out_total;  // sum of |R(u)|
+  unsigned long long bits;       // words of the bit matrix handed out
+  int num_big;                   // rows oriented by a workgroup
+  int num_mid;                   // rows oriented by a wave
+  int num_task[2], cur_task[2];  // wedge tasks: 16-bit, 32-bit
+  int num_wave, num_s16, num_s64, num_red;
+  int cur_wave, cur_red, cur_big, pad;
+  int hist[kTriBuckets];
+  int cur[kTriBuckets];
+};
+
+namespace {
+
+struct TriArgs {
+  int32_t n;
+  int64_t m;
+  const int32_t* off;
+  const int32_t* ind;
+  const float* vw;
+  TriCtl* ctl;
+  int2* rw;         // per vertex: rank, weight bits
+  int32_t* vtx;     // per rank: vertex
+  float* wr;        // per rank: weight
+  double* sr;       // per rank: row sum of the weights (unweighted: unused)
+  int32_t* dr;      // per rank: degree
+  int4* info;       // per vertex: row offset, |R|, first word of its bit matrix, weight bits
+  uint32_t* R32;    // R(u) at [off[u], off[u] + |R(u)|), later the pairs' values
+  uint16_t* R16;
+  int32_t* emap;
+  double* accw;     // per slot: sums of wedge (weighted)
+  uint32_t* accu;   // (unweighted)
+  uint32_t* bits;
+  uint64_t bits_cap;
+  int32_t* list_mid;  // vertices by class; ends of one array (orient), then reused
+  int32_t* list_big;
+  TriTask* task[2];
+  int64_t task_cap;
+  int32_t* list_wave;  // ranks
+  int32_t* list_s16;   // vertices with |R| in 1..16
+  int32_t* list_s64;   // 17..64
+  int32_t* list_red;   // > 64
+  // delivery
+  int mode;
+  const float* work32;
+  float* out32;
+  float* ws32;
+  int accumulate;
+};
+
+__device__ __forceinline__ bool tri_go(const TriArgs& a) { return a.ctl->bad == 0; }
+
+// after orient: the facts that must hold before wedge starts
+template <bool W>
+__device__ __forceinline__ bool tri_ready(const TriArgs& a) {
+  const TriCtl* c = a.ctl;
+  if (c->bad != 0 || 2ull * c->out_total != (unsigned long long)a.m || c->bits > a.bits_cap) return false;
+  if constexpr (W) return exact_sums_fit_f64(ExactInfo{c->lsb, c->maxexp, 0, 0});
+  return true;
+}
+
+__global__ void k_tri_init(TriCtl* c) {
+  int* p = reinterpret_cast<int*>(c);
+  for (int i = threadIdx.x; i < (int)(sizeof(TriCtl) / sizeof(int)); i += blockDim.x) p[i] = 0;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    c->lsb = INT32_MAX;
+    c->maxexp = INT32_MIN;
+  }
+}
+
+// Degree histogram over each workgroup's contiguous range of vertices, and
+// the finest set bit of the weights.
+template <bool W, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_tri_hist(TriArgs a) {
+  __shared__ int h[kTriBuckets];
+  for (int i = threadIdx.x; i < kTriBuckets; i += BLOCK) h[i] = 0;
+  __syncthreads();
+  const int64_t per = ((int64_t)a.n + gridDim.x - 1) / gridDim.x;
+  const int32_t r0 = (int32_t)min(per * blockIdx.x, (int64_t)a.n), r1 = (int32_t)min(per * (blockIdx.x + 1), (int64_t)a.n);
+  int lsb = INT32_MAX;
+  bool bad = false;
+  for (int32_t u = r0 + threadIdx.x; u < r1; u += BLOCK) {
+    const int d = a.off[u + 1] - a.off[u];
+    atomicAdd(&h[deg_bucket(d)], 1);
+    if constexpr (W) {
+      const uint32_t b = __float_as_uint(a.vw[u]);
+      const uint32_t ex = (b >> 23) & 0xFFu, man = b & 0x7FFFFFu;
+      if (((b >> 31) && (b << 1)) || ex == 0xFFu) bad = true;  // negative or not finite (-0 is harmless)
+      else if (ex != 0 || man != 0) lsb = min(lsb, (ex ? (int)ex - 150 : -149) + (int)__builtin_ctz(ex ? (man | 0x800000u) : man));
+    }
+  }
+  if constexpr (W) {
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) lsb = min(lsb, __shfl_xor(lsb, o));
+    if (ballot(bad) && lane_id() == 0) atomicOr(&a.ctl->bad, 1);
+    if (lane_id() == 0 && lsb < *(volatile int*)&a.ctl->lsb) atomicMin(&a.ctl->lsb, lsb);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < kTriBuckets; i += BLOCK)
+    if (h[i]) atomicAdd(&a.ctl->hist[i], h[i]);
+}
+
+// First rank of every bucket, largest degrees first.
+__global__ __launch_bounds__(kTriBuckets) void k_tri_scan(TriCtl* c) {
+  __shared__ int part[kTriBuckets / kWave];
+  const int b = kTriBuckets - 1 - threadIdx.x;
+  const int v = c->hist[b];
+  int incl = v;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int t = __shfl_up(incl, o);
+    if (lane_id() >= o) incl += t;
+  }
+  if (lane_id() == kWave - 1) part[threadIdx.x / kWave] = incl;
+  __syncthreads();
+  int base = 0;
+  for (int i = 0; i < (int)threadIdx.x / kWave; ++i) base += part[i];
+  c->cur[b] = base + incl - v;
+}
+
+// Ranks: each workgroup counts its range per bucket, reserves the places with
+// one atomic per bucket, then assigns. Also the rank-ordered copies, and the
+// lists of the rows that orient takes by wave and by workgroup.
+template <bool W, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_tri_rank(TriArgs a) {
+  __shared__ int h[kTriBuckets];
+  __shared__ int base[kTriBuckets];
+  __shared__ int s_cnt[2], s_base[2];
+  for (int i = threadIdx.x; i < kTriBuckets; i += BLOCK) h[i] = 0;
+  if (threadIdx.x < 2) s_cnt[threadIdx.x] = 0;
+  __syncthreads();
+  const int64_t per = ((int64_t)a.n + gridDim.x - 1) / gridDim.x;
+  const int32_t r0 = (int32_t)min(per * blockIdx.x, (int64_t)a.n), r1 = (int32_t)min(per * (blockIdx.x + 1), (int64_t)a.n);
+  for (int32_t u = r0 + threadIdx.x; u < r1; u += BLOCK) {
+    const int d = a.off[u + 1] - a.off[u];
+    atomicAdd(&h[deg_bucket(d)], 1);
+    if (d > kTriRowWave) atomicAdd(&s_cnt[1], 1);
+    else if (d > kWave) atomicAdd(&s_cnt[0], 1);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < kTriBuckets; i += BLOCK) {
+    base[i] = h[i] ? atomicAdd(&a.ctl->cur[i], h[i]) : 0;
+    h[i] = 0;
+  }
+  if (threadIdx.x == 0) {
+    s_base[0] = s_cnt[0] ? atomicAdd(&a.ctl->num_mid, s_cnt[0]) : 0;
+    s_base[1] = s_cnt[1] ? atomicAdd(&a.ctl->num_big, s_cnt[1]) : 0;
+    s_cnt[0] = s_cnt[1] = 0;
+  }
+  __syncthreads();
+  for (int32_t u = r0 + threadIdx.x; u < r1; u += BLOCK) {
+    const int o = a.off[u], d = a.off[u + 1] - o;
+    const int b = deg_bucket(d);
+    const int r = base[b] + atomicAdd(&h[b], 1);
+    const float w = W ? a.vw[u] : 0.0f;
+    a.rw[u] = make_int2(r, __float_as_int(w));
+    a.vtx[r] = u;
+    a.dr[r] = d;
+    if constexpr (W) a.wr[r] = w;
+    if (d > kTriRowWave) a.list_big[s_base[1] + atomicAdd(&s_cnt[1], 1)] = u;
+    else if (d > kWave) a.list_mid[s_base[0] + atomicAdd(&s_cnt[0], 1)] = u;
+    else if (d == 0) a.info[u] = make_int4(o, 0, 0, __float_as_int(w));
+  }
+}
+
+// Row sum of row u (rank ru) and the bound of all of them.
+template <bool W>
+__device__ __forceinline__ void put_row_sum(const TriArgs& a, int32_t ru, double s) {
+  if constexpr (W) {
+    a.sr[ru] = s;
+    if (!(s >= 0.0) || isinf(s)) {
+      a.ctl->bad = 1;
+    } else if (s > 0.0) {
+      const int e = ilogb(s) + 1;
+      if (e > *(volatile int*)&a.ctl->maxexp) atomicMax(&a.ctl->maxexp, e);
+    }
+  }
+}
+
+// Writes entry (rank r, row entry k) of row o at sorted position p.
+template <bool W>
+__device__ __forceinline__ void put_out(const TriArgs& a, int o, int p, uint32_t r, int k) {
+  const int e = o + p;
+  a.R32[e] = r;
+  a.R16[e] = (uint16_t)min(r, (uint32_t)kSat16);
+  a.emap[k] = e;
+  if constexpr (W) a.accw[e] = 0.0;
+  else a.accu[e] = 0u;
+}
+
+// Rows of at most 64 entries: groups of G lanes, one row each (16 lanes for
+// rows of up to 16 entries). The position of an entry among the kept ones is
+// the number of kept ranks below its own, counted over the group.
+template <bool W, int G>
+__device__ __forceinline__ void orient_group(const TriArgs& a, bool valid, int32_t u, int o, int d, int ru, float w) {
+  const int gl = lane_id() & (G - 1), gb = lane_id() & ~(G - 1);
+  bool in_row = valid && gl < d;
+  int2 rw = make_int2(0, 0);
+  int32_t x = 0;
+  if (in_row) {
+    x = a.ind[o + gl];
+    rw = a.rw[x];
+    if (x == u || (gl > 0 && a.ind[o + gl - 1] >= x)) a.ctl->bad = 1;  // a self loop; a row out of order
+  }
+  const bool keep = in_row && rw.x < ru;
+  const uint64_t km = ballot(keep);
+  // kept ranks below mine: a lane that keeps nothing offers no rank
+  const int mine = keep ? rw.x : INT32_MAX;
+  int pos = 0;
+  const int dmax = G == kWave ? d : 16;
+  for (int j = 0; j < dmax; ++j) {
+    const int rj = G == kWave ? __builtin_amdgcn_readlane(mine, j) : __shfl(mine, gb + j);
+    pos += rj < mine ? 1 : 0;
+  }
+  if (keep) put_out<W>(a, o, pos, (uint32_t)rw.x, o + gl);
+  else if (in_row) a.emap[o + gl] = -1;
+  const uint64_t gm = G == kWave ? ~0ull : ((1ull << G) - 1) << gb;
+  const int cnt = popc64(km & gm);
+  if constexpr (W) {
+    double s = in_row ? (double)__int_as_float(rw.y) : 0.0;
+#pragma unroll
+    for (int t = 1; t < G; t <<= 1) s += __shfl_xor(s, t);
+    if (valid && gl == 0) put_row_sum<W>(a, ru, s);
+  }
+  if (valid && gl == 0) a.info[u] = make_int4(o, cnt, 0, __float_as_int(w));
+}
+
+template <bool W, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_tri_orient_small(TriArgs a) {
+  if (!tri_go(a)) return;
+  const int lane = lane_id();
+  const int nw = gridDim.x * (BLOCK / kWave);
+  for (int64_t base = (int64_t)(blockIdx.x * (BLOCK / kWave) + threadIdx.x / kWave) * kWave; base < a.n;
+       base += (int64_t)nw * kWave) {
+    const int32_t u = (int32_t)base + lane;
+    int o = 0, d = 0, ru = 0;
+    float w = 0.0f;
+    if (base + lane < a.n) {
+      o = a.off[u];
+      d = a.off[u + 1] - o;
+      const int2 rw = a.rw[u];
+      ru = rw.x;
+      w = __int_as_float(rw.y);
+    }
+    uint64_t m16 = ballot(d > 0 && d <= 16), m64 = ballot(d > 16 && d <= kWave);
+    while (m16) {
+      int src = -1;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        if (m16) {
+          const int b = __ffsll((unsigned long long)m16) - 1;
+          if (lane / 16 == g) src = b;
+          m16 &= m16 - 1;
+        }
+      }
+      const int s = max(src, 0);
+      orient_group<W, 16>(a, src >= 0, __shfl(u, s), __shfl(o, s), __shfl(d, s), __shfl(ru, s), __shfl(w, s));
+    }
+    while (m64) {
+      const int s = __ffsll((unsigned long long)m64) - 1;
+      m64 &= m64 - 1;
+      orient_group<W, kWave>(a, true, __builtin_amdgcn_readlane(u, s), __builtin_amdgcn_readlane(o, s),
+                             __builtin_amdgcn_readlane(d, s), __builtin_amdgcn_readlane(ru, s), __shfl(w, s));
+    }
+  }
+}
+
+// Rows of more entries: the kept ranks are compacted into LDS, then every
+// kept entry counts the kept ranks below its own (LDS broadcasts, 16 bytes
+// per read; quadratic, but the square of |R(u)| is what wedge then tests).
+// One wave per row (T = 64 threads, up to kTriRowWave entries) or one
+// workgroup per row.
+template <bool W, int T, int CAP>
+__device__ __forceinline__ void orient_row(const TriArgs& a, int32_t u, int tid, uint32_t* s_r, uint16_t* s_k, int* s_n,
+                                           double* s_s) {
+  const int o = a.off[u], d = a.off[u + 1] - o;
+  const int2 me = a.rw[u];
+  const int ru = me.x;
+  const int lane = lane_id();
+  if (tid == 0) {
+    *s_n = 0;
+    if constexpr (W && T > kWave) *s_s = 0.0;
+  }
+  if constexpr (T > kWave) __syncthreads();
+  else lds_fence_wave();
+  double sum = 0.0;
+  int cnt = 0;  // T == 64: kept so far
+  for (int b = 0; b < d; b += 4 * T) {
+    int32_t x[4];
+    int2 rw[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) x[t] = a.ind[o + min(b + t * T + tid, d - 1)];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) rw[t] = a.rw[x[t]];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int i = b + t * T + tid;
+      const bool in_row = i < d;
+      const bool keep = in_row && rw[t].x < ru;
+      if (in_row && (x[t] == u || (i > 0 && a.ind[o + i - 1] >= x[t]))) a.ctl->bad = 1;
+      const uint64_t km = ballot(keep);
+      int at = 0;
+      if constexpr (T == kWave) {
+        at = cnt + popc64(km & ((1ull << lane) - 1));
+        cnt += popc64(km);
+      } else {
+        if (lane == 0 && km) at = atomicAdd(s_n, popc64(km));
+        at = __builtin_amdgcn_readfirstlane(at) + popc64(km & ((1ull << lane) - 1));
+      }
+      if (keep) {
+        if (at < CAP) {
+          s_r[at] = (uint32_t)rw[t].x;
+          if constexpr (T == kWave) s_k[at] = (uint16_t)i;
+          else reinterpret_cast<int32_t*>(s_k)[at] = i;
+        }
+      } else if (in_row) {
+        a.emap[o + i] = -1;
+      }
+      if constexpr (W) sum += in_row ? (double)__int_as_float(rw[t].y) : 0.0;
+    }
+  }
+  if constexpr (W) {
+#pragma unroll
+    for (int t = 1; t < kWave; t <<= 1) sum += __shfl_xor(sum, t);
+    if constexpr (T > kWave) {
+      if (lane == 0) unsafeAtomicAdd(s_s, sum);
+    }
+  }
+  if constexpr (T > kWave) {
+    __syncthreads();
+    cnt = *s_n;
+    if constexpr (W) sum = *s_s;
+  } else {
+    lds_fence_wave();
+  }
+  if (tid == 0) {
+    put_row_sum<W>(a, ru, sum);
+    a.info[u] = make_int4(o, cnt, 0, me.y);
+    if (cnt > CAP) a.ctl->bad = 1;
+  }
+  const int c = min(cnt, CAP);
+  // pad to a multiple of four with a rank that counts for nobody
+  for (int i = c + tid; i < ((c + 3) & ~3); i += T) s_r[i] = 0xFFFFFFFFu;
+  if constexpr (T > kWave) __syncthreads();
+  else lds_fence_wave();
+  for (int i0 = 0; i0 < c; i0 += 2 * T) {
+    const int ia = i0 + tid, ib = i0 + T + tid;
+    const uint32_t ra = ia < c ? s_r[ia] : 0u, rb = ib < c ? s_r[ib] : 0u;
+    int pa = 0, pb = 0;
+    for (int j = 0; j < c; j += 4) {
+      const uint4 q = *reinterpret_cast<const uint4*>(s_r + j);
+      pa += (q.x < ra) + (q.y < ra) + (q.z < ra) + (q.w < ra);
+      pb += (q.x < rb) + (q.y < rb) + (q.z < rb) + (q.w < rb);
+    }
+    const int ka = ia < c ? (T == kWave ? (int)s_k[ia] : reinterpret_cast<int32_t*>(s_k)[ia]) : 0;
+    const int kb = ib < c ? (T == kWave ? (int)s_k[ib] : reinterpret_cast<int32_t*>(s_k)[ib]) : 0;
+    if (ia < c) put_out<W>(a, o, pa, ra, o + ka);
+    if (ib < c) put_out<W>(a, o, pb, rb, o + kb);
+  }
+  if constexpr (T > kWave) __syncthreads();
+  else lds_fence_wave();
+}
+
+template <bool W, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_tri_orient_mid(TriArgs a) {
+  constexpr int NW = BLOCK / kWave;
+  __shared__ __align__(16) uint32_t s_r[NW][kTriRowWave + 4];
+  __shared__ uint16_t s_k[NW][kTriRowWave];
+  __shared__ int s_n[NW];
+  if (!tri_go(a)) return;
+  const int w = threadIdx.x / kWave;
+  const int count = a.ctl->num_mid;
+  for (int i = blockIdx.x * NW + w; i < count; i += gridDim.x * NW)
+    orient_row<W, kWave, kTriRowWave>(a, a.list_mid[i], lane_id(), s_r[w], s_k[w], &s_n[w], nullptr);
+}
+
+template <bool W, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_tri_orient_big(TriArgs a) {
+  __shared__ __align__(16) uint32_t s_r[kTriMaxOut + 4];
+  __shared__ int32_t s_k[kTriMaxOut];
+  __shared__ int s_n, s_i;
+  __shared__ double s_s;
+  if (!tri_go(a)) return;
+  const int count = a.ctl->num_big;
+  for (;;) {
+    if (threadIdx.x == 0) s_i = atomicAdd(&a.ctl->cur_big, 1);
+    __syncthreads();
+    const int i = s_i;
+    if (i >= count) return;
+    orient_row<W, BLOCK, kTriMaxOut>(a, a.list_big[i], threadIdx.x, s_r, reinterpret_cast<uint16_t*>(s_k), &s_n, &s_s);
+  }
+}
+
+// In rank order: places in the bit matrix, wedge tasks, reduce lists. Each
+// workgroup takes BLOCK ranks, scans its counts and reserves with one atomic
+// per list; workgroups start in rank order, so the heavy tasks come first.
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_tri_plan(TriArgs a) {
+  constexpr int NW = BLOCK / kWave;
+  constexpr int NL = 6;  // tasks 16-bit, 32-bit, wave list, reduce lists 16, 64, above
+  __shared__ int s_w[NL][NW];
+  __shared__ unsigned long long s_bw[NW], s_ow[NW];
+  __shared__ int s_base[NL];
+  __shared__ unsigned long long s_bbase;
+  if (!tri_go(a)) return;
+  const int lane = lane_id(), wv = threadIdx.x / kWave;
+  for (int64_t b0 = (int64_t)blockIdx.x * BLOCK; b0 < a.n; b0 += (int64_t)gridDim.x * BLOCK) {
+    const int32_t r = (int32_t)(b0 + threadIdx.x);
+    int d = 0, dp = 0;
+    int32_t u = 0;
+    if (r < a.n) {
+      u = a.vtx[r];
+      d = a.dr[r];
+      dp = a.info[u].y;
+    }
+    const int din = d - dp;
+    int c[NL] = {0, 0, 0, 0, 0, 0};
+    const bool wg = din > 0 && d >= kWgMinDeg && dp <= kAccB && r <= 32 * kTabB;
+    const int npiece = (d + kWedgeB - 1) / kWedgeB;
+    const int kind = r < kSat16 && dp <= kAccA ? 0 : 1;
+    if (wg) c[kind] = npiece;
+    else if (din > 0) c[2] = 1;
+    if (dp > 0) c[dp <= 16 ? 3 : dp <= kWave ? 4 : 5] = 1;
+    const unsigned long long words = tri_words(dp);
+    int incl[NL];
+    unsigned long long bi = words, oi = (unsigned long long)dp;
+#pragma unroll
+    for (int l = 0; l < NL; ++l) incl[l] = c[l];
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+#pragma unroll
+      for (int l = 0; l < NL; ++l) {
+        const int t = __shfl_up(incl[l], o);
+        if (lane >= o) incl[l] += t;
+      }
+      const unsigned long long tb = __shfl_up(bi, o), to = __shfl_up(oi, o);
+      if (lane >= o) {
+        bi += tb;
+        oi += to;
+      }
+    }
+    if (lane == kWave - 1) {
+#pragma unroll
+      for (int l = 0; l < NL; ++l) s_w[l][wv] = incl[l];
+      s_bw[wv] = bi;
+      s_ow[wv] = oi;
+    }
+    __syncthreads();
+    if (threadIdx.x < NL) {
+      int t = 0;
+      for (int k = 0; k < NW; ++k) {
+        const int x = s_w[threadIdx.x][k];
+        s_w[threadIdx.x][k] = t;
+        t += x;
+      }
+      int* ctr[NL] = {&a.ctl->num_task[0], &a.ctl->num_task[1], &a.ctl->num_wave,
+                      &a.ctl->num_s16, &a.ctl->num_s64, &a.ctl->num_red};
+      s_base[threadIdx.x] = t ? atomicAdd(ctr[threadIdx.x], t) : 0;
+    } else if (threadIdx.x == NL) {
+      unsigned long long t = 0, ot = 0;
+      for (int k = 0; k < NW; ++k) {
+        const unsigned long long x = s_bw[k];
+        s_bw[k] = t;
+        t += x;
+        ot += s_ow[k];
+      }
+      s_bbase = t ? atomicAdd(&a.ctl->bits, t) : 0ull;
+      if (ot) atomicAdd(&a.ctl->out_total, ot);
+    }
+    __syncthreads();
+    int at[NL];
+#pragma unroll
+    for (int l = 0; l < NL; ++l) at[l] = s_base[l] + s_w[l][wv] + incl[l] - c[l];
+    if (wg)
+      for (int p = 0; p < npiece; ++p)
+        if (at[kind] + p < a.task_cap) a.task[kind][at[kind] + p] = TriTask{r, p};
+    if (c[2]) a.list_wave[at[2]] = r;
+    if (c[3]) a.list_s16[at[3]] = u;
+    if (c[4]) a.list_s64[at[4]] = u;
+    if (c[5]) a.list_red[at[5]] = u;
+    if (dp > 0) a.info[u].z = (int)(uint32_t)(s_bbase + s_bw[wv] + bi - words);
+    __syncthreads();
+  }
+}
+
+// Position of rank r in the sorted row R[0, n), or -1.
+template <typename RT>
+__device__ __forceinline__ int find_rank(const RT* __restrict__ R, int n, uint32_t r) {
+  int lo = 0, len = n;
+  while (len > 0) {
+    const int half = len >> 1;
+    if ((uint32_t)R[lo + half] < r) {
+      lo += half + 1;
+      len -= half + 1;
+    } else {
+      len = half;
+    }
+  }
+  return lo < n && (uint32_t)R[lo] == r ? lo : -1;
+}
+
+// Eight consecutive entries of a row (any alignment).
+struct __attribute__((packed, aligned(2))) Raw16 {
+  uint32_t v[4];
+};
+struct __attribute__((packed, aligned(4))) Raw32 {
+  uint32_t v[4];
+};
+template <typename RT>
+struct Octet;
+template <>
+struct Octet<uint16_t> {
+  uint32_t v[4];
+  __device__ __forceinline__ void load(const uint16_t* p) {
+    const Raw16 x = *reinterpret_cast<const Raw16*>(p);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = x.v[i];
+  }
+  __device__ __forceinline__ uint32_t get(int t) const { return (t & 1) ? v[t >> 1] >> 16 : v[t >> 1] & 0xFFFFu; }
+};
+template <>
+struct Octet<uint32_t> {
+  uint32_t v[8];
+  __device__ __forceinline__ void load(const uint32_t* p) {
+    const Raw32 x = *reinterpret_cast<const Raw32*>(p), y = *reinterpret_cast<const Raw32*>(p + 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[i] = x.v[i];
+      v[4 + i] = y.v[i];
+    }
+  }
+  __device__ __forceinline__ uint32_t get(int t) const { return v[t]; }
+};
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t or_dpp(uint32_t v) {
+  return v | (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, false);
+}
+
+// Tests the nv (<= 8, possibly <= 0) first entries of an octet against the
+// bitmap; hits add to the LDS sums and are returned as a byte.
+template <bool W, typename RT>
+__device__ __forceinline__ uint32_t probe_octet(const Octet<RT>& y, int nv, const uint2* tab, uint32_t guard,
+                                                typename std::conditional<W, double, uint32_t>::type* acc, double w) {
+  uint2 t[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    uint32_t wi = y.get(i) >> 5;
+    if constexpr (sizeof(RT) == 4) wi = min(wi, guard);  // entries past nv may be anything
+    t[i] = tab[wi];
+  }
+  const uint32_t live = nv >= 8 ? 0xFFu : nv <= 0 ? 0u : (1u << nv) - 1u;
+  uint32_t byte = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) byte |= __builtin_amdgcn_ubfe(t[i].x, y.get(i), 1u) << i;
+  byte &= live;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if (byte & (1u << i)) {
+      const uint32_t slot = __popc(__builtin_amdgcn_ubfe(t[i].x, 0u, y.get(i))) + t[i].y;
+      if constexpr (W) unsafeAtomicAdd(&acc[slot], w);
+      else atomicAdd(&acc[slot], 1u);
+    }
+  }
+  return byte;
+}
+
+constexpr int kWClasses = 8;  // entries to test: <= 8 << c for c < 7, more
+
+// Wedge, one workgroup per task (v, 512 entries of its row).
+template <bool W, typename RT, int TAB, int ACC>
+__global__ __launch_bounds__(kWedgeB, (TAB <= kTabA ? 8 : 2)) void k_tri_wedge(TriArgs a) {
+  constexpr int NW = kWedgeB / kWave;
+  constexpr int KIND = sizeof(RT) == 2 ? 0 : 1;
+  using AT = typename std::conditional<W, double, uint32_t>::type;
+  __shared__ __align__(16) uint2 tab[TAB + 1];  // word of the bitmap, |R(v)| below it (set where the word is not 0)
+  __shared__ AT acc[ACC];
+  __shared__ int s_start[kWedgeB];
+  __shared__ uint16_t s_p[kWedgeB];
+  __shared__ uint32_t s_row[kWedgeB];
+  __shared__ float s_wt[W ? kWedgeB : 1];
+  __shared__ int s_wcnt[kWClasses][NW];
+  __shared__ int s_cbase[kWClasses + 1], s_ubase[kWClasses + 1];
+  __shared__ int s_task, s_next;
+  if (!tri_ready<W>(a)) return;
+  const int tid = threadIdx.x, lane = lane_id(), w = tid / kWave;
+  const int ntask = a.ctl->num_task[KIND];
+  const RT* __restrict__ R = KIND == 0 ? (const RT*)a.R16 : (const RT*)a.R32;
+  for (;;) {
+    if (tid == 0) s_task = atomicAdd(&a.ctl->cur_task[KIND], 1);
+    __syncthreads();
+    const int ti = s_task;
+    if (ti >= ntask) return;
+    const TriTask tk = a.task[KIND][ti];
+    const int32_t r = tk.r, v = a.vtx[r];
+    const int4 vi = a.info[v];
+    const int d = a.dr[r];
+    const int ov = vi.x, dpv = vi.y;
+    const uint32_t guard = KIND == 0 ? 0u : (uint32_t)(r + 31) >> 5;
+    for (int i = tid; i <= (r + 31) >> 5; i += kWedgeB) tab[i] = make_uint2(0u, 0u);
+    if (tid == 0) s_next = 0;
+    // the entries of v's row that are not in R(v): where v stands in R(x)
+    int cls = -1, start = 0, p = 0;
+    uint32_t row = 0;
+    float wt = 0.0f;
+    const int i = tk.piece * kWedgeB + tid;
+    if (i < d) {
+      const int k = ov + i;
+      if (a.emap[k] < 0) {
+        const int4 xi = a.info[a.ind[k]];
+        start = xi.x;
+        wt = __int_as_float(xi.w);
+        p = find_rank(R + start, xi.y, (uint32_t)r);
+        if (p < 0) {
+          a.ctl->bad = 1;  // (v, x) is stored, (x, v) is not
+        } else {
+          a.emap[k] = start + p;
+          row = (uint32_t)xi.z + tri_words(p);
+          if (p > 0) cls = p <= 8 ? 0 : p > 512 ? 7 : 29 - __clz(p - 1);
+        }
+      }
+    }
+    int rank = 0;
+#pragma unroll
+    for (int c = 0; c < kWClasses; ++c) {
+      const uint64_t bm = ballot(cls == c);
+      if (cls == c) rank = popc64(bm & ((1ull << lane) - 1));
+      if (lane == 0) s_wcnt[c][w] = popc64(bm);
+    }
+    __syncthreads();
+    for (int j = tid; j < dpv; j += kWedgeB) {
+      const uint32_t y = (uint32_t)R[ov + j];
+      const uint32_t yp = j > 0 ? (uint32_t)R[ov + j - 1] : 0u;
+      acc[j] = 0;
+      atomicOr(&tab[y >> 5].x, 1u << (y & 31u));
+      if (j == 0 || (yp >> 5) != (y >> 5)) tab[y >> 5].y = (uint32_t)j;
+    }
+    if (tid == 0) {
+      int ib = 0, ub = 0;
+      for (int c = kWClasses - 1; c >= 0; --c) {
+        int n = 0;
+        for (int k = 0; k < NW; ++k) {
+          const int x = s_wcnt[c][k];
+          s_wcnt[c][k] = n;
+          n += x;
+        }
+        s_cbase[kWClasses - 1 - c] = ib;
+        s_ubase[kWClasses - 1 - c] = ub;
+        ib += n;
+        const int per = kWave >> min(c, 6);
+        ub += (n + per - 1) / per;
+      }
+      s_cbase[kWClasses] = ib;
+      s_ubase[kWClasses] = ub;
+    }
+    __syncthreads();
+    if (cls >= 0) {
+      const int at = s_cbase[kWClasses - 1 - cls] + s_wcnt[cls][w] + rank;
+      s_start[at] = start;
+      s_p[at] = (uint16_t)p;
+      s_row[at] = row;
+      if constexpr (W) s_wt[at] = wt;
+    }
+    __syncthreads();
+    const int nunits = s_ubase[kWClasses];
+    for (;;) {
+      int un = 0;
+      if (lane == 0) un = atomicAdd(&s_next, 1);
+      un = __builtin_amdgcn_readfirstlane(un);
+      if (un >= nunits) break;
+      int k = 0;
+      while (un >= s_ubase[k + 1]) ++k;
+      const int lg = min(kWClasses - 1 - k, 6);  // log2 of the lanes per entry
+      const int gl = lane & ((1 << lg) - 1);
+      const int it = s_cbase[k] + ((un - s_ubase[k]) << (6 - lg)) + (lane >> lg);
+      const bool valid = it < s_cbase[k + 1];
+      const int st = valid ? s_start[it] : 0;
+      const int len = valid ? (int)s_p[it] : 0;
+      const uint32_t rowb = valid ? s_row[it] : 0u;
+      const double wu = W ? (double)(valid ? s_wt[W ? it : 0] : 0.0f) : 0.0;
+      Octet<RT> y;
+      if (gl * 8 < len) y.load(R + st + gl * 8);
+      for (int b = 0;;) {
+        const int at = b + gl * 8;
+        Octet<RT> yn;
+        const bool more = lg == 6 && b + 512 < len;  // wave-uniform: one entry per wave
+        if (more && at + 512 < len) yn.load(R + st + at + 512);
+        uint32_t byte = 0;
+        if (at < len) byte = probe_octet<W, RT>(y, len - at, tab, guard, acc, wu);
+        // four lanes' bytes make one word of the row
+        uint32_t word = byte << ((gl & 3) * 8);
+        if (lg >= 1) word = or_dpp<0xB1>(word);
+        if (lg >= 2) word = or_dpp<0x4E>(word);
+        if ((gl & 3) == 0 && at < len) a.bits[rowb + (uint32_t)(at >> 5)] = word;
+        if (!more) break;
+        b += 512;
+        y = yn;
+      }
+    }
+    __syncthreads();
+    // the pairs (v, w): alone on its row, or one of several pieces
+    for (int j = tid; j < dpv; j += kWedgeB) {
+      const AT s = acc[j];
+      if constexpr (W) {
+        if (d <= kWedgeB) a.accw[ov + j] = s;
+        else if (s != 0.0) unsafeAtomicAdd(&a.accw[ov + j], s);
+      } else {
+        if (d <= kWedgeB) a.accu[ov + j] = s;
+        else if (s != 0u) atomicAdd(&a.accu[ov + j], s);
+      }
+    }
+  }
+}
+
+// Wedge, one wave per v: short rows, and rows beyond the workgroup kernels'
+// tables. R(v) is searched (in LDS up to kWaveTab entries), eight lanes per
+// entry of v's row.
+template <bool W, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_tri_wedge_wave(TriArgs a) {
+  constexpr int NW = BLOCK / kWave;
+  using AT = typename std::conditional<W, double, uint32_t>::type;
+  __shared__ uint32_t s_list[NW][kWaveTab];
+  __shared__ AT s_acc[NW][kWaveTab];
+  if (!tri_ready<W>(a)) return;
+  const int lane = lane_id(), w = threadIdx.x / kWave;
+  const int gl = lane & 7;
+  const int count = a.ctl->num_wave;
+  AT* const gacc = W ? (AT*)a.accw : (AT*)a.accu;
+  for (int li = blockIdx.x * NW + w; li < count; li += gridDim.x * NW) {
+    const int32_t r = a.list_wave[li], v = a.vtx[r];
+    const int4 vi = a.info[v];
+    const int d = a.dr[r], ov = vi.x, dpv = vi.y;
+    const bool lds = dpv <= kWaveTab;
+    if (lds)
+      for (int j = lane; j < dpv; j += kWave) {
+        s_list[w][j] = a.R32[ov + j];
+        s_acc[w][j] = 0;
+      }
+    lds_fence_wave();
+    for (int b = 0; b < d; b += kWave) {
+      int start = 0, p = 0;
+      uint32_t row = 0;
+      float wt = 0.0f;
+      if (b + lane < d) {
+        const int k = ov + b + lane;
+        if (a.emap[k] < 0) {
+          const int4 xi = a.info[a.ind[k]];
+          start = xi.x;
+          wt = __int_as_float(xi.w);
+          p = find_rank(a.R32 + start, xi.y, (uint32_t)r);
+          if (p < 0) {
+            a.ctl->bad = 1;
+            p = 0;
+          } else {
+            a.emap[k] = start + p;
+            row = (uint32_t)xi.z + tri_words(p);
+          }
+        }
+      }
+      uint64_t todo = ballot(p > 0);
+      while (todo) {
+        int src = -1;
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+          if (todo) {
+            const int s = __ffsll((unsigned long long)todo) - 1;
+            if ((lane >> 3) == g) src = s;
+            todo &= todo - 1;
+          }
+        }
+        const int s = max(src, 0);
+        const int st = __shfl(start, s);
+        const int ls = __shfl(p, s);
+        const int len = src >= 0 ? ls : 0;
+        const uint32_t rowb = (uint32_t)__shfl((int)row, s);
+        const float wu = __shfl(wt, s);
+        for (int c = 0; ballot(c < len) != 0; c += 32) {
+          const int at = c + gl * 4;
+          uint32_t nib = 0;
+          if (at < len) {
+            const Raw32 y = *reinterpret_cast<const Raw32*>(a.R32 + st + at);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              if (at + t < len) {
+                const int q = lds ? find_rank(s_list[w], dpv, y.v[t]) : find_rank(a.R32 + ov, dpv, y.v[t]);
+                if (q >= 0) {
+                  nib |= 1u << t;
+                  // (separate branches: one pointer for both would be flat atomics)
+                  if (lds) {
+                    if constexpr (W) unsafeAtomicAdd(&s_acc[w][q], (double)wu);
+                    else atomicAdd(&s_acc[w][q], 1u);
+                  } else {
+                    if constexpr (W) unsafeAtomicAdd(&gacc[ov + q], (double)wu);
+                    else atomicAdd(&gacc[ov + q], 1u);
+                  }
+                }
+              }
+            }
+          }
+          uint32_t word = nib << (gl * 4);
+          word = or_dpp<0xB1>(word);
+          word = or_dpp<0x4E>(word);
+          word = or_dpp<0x141>(word);
+          if (gl == 0 && c < len) a.bits[rowb + (uint32_t)(c >> 5)] = word;
+        }
+      }
+    }
+    lds_fence_wave();
+    if (lds)
+      for (int j = lane; j < dpv; j += kWave) gacc[ov + j] = s_acc[w][j];
+    lds_fence_wave();
+  }
+}
+
+// The value of slot e (row u of rank ru, neighbour rank rv): the quotient, or
+// the intersection and the sum of the row sums for the kernel-level entry.
+template <bool W>
+__device__ __forceinline__ void put_value(const TriArgs& a, int e, int32_t u, int du, double su, uint32_t rv,
+                                          double isum, uint32_t cnt) {
+  if (a.mode == kModeIsF32) {
+    const float add = W ? (float)isum : (float)cnt;
+    const float ws = a.work32[u] + a.work32[a.vtx[rv]];
+    // the slot's sum was read before: its place takes the pair
+    if constexpr (W) reinterpret_cast<float2*>(a.accw)[e] = make_float2(add, ws);
+    else {
+      a.accu[e] = __float_as_uint(add);
+      a.R32[e] = __float_as_uint(ws);
+    }
+    return;
+  }
+  float q;
+  if constexpr (W) {
+    const double ws = su + a.sr[rv];
+    q = (float)(isum / (ws - isum));
+  } else {
+    const float fI = (float)cnt;
+    q = fI / ((float)(du + a.dr[rv]) - fI);
+  }
+  a.R32[e] = __float_as_uint(q);
+}
+
+// Reduce for |R(u)| <= G: lane p of a group holds row p of the matrix; the
+// transpose comes from one ballot per column.
+template <bool W, int G>
+__device__ __forceinline__ void reduce_group(const TriArgs& a, bool valid, int32_t u) {
+  const int lane = lane_id(), gl = lane & (G - 1), gb = lane & ~(G - 1);
+  int4 inf = make_int4(0, 0, 0, 0);
+  int2 me = make_int2(0, 0);
+  if (valid) {
+    inf = a.info[u];
+    me = a.rw[u];
+  }
+  const int o = inf.x, dp = inf.y;
+  const bool act = valid && gl < dp;
+  uint32_t rv = 0;
+  uint64_t row = 0;
+  float wv = 0.0f;
+  double sum = 0.0;
+  uint32_t cnt = 0;
+  if (act) {
+    rv = a.R32[o + gl];
+    if constexpr (W) {
+      wv = a.wr[rv];
+      sum = a.accw[o + gl];
+    } else {
+      cnt = a.accu[o + gl];
+    }
+    const uint32_t rb = (uint32_t)inf.z + tri_words(gl);
+    if (gl > 0) row = a.bits[rb];
+    if (G > 32 && gl > 32) row |= (uint64_t)a.bits[rb + 1] << 32;
+  }
+  int dmax = dp;
+  if constexpr (G < kWave) {
+    dmax = max(dmax, __shfl_xor(dmax, 16));
+    dmax = max(dmax, __shfl_xor(dmax, 32));
+  }
+  dmax = __builtin_amdgcn_readfirstlane(dmax);
+  uint64_t full = row;
+  for (int c = 0; c < dmax; ++c) {
+    const uint64_t col = ballot((row >> c) & 1ull);
+    const uint64_t mine = G == kWave ? col : (col >> gb) & ((1ull << G) - 1);
+    if (gl == c) full |= mine;
+  }
+  if constexpr (W) {
+    for (int q = 0; q < dmax; ++q) {
+      const float wq = G == kWave ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wv), q)) : __shfl(wv, gb + q);
+      if ((full >> q) & 1ull) sum += (double)wq;
+    }
+  } else {
+    cnt += (uint32_t)popc64(full);
+  }
+  if (act) {
+    const int du = a.dr[me.x];
+    const double su = W ? a.sr[me.x] : 0.0;
+    put_value<W>(a, o + gl, u, du, su, rv, sum, cnt);
+  }
+}
+
+template <bool W, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_tri_reduce_small(TriArgs a) {
+  if (!tri_ready<W>(a)) return;
+  const int lane = lane_id();
+  const int gw = blockIdx.x * (BLOCK / kWave) + threadIdx.x / kWave, nw = gridDim.x * (BLOCK / kWave);
+  const int n16 = a.ctl->num_s16, n64 = a.ctl->num_s64;
+  for (int i = gw; i < n64; i += nw) reduce_group<W, kWave>(a, true, a.list_s64[i]);
+  for (int i = gw * 4; i < n16; i += nw * 4) {
+    const int j = i + lane / 16;
+    reduce_group<W, 16>(a, j < n16, a.list_s16[min(j, n16 - 1)]);
+  }
+}
+
+// Reduce for larger |R(u)|: a workgroup per u, 64 x 64 blocks of the lower
+// triangle dealt to the waves; both halves of a block's symmetric
+// contribution are added to LDS sums.
+template <bool W, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_tri_reduce_big(TriArgs a) {
+  constexpr int NW = BLOCK / kWave;
+  using AT = typename std::conditional<W, double, uint32_t>::type;
+  __shared__ AT s_acc[kTriMaxOut];
+  __shared__ float s_wt[W ? kTriMaxOut : 1];
+  __shared__ int s_i;
+  if (!tri_ready<W>(a)) return;
+  const int tid = threadIdx.x, lane = lane_id(), w = tid / kWave;
+  const int count = a.ctl->num_red;
+  for (;;) {
+    if (tid == 0) s_i = atomicAdd(&a.ctl->cur_red, 1);
+    __syncthreads();
+    const int li = s_i;
+    if (li >= count) return;
+    const int32_t u = a.list_red[li];
+    const int4 inf = a.info[u];
+    const int ru = a.rw[u].x;
+    const int o = inf.x, dp = inf.y;
+    const int nb = (dp + kWave - 1) / kWave;
+    for (int i = tid; i < nb * kWave; i += BLOCK) {
+      if constexpr (W) {
+        s_acc[i] = i < dp ? a.accw[o + i] : 0.0;
+        s_wt[i] = i < dp ? a.wr[a.R32[o + i]] : 0.0f;
+      } else {
+        s_acc[i] = i < dp ? a.accu[o + i] : 0u;
+      }
+    }
+    __syncthreads();
+    // blocks (P, Q), Q <= P, in row order
+    const int nblk = nb * (nb + 1) / 2;
+    int P = 0, Q = 0, at = 0;
+    for (int blk = w; blk < nblk; blk += NW) {
+      while (at < blk) {
+        if (++Q > P) {
+          ++P;
+          Q = 0;
+        }
+        ++at;
+      }
+      const int p = P * kWave + lane;
+      uint32_t lo = 0, hi = 0;
+      if (p < dp) {
+        const uint32_t rb = (uint32_t)inf.z + tri_words(p);
+        const int nwords = (p + 31) >> 5;
+        if (2 * Q < nwords) lo = a.bits[rb + 2 * Q];
+        if (2 * Q + 1 < nwords) hi = a.bits[rb + 2 * Q + 1];
+      }
+      uint32_t tlo = 0, thi = 0;  // column `lane`: its rows
+      AT racc = 0, cacc = 0;
+#pragma unroll 8
+      for (int c = 0; c < kWave; ++c) {
+        const bool bit = ((c < 32 ? lo : hi) >> (c & 31)) & 1u;
+        const uint64_t col = ballot(bit);
+        if constexpr (W) {
+          const double wq = (double)s_wt[Q * kWave + c];
+          if (bit) racc += wq;
+          tlo = lane == c ? (uint32_t)col : tlo;
+          thi = lane == c ? (uint32_t)(col >> 32) : thi;
+        } else {
+          cacc = lane == c ? (uint32_t)popc64(col) : cacc;
+        }
+      }
+      if constexpr (W) {
+#pragma unroll 8
+        for (int q = 0; q < kWave; ++q) {
+          const bool bit = ((q < 32 ? tlo : thi) >> (q & 31)) & 1u;
+          const double wp = (double)s_wt[P * kWave + q];
+          if (bit) cacc += wp;
+        }
+        if (racc != 0.0) unsafeAtomicAdd(&s_acc[p], racc);
+        if (cacc != 0.0) unsafeAtomicAdd(&s_acc[Q * kWave + lane], cacc);
+      } else {
+        racc = (uint32_t)(__popc(lo) + __popc(hi));
+        if (racc) atomicAdd(&s_acc[p], racc);
+        if (cacc) atomicAdd(&s_acc[Q * kWave + lane], cacc);
+      }
+    }
+    __syncthreads();
+    const int du = a.dr[ru];
+    const double su = W ? a.sr[ru] : 0.0;
+    for (int i = tid; i < dp; i += BLOCK) {
+      const uint32_t rv = a.R32[o + i];
+      if constexpr (W) put_value<W>(a, o + i, u, du, su, rv, s_acc[i], 0u);
+      else put_value<W>(a, o + i, u, du, su, rv, 0.0, s_acc[i]);
+    }
+    __syncthreads();
+  }
+}
+
+template <bool W>
+__global__ __launch_bounds__(256) void k_tri_deliver(TriArgs a) {
+  if (!tri_ready<W>(a)) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) a.ctl->done = 1;
+  const int64_t nt = (int64_t)gridDim.x * blockDim.x;
+  if (a.mode == kModeIsF32) {
+    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < a.m; k += nt) {
+      const int e = a.emap[k];
+      float2 x;
+      if constexpr (W) x = reinterpret_cast<const float2*>(a.accw)[e];
+      else x = make_float2(__uint_as_float(a.accu[e]), __uint_as_float(a.R32[e]));
+      a.out32[k] = (a.accumulate ? a.out32[k] : 0.0f) + x.x;
+      a.ws32[k] = x.y;
+    }
+    return;
+  }
+  // four entries per thread, a stride apart: their gathers are in flight together
+  const int64_t quads = (a.m + 3) / 4;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < quads; i += nt) {
+    int e[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) e[t] = i + t * quads < a.m ? a.emap[i + t * quads] : 0;
+    uint32_t q[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) q[t] = a.R32[e[t]];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      if (i + t * quads < a.m) a.out32[i + t * quads] = __uint_as_float(q[t]);
+  }
+}
+
+size_t al256(size_t v) { return (v + 255) / 256 * 256; }
+
+constexpr uint64_t kBitsWordsPerEdge = 4;
+
+uint64_t bits_cap(int64_t m) { return std::min<uint64_t>(kBitsWordsPerEdge * (uint64_t)m, 0xFFFFFF00ull); }
+
+int64_t tri_tasks(int32_t n, int64_t m) { return m / kWedgeB + std::min<int64_t>(n, m / kWgMinDeg) + 1; }
+
+// Carves the workspace; with p == nullptr only measures it.
+size_t carve(TriArgs& a, unsigned char* p, int32_t n, int64_t m, bool weighted) {
+  size_t o = 0;
+  auto take = [&](size_t bytes) {
+    unsigned char* q = p ? p + o : nullptr;
+    o += al256(bytes);
+    return q;
+  };
+  const size_t nn = (size_t)std::max(n, 1), mm = (size_t)m;
+  a.ctl = reinterpret_cast<TriCtl*>(take(sizeof(TriCtl)));
+  a.rw = reinterpret_cast<int2*>(take(nn * sizeof(int2)));
+  a.vtx = reinterpret_cast<int32_t*>(take(nn * 4));
+  a.dr = reinterpret_cast<int32_t*>(take(nn * 4));
+  a.wr = reinterpret_cast<float*>(weighted ? take(nn * 4) : nullptr);
+  a.sr = reinterpret_cast<double*>(weighted ? take(nn * 8) : nullptr);
+  a.info = reinterpret_cast<int4*>(take(nn * sizeof(int4)));
+  a.R32 = reinterpret_cast<uint32_t*>(take((mm + 16) * 4));
+  a.R16 = reinterpret_cast<uint16_t*>(take((mm + 16) * 2));
+  a.emap = reinterpret_cast<int32_t*>(take(mm * 4));
+  unsigned char* acc = take(mm * (weighted ? 8 : 4));
+  a.accw = weighted ? reinterpret_cast<double*>(acc) : nullptr;
+  a.accu = weighted ? nullptr : reinterpret_cast<uint32_t*>(acc);
+  a.bits_cap = bits_cap(m);
+  a.bits = reinterpret_cast<uint32_t*>(take((size_t)a.bits_cap * 4));
+  a.list_mid = reinterpret_cast<int32_t*>(take(nn * 4));
+  a.list_big = reinterpret_cast<int32_t*>(take(nn * 4));
+  a.task_cap = tri_tasks(n, m);
+  a.task[0] = reinterpret_cast<TriTask*>(take((size_t)a.task_cap * sizeof(TriTask)));
+  a.task[1] = reinterpret_cast<TriTask*>(take((size_t)a.task_cap * sizeof(TriTask)));
+  a.list_wave = reinterpret_cast<int32_t*>(take(nn * 4));
+  a.list_s16 = reinterpret_cast<int32_t*>(take(nn * 4));
+  a.list_s64 = a.list_mid;  // orient is done with its lists when plan runs
+  a.list_red = a.list_big;
+  return o;
+}
+
+template <bool W>
+hipError_t tri_launch(const TriArgs& a, hipStream_t s) {
+  const int cus = device_cu_count();
+  constexpr int PB = 256;
+  auto grid = [&](int64_t items, int per, int cap) {
+    return dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>((items + per - 1) / per, (int64_t)cus * cap)));
+  };
+  {
+    ProfScope ps("tri_rank", s);
+    hipLaunchKernelGGL(k_tri_init, dim3(1), dim3(1024), 0, s, a.ctl);
+    const dim3 g = grid(a.n, PB * 4, 4);
+    hipLaunchKernelGGL((k_tri_hist<W, PB>), g, dim3(PB), 0, s, a);
+    hipLaunchKernelGGL(k_tri_scan, dim3(1), dim3(kTriBuckets), 0, s, a.ctl);
+    hipLaunchKernelGGL((k_tri_rank<W, PB>), g, dim3(PB), 0, s, a);
+  }
+  {
+    ProfScope ps("tri_orient", s);
+    hipLaunchKernelGGL((k_tri_orient_big<W, PB>), dim3(cus * 4), dim3(PB), 0, s, a);
+    hipLaunchKernelGGL((k_tri_orient_mid<W, PB>), grid(std::min<int64_t>(a.n, a.m / kWave), PB / kWave, 32), dim3(PB), 0, s, a);
+    hipLaunchKernelGGL((k_tri_orient_small<W, PB>), grid(a.n, PB, 32), dim3(PB), 0, s, a);
+  }
+  {
+    ProfScope ps("tri_plan", s);
+    hipLaunchKernelGGL((k_tri_plan<PB>), grid(a.n, PB, 64), dim3(PB), 0, s, a);
+  }
+  {
+    ProfScope ps("tri_wedge", s);
+    hipLaunchKernelGGL((k_tri_wedge<W, uint16_t, kTabA, kAccA>), dim3(cus * 4), dim3(kWedgeB), 0, s, a);
+    hipLaunchKernelGGL((k_tri_wedge<W, uint32_t, kTabB, kAccB>), dim3(cus), dim3(kWedgeB), 0, s, a);
+    hipLaunchKernelGGL((k_tri_wedge_wave<W, PB>), grid(a.n, PB / kWave, 32), dim3(PB), 0, s, a);
+  }
+  {
+    ProfScope ps("tri_reduce", s);
+    hipLaunchKernelGGL((k_tri_reduce_big<W, PB>), dim3(cus * (W ? 3 : 8)), dim3(PB), 0, s, a);
+    hipLaunchKernelGGL((k_tri_reduce_small<W, PB>), grid(a.n, 4 * PB / kWave, 32), dim3(PB), 0, s, a);
+  }
+  {
+    ProfScope ps("tri_deliver", s);
+    hipLaunchKernelGGL((k_tri_deliver<W>), grid(a.m, 1024, 32), dim3(256), 0, s, a);
+  }
+  return hipGetLastError();
+}
+
+}  // namespace
+
+size_t tri_workspace_bytes(int32_t n, int64_t m, bool weighted) {
+  TriArgs a{};
+  return carve(a, nullptr, n, m, weighted);
+}
+
+hipError_t run_tri(int mode, const EngineArgs& e, void* ws, const int** done, hipStream_t s) {
+  TriArgs a{};
+  const bool weighted = e.vw != nullptr;
+  carve(a, static_cast<unsigned char*>(ws), e.n, e.m, weighted);
+  a.n = e.n;
+  a.m = e.m;
+  a.off = e.off;
+  a.ind = e.ind;
+  a.vw = e.vw;
+  a.mode = mode;
+  a.work32 = e.work32;
+  a.out32 = e.out32;
+  a.ws32 = e.ws32;
+  a.accumulate = e.accumulate;
+  *done = &a.ctl->done;
+  return weighted ? tri_launch<true>(a, s) : tri_launch<false>(a, s);
+}
+
+}  // namespace jc
