@@ -36,9 +36,9 @@
 // above kTriMaxOut. The owner engine, launched after it, then runs; when the
 // oriented engine has delivered, the owner engine's kernels return at once.
 //
-// Measured against the owner engine (whole calls): RMAT-22 weighted 58.3 ->
-// 26.6 ms, RMAT of 200003 vertices weighted vertex-centric 1.58 -> 1.12 ms,
-// Chung-Lu 2^20 4.01 -> 3.63 ms.
+// Measured against the owner engine (whole calls): RMAT-22 weighted 58.2 ->
+// 20.6 ms, RMAT of 200003 vertices weighted vertex-centric 1.58 -> 0.96 ms,
+// Chung-Lu 2^20 4.00 -> 3.38 ms.
 #include <type_traits>
 
 #include "jc_device.hpp"
@@ -60,6 +60,8 @@ constexpr int kAccA = 1536;        // largest |R(v)| of the 16-bit wedge kernel
 constexpr int kTabB = 8192;        // the same for the 32-bit wedge kernel (262144 ranks)
 constexpr int kAccB = kTriMaxOut;
 constexpr int kWaveTab = 256;      // |R(v)| held in LDS by the one-wave wedge kernel
+constexpr int kRedWave = 256;      // |R(u)| that reduce takes by one wave
+constexpr int kRedWg = 1280;       // by a workgroup with that many weights in LDS; above, kTriMaxOut
 
 // Monotone in the degree: exact below 512, 16 steps per octave above.
 __device__ __forceinline__ int deg_bucket(int d) {
@@ -71,7 +73,7 @@ __device__ __forceinline__ int deg_bucket(int d) {
 // Words of the bit matrix rows of 0 .. L-1 columns: sum of ceil(l / 32).
 __device__ __forceinline__ uint32_t tri_words(int L) {
   const uint32_t t = (uint32_t)max(L - 1, 0), k = t >> 5;
-  return 16u * k * (k + 1u) + (t - 32u * k) * (k + 1u);
+  return (k + 1u) * (t - 16u * k);
 }
 
 struct TriTask {
@@ -90,8 +92,9 @@ struct TriCtl {
   int num_big;                   // rows oriented by a workgroup
   int num_mid;                   // rows oriented by a wave
   int num_task[2], cur_task[2];  // wedge tasks: 16-bit, 32-bit
-  int num_wave, num_s16, num_s64, num_red;
-  int cur_wave, cur_red, cur_big, pad;
+  int num_wave, num_s16, num_s64;
+  int num_red[2], cur_red[2];    // reduce by workgroup: up to kRedWg entries, more
+  int cur_big;
   int hist[kTriBuckets];
   int cur[kTriBuckets];
 };
@@ -124,8 +127,8 @@ struct TriArgs {
   int64_t task_cap;
   int32_t* list_wave;  // ranks
   int32_t* list_s16;   // vertices with |R| in 1..16
-  int32_t* list_s64;   // 17..64
-  int32_t* list_red;   // > 64
+  int32_t* list_s64;   // up to kRedWave
+  int32_t* list_red[2];  // up to kRedWg, more
   // delivery
   int mode;
   const float* work32;
@@ -484,7 +487,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_orient_big(TriArgs a) {
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_tri_plan(TriArgs a) {
   constexpr int NW = BLOCK / kWave;
-  constexpr int NL = 6;  // tasks 16-bit, 32-bit, wave list, reduce lists 16, 64, above
+  constexpr int NL = 7;  // tasks 16-bit, 32-bit, wave list, reduce lists by |R|
   __shared__ int s_w[NL][NW];
   __shared__ unsigned long long s_bw[NW], s_ow[NW];
   __shared__ int s_base[NL];
@@ -501,13 +504,13 @@ __global__ __launch_bounds__(BLOCK) void k_tri_plan(TriArgs a) {
       dp = a.info[u].y;
     }
     const int din = d - dp;
-    int c[NL] = {0, 0, 0, 0, 0, 0};
+    int c[NL] = {0, 0, 0, 0, 0, 0, 0};
     const bool wg = din > 0 && d >= kWgMinDeg && dp <= kAccB && r <= 32 * kTabB;
     const int npiece = (d + kWedgeB - 1) / kWedgeB;
     const int kind = r < kSat16 && dp <= kAccA ? 0 : 1;
     if (wg) c[kind] = npiece;
     else if (din > 0) c[2] = 1;
-    if (dp > 0) c[dp <= 16 ? 3 : dp <= kWave ? 4 : 5] = 1;
+    if (dp > 0) c[dp <= 16 ? 3 : dp <= kRedWave ? 4 : dp <= kRedWg ? 5 : 6] = 1;
     const unsigned long long words = tri_words(dp);
     int incl[NL];
     unsigned long long bi = words, oi = (unsigned long long)dp;
@@ -541,7 +544,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_plan(TriArgs a) {
         t += x;
       }
       int* ctr[NL] = {&a.ctl->num_task[0], &a.ctl->num_task[1], &a.ctl->num_wave,
-                      &a.ctl->num_s16, &a.ctl->num_s64, &a.ctl->num_red};
+                      &a.ctl->num_s16, &a.ctl->num_s64, &a.ctl->num_red[0], &a.ctl->num_red[1]};
       s_base[threadIdx.x] = t ? atomicAdd(ctr[threadIdx.x], t) : 0;
     } else if (threadIdx.x == NL) {
       unsigned long long t = 0, ot = 0;
@@ -564,7 +567,8 @@ __global__ __launch_bounds__(BLOCK) void k_tri_plan(TriArgs a) {
     if (c[2]) a.list_wave[at[2]] = r;
     if (c[3]) a.list_s16[at[3]] = u;
     if (c[4]) a.list_s64[at[4]] = u;
-    if (c[5]) a.list_red[at[5]] = u;
+    if (c[5]) a.list_red[0][at[5]] = u;
+    if (c[6]) a.list_red[1][at[6]] = u;
     if (dp > 0) a.info[u].z = (int)(uint32_t)(s_bbase + s_bw[wv] + bi - words);
     __syncthreads();
   }
@@ -926,11 +930,11 @@ __device__ __forceinline__ void put_value(const TriArgs& a, int e, int32_t u, in
   a.R32[e] = __float_as_uint(q);
 }
 
-// Reduce for |R(u)| <= G: lane p of a group holds row p of the matrix; the
-// transpose comes from one ballot per column.
-template <bool W, int G>
-__device__ __forceinline__ void reduce_group(const TriArgs& a, bool valid, int32_t u) {
-  const int lane = lane_id(), gl = lane & (G - 1), gb = lane & ~(G - 1);
+// Reduce for |R(u)| <= 16: four rows u per wave, lane p of a group holds row p
+// of the matrix; the transpose comes from one ballot per column.
+template <bool W>
+__device__ __forceinline__ void reduce_16(const TriArgs& a, bool valid, int32_t u) {
+  const int lane = lane_id(), gl = lane & 15, gb = lane & ~15;
   int4 inf = make_int4(0, 0, 0, 0);
   int2 me = make_int2(0, 0);
   if (valid) {
@@ -939,11 +943,9 @@ __device__ __forceinline__ void reduce_group(const TriArgs& a, bool valid, int32
   }
   const int o = inf.x, dp = inf.y;
   const bool act = valid && gl < dp;
-  uint32_t rv = 0;
-  uint64_t row = 0;
+  uint32_t rv = 0, row = 0, cnt = 0;
   float wv = 0.0f;
   double sum = 0.0;
-  uint32_t cnt = 0;
   if (act) {
     rv = a.R32[o + gl];
     if constexpr (W) {
@@ -952,140 +954,240 @@ __device__ __forceinline__ void reduce_group(const TriArgs& a, bool valid, int32
     } else {
       cnt = a.accu[o + gl];
     }
-    const uint32_t rb = (uint32_t)inf.z + tri_words(gl);
-    if (gl > 0) row = a.bits[rb];
-    if (G > 32 && gl > 32) row |= (uint64_t)a.bits[rb + 1] << 32;
+    if (gl > 0) row = a.bits[(uint32_t)inf.z + tri_words(gl)];
   }
   int dmax = dp;
-  if constexpr (G < kWave) {
-    dmax = max(dmax, __shfl_xor(dmax, 16));
-    dmax = max(dmax, __shfl_xor(dmax, 32));
-  }
+  dmax = max(dmax, __shfl_xor(dmax, 16));
+  dmax = max(dmax, __shfl_xor(dmax, 32));
   dmax = __builtin_amdgcn_readfirstlane(dmax);
-  uint64_t full = row;
+  uint32_t full = row;
   for (int c = 0; c < dmax; ++c) {
-    const uint64_t col = ballot((row >> c) & 1ull);
-    const uint64_t mine = G == kWave ? col : (col >> gb) & ((1ull << G) - 1);
-    if (gl == c) full |= mine;
+    const uint64_t col = ballot((row >> c) & 1u);
+    if (gl == c) full |= (uint32_t)(col >> gb) & 0xFFFFu;
   }
   if constexpr (W) {
     for (int q = 0; q < dmax; ++q) {
-      const float wq = G == kWave ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wv), q)) : __shfl(wv, gb + q);
-      if ((full >> q) & 1ull) sum += (double)wq;
+      const float wq = __shfl(wv, gb + q);
+      if ((full >> q) & 1u) sum += (double)wq;
     }
   } else {
-    cnt += (uint32_t)popc64(full);
+    cnt += (uint32_t)__popc(full);
   }
-  if (act) {
-    const int du = a.dr[me.x];
-    const double su = W ? a.sr[me.x] : 0.0;
-    put_value<W>(a, o + gl, u, du, su, rv, sum, cnt);
-  }
+  if (act) put_value<W>(a, o + gl, u, a.dr[me.x], W ? a.sr[me.x] : 0.0, rv, sum, cnt);
 }
 
 template <bool W, int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_tri_reduce_small(TriArgs a) {
+__global__ __launch_bounds__(BLOCK) void k_tri_reduce_16(TriArgs a) {
   if (!tri_ready<W>(a)) return;
-  const int lane = lane_id();
   const int gw = blockIdx.x * (BLOCK / kWave) + threadIdx.x / kWave, nw = gridDim.x * (BLOCK / kWave);
-  const int n16 = a.ctl->num_s16, n64 = a.ctl->num_s64;
-  for (int i = gw; i < n64; i += nw) reduce_group<W, kWave>(a, true, a.list_s64[i]);
+  const int n16 = a.ctl->num_s16;
   for (int i = gw * 4; i < n16; i += nw * 4) {
-    const int j = i + lane / 16;
-    reduce_group<W, 16>(a, j < n16, a.list_s16[min(j, n16 - 1)]);
+    const int j = i + lane_id() / 16;
+    reduce_16<W>(a, j < n16, a.list_s16[min(j, n16 - 1)]);
   }
 }
 
-// Reduce for larger |R(u)|: a workgroup per u, 64 x 64 blocks of the lower
-// triangle dealt to the waves; both halves of a block's symmetric
-// contribution are added to LDS sums.
+// Reduce for larger |R(u)|. I = M w for the symmetric 0/1 matrix M whose lower
+// triangle is stored. A wave takes 64 rows P and runs over all 64-column
+// blocks Q: the stored block (P, Q) for Q <= P and the transpose of the stored
+// block (Q, P) for Q >= P. A block is held as 16-bit chunks, chunk h (columns
+// 16h ..) of row 16g + r in lane 16h + r, register g. Bits are transposed
+// inside 16 lanes by four butterfly steps (DPP), two registers packed in one,
+// and register and lane group change places by the gfx950 row swaps: about 35
+// instructions for 4096 bits.
+//   Unweighted: the chunks' bit counts.
+//   Weighted: matrix products of the bits, spread to bytes, with the weights
+// as integers of 7-bit digits (weight = sum digit_n 2^(7n) 2^lsb, eight digits
+// hold the 53 bits that tri_ready admits), int8 MFMA 16x16x64 with int32 sums,
+// which are exact; each row's digit sums are put together in fp64, exactly.
+// Both operands use the same order of k, so the product does not depend on it.
+// (Adding the weights bit by bit in fp64 took 24 instructions per 64 bits:
+// RMAT-22 9.8 ms for all of reduce, 3.9 with the products; Chung-Lu 2^20
+// unweighted 0.61 and 0.36.)
+struct Chunks {
+  uint32_t x[2];  // registers g = 0, 1 and g = 2, 3, 16 bits each
+};
+
+__device__ __forceinline__ Chunks transpose_block(Chunks c) {
+  const int r = lane_id() & 15;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    uint32_t x = c.x[i];
+    auto step = [&](uint32_t t, int s, uint32_t low) {
+      const bool up = (r & s) != 0;
+      const uint32_t own = up ? ~low : low;  // columns this lane keeps
+      const uint32_t rot = __builtin_amdgcn_alignbit(t, t, up ? s : 32 - s);
+      x = (x & own) | (rot & ~own);
+    };
+    step((uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x128, 0xF, 0xF, false), 8, 0x00FF00FFu);  // row_ror:8
+    int t = __builtin_amdgcn_update_dpp(0, (int)x, 0x104, 0xF, 0x5, false);                    // row_shl:4
+    t = __builtin_amdgcn_update_dpp(t, (int)x, 0x114, 0xF, 0xA, false);                        // row_shr:4
+    step((uint32_t)t, 4, 0x0F0F0F0Fu);
+    step((uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x4E, 0xF, 0xF, false), 2, 0x33333333u);
+    step((uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xB1, 0xF, 0xF, false), 1, 0x55555555u);
+    c.x[i] = x;
+  }
+  const auto s32 = __builtin_amdgcn_permlane32_swap(c.x[0], c.x[1], false, false);
+  const uint32_t sel = (lane_id() & 16) ? 0x07060302u : 0x05040100u;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const auto s16 = __builtin_amdgcn_permlane16_swap(s32[i], s32[i], false, false);
+    c.x[i] = __builtin_amdgcn_perm(s16[1], s16[0], sel);
+  }
+  return c;
+}
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+
+// The 16 bits at `sh` of x as 16 bytes of 0 or 1.
+__device__ __forceinline__ v4i spread16(uint32_t x, int sh) {
+  v4i v;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t nib = __builtin_amdgcn_ubfe(x, sh + 4 * j, 4);
+    v[j] = (int)((nib * 0x204081u) & 0x01010101u);
+  }
+  return v;
+}
+
+constexpr int kDigits = 8;      // 7-bit digits of a weight
+constexpr int kRedRow = 64 + 4; // ints per digit of a wave's 64 row sums (padded)
+
+// Digits of the weight of row entry k, to digit arrays in blocks of 16 entries
+// (16 bytes per digit).
+__device__ __forceinline__ void put_digits(unsigned char* dig, int k, float w, int lsb) {
+  const uint32_t b = __float_as_uint(w);
+  const int ex = (int)((b >> 23) & 0xFFu);
+  const uint64_t full = ex ? (b & 0x7FFFFFu) | 0x800000u : b & 0x7FFFFFu;
+  const int sh = (ex ? ex - 150 : -149) - lsb;
+  uint64_t v = full == 0 ? 0ull : sh >= 0 ? full << sh : full >> -sh;  // (trailing zeros shifted out)
+#pragma unroll
+  for (int n = 0; n < kDigits; ++n) {
+    dig[(k >> 4) * (16 * kDigits) + n * 16 + (k & 15)] = (unsigned char)(v & 127u);
+    v >>= 7;
+  }
+}
+
+// Rows [64 P, 64 P + 64) of u's product; returns the lane's row's result
+// (lane = row), without the wedge part.
+template <bool W>
+__device__ __forceinline__ void reduce_rows(const TriArgs& a, uint32_t z, int dp, int P, const unsigned char* dig,
+                                            int* stage, double unit, double& sum, uint32_t& cnt) {
+  const int lane = lane_id(), r = lane & 15, h = lane >> 4;
+  const int nb = (dp + 63) >> 6;
+  const uint16_t* __restrict__ hw = reinterpret_cast<const uint16_t*>(a.bits);
+  v4i acc[4];
+  uint32_t c16[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int g = 0; g < 4; ++g) acc[g] = v4i{0, 0, 0, 0};
+  auto use = [&](const Chunks& c, int Q) {
+    if constexpr (W) {
+      const v4i bq = *reinterpret_cast<const v4i*>(dig + (4 * Q + h) * (16 * kDigits) + (r & 7) * 16);
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        acc[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(spread16(c.x[g >> 1], 16 * (g & 1)), bq, acc[g], 0, 0, 0);
+    } else {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) c16[g] += (uint32_t)__popc(g & 1 ? c.x[g >> 1] >> 16 : c.x[g >> 1] & 0xFFFFu);
+    }
+  };
+  // 16 columns from 16 * (4 C + h) of the rows 64 B + 16 g + r
+  auto load = [&](int B, int C) {
+    uint32_t v[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int p = 64 * B + 16 * g + r, c0 = 64 * C + 16 * h;
+      v[g] = 0u;
+      if (p < dp && c0 < p) v[g] = hw[2 * (size_t)(z + tri_words(p)) + (size_t)(4 * C + h)];
+    }
+    return Chunks{{v[0] | (v[1] << 16), v[2] | (v[3] << 16)}};
+  };
+  for (int Q = 0; Q <= P; ++Q) use(load(P, Q), Q);
+  for (int Q = P; Q < nb; ++Q) use(transpose_block(load(Q, P)), Q);
+  if constexpr (W) {
+    // acc[g][i]: row 16 g + 4 h + i, digit r (r < 8)
+    if (r < kDigits) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) *reinterpret_cast<v4i*>(stage + r * kRedRow + 16 * g + 4 * h) = acc[g];
+    }
+    lds_fence_wave();
+    double t = 0.0;
+#pragma unroll
+    for (int n = kDigits - 1; n >= 0; --n) t = t * 128.0 + (double)stage[n * kRedRow + lane];
+    sum = t * unit;
+    lds_fence_wave();
+  } else {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      c16[g] += __shfl_xor(c16[g], 16);
+      c16[g] += __shfl_xor(c16[g], 32);
+    }
+    cnt = h == 0 ? c16[0] : h == 1 ? c16[1] : h == 2 ? c16[2] : c16[3];
+  }
+}
+
+// All rows of u, by the T threads of a wave or workgroup.
+template <bool W, int T>
+__device__ __forceinline__ void reduce_vertex(const TriArgs& a, int32_t u, int tid, unsigned char* dig, int* stage) {
+  constexpr int NW = T / kWave;
+  const int lane = lane_id(), w = tid / kWave;
+  const int4 inf = a.info[u];
+  const int ru = a.rw[u].x;
+  const int o = inf.x, dp = inf.y;
+  const int nb = (dp + 63) >> 6;
+  double unit = 1.0;
+  if constexpr (W) {
+    const int lsb = a.ctl->lsb == INT32_MAX ? 0 : a.ctl->lsb;
+    unit = ldexp(1.0, lsb);
+    for (int k = tid; k < nb * 64; k += T) put_digits(dig, k, k < dp ? a.wr[a.R32[o + k]] : 0.0f, lsb);
+    if constexpr (T > kWave) __syncthreads();
+    else lds_fence_wave();
+  }
+  const int du = a.dr[ru];
+  const double su = W ? a.sr[ru] : 0.0;
+  for (int P = w; P < nb; P += NW) {
+    double sum = 0.0;
+    uint32_t cnt = 0;
+    reduce_rows<W>(a, (uint32_t)inf.z, dp, P, dig, stage, unit, sum, cnt);
+    const int p = P * 64 + lane;
+    if (p < dp) {
+      const uint32_t rv = a.R32[o + p];
+      if constexpr (W) sum += a.accw[o + p];
+      else cnt += a.accu[o + p];
+      put_value<W>(a, o + p, u, du, su, rv, sum, cnt);
+    }
+  }
+  if constexpr (T > kWave) __syncthreads();
+  else lds_fence_wave();
+}
+
 template <bool W, int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_tri_reduce_big(TriArgs a) {
+__global__ __launch_bounds__(BLOCK) void k_tri_reduce_wave(TriArgs a) {
   constexpr int NW = BLOCK / kWave;
-  using AT = typename std::conditional<W, double, uint32_t>::type;
-  __shared__ AT s_acc[kTriMaxOut];
-  __shared__ float s_wt[W ? kTriMaxOut : 1];
+  __shared__ __align__(16) unsigned char dig[W ? NW : 1][W ? kRedWave * kDigits : 16];
+  __shared__ __align__(16) int stage[W ? NW : 1][W ? kDigits * kRedRow : 4];
+  if (!tri_ready<W>(a)) return;
+  const int w = threadIdx.x / kWave;
+  const int count = a.ctl->num_s64;
+  for (int i = blockIdx.x * NW + w; i < count; i += gridDim.x * NW)
+    reduce_vertex<W, kWave>(a, a.list_s64[i], lane_id(), dig[W ? w : 0], stage[W ? w : 0]);
+}
+
+template <bool W, int BLOCK, int CAP>
+__global__ __launch_bounds__(BLOCK) void k_tri_reduce_wg(TriArgs a) {
+  constexpr int NW = BLOCK / kWave;
+  constexpr int L = CAP > kRedWg ? 1 : 0;
+  __shared__ __align__(16) unsigned char dig[W ? CAP * kDigits : 16];
+  __shared__ __align__(16) int stage[W ? NW : 1][W ? kDigits * kRedRow : 4];
   __shared__ int s_i;
   if (!tri_ready<W>(a)) return;
-  const int tid = threadIdx.x, lane = lane_id(), w = tid / kWave;
-  const int count = a.ctl->num_red;
+  const int count = a.ctl->num_red[L];
   for (;;) {
-    if (tid == 0) s_i = atomicAdd(&a.ctl->cur_red, 1);
+    if (threadIdx.x == 0) s_i = atomicAdd(&a.ctl->cur_red[L], 1);
     __syncthreads();
-    const int li = s_i;
-    if (li >= count) return;
-    const int32_t u = a.list_red[li];
-    const int4 inf = a.info[u];
-    const int ru = a.rw[u].x;
-    const int o = inf.x, dp = inf.y;
-    const int nb = (dp + kWave - 1) / kWave;
-    for (int i = tid; i < nb * kWave; i += BLOCK) {
-      if constexpr (W) {
-        s_acc[i] = i < dp ? a.accw[o + i] : 0.0;
-        s_wt[i] = i < dp ? a.wr[a.R32[o + i]] : 0.0f;
-      } else {
-        s_acc[i] = i < dp ? a.accu[o + i] : 0u;
-      }
-    }
-    __syncthreads();
-    // blocks (P, Q), Q <= P, in row order
-    const int nblk = nb * (nb + 1) / 2;
-    int P = 0, Q = 0, at = 0;
-    for (int blk = w; blk < nblk; blk += NW) {
-      while (at < blk) {
-        if (++Q > P) {
-          ++P;
-          Q = 0;
-        }
-        ++at;
-      }
-      const int p = P * kWave + lane;
-      uint32_t lo = 0, hi = 0;
-      if (p < dp) {
-        const uint32_t rb = (uint32_t)inf.z + tri_words(p);
-        const int nwords = (p + 31) >> 5;
-        if (2 * Q < nwords) lo = a.bits[rb + 2 * Q];
-        if (2 * Q + 1 < nwords) hi = a.bits[rb + 2 * Q + 1];
-      }
-      uint32_t tlo = 0, thi = 0;  // column `lane`: its rows
-      AT racc = 0, cacc = 0;
-#pragma unroll 8
-      for (int c = 0; c < kWave; ++c) {
-        const bool bit = ((c < 32 ? lo : hi) >> (c & 31)) & 1u;
-        const uint64_t col = ballot(bit);
-        if constexpr (W) {
-          const double wq = (double)s_wt[Q * kWave + c];
-          if (bit) racc += wq;
-          tlo = lane == c ? (uint32_t)col : tlo;
-          thi = lane == c ? (uint32_t)(col >> 32) : thi;
-        } else {
-          cacc = lane == c ? (uint32_t)popc64(col) : cacc;
-        }
-      }
-      if constexpr (W) {
-#pragma unroll 8
-        for (int q = 0; q < kWave; ++q) {
-          const bool bit = ((q < 32 ? tlo : thi) >> (q & 31)) & 1u;
-          const double wp = (double)s_wt[P * kWave + q];
-          if (bit) cacc += wp;
-        }
-        if (racc != 0.0) unsafeAtomicAdd(&s_acc[p], racc);
-        if (cacc != 0.0) unsafeAtomicAdd(&s_acc[Q * kWave + lane], cacc);
-      } else {
-        racc = (uint32_t)(__popc(lo) + __popc(hi));
-        if (racc) atomicAdd(&s_acc[p], racc);
-        if (cacc) atomicAdd(&s_acc[Q * kWave + lane], cacc);
-      }
-    }
-    __syncthreads();
-    const int du = a.dr[ru];
-    const double su = W ? a.sr[ru] : 0.0;
-    for (int i = tid; i < dp; i += BLOCK) {
-      const uint32_t rv = a.R32[o + i];
-      if constexpr (W) put_value<W>(a, o + i, u, du, su, rv, s_acc[i], 0u);
-      else put_value<W>(a, o + i, u, du, su, rv, 0.0, s_acc[i]);
-    }
-    __syncthreads();
+    const int i = s_i;
+    if (i >= count) return;
+    reduce_vertex<W, BLOCK>(a, a.list_red[L][i], threadIdx.x, dig, stage[W ? threadIdx.x / kWave : 0]);
   }
 }
 
@@ -1160,7 +1262,8 @@ size_t carve(TriArgs& a, unsigned char* p, int32_t n, int64_t m, bool weighted) 
   a.list_wave = reinterpret_cast<int32_t*>(take(nn * 4));
   a.list_s16 = reinterpret_cast<int32_t*>(take(nn * 4));
   a.list_s64 = a.list_mid;  // orient is done with its lists when plan runs
-  a.list_red = a.list_big;
+  a.list_red[0] = a.list_big;
+  a.list_red[1] = reinterpret_cast<int32_t*>(take((size_t)std::min<int64_t>(nn, m / kRedWg + 1) * 4));
   return o;
 }
 
@@ -1197,8 +1300,10 @@ hipError_t tri_launch(const TriArgs& a, hipStream_t s) {
   }
   {
     ProfScope ps("tri_reduce", s);
-    hipLaunchKernelGGL((k_tri_reduce_big<W, PB>), dim3(cus * (W ? 3 : 8)), dim3(PB), 0, s, a);
-    hipLaunchKernelGGL((k_tri_reduce_small<W, PB>), grid(a.n, 4 * PB / kWave, 32), dim3(PB), 0, s, a);
+    hipLaunchKernelGGL((k_tri_reduce_wg<W, PB, kTriMaxOut>), dim3(cus * (W ? 3 : 8)), dim3(PB), 0, s, a);
+    hipLaunchKernelGGL((k_tri_reduce_wg<W, PB, kRedWg>), dim3(cus * 8), dim3(PB), 0, s, a);
+    hipLaunchKernelGGL((k_tri_reduce_wave<W, PB>), grid(a.n, PB / kWave, 32), dim3(PB), 0, s, a);
+    hipLaunchKernelGGL((k_tri_reduce_16<W, PB>), grid(a.n, 4 * PB / kWave, 32), dim3(PB), 0, s, a);
   }
   {
     ProfScope ps("tri_deliver", s);
