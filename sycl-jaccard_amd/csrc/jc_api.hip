@@ -82,6 +82,7 @@ constexpr int32_t kTriMinEdges = 1 << 22;
 
 bool tri_wanted(const jc_csr* g, const jc_tuning* t) {
   if (t && (t->engine == JC_ENGINE_OWNER || t->wide_index || t->hash_table == 1 || t->quot_max_disp > 0)) return false;
+  if (g->n > jc::kTriMaxN) return false;
   return (t && t->engine == JC_ENGINE_ORIENTED) || (!t && g->m >= kTriMinEdges);
 }
 

@@ -106,6 +106,7 @@ struct EngineArgs {
 // decides; *done then receives the address (in ws) of a flag that is set when
 // the results were written, for EngineArgs::skip of the owner engine that
 // must follow. ws holds tri_workspace_bytes(n, m, weighted) bytes.
+constexpr int32_t kTriMaxN = 1 << 26;  // its hash keys hold 26-bit ranks
 size_t tri_workspace_bytes(int32_t n, int64_t m, bool weighted);
 hipError_t run_tri(int mode, const EngineArgs& base, void* ws, const int** done, hipStream_t s);
 

@@ -37,11 +37,12 @@
 // oriented engine has delivered, the owner engine's kernels return at once.
 //
 // Measured against the owner engine (whole calls): RMAT-22 weighted 58.2 ->
-// 20.6 ms, RMAT of 200003 vertices weighted vertex-centric 1.58 -> 0.96 ms,
-// Chung-Lu 2^20 4.00 -> 3.38 ms.
+// 18.0 ms, RMAT of 200003 vertices weighted vertex-centric 1.58 -> 0.91 ms,
+// Chung-Lu 2^20 4.00 -> 3.09 ms.
 #include <type_traits>
 
 #include "jc_device.hpp"
+#include "jc_hash.hpp"
 #include "jc_internal.hpp"
 #include "jc_profile.hpp"
 
@@ -53,13 +54,16 @@ constexpr int kTriBuckets = 1024;
 constexpr int kTriMaxOut = 4096;   // largest |R(u)|: the sort and reduce buffers in LDS
 constexpr int kTriRowWave = 1024;  // rows up to this many entries are oriented by one wave
 constexpr int kSat16 = 65535;      // 16-bit ranks saturate here
+constexpr int kPivotMin = 16;      // rows up to this are searched whole
 constexpr int kWgMinDeg = 192;     // rows of at least this many entries get a workgroup in wedge
 constexpr int kWedgeB = 512;       // threads of a wedge workgroup, entries of a wedge task
+constexpr int kGroupMax = 512;     // shorter rows are taken several to a workgroup
+constexpr int kGroupRows = 64;     // at most that many
 constexpr int kTabA = 2048;        // bitmap words of the 16-bit wedge kernel (65536 ranks)
-constexpr int kAccA = 1536;        // largest |R(v)| of the 16-bit wedge kernel
+constexpr int kAccA = 1408;        // largest |R(v)| of the 16-bit wedge kernel
 constexpr int kTabB = 8192;        // the same for the 32-bit wedge kernel (262144 ranks)
 constexpr int kAccB = kTriMaxOut;
-constexpr int kWaveTab = 256;      // |R(v)| held in LDS by the one-wave wedge kernel
+constexpr int kWaveTab = 256;      // largest |R(v)| hashed in LDS by the one-wave wedge kernel
 constexpr int kRedWave = 256;      // |R(u)| that reduce takes by one wave
 constexpr int kRedWg = 1280;       // by a workgroup with that many weights in LDS; above, kTriMaxOut
 
@@ -76,9 +80,24 @@ __device__ __forceinline__ uint32_t tri_words(int L) {
   return (k + 1u) * (t - 16u * k);
 }
 
-struct TriTask {
-  int32_t r;      // rank of v
-  int32_t piece;  // entries [piece * kWedgeB, ...) of v's row
+// Row u of the 16-bit ranks, in units of 16 bytes: a header of two units, then
+// the entries, eight to a unit, and at least eight more, which hold kSat16 (no
+// bitmap has that bit), so a group of eight may be read past the end. The
+// header is what wedge needs of u: row offset, |R(u)|, first word of its bit
+// matrix, weight bits; then the ranks at |R| k / 8, k = 1 .. 7, for the search.
+// An entry that leads to u carries the header's place (emap). Rows start on
+// 128-byte lines, the unit of what the cache fetches: wedge is bound by the
+// lines it touches (RMAT-22: 34.5 GB at 5.5 TB/s with rows on 16 bytes).
+__host__ __device__ __forceinline__ uint64_t row16_line(uint64_t o, uint64_t u) { return ((o + 24 * u) >> 6) + u; }
+__device__ __forceinline__ uint32_t row16(int o, int32_t u) { return 8u * (uint32_t)row16_line((uint64_t)o, (uint64_t)u); }
+constexpr int kHead = 2;
+
+// A task of the bitmap wedge kernels.
+struct __attribute__((aligned(32))) TriTask {
+  int32_t r, o, d, dp;  // v: rank, row offset, row entries, |R(v)|
+  int32_t piece;        // entries [piece * kWedgeB, ...) of v's row
+  int32_t row;          // row16 of v
+  int32_t pad[2];
 };
 
 }  // namespace
@@ -95,6 +114,9 @@ struct TriCtl {
   int num_wave, num_s16, num_s64;
   int num_red[2], cur_red[2];    // reduce by workgroup: up to kRedWg entries, more
   int cur_big;
+  int num_group, cur_group;      // group tasks of wedge: rows of fewer than kGroupMax entries
+  int grp_task[kGroupMax];       // first task of the rows of each length
+  int grp_rank[kGroupMax];       // first rank among them that is taken in groups
   int hist[kTriBuckets];
   int cur[kTriBuckets];
 };
@@ -108,15 +130,16 @@ struct TriArgs {
   const int32_t* ind;
   const float* vw;
   TriCtl* ctl;
-  int2* rw;         // per vertex: rank, weight bits
+  int4* rw;         // per vertex: rank, weight bits, place of its 16-bit row
   int32_t* vtx;     // per rank: vertex
   float* wr;        // per rank: weight
   double* sr;       // per rank: row sum of the weights (unweighted: unused)
   int32_t* dr;      // per rank: degree
-  int4* info;       // per vertex: row offset, |R|, first word of its bit matrix, weight bits
+  int4* info;       // per vertex: row offset, |R|, first word of its bit matrix
+  int2* rinfo;      // per rank: row offset, |R|
   uint32_t* R32;    // R(u) at [off[u], off[u] + |R(u)|), later the pairs' values
-  uint16_t* R16;
-  int32_t* emap;
+  uint16_t* R16;    // the same, saturated, at row16 with headers
+  int32_t* emap;    // per stored entry (u, x): its slot, or until wedge ~row16 of x if x ranks after u
   double* accw;     // per slot: sums of wedge (weighted)
   uint32_t* accu;   // (unweighted)
   uint32_t* bits;
@@ -190,6 +213,9 @@ __global__ __launch_bounds__(BLOCK) void k_tri_hist(TriArgs a) {
     if (h[i]) atomicAdd(&a.ctl->hist[i], h[i]);
 }
 
+// Vertices of degree d in a group task of wedge.
+__device__ __forceinline__ int group_rows(int d) { return min(kGroupRows, kWedgeB / d); }
+
 // First rank of every bucket, largest degrees first.
 __global__ __launch_bounds__(kTriBuckets) void k_tri_scan(TriCtl* c) {
   __shared__ int part[kTriBuckets / kWave];
@@ -206,6 +232,29 @@ __global__ __launch_bounds__(kTriBuckets) void k_tri_scan(TriCtl* c) {
   int base = 0;
   for (int i = 0; i < (int)threadIdx.x / kWave; ++i) base += part[i];
   c->cur[b] = base + incl - v;
+  // Group tasks of wedge. Buckets below kGroupMax hold one degree each, so a
+  // group is group_rows(b) vertices of consecutive ranks and equal degree;
+  // long rows of low rank go to the bitmap kernel instead.
+  int ng = 0;
+  if (b > 0 && b < kGroupMax) {
+    const int first = b >= kWgMinDeg ? max(base + incl - v, kSat16) : base + incl - v;
+    const int cnt = max(0, base + incl - first);
+    c->grp_rank[b] = first;
+    ng = (cnt + group_rows(b) - 1) / group_rows(b);
+  }
+  int gi = ng;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int t = __shfl_up(gi, o);
+    if (lane_id() >= o) gi += t;
+  }
+  __syncthreads();
+  if (lane_id() == kWave - 1) part[threadIdx.x / kWave] = gi;
+  __syncthreads();
+  int gbase = 0;
+  for (int i = 0; i < (int)threadIdx.x / kWave; ++i) gbase += part[i];
+  if (b < kGroupMax) c->grp_task[b] = gbase + gi - ng;
+  if (b == 0) c->num_group = gbase + gi;
 }
 
 // Ranks: each workgroup counts its range per bucket, reserves the places with
@@ -243,13 +292,13 @@ __global__ __launch_bounds__(BLOCK) void k_tri_rank(TriArgs a) {
     const int b = deg_bucket(d);
     const int r = base[b] + atomicAdd(&h[b], 1);
     const float w = W ? a.vw[u] : 0.0f;
-    a.rw[u] = make_int2(r, __float_as_int(w));
+    a.rw[u] = make_int4(r, __float_as_int(w), (int)row16(o, u), 0);
     a.vtx[r] = u;
     a.dr[r] = d;
     if constexpr (W) a.wr[r] = w;
     if (d > kTriRowWave) a.list_big[s_base[1] + atomicAdd(&s_cnt[1], 1)] = u;
     else if (d > kWave) a.list_mid[s_base[0] + atomicAdd(&s_cnt[0], 1)] = u;
-    else if (d == 0) a.info[u] = make_int4(o, 0, 0, __float_as_int(w));
+    else if (d == 0) a.info[u] = make_int4(o, 0, 0, 0);
   }
 }
 
@@ -267,15 +316,31 @@ __device__ __forceinline__ void put_row_sum(const TriArgs& a, int32_t ru, double
   }
 }
 
-// Writes entry (rank r, row entry k) of row o at sorted position p.
+// Writes entry (rank r, row entry k) of row u at sorted position p.
 template <bool W>
-__device__ __forceinline__ void put_out(const TriArgs& a, int o, int p, uint32_t r, int k) {
+__device__ __forceinline__ void put_out(const TriArgs& a, int32_t u, int o, int p, uint32_t r, int k) {
   const int e = o + p;
   a.R32[e] = r;
-  a.R16[e] = (uint16_t)min(r, (uint32_t)kSat16);
+  a.R16[8 * ((size_t)row16(o, u) + kHead) + p] = (uint16_t)min(r, (uint32_t)kSat16);
   a.emap[k] = e;
   if constexpr (W) a.accw[e] = 0.0;
   else a.accu[e] = 0u;
+}
+
+// Position p of n: where it is an eighth of the row, its rank goes to the
+// header (rows of more than kPivotMin entries have these).
+__device__ __forceinline__ void put_pivot(const TriArgs& a, int32_t u, int o, int n, int p, uint32_t r) {
+  if (n <= kPivotMin) return;
+  uint16_t* pv = a.R16 + 8 * ((size_t)row16(o, u) + 1);
+#pragma unroll
+  for (int k = 1; k <= 7; ++k)
+    if (((n * k) >> 3) == p) pv[k - 1] = (uint16_t)min(r, (uint32_t)kSat16);
+}
+
+// Row u's facts (one lane).
+__device__ __forceinline__ void put_info(const TriArgs& a, int32_t u, int o, int cnt, int wbits) {
+  a.info[u] = make_int4(o, cnt, 0, 0);
+  reinterpret_cast<int4*>(a.R16)[row16(o, u)] = make_int4(o, cnt, 0, wbits);
 }
 
 // Rows of at most 64 entries: groups of G lanes, one row each (16 lanes for
@@ -285,7 +350,7 @@ template <bool W, int G>
 __device__ __forceinline__ void orient_group(const TriArgs& a, bool valid, int32_t u, int o, int d, int ru, float w) {
   const int gl = lane_id() & (G - 1), gb = lane_id() & ~(G - 1);
   bool in_row = valid && gl < d;
-  int2 rw = make_int2(0, 0);
+  int4 rw = make_int4(0, 0, 0, 0);
   int32_t x = 0;
   if (in_row) {
     x = a.ind[o + gl];
@@ -302,8 +367,8 @@ __device__ __forceinline__ void orient_group(const TriArgs& a, bool valid, int32
     const int rj = G == kWave ? __builtin_amdgcn_readlane(mine, j) : __shfl(mine, gb + j);
     pos += rj < mine ? 1 : 0;
   }
-  if (keep) put_out<W>(a, o, pos, (uint32_t)rw.x, o + gl);
-  else if (in_row) a.emap[o + gl] = -1;
+  if (keep) put_out<W>(a, u, o, pos, (uint32_t)rw.x, o + gl);
+  else if (in_row) a.emap[o + gl] = ~rw.z;
   const uint64_t gm = G == kWave ? ~0ull : ((1ull << G) - 1) << gb;
   const int cnt = popc64(km & gm);
   if constexpr (W) {
@@ -312,7 +377,9 @@ __device__ __forceinline__ void orient_group(const TriArgs& a, bool valid, int32
     for (int t = 1; t < G; t <<= 1) s += __shfl_xor(s, t);
     if (valid && gl == 0) put_row_sum<W>(a, ru, s);
   }
-  if (valid && gl == 0) a.info[u] = make_int4(o, cnt, 0, __float_as_int(w));
+  if (valid && gl == 0) put_info(a, u, o, cnt, __float_as_int(w));
+  if (keep) put_pivot(a, u, o, cnt, pos, (uint32_t)rw.x);
+  if (valid && gl < 8) a.R16[8 * ((size_t)row16(o, u) + kHead) + cnt + gl] = (uint16_t)kSat16;
 }
 
 template <bool W, int BLOCK>
@@ -328,7 +395,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_orient_small(TriArgs a) {
     if (base + lane < a.n) {
       o = a.off[u];
       d = a.off[u + 1] - o;
-      const int2 rw = a.rw[u];
+      const int4 rw = a.rw[u];
       ru = rw.x;
       w = __int_as_float(rw.y);
     }
@@ -364,7 +431,7 @@ template <bool W, int T, int CAP>
 __device__ __forceinline__ void orient_row(const TriArgs& a, int32_t u, int tid, uint32_t* s_r, uint16_t* s_k, int* s_n,
                                            double* s_s) {
   const int o = a.off[u], d = a.off[u + 1] - o;
-  const int2 me = a.rw[u];
+  const int4 me = a.rw[u];
   const int ru = me.x;
   const int lane = lane_id();
   if (tid == 0) {
@@ -377,7 +444,7 @@ __device__ __forceinline__ void orient_row(const TriArgs& a, int32_t u, int tid,
   int cnt = 0;  // T == 64: kept so far
   for (int b = 0; b < d; b += 4 * T) {
     int32_t x[4];
-    int2 rw[4];
+    int4 rw[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) x[t] = a.ind[o + min(b + t * T + tid, d - 1)];
 #pragma unroll
@@ -404,7 +471,7 @@ __device__ __forceinline__ void orient_row(const TriArgs& a, int32_t u, int tid,
           else reinterpret_cast<int32_t*>(s_k)[at] = i;
         }
       } else if (in_row) {
-        a.emap[o + i] = -1;
+        a.emap[o + i] = ~rw[t].z;
       }
       if constexpr (W) sum += in_row ? (double)__int_as_float(rw[t].y) : 0.0;
     }
@@ -425,10 +492,11 @@ __device__ __forceinline__ void orient_row(const TriArgs& a, int32_t u, int tid,
   }
   if (tid == 0) {
     put_row_sum<W>(a, ru, sum);
-    a.info[u] = make_int4(o, cnt, 0, me.y);
+    put_info(a, u, o, cnt, me.y);
     if (cnt > CAP) a.ctl->bad = 1;
   }
   const int c = min(cnt, CAP);
+  if (tid < 8) a.R16[8 * ((size_t)row16(o, u) + kHead) + c + tid] = (uint16_t)kSat16;
   // pad to a multiple of four with a rank that counts for nobody
   for (int i = c + tid; i < ((c + 3) & ~3); i += T) s_r[i] = 0xFFFFFFFFu;
   if constexpr (T > kWave) __syncthreads();
@@ -444,8 +512,14 @@ __device__ __forceinline__ void orient_row(const TriArgs& a, int32_t u, int tid,
     }
     const int ka = ia < c ? (T == kWave ? (int)s_k[ia] : reinterpret_cast<int32_t*>(s_k)[ia]) : 0;
     const int kb = ib < c ? (T == kWave ? (int)s_k[ib] : reinterpret_cast<int32_t*>(s_k)[ib]) : 0;
-    if (ia < c) put_out<W>(a, o, pa, ra, o + ka);
-    if (ib < c) put_out<W>(a, o, pb, rb, o + kb);
+    if (ia < c) {
+      put_out<W>(a, u, o, pa, ra, o + ka);
+      put_pivot(a, u, o, c, pa, ra);
+    }
+    if (ib < c) {
+      put_out<W>(a, u, o, pb, rb, o + kb);
+      put_pivot(a, u, o, c, pb, rb);
+    }
   }
   if constexpr (T > kWave) __syncthreads();
   else lds_fence_wave();
@@ -496,20 +570,29 @@ __global__ __launch_bounds__(BLOCK) void k_tri_plan(TriArgs a) {
   const int lane = lane_id(), wv = threadIdx.x / kWave;
   for (int64_t b0 = (int64_t)blockIdx.x * BLOCK; b0 < a.n; b0 += (int64_t)gridDim.x * BLOCK) {
     const int32_t r = (int32_t)(b0 + threadIdx.x);
-    int d = 0, dp = 0;
+    int d = 0, dp = 0, o = 0;
     int32_t u = 0;
     if (r < a.n) {
-      u = a.vtx[r];
       d = a.dr[r];
-      dp = a.info[u].y;
+      if (d > 0) {
+        u = a.vtx[r];
+        const int4 inf = a.info[u];
+        o = inf.x;
+        dp = inf.y;
+        a.rinfo[r] = make_int2(o, dp);
+      }
     }
     const int din = d - dp;
     int c[NL] = {0, 0, 0, 0, 0, 0, 0};
-    const bool wg = din > 0 && d >= kWgMinDeg && dp <= kAccB && r <= 32 * kTabB;
+    // v by a workgroup where its row is worth a bitmap: 16-bit ranks, or a
+    // larger table for what the one-wave kernel's hash does not hold; short
+    // rows are in the group tasks (k_tri_scan has the same rule)
     const int npiece = (d + kWedgeB - 1) / kWedgeB;
     const int kind = r < kSat16 && dp <= kAccA ? 0 : 1;
+    const bool grp = d < kGroupMax && (d < kWgMinDeg || r >= kSat16);
+    const bool wg = din > 0 && !grp && (kind == 0 || (dp > kWaveTab && dp <= kAccB && r <= 32 * kTabB));
     if (wg) c[kind] = npiece;
-    else if (din > 0) c[2] = 1;
+    else if (din > 0 && !grp) c[2] = 1;
     if (dp > 0) c[dp <= 16 ? 3 : dp <= kRedWave ? 4 : dp <= kRedWg ? 5 : 6] = 1;
     const unsigned long long words = tri_words(dp);
     int incl[NL];
@@ -563,13 +646,17 @@ __global__ __launch_bounds__(BLOCK) void k_tri_plan(TriArgs a) {
     for (int l = 0; l < NL; ++l) at[l] = s_base[l] + s_w[l][wv] + incl[l] - c[l];
     if (wg)
       for (int p = 0; p < npiece; ++p)
-        if (at[kind] + p < a.task_cap) a.task[kind][at[kind] + p] = TriTask{r, p};
+        if (at[kind] + p < a.task_cap) a.task[kind][at[kind] + p] = TriTask{r, o, d, dp, p, (int32_t)row16(o, u), {0, 0}};
     if (c[2]) a.list_wave[at[2]] = r;
     if (c[3]) a.list_s16[at[3]] = u;
     if (c[4]) a.list_s64[at[4]] = u;
     if (c[5]) a.list_red[0][at[5]] = u;
     if (c[6]) a.list_red[1][at[6]] = u;
-    if (dp > 0) a.info[u].z = (int)(uint32_t)(s_bbase + s_bw[wv] + bi - words);
+    if (dp > 0) {
+      const int z = (int)(uint32_t)(s_bbase + s_bw[wv] + bi - words);
+      a.info[u].z = z;
+      reinterpret_cast<int4*>(a.R16)[row16(o, u)].z = z;
+    }
     __syncthreads();
   }
 }
@@ -590,37 +677,47 @@ __device__ __forceinline__ int find_rank(const RT* __restrict__ R, int n, uint32
   return lo < n && (uint32_t)R[lo] == r ? lo : -1;
 }
 
-// Eight consecutive entries of a row (any alignment).
-struct __attribute__((packed, aligned(2))) Raw16 {
-  uint32_t v[4];
-};
-struct __attribute__((packed, aligned(4))) Raw32 {
-  uint32_t v[4];
-};
+// The same in 16-bit ranks (r < kSat16), the eighth of the row taken from the
+// pivots in its header: the search then stays in about one cache line.
+__device__ __forceinline__ int find_rank16(const uint16_t* __restrict__ R, int n, uint32_t r, const int4& pv) {
+  if (n <= kPivotMin) return find_rank(R, n, r);
+  const uint32_t w[4] = {(uint32_t)pv.x, (uint32_t)pv.y, (uint32_t)pv.z, (uint32_t)pv.w};
+  int c = 0;
+#pragma unroll
+  for (int k = 0; k < 7; ++k) c += ((k & 1) ? w[k >> 1] >> 16 : w[k >> 1] & 0xFFFFu) <= r ? 1 : 0;
+  const int lo = (n * c) >> 3, hi = (n * (c + 1)) >> 3;
+  const int p = find_rank(R + lo, hi - lo, r);
+  return p < 0 ? -1 : lo + p;
+}
+
+// Eight consecutive entries of a row.
 template <typename RT>
 struct Octet;
 template <>
 struct Octet<uint16_t> {
   uint32_t v[4];
-  __device__ __forceinline__ void load(const uint16_t* p) {
-    const Raw16 x = *reinterpret_cast<const Raw16*>(p);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = x.v[i];
+  __device__ __forceinline__ void load(const uint16_t* p) {  // 16-byte aligned
+    const uint4 x = *reinterpret_cast<const uint4*>(p);
+    v[0] = x.x;
+    v[1] = x.y;
+    v[2] = x.z;
+    v[3] = x.w;
   }
-  __device__ __forceinline__ uint32_t get(int t) const { return (t & 1) ? v[t >> 1] >> 16 : v[t >> 1] & 0xFFFFu; }
 };
 template <>
 struct Octet<uint32_t> {
   uint32_t v[8];
-  __device__ __forceinline__ void load(const uint32_t* p) {
-    const Raw32 x = *reinterpret_cast<const Raw32*>(p), y = *reinterpret_cast<const Raw32*>(p + 4);
+  struct __attribute__((packed, aligned(4))) Raw {
+    uint32_t v[4];
+  };
+  __device__ __forceinline__ void load(const uint32_t* p) {  // any alignment
+    const Raw x = *reinterpret_cast<const Raw*>(p), y = *reinterpret_cast<const Raw*>(p + 4);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       v[i] = x.v[i];
       v[4 + i] = y.v[i];
     }
   }
-  __device__ __forceinline__ uint32_t get(int t) const { return v[t]; }
 };
 
 template <int CTRL>
@@ -628,166 +725,186 @@ __device__ __forceinline__ uint32_t or_dpp(uint32_t v) {
   return v | (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, false);
 }
 
-// Tests the nv (<= 8, possibly <= 0) first entries of an octet against the
-// bitmap; hits add to the LDS sums and are returned as a byte.
-template <bool W, typename RT>
-__device__ __forceinline__ uint32_t probe_octet(const Octet<RT>& y, int nv, const uint2* tab, uint32_t guard,
-                                                typename std::conditional<W, double, uint32_t>::type* acc, double w) {
-  uint2 t[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    uint32_t wi = y.get(i) >> 5;
-    if constexpr (sizeof(RT) == 4) wi = min(wi, guard);  // entries past nv may be anything
-    t[i] = tab[wi];
-  }
-  const uint32_t live = nv >= 8 ? 0xFFu : nv <= 0 ? 0u : (1u << nv) - 1u;
+// Tests an octet against the bitmap; hits add w to the LDS sums and come back
+// as a byte. A table word is 8 bytes: 32 bits and the byte offset of the sum
+// before the one of its lowest bit. Shifting the word left so that the
+// entry's own bit is the sign gives the test, and the count of the bits that
+// stay is the entry's place: about 8 instructions per entry. 16-bit entries
+// past the row's part are ranks of v and above, whose bits are 0; 32-bit ones
+// (only nv are valid) read the guard word.
+template <typename RT, typename AT>
+__device__ __forceinline__ uint32_t probe_octet(const Octet<RT>& y, int nv, const unsigned char* tab, uint32_t guard,
+                                                unsigned char* acc, AT w) {
   uint32_t byte = 0;
+  // four entries at a time: eight would take the kernel's registers past eight
+  // waves per SIMD
 #pragma unroll
-  for (int i = 0; i < 8; ++i) byte |= __builtin_amdgcn_ubfe(t[i].x, y.get(i), 1u) << i;
-  byte &= live;
+  for (int h = 1; h >= 0; --h) {
+    uint2 t[4];
+    uint32_t sh[4];
+    if constexpr (sizeof(RT) == 2) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    if (byte & (1u << i)) {
-      const uint32_t slot = __popc(__builtin_amdgcn_ubfe(t[i].x, 0u, y.get(i))) + t[i].y;
-      if constexpr (W) unsafeAtomicAdd(&acc[slot], w);
-      else atomicAdd(&acc[slot], 1u);
+      for (int i = 0; i < 2; ++i) {
+        const uint32_t d = y.v[2 * h + i];
+        t[2 * i] = *reinterpret_cast<const uint2*>(tab + ((d >> 2) & 0x3FF8u));
+        t[2 * i + 1] = *reinterpret_cast<const uint2*>(tab + ((d >> 18) & 0x3FF8u));
+        sh[2 * i] = ~d;
+        sh[2 * i + 1] = ~d >> 16;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t wi = 4 * h + i < nv ? min(y.v[4 * h + i] >> 5, guard) : guard;
+        t[i] = *reinterpret_cast<const uint2*>(tab + 8u * wi);
+        sh[i] = ~y.v[4 * h + i];
+      }
+    }
+#pragma unroll
+    for (int i = 3; i >= 0; --i) {
+      t[i].x <<= sh[i] & 31u;
+      byte = __builtin_amdgcn_alignbit(byte, t[i].x, 31);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if ((int32_t)t[i].x < 0) {
+        AT* s = reinterpret_cast<AT*>(acc + ((uint32_t)__popc(t[i].x) * (uint32_t)sizeof(AT) + t[i].y));
+        if constexpr (sizeof(AT) == 8) unsafeAtomicAdd(s, w);
+        else atomicAdd(s, w);
+      }
     }
   }
   return byte;
 }
 
-constexpr int kWClasses = 8;  // entries to test: <= 8 << c for c < 7, more
+constexpr int kMapCap = 2048;  // words of a task looked at together
 
-// Wedge, one workgroup per task (v, 512 entries of its row).
+// Wedge, one workgroup per task (v, 512 entries of its row). The entries to
+// test, rows of p ranks, are cut into words of 32; a map from word to (row,
+// word of the row) deals the words to groups of four lanes, eight ranks each,
+// so rows of all lengths fill the lanes (dealing rows to 8-lane and larger
+// groups by length left half of them idle: RMAT-22 7.9 ms, this 6.1). What is
+// left is spread over the lines touched (30 GB at 5 TB/s), the LDS (half of
+// the time busy) and the chain of a task's steps.
 template <bool W, typename RT, int TAB, int ACC>
 __global__ __launch_bounds__(kWedgeB, (TAB <= kTabA ? 8 : 2)) void k_tri_wedge(TriArgs a) {
   constexpr int NW = kWedgeB / kWave;
   constexpr int KIND = sizeof(RT) == 2 ? 0 : 1;
   using AT = typename std::conditional<W, double, uint32_t>::type;
-  __shared__ __align__(16) uint2 tab[TAB + 1];  // word of the bitmap, |R(v)| below it (set where the word is not 0)
-  __shared__ AT acc[ACC];
-  __shared__ int s_start[kWedgeB];
-  __shared__ uint16_t s_p[kWedgeB];
-  __shared__ uint32_t s_row[kWedgeB];
-  __shared__ float s_wt[W ? kWedgeB : 1];
-  __shared__ int s_wcnt[kWClasses][NW];
-  __shared__ int s_cbase[kWClasses + 1], s_ubase[kWClasses + 1];
-  __shared__ int s_task, s_next;
+  __shared__ __align__(16) uint2 tab[TAB + (KIND == 0 ? 0 : 2)];
+  __shared__ __align__(16) AT acc[ACC];
+  __shared__ int4 s_item[kWedgeB];  // row (units of 8 entries, or entries), word of the bit matrix, weight, p
+  __shared__ uint16_t s_map[kMapCap];  // item | word << 9
+  __shared__ int s_wsum[NW];
+  __shared__ int s_task;
   if (!tri_ready<W>(a)) return;
   const int tid = threadIdx.x, lane = lane_id(), w = tid / kWave;
   const int ntask = a.ctl->num_task[KIND];
-  const RT* __restrict__ R = KIND == 0 ? (const RT*)a.R16 : (const RT*)a.R32;
+  const unsigned char* const tabp = reinterpret_cast<const unsigned char*>(tab);
+  unsigned char* const accp = reinterpret_cast<unsigned char*>(acc);
+  // first entry of a row, from its place in s_item
+  auto row_at = [&](uint32_t q) -> const RT* {
+    if constexpr (KIND == 0) return a.R16 + 8 * (size_t)q;
+    else return a.R32 + q;
+  };
+  // The next task's record and this thread's entry of it are loaded while a
+  // task runs, and the task after that is reserved, so a task starts with the
+  // headers of its entries.
+  auto entry_of = [&](const TriTask& t, bool any) -> int {
+    const int i = t.piece * kWedgeB + tid;
+    return any && i < t.d ? a.emap[t.o + i] : 0;
+  };
+  if (tid == 0) {
+    s_task = atomicAdd(&a.ctl->cur_task[KIND], 2);
+  }
+  __syncthreads();
+  int ti = s_task, ti1 = ti + 1;
+  if (ti >= ntask) return;
+  TriTask tk = a.task[KIND][ti];
+  int e = entry_of(tk, true);
   for (;;) {
-    if (tid == 0) s_task = atomicAdd(&a.ctl->cur_task[KIND], 1);
-    __syncthreads();
-    const int ti = s_task;
-    if (ti >= ntask) return;
-    const TriTask tk = a.task[KIND][ti];
-    const int32_t r = tk.r, v = a.vtx[r];
-    const int4 vi = a.info[v];
-    const int d = a.dr[r];
-    const int ov = vi.x, dpv = vi.y;
+    const bool more = ti1 < ntask;
+    const TriTask tk1 = a.task[KIND][more ? ti1 : ti];
+    int ti2 = 0;
+    if (tid == 0) ti2 = atomicAdd(&a.ctl->cur_task[KIND], 1);
+    const int32_t r = tk.r;
+    const int d = tk.d, ov = tk.o, dpv = tk.dp;
     const uint32_t guard = KIND == 0 ? 0u : (uint32_t)(r + 31) >> 5;
-    for (int i = tid; i <= (r + 31) >> 5; i += kWedgeB) tab[i] = make_uint2(0u, 0u);
-    if (tid == 0) s_next = 0;
+    // 16-bit: the whole table, so that ranks of r and above find 0
+    const int nclear = KIND == 0 ? TAB / 2 : (int)guard / 2 + 1;
+    for (int i = tid; i < nclear; i += kWedgeB) reinterpret_cast<uint4*>(tab)[i] = make_uint4(0u, 0u, 0u, 0u);
+    const RT* const Rv = row_at(KIND == 0 ? (uint32_t)(tk.row + kHead) : (uint32_t)ov);
+    uint32_t y0 = 0, y0p = 0;
+    if (tid < dpv) {
+      y0 = (uint32_t)Rv[tid];
+      y0p = tid > 0 ? (uint32_t)Rv[tid - 1] : 0u;
+    }
     // the entries of v's row that are not in R(v): where v stands in R(x)
-    int cls = -1, start = 0, p = 0;
-    uint32_t row = 0;
-    float wt = 0.0f;
-    const int i = tk.piece * kWedgeB + tid;
-    if (i < d) {
-      const int k = ov + i;
-      if (a.emap[k] < 0) {
-        const int4 xi = a.info[a.ind[k]];
-        start = xi.x;
-        wt = __int_as_float(xi.w);
-        p = find_rank(R + start, xi.y, (uint32_t)r);
+    int p = 0;
+    {
+      const int k = ov + tk.piece * kWedgeB + tid;
+      if (e < 0) {
+        const int4* const hd = reinterpret_cast<const int4*>(a.R16) + ~e;
+        const int4 xi = hd[0];
+        const uint32_t q = KIND == 0 ? (uint32_t)(~e + kHead) : (uint32_t)xi.x;
+        if constexpr (KIND == 0) p = find_rank16(row_at(q), xi.y, (uint32_t)r, hd[1]);
+        else p = find_rank(row_at(q), xi.y, (uint32_t)r);
         if (p < 0) {
           a.ctl->bad = 1;  // (v, x) is stored, (x, v) is not
+          p = 0;
         } else {
-          a.emap[k] = start + p;
-          row = (uint32_t)xi.z + tri_words(p);
-          if (p > 0) cls = p <= 8 ? 0 : p > 512 ? 7 : 29 - __clz(p - 1);
+          a.emap[k] = xi.x + p;
+          s_item[tid] = make_int4((int)q, (int)((uint32_t)xi.z + tri_words(p)), xi.w, p);
         }
       }
     }
-    int rank = 0;
+    const int nw = (p + 31) >> 5;
+    int incl = nw;
 #pragma unroll
-    for (int c = 0; c < kWClasses; ++c) {
-      const uint64_t bm = ballot(cls == c);
-      if (cls == c) rank = popc64(bm & ((1ull << lane) - 1));
-      if (lane == 0) s_wcnt[c][w] = popc64(bm);
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int t = __shfl_up(incl, o);
+      if (lane >= o) incl += t;
     }
+    if (lane == kWave - 1) s_wsum[w] = incl;
     __syncthreads();
     for (int j = tid; j < dpv; j += kWedgeB) {
-      const uint32_t y = (uint32_t)R[ov + j];
-      const uint32_t yp = j > 0 ? (uint32_t)R[ov + j - 1] : 0u;
+      const uint32_t y = j < kWedgeB ? y0 : (uint32_t)Rv[j];
+      const uint32_t yp = j < kWedgeB ? y0p : (uint32_t)Rv[j - 1];
       acc[j] = 0;
       atomicOr(&tab[y >> 5].x, 1u << (y & 31u));
-      if (j == 0 || (yp >> 5) != (y >> 5)) tab[y >> 5].y = (uint32_t)j;
+      if (j == 0 || (yp >> 5) != (y >> 5)) tab[y >> 5].y = (uint32_t)((j - 1) * (int)sizeof(AT));
     }
-    if (tid == 0) {
-      int ib = 0, ub = 0;
-      for (int c = kWClasses - 1; c >= 0; --c) {
-        int n = 0;
-        for (int k = 0; k < NW; ++k) {
-          const int x = s_wcnt[c][k];
-          s_wcnt[c][k] = n;
-          n += x;
-        }
-        s_cbase[kWClasses - 1 - c] = ib;
-        s_ubase[kWClasses - 1 - c] = ub;
-        ib += n;
-        const int per = kWave >> min(c, 6);
-        ub += (n + per - 1) / per;
-      }
-      s_cbase[kWClasses] = ib;
-      s_ubase[kWClasses] = ub;
+    int wbase = incl - nw, total = 0;
+#pragma unroll
+    for (int k = 0; k < NW; ++k) {
+      const int x = s_wsum[k];
+      wbase += k < w ? x : 0;
+      total += x;
     }
-    __syncthreads();
-    if (cls >= 0) {
-      const int at = s_cbase[kWClasses - 1 - cls] + s_wcnt[cls][w] + rank;
-      s_start[at] = start;
-      s_p[at] = (uint16_t)p;
-      s_row[at] = row;
-      if constexpr (W) s_wt[at] = wt;
-    }
-    __syncthreads();
-    const int nunits = s_ubase[kWClasses];
-    for (;;) {
-      int un = 0;
-      if (lane == 0) un = atomicAdd(&s_next, 1);
-      un = __builtin_amdgcn_readfirstlane(un);
-      if (un >= nunits) break;
-      int k = 0;
-      while (un >= s_ubase[k + 1]) ++k;
-      const int lg = min(kWClasses - 1 - k, 6);  // log2 of the lanes per entry
-      const int gl = lane & ((1 << lg) - 1);
-      const int it = s_cbase[k] + ((un - s_ubase[k]) << (6 - lg)) + (lane >> lg);
-      const bool valid = it < s_cbase[k + 1];
-      const int st = valid ? s_start[it] : 0;
-      const int len = valid ? (int)s_p[it] : 0;
-      const uint32_t rowb = valid ? s_row[it] : 0u;
-      const double wu = W ? (double)(valid ? s_wt[W ? it : 0] : 0.0f) : 0.0;
-      Octet<RT> y;
-      if (gl * 8 < len) y.load(R + st + gl * 8);
-      for (int b = 0;;) {
-        const int at = b + gl * 8;
-        Octet<RT> yn;
-        const bool more = lg == 6 && b + 512 < len;  // wave-uniform: one entry per wave
-        if (more && at + 512 < len) yn.load(R + st + at + 512);
+    const int e1 = entry_of(tk1, more);
+    for (int w0 = 0; w0 < total; w0 += kMapCap) {
+      if (w0 > 0) __syncthreads();  // the words of the last round are done
+      const int t1 = min(nw, w0 + kMapCap - wbase);
+      for (int t = max(0, w0 - wbase); t < t1; ++t) s_map[wbase + t - w0] = (uint16_t)(tid | (t << 9));
+      __syncthreads();
+      const int end = min(total - w0, kMapCap);
+      for (int j = w * (kWave / 4) + (lane >> 2); j < end; j += kWedgeB / 4) {
+        const uint32_t me = s_map[j];
+        const int4 it = s_item[me & 511u];
+        const int t = (int)(me >> 9), at = 32 * t + 8 * (lane & 3);
         uint32_t byte = 0;
-        if (at < len) byte = probe_octet<W, RT>(y, len - at, tab, guard, acc, wu);
+        if (at < it.w) {
+          Octet<RT> y;
+          y.load(row_at((uint32_t)it.x) + at);
+          byte = probe_octet<RT, AT>(y, it.w - at, tabp, guard, accp, W ? (AT)__int_as_float(it.z) : (AT)1);
+        }
         // four lanes' bytes make one word of the row
-        uint32_t word = byte << ((gl & 3) * 8);
-        if (lg >= 1) word = or_dpp<0xB1>(word);
-        if (lg >= 2) word = or_dpp<0x4E>(word);
-        if ((gl & 3) == 0 && at < len) a.bits[rowb + (uint32_t)(at >> 5)] = word;
-        if (!more) break;
-        b += 512;
-        y = yn;
+        uint32_t word = byte << ((lane & 3) * 8);
+        word = or_dpp<0xB1>(word);
+        word = or_dpp<0x4E>(word);
+        if ((lane & 3) == 0) a.bits[(uint32_t)it.y + (uint32_t)t] = word;
       }
     }
+    if (tid == 0) s_task = ti2;
     __syncthreads();
     // the pairs (v, w): alone on its row, or one of several pieces
     for (int j = tid; j < dpv; j += kWedgeB) {
@@ -800,21 +917,222 @@ __global__ __launch_bounds__(kWedgeB, (TAB <= kTabA ? 8 : 2)) void k_tri_wedge(T
         else if (s != 0u) atomicAdd(&a.accu[ov + j], s);
       }
     }
+    if (!more) return;
+    ti = ti1;
+    ti1 = s_task;
+    tk = tk1;
+    e = e1;
   }
 }
 
-// Wedge, one wave per v: short rows, and rows beyond the workgroup kernels'
-// tables. R(v) is searched (in LDS up to kWaveTab entries), eight lanes per
-// entry of v's row.
+// Wedge for short rows: group_rows(d) vertices v of degree d per task, a thread
+// per entry of their rows. The R(v) of the group share one hash table in LDS
+// (key: rank and place of v in the group; at most half full, linear probing).
+// What a task costs is the chain of dependent reads from its first to its last
+// step, which one wave per v paid for every v (RMAT-22 3.0 ms, Chung-Lu 2^20
+// 1.0 ms; here 2.4 and 0.63, of which looking a task ahead is 0.6 and 0.17).
+constexpr int kGroupSlots = 2 * kWedgeB;
+constexpr int kGroupLb = 10;
+static_assert(kGroupSlots == 1 << kGroupLb, "slots");
+
+template <bool W>
+__global__ __launch_bounds__(kWedgeB, 8) void k_tri_wedge_group(TriArgs a) {
+  constexpr int NW = kWedgeB / kWave;
+  constexpr uint32_t kNone = 0xFFFFFFFFu;
+  using AT = typename std::conditional<W, double, uint32_t>::type;
+  __shared__ __align__(16) uint32_t s_key[kGroupSlots];
+  __shared__ uint16_t s_slot[kGroupSlots];
+  __shared__ AT acc[kWedgeB];
+  __shared__ int4 s_item[kWedgeB];  // row, word of the bit matrix, weight, p | place of v << 16
+  __shared__ uint16_t s_map[kMapCap];
+  __shared__ int s_wsum[NW];
+  __shared__ int s_task, s_d;
+  __shared__ int s_gt[kGroupMax], s_gr[kGroupMax], s_ge[kGroupMax];  // per length: first task, first and end rank
+  if (!tri_ready<W>(a)) return;
+  const int tid = threadIdx.x, lane = lane_id(), w = tid / kWave;
+  const int ntask = a.ctl->num_group;
+  s_gt[tid] = a.ctl->grp_task[tid];
+  s_gr[tid] = a.ctl->grp_rank[tid];
+  s_ge[tid] = a.ctl->cur[tid];  // where the ranks of the next shorter length begin
+  if (tid == 0) s_task = atomicAdd(&a.ctl->cur_group, 2);
+  __syncthreads();
+  // As the bitmap kernel, a task ahead: its length, then its rows, then this
+  // thread's entry are looked up while the task before it runs. Lengths
+  // descend with the tasks: a task's is the one whose tasks start at or before
+  // it and whose next shorter length's start after it.
+  auto find_length = [&](int t) {
+    if (tid > 0 && s_gt[tid] <= t && t < s_gt[tid - 1]) s_d = tid;
+  };
+  struct Mine {
+    int d, vl, i, nv;  // length, place of this thread's row, its entry of it, rows of the task
+    int32_t r;         // rank of the row
+    int2 v;            // row offset, |R(v)|
+  };
+  auto rows_of = [&](int t, int d) {
+    Mine m;
+    const int rows = group_rows(d);
+    const int r0 = s_gr[d] + (t - s_gt[d]) * rows;
+    m.d = d;
+    m.nv = min(rows, s_ge[d] - r0);
+    m.vl = tid / d;
+    m.i = tid - m.vl * d;
+    m.r = r0 + m.vl;
+    m.v = m.vl < m.nv ? a.rinfo[m.r] : make_int2(0, 0);
+    return m;
+  };
+  int ti = s_task, ti1 = ti + 1;
+  if (ti >= ntask) return;
+  find_length(ti);
+  __syncthreads();
+  Mine me = rows_of(ti, s_d);
+  int e = me.vl < me.nv ? a.emap[me.v.x + me.i] : 0;
+  for (;;) {
+    const bool more = ti1 < ntask;
+    int ti2 = 0;
+    if (tid == 0) ti2 = atomicAdd(&a.ctl->cur_group, 1);
+    for (int i = tid; i < kGroupSlots / 4; i += kWedgeB)
+      reinterpret_cast<uint4*>(s_key)[i] = make_uint4(kNone, kNone, kNone, kNone);
+    acc[tid] = 0;
+    __syncthreads();  // (also: every thread has read s_d)
+    if (more) find_length(ti1);
+    const bool use16 = me.r - me.vl + me.nv <= kSat16;  // every rank of the group below kSat16
+    const bool mine = me.vl < me.nv;
+    const uint32_t r = (uint32_t)me.r;
+    int p = 0;
+    if (mine) {
+      const int ov = me.v.x, vl = me.vl;
+      if (e >= 0) {
+        const uint32_t y = a.R32[e];
+        const uint32_t key = y | ((uint32_t)vl << 26);
+        uint32_t q = hash_bucket((int32_t)(y ^ ((uint32_t)vl * 0x9E3B5u)), kGroupLb);
+        while (atomicCAS(&s_key[q], kNone, key) != kNone) q = (q + 1) & (kGroupSlots - 1);  // at most half full: ends
+        s_slot[q] = (uint16_t)(vl * me.d + (e - ov));
+      } else {
+        const int4* const hd = reinterpret_cast<const int4*>(a.R16) + ~e;
+        const int4 xi = hd[0];
+        if (use16) p = find_rank16(reinterpret_cast<const uint16_t*>(hd + kHead), xi.y, r, hd[1]);
+        else p = find_rank(a.R32 + xi.x, xi.y, r);
+        if (p < 0) {
+          a.ctl->bad = 1;  // (v, x) is stored, (x, v) is not
+          p = 0;
+        } else {
+          a.emap[ov + me.i] = xi.x + p;
+          s_item[tid] = make_int4(use16 ? ~e + kHead : xi.x, (int)((uint32_t)xi.z + tri_words(p)), xi.w, p | (vl << 16));
+        }
+      }
+    }
+    const int nw = (p + 31) >> 5;
+    int incl = nw;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int t = __shfl_up(incl, o);
+      if (lane >= o) incl += t;
+    }
+    if (lane == kWave - 1) s_wsum[w] = incl;
+    __syncthreads();
+    int wbase = incl - nw, total = 0;
+#pragma unroll
+    for (int k = 0; k < NW; ++k) {
+      const int x = s_wsum[k];
+      wbase += k < w ? x : 0;
+      total += x;
+    }
+    Mine me1 = me;
+    int e1 = 0;
+    if (more) {
+      me1 = rows_of(ti1, s_d);
+      if (me1.vl < me1.nv) e1 = a.emap[me1.v.x + me1.i];
+    }
+    for (int w0 = 0; w0 < total; w0 += kMapCap) {
+      if (w0 > 0) __syncthreads();
+      const int t1 = min(nw, w0 + kMapCap - wbase);
+      for (int t = max(0, w0 - wbase); t < t1; ++t) s_map[wbase + t - w0] = (uint16_t)(tid | (t << 9));
+      __syncthreads();
+      const int end = min(total - w0, kMapCap);
+      for (int j = w * (kWave / 4) + (lane >> 2); j < end; j += kWedgeB / 4) {
+        const uint32_t mp = s_map[j];
+        const int4 it = s_item[mp & 511u];
+        const int t = (int)(mp >> 9), at = 32 * t + 8 * (lane & 3), nvalid = (it.w & 0xFFFF) - at;
+        uint32_t byte = 0;
+        if (nvalid > 0) {
+          const uint32_t vt = (uint32_t)it.w >> 16, mix = vt * 0x9E3B5u, tag = vt << 26;
+          uint32_t y[8];
+          if (use16) {
+            Octet<uint16_t> o;
+            o.load(a.R16 + 8 * (size_t)(uint32_t)it.x + at);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) y[k] = (k & 1) ? o.v[k >> 1] >> 16 : o.v[k >> 1] & 0xFFFFu;
+          } else {
+            Octet<uint32_t> o;
+            o.load(a.R32 + it.x + at);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) y[k] = o.v[k];
+          }
+          const AT wu = W ? (AT)__int_as_float(it.z) : (AT)1;
+#pragma unroll
+          for (int h = 0; h < 8; h += 4) {
+            uint32_t q[4], key[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              q[k] = hash_bucket((int32_t)(y[h + k] ^ mix), kGroupLb);
+              key[k] = s_key[q[k]];
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              // an entry past the row's part looks like an empty slot
+              const uint32_t want = h + k < nvalid ? y[h + k] | tag : kNone;
+              while (key[k] != want && key[k] != kNone && want != kNone) {
+                q[k] = (q[k] + 1) & (kGroupSlots - 1);
+                key[k] = s_key[q[k]];
+              }
+              if (key[k] == want && want != kNone) {
+                byte |= 1u << (h + k);
+                AT* s = &acc[s_slot[q[k]]];
+                if constexpr (W) unsafeAtomicAdd(s, wu);
+                else atomicAdd(s, wu);
+              }
+            }
+          }
+        }
+        uint32_t word = byte << ((lane & 3) * 8);
+        word = or_dpp<0xB1>(word);
+        word = or_dpp<0x4E>(word);
+        if ((lane & 3) == 0) a.bits[(uint32_t)it.y + (uint32_t)t] = word;
+      }
+    }
+    if (tid == 0) s_task = ti2;
+    __syncthreads();
+    if (mine && me.i < me.v.y) {
+      AT* const gacc = W ? (AT*)a.accw : (AT*)a.accu;
+      gacc[me.v.x + me.i] = acc[tid];
+    }
+    if (!more) return;
+    ti = ti1;
+    ti1 = s_task;
+    me = me1;
+    e = e1;
+  }
+}
+
+// Wedge, one wave per v: long rows of ranks beyond the workgroup kernels' tables. R(v)
+// is hashed in LDS (at most half full, linear probing); longer R(v) that the
+// workgroup kernels cannot take are searched in memory. 64 entries of v's row
+// at a time, their words dealt to groups of four lanes as above.
+constexpr int kWaveSlots = 2 * kWaveTab;
+constexpr int kWaveMap = 512;
+
 template <bool W, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_tri_wedge_wave(TriArgs a) {
   constexpr int NW = BLOCK / kWave;
   using AT = typename std::conditional<W, double, uint32_t>::type;
-  __shared__ uint32_t s_list[NW][kWaveTab];
+  constexpr uint32_t kNone = 0xFFFFFFFFu;
+  __shared__ uint32_t s_key[NW][kWaveSlots];
+  __shared__ uint8_t s_pos[NW][kWaveSlots];
   __shared__ AT s_acc[NW][kWaveTab];
+  __shared__ int4 s_item[NW][kWave];
+  __shared__ uint16_t s_map[NW][kWaveMap];  // item | word << 6
   if (!tri_ready<W>(a)) return;
   const int lane = lane_id(), w = threadIdx.x / kWave;
-  const int gl = lane & 7;
   const int count = a.ctl->num_wave;
   AT* const gacc = W ? (AT*)a.accw : (AT*)a.accu;
   for (int li = blockIdx.x * NW + w; li < count; li += gridDim.x * NW) {
@@ -822,81 +1140,103 @@ __global__ __launch_bounds__(BLOCK) void k_tri_wedge_wave(TriArgs a) {
     const int4 vi = a.info[v];
     const int d = a.dr[r], ov = vi.x, dpv = vi.y;
     const bool lds = dpv <= kWaveTab;
-    if (lds)
+    const int lb = max(ceil_log2(2 * dpv), 4);
+    const uint32_t mask = (1u << lb) - 1u;
+    if (lds) {
+      for (int j = lane; j <= (int)mask; j += kWave) s_key[w][j] = kNone;
+      lds_fence_wave();
       for (int j = lane; j < dpv; j += kWave) {
-        s_list[w][j] = a.R32[ov + j];
+        const uint32_t y = a.R32[ov + j];
         s_acc[w][j] = 0;
+        uint32_t q = hash_bucket((int32_t)y, lb);
+        while (atomicCAS(&s_key[w][q], kNone, y) != kNone) q = (q + 1) & mask;  // at most half full: ends
+        s_pos[w][q] = (uint8_t)j;
       }
-    lds_fence_wave();
+    }
     for (int b = 0; b < d; b += kWave) {
-      int start = 0, p = 0;
-      uint32_t row = 0;
-      float wt = 0.0f;
+      int p = 0;
       if (b + lane < d) {
         const int k = ov + b + lane;
-        if (a.emap[k] < 0) {
-          const int4 xi = a.info[a.ind[k]];
-          start = xi.x;
-          wt = __int_as_float(xi.w);
-          p = find_rank(a.R32 + start, xi.y, (uint32_t)r);
+        const int e = a.emap[k];
+        if (e < 0) {
+          const int4* const hd = reinterpret_cast<const int4*>(a.R16) + ~e;
+          const int4 xi = hd[0];
+          if (r < kSat16)
+            p = find_rank16(reinterpret_cast<const uint16_t*>(hd + kHead), xi.y, (uint32_t)r, hd[1]);
+          else
+            p = find_rank(a.R32 + xi.x, xi.y, (uint32_t)r);
           if (p < 0) {
             a.ctl->bad = 1;
             p = 0;
           } else {
-            a.emap[k] = start + p;
-            row = (uint32_t)xi.z + tri_words(p);
+            a.emap[k] = xi.x + p;
+            s_item[w][lane] = make_int4(xi.x, (int)((uint32_t)xi.z + tri_words(p)), xi.w, p);
           }
         }
       }
-      uint64_t todo = ballot(p > 0);
-      while (todo) {
-        int src = -1;
+      const int nw = (p + 31) >> 5;
+      int incl = nw;
 #pragma unroll
-        for (int g = 0; g < 8; ++g) {
-          if (todo) {
-            const int s = __ffsll((unsigned long long)todo) - 1;
-            if ((lane >> 3) == g) src = s;
-            todo &= todo - 1;
-          }
-        }
-        const int s = max(src, 0);
-        const int st = __shfl(start, s);
-        const int ls = __shfl(p, s);
-        const int len = src >= 0 ? ls : 0;
-        const uint32_t rowb = (uint32_t)__shfl((int)row, s);
-        const float wu = __shfl(wt, s);
-        for (int c = 0; ballot(c < len) != 0; c += 32) {
-          const int at = c + gl * 4;
-          uint32_t nib = 0;
-          if (at < len) {
-            const Raw32 y = *reinterpret_cast<const Raw32*>(a.R32 + st + at);
+      for (int o = 1; o < kWave; o <<= 1) {
+        const int t = __shfl_up(incl, o);
+        if (lane >= o) incl += t;
+      }
+      const int total = __builtin_amdgcn_readlane(incl, kWave - 1), wbase = incl - nw;
+      for (int w0 = 0; w0 < total; w0 += kWaveMap) {
+        lds_fence_wave();
+        const int t1 = min(nw, w0 + kWaveMap - wbase);
+        for (int t = max(0, w0 - wbase); t < t1; ++t) s_map[w][wbase + t - w0] = (uint16_t)(lane | (t << 6));
+        lds_fence_wave();
+        const int end = min(total - w0, kWaveMap);
+        for (int j = lane >> 2; j < end; j += kWave / 4) {
+          const uint32_t e = s_map[w][j];
+          const int4 it = s_item[w][e & 63u];
+          const int t = (int)(e >> 6), at = 32 * t + 8 * (lane & 3);
+          uint32_t byte = 0;
+          if (at < it.w) {
+            const AT wu = W ? (AT)__int_as_float(it.z) : (AT)1;
+            Octet<uint32_t> y;
+            y.load(a.R32 + it.x + at);
+            if (lds) {
+              uint32_t q[8], key[8];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-              if (at + t < len) {
-                const int q = lds ? find_rank(s_list[w], dpv, y.v[t]) : find_rank(a.R32 + ov, dpv, y.v[t]);
+              for (int i = 0; i < 8; ++i) {
+                q[i] = hash_bucket((int32_t)y.v[i], lb);
+                key[i] = s_key[w][q[i]];
+              }
+#pragma unroll
+              for (int i = 0; i < 8; ++i) {
+                const bool live = at + i < it.w;
+                while (live && key[i] != y.v[i] && key[i] != kNone) {
+                  q[i] = (q[i] + 1) & mask;
+                  key[i] = s_key[w][q[i]];
+                }
+                if (live && key[i] == y.v[i]) {
+                  byte |= 1u << i;
+                  AT* s = &s_acc[w][s_pos[w][q[i]]];
+                  if constexpr (W) unsafeAtomicAdd(s, wu);
+                  else atomicAdd(s, wu);
+                }
+              }
+            } else {
+              for (int i = 0; i < 8 && at + i < it.w; ++i) {
+                const int q = find_rank(a.R32 + ov, dpv, y.v[i]);
                 if (q >= 0) {
-                  nib |= 1u << t;
-                  // (separate branches: one pointer for both would be flat atomics)
-                  if (lds) {
-                    if constexpr (W) unsafeAtomicAdd(&s_acc[w][q], (double)wu);
-                    else atomicAdd(&s_acc[w][q], 1u);
-                  } else {
-                    if constexpr (W) unsafeAtomicAdd(&gacc[ov + q], (double)wu);
-                    else atomicAdd(&gacc[ov + q], 1u);
-                  }
+                  byte |= 1u << i;
+                  if constexpr (W) unsafeAtomicAdd(&gacc[ov + q], wu);
+                  else atomicAdd(&gacc[ov + q], wu);
                 }
               }
             }
           }
-          uint32_t word = nib << (gl * 4);
+          uint32_t word = byte << ((lane & 3) * 8);
           word = or_dpp<0xB1>(word);
           word = or_dpp<0x4E>(word);
-          word = or_dpp<0x141>(word);
-          if (gl == 0 && c < len) a.bits[rowb + (uint32_t)(c >> 5)] = word;
+          if ((lane & 3) == 0) a.bits[(uint32_t)it.y + (uint32_t)t] = word;
         }
       }
+      lds_fence_wave();
     }
-    lds_fence_wave();
     if (lds)
       for (int j = lane; j < dpv; j += kWave) gacc[ov + j] = s_acc[w][j];
     lds_fence_wave();
@@ -936,7 +1276,7 @@ template <bool W>
 __device__ __forceinline__ void reduce_16(const TriArgs& a, bool valid, int32_t u) {
   const int lane = lane_id(), gl = lane & 15, gb = lane & ~15;
   int4 inf = make_int4(0, 0, 0, 0);
-  int2 me = make_int2(0, 0);
+  int4 me = make_int4(0, 0, 0, 0);
   if (valid) {
     inf = a.info[u];
     me = a.rw[u];
@@ -1240,14 +1580,15 @@ size_t carve(TriArgs& a, unsigned char* p, int32_t n, int64_t m, bool weighted) 
   };
   const size_t nn = (size_t)std::max(n, 1), mm = (size_t)m;
   a.ctl = reinterpret_cast<TriCtl*>(take(sizeof(TriCtl)));
-  a.rw = reinterpret_cast<int2*>(take(nn * sizeof(int2)));
+  a.rw = reinterpret_cast<int4*>(take(nn * sizeof(int4)));
   a.vtx = reinterpret_cast<int32_t*>(take(nn * 4));
   a.dr = reinterpret_cast<int32_t*>(take(nn * 4));
   a.wr = reinterpret_cast<float*>(weighted ? take(nn * 4) : nullptr);
   a.sr = reinterpret_cast<double*>(weighted ? take(nn * 8) : nullptr);
   a.info = reinterpret_cast<int4*>(take(nn * sizeof(int4)));
+  a.rinfo = reinterpret_cast<int2*>(take(nn * sizeof(int2)));
   a.R32 = reinterpret_cast<uint32_t*>(take((mm + 16) * 4));
-  a.R16 = reinterpret_cast<uint16_t*>(take((mm + 16) * 2));
+  a.R16 = reinterpret_cast<uint16_t*>(take((size_t)(row16_line(mm, nn) + 1) * 128));
   a.emap = reinterpret_cast<int32_t*>(take(mm * 4));
   unsigned char* acc = take(mm * (weighted ? 8 : 4));
   a.accw = weighted ? reinterpret_cast<double*>(acc) : nullptr;
@@ -1296,7 +1637,8 @@ hipError_t tri_launch(const TriArgs& a, hipStream_t s) {
     ProfScope ps("tri_wedge", s);
     hipLaunchKernelGGL((k_tri_wedge<W, uint16_t, kTabA, kAccA>), dim3(cus * 4), dim3(kWedgeB), 0, s, a);
     hipLaunchKernelGGL((k_tri_wedge<W, uint32_t, kTabB, kAccB>), dim3(cus), dim3(kWedgeB), 0, s, a);
-    hipLaunchKernelGGL((k_tri_wedge_wave<W, PB>), grid(a.n, PB / kWave, 32), dim3(PB), 0, s, a);
+    hipLaunchKernelGGL((k_tri_wedge_group<W>), dim3(cus * 4), dim3(kWedgeB), 0, s, a);
+    hipLaunchKernelGGL((k_tri_wedge_wave<W, PB>), grid(std::min<int64_t>(a.n, a.m / kGroupMax), PB / kWave, 16), dim3(PB), 0, s, a);
   }
   {
     ProfScope ps("tri_reduce", s);
