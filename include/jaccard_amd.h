@@ -129,7 +129,9 @@ typedef struct jc_tuning {
                                   chunk with a full bucket) */
   int32_t engine;              /* 0 (default), JC_ENGINE_OWNER or JC_ENGINE_ORIENTED (then
                                   the owner engine for what that one cannot do) */
-  int32_t reserved[1];
+  int32_t members;             /* nonzero: the graph is a disjoint union of many graphs of at
+                                  most 65536 vertices, with consecutive ids (a batch); the
+                                  oriented engine then ranks each by itself */
 } jc_tuning;
 #define JC_ENGINE_OWNER 1    /* each pair by streaming its shorter row */
 #define JC_ENGINE_ORIENTED 2 /* from the triangles, where that applies */

@@ -75,15 +75,16 @@ Layout layout(int32_t n, int32_t m, bool weighted, bool ec) {
 }
 
 // Oriented engine (jc_tri.hip) before the owner engine: from kTriMinEdges
-// stored edges on, where no tuning is given. Measured: RMAT-16 (1.8M entries)
-// 0.27 ms by the owner engine, 0.40 by this one, whose two dozen dependent
-// launches are then most of it; RMAT of 200003 vertices (5.7M) 1.58 and 1.12.
+// stored edges on, where no tuning is given or it names a batch. Measured:
+// RMAT-16 (1.8M entries) 0.27 ms by the owner engine, 0.40 by this one, whose
+// two dozen dependent launches are then most of it; RMAT of 200003 vertices
+// (5.7M) 1.58 and 0.90, the kernel-level sequence on 150001 (4.3M) 1.26 and 0.77.
 constexpr int32_t kTriMinEdges = 1 << 22;
 
 bool tri_wanted(const jc_csr* g, const jc_tuning* t) {
   if (t && (t->engine == JC_ENGINE_OWNER || t->wide_index || t->hash_table == 1 || t->quot_max_disp > 0)) return false;
   if (g->n > jc::kTriMaxN) return false;
-  return (t && t->engine == JC_ENGINE_ORIENTED) || (!t && g->m >= kTriMinEdges);
+  return (t && t->engine == JC_ENGINE_ORIENTED) || ((!t || t->members) && g->m >= kTriMinEdges);
 }
 
 // RAII for a stream-ordered allocation.
@@ -119,6 +120,7 @@ int run_jaccard(const jc_csr* g, const float* vw, float* result, bool ec, unsign
     // quotients are the vertex-centric pipeline's values
     jc::EngineArgs t = a;
     t.out32 = result;
+    t.members = tuning ? tuning->members != 0 : 0;
     JC_TRY(jc::run_tri(weighted ? jc::kModeEcW : jc::kModeEcU, t, tri_ws, &a.skip, s));
   }
   double* S64 = weighted ? reinterpret_cast<double*>(ws + L.s64) : nullptr;
@@ -335,9 +337,16 @@ int jc_intersect(int32_t n, int32_t m, const int32_t* offsets, const int32_t* in
   if (!csr_args_ok(&g) || (m > 0 && (!work || !weight_i || !weight_s))) return JC_ERR_INVALID_ARG;
   if (n == 0 || m == 0) return JC_OK;
   hipStream_t s = hs(stream);
+  const size_t need = al(jc::engine_workspace_bytes(n, m));
   AsyncBuf buf;
   buf.s = s;
-  JC_TRY(hipMallocAsync(&buf.p, jc::engine_workspace_bytes(n, m), s));
+  bool tri = tri_wanted(&g, nullptr);
+  if (tri && hipMallocAsync(&buf.p, need + jc::tri_workspace_bytes(n, m, v != nullptr), s) != hipSuccess) {
+    (void)hipGetLastError();
+    buf.p = nullptr;
+    tri = false;
+  }
+  if (!tri) JC_TRY(hipMallocAsync(&buf.p, need, s));
   jc::EngineArgs a{};
   a.n = n;
   a.m = m;
@@ -350,7 +359,9 @@ int jc_intersect(int32_t n, int32_t m, const int32_t* offsets, const int32_t* in
   a.accumulate = 1;
   a.small_max = 0;
   a.small_blocks_per_cu = 0;
-  JC_TRY(jc::launch_fill_u32(reinterpret_cast<uint32_t*>(weight_s), m, jc::kSentinel32, s));
+  if (tri)
+    JC_TRY(jc::run_tri(jc::kModeIsF32, a, static_cast<unsigned char*>(buf.p) + need, &a.skip, s));
+  JC_TRY(jc::launch_fill_u32(reinterpret_cast<uint32_t*>(weight_s), m, jc::kSentinel32, s, a.skip));
   JC_TRY(jc::run_engine(jc::kModeIsF32, v != nullptr, a, buf.p, true, s));
   return JC_OK;
 }

@@ -99,6 +99,7 @@ struct EngineArgs {
   // Device flag, or nullptr: when it is not 0 the results are already there
   // (the oriented engine delivered them) and the pass does nothing.
   const int* skip;
+  int members;  // the graph is a union of many small graphs (oriented engine)
 };
 
 // Oriented engine (jc_tri.hip): kModeEcU / kModeEcW (out32 the result) and

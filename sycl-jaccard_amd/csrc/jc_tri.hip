@@ -11,6 +11,9 @@
 // over the ranks below v, which for the vertices that matter is a few KiB.
 //
 //   rank     degree-bucket counting sort of the vertices
+//            (a batch of small graphs, EngineArgs::members: the disjoint parts
+//            are found from the reach of the rows, and each is ranked by
+//            itself, so that its 16-bit ranks start at its own first)
 //   orient   per row: R(u) sorted by rank (32-bit and, saturated, 16-bit
 //            copies, at the row's own offset), the row sum of the weights,
 //            and emap[k], the oriented slot of a stored entry (u, v in R(u))
@@ -51,6 +54,8 @@ namespace jc {
 namespace {
 
 constexpr int kTriBuckets = 1024;
+constexpr int kTriParts = 1024;    // vertex ranges of the rank kernels, at most
+constexpr int kPartMax = 65536;    // vertices of a disjoint part
 constexpr int kTriMaxOut = 4096;   // largest |R(u)|: the sort and reduce buffers in LDS
 constexpr int kTriRowWave = 1024;  // rows up to this many entries are oriented by one wave
 constexpr int kSat16 = 65535;      // 16-bit ranks saturate here
@@ -94,7 +99,7 @@ constexpr int kHead = 2;
 
 // A task of the bitmap wedge kernels.
 struct __attribute__((aligned(32))) TriTask {
-  int32_t r, o, d, dp;  // v: rank, row offset, row entries, |R(v)|
+  int32_t r, o, d, dp;  // v: rank (16-bit kernel: in its part), row offset, row entries, |R(v)|
   int32_t piece;        // entries [piece * kWedgeB, ...) of v's row
   int32_t row;          // row16 of v
   int32_t pad[2];
@@ -114,11 +119,13 @@ struct TriCtl {
   int num_wave, num_s16, num_s64;
   int num_red[2], cur_red[2];    // reduce by workgroup: up to kRedWg entries, more
   int cur_big;
+  int num_part, cur_part;        // disjoint parts (members)
   int num_group, cur_group;      // group tasks of wedge: rows of fewer than kGroupMax entries
   int grp_task[kGroupMax];       // first task of the rows of each length
   int grp_rank[kGroupMax];       // first rank among them that is taken in groups
   int hist[kTriBuckets];
   int cur[kTriBuckets];
+  int reach[kTriParts], nstart[kTriParts];  // per vertex range: largest neighbour id (then of all ranges before), parts begun
 };
 
 namespace {
@@ -130,13 +137,19 @@ struct TriArgs {
   const int32_t* ind;
   const float* vw;
   TriCtl* ctl;
-  int4* rw;         // per vertex: rank, weight bits, place of its 16-bit row
+  int4* rw;         // per vertex: rank, weight bits, place of its 16-bit row, first rank of its part
   int32_t* vtx;     // per rank: vertex
   float* wr;        // per rank: weight
   double* sr;       // per rank: row sum of the weights (unweighted: unused)
   int32_t* dr;      // per rank: degree
-  int4* info;       // per vertex: row offset, |R|, first word of its bit matrix
-  int2* rinfo;      // per rank: row offset, |R|
+  int32_t* ord;     // vertices and their degrees by descending degree bucket: vtx
+  int32_t* dord;    // and dr, but for disjoint parts, whose ranks are in id order
+  int members;      // rank disjoint parts by themselves
+  int32_t grp_from; // place in ord from which longer rows than kWgMinDeg are taken in groups too
+  int32_t* starts;  // first vertices of the parts: per vertex range, then
+  int32_t* parts;   // all of them
+  int4* info;       // per vertex: row offset, |R|, first word of its bit matrix, rank
+  int4* rinfo;      // per place in ord: row offset, |R|, rank, first rank of the part
   uint32_t* R32;    // R(u) at [off[u], off[u] + |R(u)|), later the pairs' values
   uint16_t* R16;    // the same, saturated, at row16 with headers
   int32_t* emap;    // per stored entry (u, x): its slot, or until wedge ~row16 of x if x ranks after u
@@ -148,7 +161,7 @@ struct TriArgs {
   int32_t* list_big;
   TriTask* task[2];
   int64_t task_cap;
-  int32_t* list_wave;  // ranks
+  int32_t* list_wave;  // places in ord
   int32_t* list_s16;   // vertices with |R| in 1..16
   int32_t* list_s64;   // up to kRedWave
   int32_t* list_red[2];  // up to kRedWg, more
@@ -217,7 +230,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_hist(TriArgs a) {
 __device__ __forceinline__ int group_rows(int d) { return min(kGroupRows, kWedgeB / d); }
 
 // First rank of every bucket, largest degrees first.
-__global__ __launch_bounds__(kTriBuckets) void k_tri_scan(TriCtl* c) {
+__global__ __launch_bounds__(kTriBuckets) void k_tri_scan(TriCtl* c, int grp_from) {
   __shared__ int part[kTriBuckets / kWave];
   const int b = kTriBuckets - 1 - threadIdx.x;
   const int v = c->hist[b];
@@ -237,7 +250,7 @@ __global__ __launch_bounds__(kTriBuckets) void k_tri_scan(TriCtl* c) {
   // long rows of low rank go to the bitmap kernel instead.
   int ng = 0;
   if (b > 0 && b < kGroupMax) {
-    const int first = b >= kWgMinDeg ? max(base + incl - v, kSat16) : base + incl - v;
+    const int first = b >= kWgMinDeg ? max(base + incl - v, grp_from) : base + incl - v;
     const int cnt = max(0, base + incl - first);
     c->grp_rank[b] = first;
     ng = (cnt + group_rows(b) - 1) / group_rows(b);
@@ -291,14 +304,194 @@ __global__ __launch_bounds__(BLOCK) void k_tri_rank(TriArgs a) {
     const int o = a.off[u], d = a.off[u + 1] - o;
     const int b = deg_bucket(d);
     const int r = base[b] + atomicAdd(&h[b], 1);
-    const float w = W ? a.vw[u] : 0.0f;
-    a.rw[u] = make_int4(r, __float_as_int(w), (int)row16(o, u), 0);
-    a.vtx[r] = u;
-    a.dr[r] = d;
-    if constexpr (W) a.wr[r] = w;
+    a.ord[r] = u;
+    a.dord[r] = d;
+    if (!a.members) {
+      const float w = W ? a.vw[u] : 0.0f;
+      a.rw[u] = make_int4(r, __float_as_int(w), (int)row16(o, u), 0);
+      if constexpr (W) a.wr[r] = w;
+    }
     if (d > kTriRowWave) a.list_big[s_base[1] + atomicAdd(&s_cnt[1], 1)] = u;
     else if (d > kWave) a.list_mid[s_base[0] + atomicAdd(&s_cnt[0], 1)] = u;
-    else if (d == 0) a.info[u] = make_int4(o, 0, 0, 0);
+  }
+}
+
+// Disjoint parts of a batch. A part begins at a vertex with neighbours that no
+// row before it reaches past; vertices without neighbours belong to the part
+// before them. Per contiguous range of vertices: the largest neighbour id ...
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_tri_reach(TriArgs a) {
+  __shared__ int s_max;
+  if (threadIdx.x == 0) s_max = -1;
+  __syncthreads();
+  const int64_t per = ((int64_t)a.n + gridDim.x - 1) / gridDim.x;
+  const int32_t r0 = (int32_t)min(per * blockIdx.x, (int64_t)a.n), r1 = (int32_t)min(per * (blockIdx.x + 1), (int64_t)a.n);
+  int m = -1;
+  for (int32_t u = r0 + threadIdx.x; u < r1; u += BLOCK) {
+    const int e = a.off[u + 1];
+    if (e > a.off[u]) m = max(m, max(u, a.ind[e - 1]));
+  }
+  atomicMax(&s_max, m);
+  __syncthreads();
+  if (threadIdx.x == 0) a.ctl->reach[blockIdx.x] = s_max;
+}
+
+// ... then of all ranges before ...
+__global__ __launch_bounds__(kTriParts) void k_tri_reach_scan(TriCtl* c, int ranges) {
+  __shared__ int s[2][kTriParts];
+  const int t = threadIdx.x;
+  s[0][t] = t < ranges ? c->reach[t] : -1;
+  int b = 0;
+  for (int o = 1; o < kTriParts; o <<= 1) {
+    __syncthreads();
+    s[b ^ 1][t] = t >= o ? max(s[b][t], s[b][t - o]) : s[b][t];
+    b ^= 1;
+  }
+  __syncthreads();
+  if (t < ranges) c->reach[t] = t > 0 ? s[b][t - 1] : -1;
+}
+
+// ... then the parts that begin in the range, in order.
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_tri_starts(TriArgs a) {
+  constexpr int NW = BLOCK / kWave;
+  __shared__ int s_m[NW], s_c[NW];
+  const int lane = lane_id(), w = threadIdx.x / kWave;
+  const int64_t per = ((int64_t)a.n + gridDim.x - 1) / gridDim.x;
+  const int32_t r0 = (int32_t)min(per * blockIdx.x, (int64_t)a.n), r1 = (int32_t)min(per * (blockIdx.x + 1), (int64_t)a.n);
+  int before = a.ctl->reach[blockIdx.x], count = 0;
+  for (int32_t b = r0; b < r1; b += BLOCK) {
+    const int32_t u = b + threadIdx.x;
+    int m = -1;
+    if (u < r1) {
+      const int e = a.off[u + 1];
+      if (e > a.off[u]) m = max(u, a.ind[e - 1]);
+    }
+    int incl = m;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int t = __shfl_up(incl, o);
+      if (lane >= o) incl = max(incl, t);
+    }
+    if (lane == kWave - 1) s_m[w] = incl;
+    __syncthreads();
+    int excl = __shfl_up(incl, 1);
+    if (lane == 0) excl = -1;
+    excl = max(excl, before);
+    int all = before;
+    for (int k = 0; k < NW; ++k) {
+      if (k < w) excl = max(excl, s_m[k]);
+      all = max(all, s_m[k]);
+    }
+    const bool start = m >= 0 && u > excl;
+    const uint64_t sm = ballot(start);
+    if (lane == 0) s_c[w] = popc64(sm);
+    __syncthreads();
+    int at = count + popc64(sm & ((1ull << lane) - 1)), tot = 0;
+    for (int k = 0; k < NW; ++k) {
+      if (k < w) at += s_c[k];
+      tot += s_c[k];
+    }
+    if (start) a.starts[r0 + at] = u;
+    count += tot;
+    before = all;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) a.ctl->nstart[blockIdx.x] = count;
+}
+
+// All parts in one list.
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_tri_parts(TriArgs a) {
+  __shared__ int s_at, s_all;
+  if (threadIdx.x == 0) s_at = s_all = 0;
+  __syncthreads();
+  int at = 0, all = 0;
+  for (int k = threadIdx.x; k < (int)gridDim.x; k += BLOCK) {
+    const int c = a.ctl->nstart[k];
+    all += c;
+    if (k < (int)blockIdx.x) at += c;
+  }
+  atomicAdd(&s_at, at);
+  atomicAdd(&s_all, all);
+  __syncthreads();
+  const int64_t per = ((int64_t)a.n + gridDim.x - 1) / gridDim.x;
+  const int32_t r0 = (int32_t)min(per * blockIdx.x, (int64_t)a.n);
+  for (int i = threadIdx.x; i < a.ctl->nstart[blockIdx.x]; i += BLOCK) a.parts[s_at + i] = a.starts[r0 + i];
+  if (blockIdx.x == 0 && threadIdx.x == 0) a.ctl->num_part = s_all;
+}
+
+// Ranks of a part's vertices, [first vertex, ...): one workgroup sorts it by
+// degree bucket. The vertex weights' finest bit is k_tri_hist's.
+template <bool W>
+__global__ __launch_bounds__(kTriBuckets) void k_tri_rank_parts(TriArgs a) {
+  __shared__ int h[kTriBuckets], base[kTriBuckets];
+  __shared__ int part[kTriBuckets / kWave];
+  __shared__ int s_i;
+  const int tid = threadIdx.x, lane = lane_id();
+  const int count = a.ctl->num_part;
+  for (;;) {
+    if (tid == 0) s_i = atomicAdd(&a.ctl->cur_part, 1);
+    h[tid] = 0;
+    __syncthreads();
+    const int i = s_i;
+    if (i >= count) return;
+    const int32_t b0 = a.parts[i], b1 = i + 1 < count ? a.parts[i + 1] : a.n;
+    if (b1 - b0 > kPartMax) {
+      if (tid == 0) a.ctl->bad = 1;
+      return;
+    }
+    for (int32_t u0 = b0; u0 < b1; u0 += 4 * kTriBuckets) {
+      int d[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int32_t u = min(u0 + t * kTriBuckets + tid, b1 - 1);
+        d[t] = a.off[u + 1] - a.off[u];
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        if (u0 + t * kTriBuckets + tid < b1) atomicAdd(&h[deg_bucket(d[t])], 1);
+    }
+    __syncthreads();
+    const int b = kTriBuckets - 1 - tid;
+    const int v = h[b];
+    int incl = v;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int t = __shfl_up(incl, o);
+      if (lane >= o) incl += t;
+    }
+    if (lane == kWave - 1) part[tid / kWave] = incl;
+    __syncthreads();
+    int before = 0;
+    for (int k = 0; k < tid / kWave; ++k) before += part[k];
+    base[b] = b0 + before + incl - v;
+    // 16-bit ranks: every vertex with neighbours below kSat16
+    if (b == 0 && before + incl - v > kSat16) a.ctl->bad = 1;
+    __syncthreads();
+    for (int32_t u0 = b0; u0 < b1; u0 += 4 * kTriBuckets) {
+      int o[4], d[4];
+      float w[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int32_t u = min(u0 + t * kTriBuckets + tid, b1 - 1);
+        o[t] = a.off[u];
+        d[t] = a.off[u + 1] - o[t];
+        if constexpr (W) w[t] = a.vw[u];
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int32_t u = u0 + t * kTriBuckets + tid;
+        if (u < b1) {
+          const int r = atomicAdd(&base[deg_bucket(d[t])], 1);
+          a.rw[u] = make_int4(r, __float_as_int(w[t]), (int)row16(o[t], u), b0);
+          a.vtx[r] = u;
+          a.dr[r] = d[t];
+          if constexpr (W) a.wr[r] = w[t];
+        }
+      }
+    }
+    __syncthreads();
   }
 }
 
@@ -316,12 +509,13 @@ __device__ __forceinline__ void put_row_sum(const TriArgs& a, int32_t ru, double
   }
 }
 
-// Writes entry (rank r, row entry k) of row u at sorted position p.
+// Writes entry (rank r, row entry k) of row u at sorted position p; cb: the
+// first rank of its part.
 template <bool W>
-__device__ __forceinline__ void put_out(const TriArgs& a, int32_t u, int o, int p, uint32_t r, int k) {
+__device__ __forceinline__ void put_out(const TriArgs& a, int32_t u, int o, int p, uint32_t r, int k, uint32_t cb) {
   const int e = o + p;
   a.R32[e] = r;
-  a.R16[8 * ((size_t)row16(o, u) + kHead) + p] = (uint16_t)min(r, (uint32_t)kSat16);
+  a.R16[8 * ((size_t)row16(o, u) + kHead) + p] = (uint16_t)min(r - cb, (uint32_t)kSat16);
   a.emap[k] = e;
   if constexpr (W) a.accw[e] = 0.0;
   else a.accu[e] = 0u;
@@ -338,8 +532,8 @@ __device__ __forceinline__ void put_pivot(const TriArgs& a, int32_t u, int o, in
 }
 
 // Row u's facts (one lane).
-__device__ __forceinline__ void put_info(const TriArgs& a, int32_t u, int o, int cnt, int wbits) {
-  a.info[u] = make_int4(o, cnt, 0, 0);
+__device__ __forceinline__ void put_info(const TriArgs& a, int32_t u, int o, int cnt, int wbits, int ru) {
+  a.info[u] = make_int4(o, cnt, 0, ru);
   reinterpret_cast<int4*>(a.R16)[row16(o, u)] = make_int4(o, cnt, 0, wbits);
 }
 
@@ -347,7 +541,8 @@ __device__ __forceinline__ void put_info(const TriArgs& a, int32_t u, int o, int
 // rows of up to 16 entries). The position of an entry among the kept ones is
 // the number of kept ranks below its own, counted over the group.
 template <bool W, int G>
-__device__ __forceinline__ void orient_group(const TriArgs& a, bool valid, int32_t u, int o, int d, int ru, float w) {
+__device__ __forceinline__ void orient_group(const TriArgs& a, bool valid, int32_t u, int o, int d, int ru, float w,
+                                             int cb) {
   const int gl = lane_id() & (G - 1), gb = lane_id() & ~(G - 1);
   bool in_row = valid && gl < d;
   int4 rw = make_int4(0, 0, 0, 0);
@@ -367,7 +562,7 @@ __device__ __forceinline__ void orient_group(const TriArgs& a, bool valid, int32
     const int rj = G == kWave ? __builtin_amdgcn_readlane(mine, j) : __shfl(mine, gb + j);
     pos += rj < mine ? 1 : 0;
   }
-  if (keep) put_out<W>(a, u, o, pos, (uint32_t)rw.x, o + gl);
+  if (keep) put_out<W>(a, u, o, pos, (uint32_t)rw.x, o + gl, (uint32_t)cb);
   else if (in_row) a.emap[o + gl] = ~rw.z;
   const uint64_t gm = G == kWave ? ~0ull : ((1ull << G) - 1) << gb;
   const int cnt = popc64(km & gm);
@@ -377,8 +572,8 @@ __device__ __forceinline__ void orient_group(const TriArgs& a, bool valid, int32
     for (int t = 1; t < G; t <<= 1) s += __shfl_xor(s, t);
     if (valid && gl == 0) put_row_sum<W>(a, ru, s);
   }
-  if (valid && gl == 0) put_info(a, u, o, cnt, __float_as_int(w));
-  if (keep) put_pivot(a, u, o, cnt, pos, (uint32_t)rw.x);
+  if (valid && gl == 0) put_info(a, u, o, cnt, __float_as_int(w), ru);
+  if (keep) put_pivot(a, u, o, cnt, pos, (uint32_t)(rw.x - cb));
   if (valid && gl < 8) a.R16[8 * ((size_t)row16(o, u) + kHead) + cnt + gl] = (uint16_t)kSat16;
 }
 
@@ -390,7 +585,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_orient_small(TriArgs a) {
   for (int64_t base = (int64_t)(blockIdx.x * (BLOCK / kWave) + threadIdx.x / kWave) * kWave; base < a.n;
        base += (int64_t)nw * kWave) {
     const int32_t u = (int32_t)base + lane;
-    int o = 0, d = 0, ru = 0;
+    int o = 0, d = 0, ru = 0, cb = 0;
     float w = 0.0f;
     if (base + lane < a.n) {
       o = a.off[u];
@@ -398,6 +593,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_orient_small(TriArgs a) {
       const int4 rw = a.rw[u];
       ru = rw.x;
       w = __int_as_float(rw.y);
+      cb = rw.w;
     }
     uint64_t m16 = ballot(d > 0 && d <= 16), m64 = ballot(d > 16 && d <= kWave);
     while (m16) {
@@ -411,13 +607,15 @@ __global__ __launch_bounds__(BLOCK) void k_tri_orient_small(TriArgs a) {
         }
       }
       const int s = max(src, 0);
-      orient_group<W, 16>(a, src >= 0, __shfl(u, s), __shfl(o, s), __shfl(d, s), __shfl(ru, s), __shfl(w, s));
+      orient_group<W, 16>(a, src >= 0, __shfl(u, s), __shfl(o, s), __shfl(d, s), __shfl(ru, s), __shfl(w, s),
+                          __shfl(cb, s));
     }
     while (m64) {
       const int s = __ffsll((unsigned long long)m64) - 1;
       m64 &= m64 - 1;
       orient_group<W, kWave>(a, true, __builtin_amdgcn_readlane(u, s), __builtin_amdgcn_readlane(o, s),
-                             __builtin_amdgcn_readlane(d, s), __builtin_amdgcn_readlane(ru, s), __shfl(w, s));
+                             __builtin_amdgcn_readlane(d, s), __builtin_amdgcn_readlane(ru, s), __shfl(w, s),
+                             __builtin_amdgcn_readlane(cb, s));
     }
   }
 }
@@ -433,6 +631,7 @@ __device__ __forceinline__ void orient_row(const TriArgs& a, int32_t u, int tid,
   const int o = a.off[u], d = a.off[u + 1] - o;
   const int4 me = a.rw[u];
   const int ru = me.x;
+  const uint32_t cb = (uint32_t)me.w;
   const int lane = lane_id();
   if (tid == 0) {
     *s_n = 0;
@@ -492,7 +691,7 @@ __device__ __forceinline__ void orient_row(const TriArgs& a, int32_t u, int tid,
   }
   if (tid == 0) {
     put_row_sum<W>(a, ru, sum);
-    put_info(a, u, o, cnt, me.y);
+    put_info(a, u, o, cnt, me.y, ru);
     if (cnt > CAP) a.ctl->bad = 1;
   }
   const int c = min(cnt, CAP);
@@ -513,12 +712,12 @@ __device__ __forceinline__ void orient_row(const TriArgs& a, int32_t u, int tid,
     const int ka = ia < c ? (T == kWave ? (int)s_k[ia] : reinterpret_cast<int32_t*>(s_k)[ia]) : 0;
     const int kb = ib < c ? (T == kWave ? (int)s_k[ib] : reinterpret_cast<int32_t*>(s_k)[ib]) : 0;
     if (ia < c) {
-      put_out<W>(a, u, o, pa, ra, o + ka);
-      put_pivot(a, u, o, c, pa, ra);
+      put_out<W>(a, u, o, pa, ra, o + ka, cb);
+      put_pivot(a, u, o, c, pa, ra - cb);
     }
     if (ib < c) {
-      put_out<W>(a, u, o, pb, rb, o + kb);
-      put_pivot(a, u, o, c, pb, rb);
+      put_out<W>(a, u, o, pb, rb, o + kb, cb);
+      put_pivot(a, u, o, c, pb, rb - cb);
     }
   }
   if constexpr (T > kWave) __syncthreads();
@@ -569,17 +768,20 @@ __global__ __launch_bounds__(BLOCK) void k_tri_plan(TriArgs a) {
   if (!tri_go(a)) return;
   const int lane = lane_id(), wv = threadIdx.x / kWave;
   for (int64_t b0 = (int64_t)blockIdx.x * BLOCK; b0 < a.n; b0 += (int64_t)gridDim.x * BLOCK) {
-    const int32_t r = (int32_t)(b0 + threadIdx.x);
-    int d = 0, dp = 0, o = 0;
+    const int32_t at_ord = (int32_t)(b0 + threadIdx.x);
+    int d = 0, dp = 0, o = 0, r = 0, lr = 0;  // lr: rank in the part
     int32_t u = 0;
-    if (r < a.n) {
-      d = a.dr[r];
+    if (at_ord < a.n) {
+      d = a.dord[at_ord];
       if (d > 0) {
-        u = a.vtx[r];
+        u = a.ord[at_ord];
         const int4 inf = a.info[u];
+        const int cb = a.members ? a.rw[u].w : 0;
         o = inf.x;
         dp = inf.y;
-        a.rinfo[r] = make_int2(o, dp);
+        r = inf.w;
+        lr = r - cb;
+        a.rinfo[at_ord] = make_int4(o, dp, r, cb);
       }
     }
     const int din = d - dp;
@@ -588,8 +790,8 @@ __global__ __launch_bounds__(BLOCK) void k_tri_plan(TriArgs a) {
     // larger table for what the one-wave kernel's hash does not hold; short
     // rows are in the group tasks (k_tri_scan has the same rule)
     const int npiece = (d + kWedgeB - 1) / kWedgeB;
-    const int kind = r < kSat16 && dp <= kAccA ? 0 : 1;
-    const bool grp = d < kGroupMax && (d < kWgMinDeg || r >= kSat16);
+    const int kind = lr < kSat16 && dp <= kAccA ? 0 : 1;
+    const bool grp = d < kGroupMax && (d < kWgMinDeg || at_ord >= a.grp_from);
     const bool wg = din > 0 && !grp && (kind == 0 || (dp > kWaveTab && dp <= kAccB && r <= 32 * kTabB));
     if (wg) c[kind] = npiece;
     else if (din > 0 && !grp) c[2] = 1;
@@ -646,8 +848,8 @@ __global__ __launch_bounds__(BLOCK) void k_tri_plan(TriArgs a) {
     for (int l = 0; l < NL; ++l) at[l] = s_base[l] + s_w[l][wv] + incl[l] - c[l];
     if (wg)
       for (int p = 0; p < npiece; ++p)
-        if (at[kind] + p < a.task_cap) a.task[kind][at[kind] + p] = TriTask{r, o, d, dp, p, (int32_t)row16(o, u), {0, 0}};
-    if (c[2]) a.list_wave[at[2]] = r;
+        if (at[kind] + p < a.task_cap) a.task[kind][at[kind] + p] = TriTask{kind == 0 ? lr : r, o, d, dp, p, (int32_t)row16(o, u), {0, 0}};
+    if (c[2]) a.list_wave[at[2]] = at_ord;
     if (c[3]) a.list_s16[at[3]] = u;
     if (c[4]) a.list_s64[at[4]] = u;
     if (c[5]) a.list_red[0][at[5]] = u;
@@ -965,8 +1167,8 @@ __global__ __launch_bounds__(kWedgeB, 8) void k_tri_wedge_group(TriArgs a) {
   };
   struct Mine {
     int d, vl, i, nv;  // length, place of this thread's row, its entry of it, rows of the task
-    int32_t r;         // rank of the row
-    int2 v;            // row offset, |R(v)|
+    int r0;            // place in ord of the task's first row
+    int4 v;            // the row's rinfo
   };
   auto rows_of = [&](int t, int d) {
     Mine m;
@@ -976,8 +1178,8 @@ __global__ __launch_bounds__(kWedgeB, 8) void k_tri_wedge_group(TriArgs a) {
     m.nv = min(rows, s_ge[d] - r0);
     m.vl = tid / d;
     m.i = tid - m.vl * d;
-    m.r = r0 + m.vl;
-    m.v = m.vl < m.nv ? a.rinfo[m.r] : make_int2(0, 0);
+    m.r0 = r0;
+    m.v = m.vl < m.nv ? a.rinfo[r0 + m.vl] : make_int4(0, 0, 0, 0);
     return m;
   };
   int ti = s_task, ti1 = ti + 1;
@@ -995,14 +1197,16 @@ __global__ __launch_bounds__(kWedgeB, 8) void k_tri_wedge_group(TriArgs a) {
     acc[tid] = 0;
     __syncthreads();  // (also: every thread has read s_d)
     if (more) find_length(ti1);
-    const bool use16 = me.r - me.vl + me.nv <= kSat16;  // every rank of the group below kSat16
+    // 16-bit ranks where every row of the task ranks below kSat16 in its part
+    const bool use16 = a.members || me.r0 + me.nv <= kSat16;
+    const uint32_t cb = use16 ? (uint32_t)me.v.w : 0u;
     const bool mine = me.vl < me.nv;
-    const uint32_t r = (uint32_t)me.r;
+    const uint32_t r = (uint32_t)me.v.z - cb;
     int p = 0;
     if (mine) {
       const int ov = me.v.x, vl = me.vl;
       if (e >= 0) {
-        const uint32_t y = a.R32[e];
+        const uint32_t y = a.R32[e] - cb;
         const uint32_t key = y | ((uint32_t)vl << 26);
         uint32_t q = hash_bucket((int32_t)(y ^ ((uint32_t)vl * 0x9E3B5u)), kGroupLb);
         while (atomicCAS(&s_key[q], kNone, key) != kNone) q = (q + 1) & (kGroupSlots - 1);  // at most half full: ends
@@ -1136,9 +1340,9 @@ __global__ __launch_bounds__(BLOCK) void k_tri_wedge_wave(TriArgs a) {
   const int count = a.ctl->num_wave;
   AT* const gacc = W ? (AT*)a.accw : (AT*)a.accu;
   for (int li = blockIdx.x * NW + w; li < count; li += gridDim.x * NW) {
-    const int32_t r = a.list_wave[li], v = a.vtx[r];
-    const int4 vi = a.info[v];
-    const int d = a.dr[r], ov = vi.x, dpv = vi.y;
+    const int place = a.list_wave[li];
+    const int4 vi = a.rinfo[place];
+    const int d = a.dord[place], ov = vi.x, dpv = vi.y, r = vi.z, lr = vi.z - vi.w;
     const bool lds = dpv <= kWaveTab;
     const int lb = max(ceil_log2(2 * dpv), 4);
     const uint32_t mask = (1u << lb) - 1u;
@@ -1161,8 +1365,8 @@ __global__ __launch_bounds__(BLOCK) void k_tri_wedge_wave(TriArgs a) {
         if (e < 0) {
           const int4* const hd = reinterpret_cast<const int4*>(a.R16) + ~e;
           const int4 xi = hd[0];
-          if (r < kSat16)
-            p = find_rank16(reinterpret_cast<const uint16_t*>(hd + kHead), xi.y, (uint32_t)r, hd[1]);
+          if (lr < kSat16)
+            p = find_rank16(reinterpret_cast<const uint16_t*>(hd + kHead), xi.y, (uint32_t)lr, hd[1]);
           else
             p = find_rank(a.R32 + xi.x, xi.y, (uint32_t)r);
           if (p < 0) {
@@ -1586,7 +1790,9 @@ size_t carve(TriArgs& a, unsigned char* p, int32_t n, int64_t m, bool weighted) 
   a.wr = reinterpret_cast<float*>(weighted ? take(nn * 4) : nullptr);
   a.sr = reinterpret_cast<double*>(weighted ? take(nn * 8) : nullptr);
   a.info = reinterpret_cast<int4*>(take(nn * sizeof(int4)));
-  a.rinfo = reinterpret_cast<int2*>(take(nn * sizeof(int2)));
+  a.rinfo = reinterpret_cast<int4*>(take(nn * sizeof(int4)));
+  a.ord = reinterpret_cast<int32_t*>(take(nn * 4));
+  a.dord = reinterpret_cast<int32_t*>(take(nn * 4));
   a.R32 = reinterpret_cast<uint32_t*>(take((mm + 16) * 4));
   a.R16 = reinterpret_cast<uint16_t*>(take((size_t)(row16_line(mm, nn) + 1) * 128));
   a.emap = reinterpret_cast<int32_t*>(take(mm * 4));
@@ -1602,6 +1808,8 @@ size_t carve(TriArgs& a, unsigned char* p, int32_t n, int64_t m, bool weighted) 
   a.task[1] = reinterpret_cast<TriTask*>(take((size_t)a.task_cap * sizeof(TriTask)));
   a.list_wave = reinterpret_cast<int32_t*>(take(nn * 4));
   a.list_s16 = reinterpret_cast<int32_t*>(take(nn * 4));
+  a.starts = a.list_wave;  // (rank is done with them when plan runs)
+  a.parts = a.list_s16;
   a.list_s64 = a.list_mid;  // orient is done with its lists when plan runs
   a.list_red[0] = a.list_big;
   a.list_red[1] = reinterpret_cast<int32_t*>(take((size_t)std::min<int64_t>(nn, m / kRedWg + 1) * 4));
@@ -1618,10 +1826,19 @@ hipError_t tri_launch(const TriArgs& a, hipStream_t s) {
   {
     ProfScope ps("tri_rank", s);
     hipLaunchKernelGGL(k_tri_init, dim3(1), dim3(1024), 0, s, a.ctl);
-    const dim3 g = grid(a.n, PB * 4, 4);
+    const dim3 g = grid(a.n, PB * 4, kTriParts / 256);
+    static_assert(kTriParts % 256 == 0, "ranges");
     hipLaunchKernelGGL((k_tri_hist<W, PB>), g, dim3(PB), 0, s, a);
-    hipLaunchKernelGGL(k_tri_scan, dim3(1), dim3(kTriBuckets), 0, s, a.ctl);
+    hipLaunchKernelGGL(k_tri_scan, dim3(1), dim3(kTriBuckets), 0, s, a.ctl, a.grp_from);
     hipLaunchKernelGGL((k_tri_rank<W, PB>), g, dim3(PB), 0, s, a);
+    if (a.members) {
+      const dim3 gp((unsigned)std::min<int64_t>(g.x, kTriParts));
+      hipLaunchKernelGGL((k_tri_reach<PB>), gp, dim3(PB), 0, s, a);
+      hipLaunchKernelGGL(k_tri_reach_scan, dim3(1), dim3(kTriParts), 0, s, a.ctl, (int)gp.x);
+      hipLaunchKernelGGL((k_tri_starts<PB>), gp, dim3(PB), 0, s, a);
+      hipLaunchKernelGGL((k_tri_parts<PB>), gp, dim3(PB), 0, s, a);
+      hipLaunchKernelGGL((k_tri_rank_parts<W>), dim3(cus * 2), dim3(kTriBuckets), 0, s, a);
+    }
   }
   {
     ProfScope ps("tri_orient", s);
@@ -1675,6 +1892,13 @@ hipError_t run_tri(int mode, const EngineArgs& e, void* ws, const int** done, hi
   a.out32 = e.out32;
   a.ws32 = e.ws32;
   a.accumulate = e.accumulate;
+  a.members = e.members;
+  if (!a.members) {
+    a.ord = a.vtx;
+    a.dord = a.dr;
+  }
+  // (all parts' ranks are below kSat16)
+  a.grp_from = a.members ? e.n : kSat16;
   *done = &a.ctl->done;
   return weighted ? tri_launch<true>(a, s) : tri_launch<false>(a, s);
 }

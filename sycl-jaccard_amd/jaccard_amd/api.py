@@ -140,7 +140,7 @@ class JcTuning(ctypes.Structure):
     _fields_ = [("small_max", ctypes.c_int32), ("small_blocks_per_cu", ctypes.c_int32),
                 ("wide_index", ctypes.c_int32), ("bitmap_blocks_per_cu", ctypes.c_int32),
                 ("hash_table", ctypes.c_int32), ("quot_max_disp", ctypes.c_int32),
-                ("engine", ctypes.c_int32), ("reserved", ctypes.c_int32 * 1)]
+                ("engine", ctypes.c_int32), ("members", ctypes.c_int32)]
 
 
 ENGINE_OWNER = 1

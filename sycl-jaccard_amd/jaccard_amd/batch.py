@@ -103,8 +103,12 @@ JcTuning = api.JcTuning
 def _tuned(dg, weights, out, ws, tuning, stream):
     lib = load_jaccard_lib()
     g = dg.c_struct()
-    t = None if tuning is None else ctypes.byref(
-        JcTuning(small_max=tuning[0], small_blocks_per_cu=tuning[1], bitmap_blocks_per_cu=tuning[2]))
+    # members: from 2^22 stored edges on the oriented engine ranks every graph by
+    # itself (128 graphs, 4.4e7 stored edges in two unions: 5.66 ms by the owner
+    # engine, 4.66 by this). tuning is None only before autotune or select.
+    tuning = tuning or (0, 0, 0)
+    t = ctypes.byref(
+        JcTuning(small_max=tuning[0], small_blocks_per_cu=tuning[1], bitmap_blocks_per_cu=tuning[2], members=1))
     code = lib.jc_jaccard_tuned(ctypes.byref(g), None if weights is None else weights.data_ptr(), out.data_ptr(),
                                 1, api.FLAG_ASSUME_SYMMETRIC, ws.data_ptr(), ws.numel(), t, api._stream(stream))
     if code != 0:

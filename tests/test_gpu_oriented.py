@@ -82,17 +82,28 @@ GRAPHS = {
 }
 
 
-def run(dg, W, engine, device):
+def union(weighted):
+    """Small graphs side by side, ids without neighbours before, between and
+    after them, a part of two vertices, one of 9001."""
+    from jaccard_amd import batch
+    b = batch.rmat_batch([256, 2, 700, 9001, 300, 4096], [4.0, 1.0, 9.0, 12.0, 30.0, 16.0], [1, 2, 3, 4, 5, 6], weighted)
+    g = b.union
+    pad = 37
+    off = np.concatenate([np.zeros(pad, np.int32), g.offsets, np.full(5, g.offsets[-1], np.int32)])
+    return graphs.CSRGraph(g.n + pad + 5, off.astype(np.int32), (g.indices + pad).astype(np.int32))
+
+
+def run(dg, W, engine, device, members=0):
     """Result and, for the oriented engine, whether it delivered."""
     import torch
     n, m, weighted = dg.n, dg.m, W is not None
     need = api.workspace_size(n, min(m, 1 << 20), weighted, True) if m <= 1 << 20 else 0
     if engine == api.ENGINE_ORIENTED and need:
         ws = torch.zeros(need + 64 * m + 256 * n + (1 << 20), dtype=torch.uint8, device=device)
-        out = api.jaccard(dg, weights=W, workspace=ws, tuning=dict(engine=engine))
+        out = api.jaccard(dg, weights=W, workspace=ws, tuning=dict(engine=engine, members=members))
         done = int(ws[need + 4:need + 8].view(torch.int32))  # the engine's flag, second word of its area
         return out, done == 1
-    return api.jaccard(dg, weights=W, tuning=dict(engine=engine)), None
+    return api.jaccard(dg, weights=W, tuning=dict(engine=engine, members=members)), None
 
 
 def same(a, b):
@@ -122,6 +133,61 @@ def test_oriented_equals_owner_and_oracle(name, cuda):
         elif kind == "weighted":
             ref = oracle.weighted_f64(g, W.cpu().numpy().astype(np.float64))
             assert np.all(np.abs(host - ref) <= 1e-6 * np.abs(ref))
+
+
+# name: (graph, engine delivers with every part ranked by itself)
+MEMBERS = {
+    "union": (lambda: union(False), True),
+    "one_graph": (lambda: graphs.rmat(14, 16, seed=4), True),
+    "edgeless_tail": (lambda: graphs.from_edges(5000, [0, 1], [1, 2]), True),
+    "too_large_a_part": (lambda: cases.star(70000), False),
+    "asymmetric": (asymmetric, False),
+}
+
+
+@pytest.mark.parametrize("name", list(MEMBERS))
+def test_members(name, cuda):
+    make, delivers = MEMBERS[name]
+    g = make()
+    print(f"[gpu] oriented members {name} n={g.n} m={g.m}", flush=True)
+    dg = api.DeviceCSR.from_host(g, cuda)
+    import torch
+    for W in (None, torch.from_numpy(grid_weights(g.n, 7)).to(cuda)):
+        out, done = run(dg, W, api.ENGINE_ORIENTED, cuda, members=1)
+        assert done == delivers
+        assert same(out, run(dg, W, api.ENGINE_OWNER, cuda)[0])
+        if W is None:
+            assert np.array_equal(out.cpu().numpy().view(np.uint32), oracle.ec_unweighted(g).view(np.uint32))
+
+
+def test_kernel_level_intersection(cuda):
+    """jc_intersect from its size on: adds into weight_i, writes weight_s, the
+    same bits as below that size by the owner engine (a tuning the kernel-level
+    entry does not take, so a part of the graph is compared with the oracle)."""
+    import torch
+    g = graphs.rmat(18, 16, seed=12)
+    dg = api.DeviceCSR.from_host(g, cuda)
+    for weighted in (False, True):
+        v = torch.from_numpy(grid_weights(g.n, 2)).to(cuda) if weighted else None
+        work = torch.empty(g.n, dtype=torch.float32, device=cuda)
+        wi = torch.full((g.m,), 2.0, dtype=torch.float32, device=cuda)
+        ws = torch.empty(g.m, dtype=torch.float32, device=cuda)
+        api.rowsum(dg, work, v=v)
+        api.intersect(dg, work, wi, ws, v=v)
+        rows = np.repeat(np.arange(g.n), np.diff(g.offsets))
+        wk = work.cpu().numpy()
+        assert np.array_equal(ws.cpu().numpy(), wk[rows] + wk[g.indices])
+        # J = I / (S - I) gives I back: the oracle's quotients of the same edges
+        e = np.random.default_rng(1).choice(g.m, 20000, replace=False)
+        got = wi.cpu().numpy()[e].astype(np.float64) - 2.0
+        s = (wk[rows[e]].astype(np.float64) + wk[g.indices[e]])
+        if weighted:
+            J = oracle.pairs_weighted_f64(g, v.cpu().numpy().astype(np.float64), rows[e], g.indices[e])
+        else:
+            J = oracle.pairs_unweighted(g, rows[e], g.indices[e]).astype(np.float64)
+        I = J / (1.0 + J) * s
+        # fp32 row sums, quotient and 2 + I: a few roundings of 2^-24 of I + 2 and S J
+        assert np.all(np.abs(got - I) <= 8 * 2.0 ** -24 * (np.abs(I) + 2.0 + s * np.abs(J)))
 
 
 @pytest.mark.parametrize("name", ["wide", "negative", "infinite", "nan"])
