@@ -81,6 +81,12 @@ Layout layout(int32_t n, int32_t m, bool weighted, bool ec) {
 // (5.7M) 1.58 and 0.90, the kernel-level sequence on 150001 (4.3M) 1.26 and 0.77.
 constexpr int32_t kTriMinEdges = 1 << 22;
 
+// The one-launch kernel for graphs that fit the LDS, where the caller names
+// nothing of the owner engine.
+bool tiny_wanted(const jc_csr* g, bool weighted, const jc_tuning* t) {
+  return !t && jc::tiny_fits(g->n, g->m, weighted);
+}
+
 bool tri_wanted(const jc_csr* g, const jc_tuning* t) {
   if (t && (t->engine == JC_ENGINE_OWNER || t->wide_index || t->hash_table == 1 || t->quot_max_disp > 0)) return false;
   if (g->n > jc::kTriMaxN) return false;
@@ -124,10 +130,23 @@ int run_jaccard(const jc_csr* g, const float* vw, float* result, bool ec, unsign
     JC_TRY(jc::run_tri(weighted ? jc::kModeEcW : jc::kModeEcU, t, tri_ws, &a.skip, s));
   }
   double* S64 = weighted ? reinterpret_cast<double*>(ws + L.s64) : nullptr;
+  if (ec && !tri_ws) {
+    // one launch: the sentinels, the schedule's counters, the range facts
+    const bool ex = weighted && jc::rowsum_one_launch(g->m);
+    JC_TRY(jc::launch_prepare(fixup ? reinterpret_cast<uint32_t*>(result) : nullptr, g->m, jc::kSentinel32,
+                              reinterpret_cast<int*>(ws + L.engine), jc::engine_counter_words(),
+                              ex ? reinterpret_cast<jc::ExactInfo*>(ws + L.exact) : nullptr, s));
+    a.counters_ready = 1;
+  }
   if (weighted) {
     jc::ExactInfo* ex = reinterpret_cast<jc::ExactInfo*>(ws + L.exact);
-    JC_TRY(jc::launch_rowsum_f64(g->n, g->offsets, g->indices, vw, S64, ws + L.rows, s, a.skip));
-    JC_TRY(jc::launch_exact_info(g->n, vw, S64, ex, s, a.skip));
+    if (!tri_ws && jc::rowsum_one_launch(g->m)) {
+      if (!ec) JC_TRY(jc::launch_prepare(nullptr, 0, 0u, nullptr, 0, ex, s));
+      JC_TRY(jc::launch_rowsum_exact(g->n, g->offsets, g->indices, vw, S64, ex, s));
+    } else {
+      JC_TRY(jc::launch_rowsum_f64(g->n, g->m, g->offsets, g->indices, vw, S64, ws + L.rows, s, a.skip));
+      JC_TRY(jc::launch_exact_info(g->n, vw, S64, ex, s, a.skip));
+    }
     a.exact = ex;
   }
   a.S64 = S64;
@@ -135,7 +154,7 @@ int run_jaccard(const jc_csr* g, const float* vw, float* result, bool ec, unsign
     // (vertex-centric after the oriented engine: what that left is computed
     // by the fused pass, with the same bits)
     a.out32 = result;
-    if (fixup)
+    if (fixup && tri_ws)
       JC_TRY(jc::launch_fill_u32(reinterpret_cast<uint32_t*>(result), g->m, jc::kSentinel32, s, a.skip));
     JC_TRY(jc::run_engine(weighted ? jc::kModeEcW : jc::kModeEcU, weighted, a, ws + L.engine, fixup, s));
     return JC_OK;
@@ -153,7 +172,7 @@ int run_jaccard(const jc_csr* g, const float* vw, float* result, bool ec, unsign
   float* work = reinterpret_cast<float*>(ws + L.work32);
   float* wi = reinterpret_cast<float*>(ws + L.wi);
   float* wsum = reinterpret_cast<float*>(ws + L.ws);
-  JC_TRY(jc::launch_rowsum_f32(g->n, g->offsets, g->indices, nullptr, work, nullptr, s));
+  JC_TRY(jc::launch_rowsum_f32(g->n, g->m, g->offsets, g->indices, nullptr, work, nullptr, s));
   a.work32 = work;
   a.out32 = wi;
   a.ws32 = wsum;
@@ -219,9 +238,13 @@ int jc_jaccard_tuned(const jc_csr* g, const float* vertex_weights, float* result
   const size_t need = layout(g->n, g->m, weighted, ec).total;
   const size_t full = need + al(jc::tri_workspace_bytes(g->n, g->m, weighted));
   hipStream_t s = hs(stream);
+  if (workspace && workspace_bytes < need) return JC_ERR_WORKSPACE;
+  if (tiny_wanted(g, weighted, tuning)) {
+    JC_TRY(jc::run_tiny(g->n, g->m, g->offsets, g->indices, vertex_weights, result, s));
+    return JC_OK;
+  }
   bool tri = tri_wanted(g, tuning);
   if (workspace) {
-    if (workspace_bytes < need) return JC_ERR_WORKSPACE;
     unsigned char* ws = static_cast<unsigned char*>(workspace);
     return run_jaccard(g, vertex_weights, result, ec, flags, ws,
                        tri && workspace_bytes >= full ? ws + need : nullptr, tuning, s);
@@ -256,6 +279,10 @@ int jc_jaccard_noalloc(const jc_csr* g, const float* vertex_weights, float* resu
   const bool ec = edge_centric != 0;
   if (layout(g->n, g->m, vertex_weights != nullptr, ec).total > (size_t)JC_NOALLOC_SCRATCH_BYTES)
     return JC_ERR_SCRATCH_LIMIT;
+  if (tiny_wanted(g, vertex_weights != nullptr, nullptr)) {
+    JC_TRY(jc::run_tiny(g->n, g->m, g->offsets, g->indices, vertex_weights, result, hs(stream)));
+    return JC_OK;
+  }
   void* ws = nullptr;
   JC_TRY(scratch_address(&ws));
   // Every part of the workspace that must start at zero (schedule counters,
@@ -282,7 +309,7 @@ int jc_vertex_weights(const jc_csr* g, float* W, jc_stream_t stream) {
     JC_TRY(jc::launch_fill_f32(W, g->n, 0.0f, hs(stream)));
     return JC_OK;
   }
-  JC_TRY(jc::launch_vertex_weights(g->n, g->offsets, g->edge_w, W, nullptr, hs(stream)));
+  JC_TRY(jc::launch_vertex_weights(g->n, g->m, g->offsets, g->edge_w, W, nullptr, hs(stream)));
   return JC_OK;
 }
 
@@ -296,7 +323,7 @@ int jc_vertex_weights_ex(const jc_csr* g, float* W, void* workspace, size_t work
     JC_TRY(jc::launch_fill_f32(W, g->n, 0.0f, hs(stream)));
     return JC_OK;
   }
-  JC_TRY(jc::launch_vertex_weights(g->n, g->offsets, g->edge_w, W, workspace, hs(stream)));
+  JC_TRY(jc::launch_vertex_weights(g->n, g->m, g->offsets, g->edge_w, W, workspace, hs(stream)));
   return JC_OK;
 }
 
@@ -327,7 +354,7 @@ int jc_fill(int64_t n, float* x, float value, jc_stream_t stream) {
 int jc_rowsum(int32_t n, int32_t m, const int32_t* offsets, const int32_t* indices, const float* v,
               float* work, jc_stream_t stream) {
   if (n < 0 || m < 0 || (n > 0 && (!offsets || !work)) || (m > 0 && v && !indices)) return JC_ERR_INVALID_ARG;
-  JC_TRY(jc::launch_rowsum_f32(n, offsets, indices, v, work, nullptr, hs(stream)));
+  JC_TRY(jc::launch_rowsum_f32(n, m, offsets, indices, v, work, nullptr, hs(stream)));
   return JC_OK;
 }
 
@@ -411,7 +438,7 @@ int jc_weighted_sum_mode(const jc_csr* g, const float* vertex_weights, int* mode
   unsigned char* p = static_cast<unsigned char*>(buf.p);
   double* S64 = reinterpret_cast<double*>(p + rows_b);
   jc::ExactInfo* ex = reinterpret_cast<jc::ExactInfo*>(p + rows_b + s64_b);
-  JC_TRY(jc::launch_rowsum_f64(g->n, g->offsets, g->indices, vertex_weights, S64, p, s));
+  JC_TRY(jc::launch_rowsum_f64(g->n, g->m, g->offsets, g->indices, vertex_weights, S64, p, s));
   JC_TRY(jc::launch_exact_info(g->n, vertex_weights, S64, ex, s));
   jc::ExactInfo h{};
   JC_TRY(hipMemcpyAsync(&h, ex, sizeof(h), hipMemcpyDeviceToHost, s));

@@ -311,13 +311,195 @@ __global__ __launch_bounds__(BLOCK) void k_rowsum_w_long(const int32_t* __restri
   }
 }
 
+// Row sums of a small graph in one launch: the five launches of the way above
+// take 40 us however small the graph, this 6 to 8 (9001 vertices, 2.4e5
+// entries). Workgroup b takes the rows b, b + G, ... (consecutive rows would
+// put the hubs of RMAT-like graphs, ids with many trailing zeros, into one
+// workgroup), 64 at a time: rows up to kRowShort entries by 4 lanes each, up to
+// kOneWave by a wave, longer ones by the workgroup. EX: also the range facts
+// of v and the sums (k_exact_scan).
+constexpr int kOneWave = 1024;
+constexpr int64_t kOneMaxEdges = 1 << 21;  // above, hub rows outlast one workgroup
+
+__device__ __forceinline__ void exact_fact(float w, int& lsb, int& bad) {
+  const uint32_t b = __float_as_uint(w);
+  const uint32_t ex = (b >> 23) & 0xFFu, man = b & 0x7FFFFFu;
+  if ((b >> 31) && (b << 1)) bad = 1;  // negative (-0 is harmless)
+  if (ex == 0xFFu) {
+    bad = 1;
+  } else if (ex != 0 || man != 0) {
+    const uint32_t full = ex ? (man | 0x800000u) : man;
+    lsb = min(lsb, (ex ? (int)ex - 150 : -149) + __builtin_ctz(full));
+  }
+}
+
+__device__ __forceinline__ void exact_sum_fact(double sv, int& mx, int& bad) {
+  if (!(sv >= 0.0) || isinf(sv))
+    bad = 1;
+  else if (sv > 0.0)
+    mx = max(mx, ilogb(sv) + 1);
+}
+
+template <typename OutT, bool IDX, bool EX>
+__global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __restrict__ off,
+                                                    const int32_t* __restrict__ ind, const float* __restrict__ v,
+                                                    OutT* __restrict__ out, ExactInfo* info, const int* skip) {
+  if (skip && *skip) return;
+  constexpr int BLOCK = 256, NW = BLOCK / kWave, R = BLOCK / kRowGroup;
+  __shared__ int s_long[R], s_nlong;
+  __shared__ double part[2][NW];
+  __shared__ int s_r[3][NW];
+  const int tid = threadIdx.x, lane = lane_id(), w = tid / kWave, gl = lane % kRowGroup;
+  int lsb = INT32_MAX, mx = INT32_MIN, bad = 0;
+  auto put = [&](int32_t u, double sum) {
+    out[u] = (OutT)sum;
+    if constexpr (EX) exact_sum_fact(sum, mx, bad);
+  };
+  const int64_t G = gridDim.x;
+  for (int64_t i0 = 0; i0 * G + blockIdx.x < n; i0 += R) {
+    if (tid == 0) s_nlong = 0;
+    __syncthreads();
+    const int64_t ul = (i0 + tid / kRowGroup) * G + blockIdx.x;
+    const int32_t u = (int32_t)ul;
+    int o = 0, d = 0;
+    const bool live = ul < n;
+    if (live) {
+      o = off[u];
+      d = off[u + 1] - o;
+      if constexpr (EX) {
+        if (gl == 0) exact_fact(v[u], lsb, bad);
+      }
+    }
+    const int ds = live && d <= kRowShort ? d : 0;
+    DD2 acc{0.0, 0.0};
+    for (int p0 = o; p0 < o + ds; p0 += kRowGroup * kRowU) {
+      float x[kRowU];
+      gather_step<IDX, kRowU>(ind, v, p0, kRowGroup, gl, o + ds, x);
+#pragma unroll
+      for (int t = 0; t < kRowU; ++t) acc = add_d(acc, (double)x[t]);
+    }
+#pragma unroll
+    for (int sh = 1; sh < kRowGroup; sh <<= 1) acc = add_dd(acc, DD2{__shfl_xor(acc.hi, sh), __shfl_xor(acc.lo, sh)});
+    if (live && gl == 0) {
+      if (d <= kRowShort) put(u, acc.hi);
+      else s_long[atomicAdd(&s_nlong, 1)] = u;
+    }
+    __syncthreads();
+    const int nl = s_nlong;
+    for (int j = w; j < nl; j += NW) {
+      const int32_t q = s_long[j];
+      const int qo = off[q], qe = off[q + 1];
+      if (qe - qo > kOneWave) continue;
+      DD2 a2{0.0, 0.0};
+      for (int p0 = qo; p0 < qe; p0 += kWave * kRowU) {
+        float x[kRowU];
+        gather_step<IDX, kRowU>(ind, v, p0, kWave, lane, qe, x);
+#pragma unroll
+        for (int t = 0; t < kRowU; ++t) a2 = add_d(a2, (double)x[t]);
+      }
+#pragma unroll
+      for (int sh = 1; sh < kWave; sh <<= 1) a2 = add_dd(a2, DD2{__shfl_xor(a2.hi, sh), __shfl_xor(a2.lo, sh)});
+      if (lane == 0) put(q, a2.hi);
+    }
+    for (int j = 0; j < nl; ++j) {
+      const int32_t q = s_long[j];
+      const int qo = off[q], qe = off[q + 1];
+      if (qe - qo <= kOneWave) continue;  // uniform over the workgroup
+      DD2 a2{0.0, 0.0};
+      for (int p0 = qo; p0 < qe; p0 += BLOCK * kRowU) {
+        float x[kRowU];
+        gather_step<IDX, kRowU>(ind, v, p0, BLOCK, tid, qe, x);
+#pragma unroll
+        for (int t = 0; t < kRowU; ++t) a2 = add_d(a2, (double)x[t]);
+      }
+#pragma unroll
+      for (int sh = 1; sh < kWave; sh <<= 1) a2 = add_dd(a2, DD2{__shfl_xor(a2.hi, sh), __shfl_xor(a2.lo, sh)});
+      if (lane == 0) {
+        part[0][w] = a2.hi;
+        part[1][w] = a2.lo;
+      }
+      __syncthreads();
+      if (tid == 0) {
+        DD2 t{0.0, 0.0};
+        for (int k = 0; k < NW; ++k) t = add_dd(t, DD2{part[0][k], part[1][k]});
+        put(q, t.hi);
+      }
+      __syncthreads();
+    }
+    __syncthreads();  // the list is read before it is begun again
+  }
+  if constexpr (EX) {
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      lsb = min(lsb, __shfl_xor(lsb, o));
+      mx = max(mx, __shfl_xor(mx, o));
+      bad |= __shfl_xor(bad, o);
+    }
+    if (lane == 0) {
+      s_r[0][w] = lsb;
+      s_r[1][w] = mx;
+      s_r[2][w] = bad;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      for (int k = 1; k < NW; ++k) {
+        lsb = min(lsb, s_r[0][k]);
+        mx = max(mx, s_r[1][k]);
+        bad |= s_r[2][k];
+      }
+      if (lsb != INT32_MAX) atomicMin(&info->min_lsb, lsb);
+      if (mx != INT32_MIN) atomicMax(&info->max_exp, mx);
+      if (bad) atomicOr(&info->bad, 1);
+    }
+  }
+}
+
+int grid_one(int32_t n) { return grid_rows((n + 63) / 64, 1, 4); }
+
+bool rowsum_one_launch(int64_t m) { return m <= kOneMaxEdges; }
+
+hipError_t launch_rowsum_exact(int32_t n, const int32_t* off, const int32_t* ind, const float* v, double* S,
+                               ExactInfo* info, hipStream_t s) {
+  ProfScope ps_("rowsum", s);
+  hipLaunchKernelGGL((k_rowsum_one<double, true, true>), dim3(grid_one(n)), dim3(256), 0, s, n, off, ind, v, S, info,
+                     (const int*)nullptr);
+  return hipGetLastError();
+}
+
+// Sentinel fill of the result (when x is not null) and the start values of a
+// pass's counters and range facts, in one launch.
+__global__ void k_prepare(uint32_t* __restrict__ x, int64_t n, uint32_t v, int* __restrict__ z, int nz, ExactInfo* info) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (x)
+    for (int64_t i = t; i < n; i += (int64_t)gridDim.x * blockDim.x) x[i] = v;
+  if (blockIdx.x == 0) {
+    for (int i = threadIdx.x; i < nz; i += blockDim.x) z[i] = 0;
+    if (info && threadIdx.x == 0) *info = ExactInfo{INT32_MAX, INT32_MIN, 0, 0};
+  }
+}
+
+hipError_t launch_prepare(uint32_t* x, int64_t n, uint32_t v, int* zero, int nzero, ExactInfo* info, hipStream_t s) {
+  ProfScope ps_("fill", s);
+  hipLaunchKernelGGL(k_prepare, dim3(x ? grid_for(n, 256 * 4, 32) : 1), dim3(256), 0, s, x, n, v, zero, nzero, info);
+  return hipGetLastError();
+}
+
 size_t rowsum_scratch_bytes(int32_t n) { return ((size_t)std::max(n, 1) + 4) * sizeof(int); }
 
 // scratch: rowsum_scratch_bytes(n) bytes, or nullptr to use a stream-ordered
 // allocation for the call.
 template <typename OutT>
-static hipError_t rowsum_both(int32_t n, const int32_t* off, const int32_t* ind, const float* v, OutT* out,
+static hipError_t rowsum_both(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* v, OutT* out,
                               void* scratch, hipStream_t s, const int* skip = nullptr) {
+  if (rowsum_one_launch(m)) {
+    if (ind)
+      hipLaunchKernelGGL((k_rowsum_one<OutT, true, false>), dim3(grid_one(n)), dim3(256), 0, s, n, off, ind, v, out,
+                         (ExactInfo*)nullptr, skip);
+    else
+      hipLaunchKernelGGL((k_rowsum_one<OutT, false, false>), dim3(grid_one(n)), dim3(256), 0, s, n, off, ind, v, out,
+                         (ExactInfo*)nullptr, skip);
+    return hipGetLastError();
+  }
   void* own = nullptr;
   hipError_t err;
   if (!scratch) {
@@ -354,7 +536,7 @@ static hipError_t rowsum_both(int32_t n, const int32_t* off, const int32_t* ind,
   return err;
 }
 
-hipError_t launch_rowsum_f32(int32_t n, const int32_t* off, const int32_t* ind, const float* v,
+hipError_t launch_rowsum_f32(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* v,
                              float* work, void* scratch, hipStream_t s) {
   ProfScope ps_("rowsum", s);
   if (n <= 0) return hipSuccess;
@@ -362,21 +544,21 @@ hipError_t launch_rowsum_f32(int32_t n, const int32_t* off, const int32_t* ind, 
     hipLaunchKernelGGL(k_rowsum_deg, dim3(grid_for(n, 256, 32)), dim3(256), 0, s, n, off, work);
     return hipGetLastError();
   }
-  return rowsum_both<float>(n, off, ind, v, work, scratch, s);
+  return rowsum_both<float>(n, m, off, ind, v, work, scratch, s);
 }
 
-hipError_t launch_rowsum_f64(int32_t n, const int32_t* off, const int32_t* ind, const float* v,
+hipError_t launch_rowsum_f64(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* v,
                              double* S, void* scratch, hipStream_t s, const int* skip) {
   ProfScope ps_("rowsum", s);
   if (n <= 0) return hipSuccess;
-  return rowsum_both<double>(n, off, ind, v, S, scratch, s, skip);
+  return rowsum_both<double>(n, m, off, ind, v, S, scratch, s, skip);
 }
 
-hipError_t launch_vertex_weights(int32_t n, const int32_t* off, const float* edge_w, float* W,
+hipError_t launch_vertex_weights(int32_t n, int64_t m, const int32_t* off, const float* edge_w, float* W,
                                  void* scratch, hipStream_t s) {
   ProfScope ps_("vertex_weights", s);
   if (n <= 0) return hipSuccess;
-  return rowsum_both<float>(n, off, nullptr, edge_w, W, scratch, s);
+  return rowsum_both<float>(n, m, off, nullptr, edge_w, W, scratch, s);
 }
 
 // Jaccard weight: weight_j = Wi / (Ws - Wi) (jaccard.cpp:614-619).
@@ -533,20 +715,8 @@ __global__ __launch_bounds__(256) void k_exact_scan(int32_t n, const float* __re
   if (skip && *skip) return;
   int lsb = INT32_MAX, mx = INT32_MIN, bad = 0;
   for (int32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const uint32_t b = __float_as_uint(vw[i]);
-    const uint32_t ex = (b >> 23) & 0xFFu, man = b & 0x7FFFFFu;
-    if ((b >> 31) && (b << 1)) bad = 1;  // negative (-0 is harmless)
-    if (ex == 0xFFu) {
-      bad = 1;
-    } else if (ex != 0 || man != 0) {
-      const uint32_t full = ex ? (man | 0x800000u) : man;
-      lsb = min(lsb, (ex ? (int)ex - 150 : -149) + __builtin_ctz(full));
-    }
-    const double sv = S[i];
-    if (!(sv >= 0.0) || isinf(sv))
-      bad = 1;
-    else if (sv > 0.0)
-      mx = max(mx, ilogb(sv) + 1);
+    exact_fact(vw[i], lsb, bad);
+    exact_sum_fact(S[i], mx, bad);
   }
 #pragma unroll
   for (int o = 1; o < kWave; o <<= 1) {

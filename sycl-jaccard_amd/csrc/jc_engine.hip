@@ -12,6 +12,8 @@ extern template hipError_t run_engine_t<kModeIsF32, false>(const EngineArgs&, vo
 extern template hipError_t run_engine_t<kModeIsF32, true>(const EngineArgs&, void*, bool, hipStream_t);
 extern template hipError_t run_engine_t<kModeIsF64, true>(const EngineArgs&, void*, bool, hipStream_t);
 
+int engine_counter_words() { return (int)(sizeof(Sched) / sizeof(int)); }
+
 size_t engine_workspace_bytes(int32_t n, int64_t m) {
   size_t b = align_up(sizeof(Sched), 256);
   b += align_up((size_t)max_tasks(n, m) * sizeof(int2), 256);

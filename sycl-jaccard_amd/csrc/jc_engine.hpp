@@ -1462,8 +1462,12 @@ __global__ __launch_bounds__(BLOCK) void k_owner_block(EngineArgs a) {
   const int lane = lane_id();
   const int w = tid / kWave;
   const bool redo = KIND == 0 && a.redo_pass != 0;
-  const int ntasks = KIND == 1 ? a.num_tasks[1] : redo ? *a.num_redo : a.num_tasks[0];
+  // bitmap tasks: list 1 after list 0, or (task_cap) the one-pass schedule's
+  // longer rows from the front of the array and the others from its back
+  const bool one_pass = KIND == 1 && a.task_cap > 0;
+  const int ntasks = KIND == 1 ? a.num_tasks[1] + (one_pass ? a.num_tasks[0] : 0) : redo ? *a.num_redo : a.num_tasks[0];
   const int tbase = KIND == 1 ? a.num_tasks[0] : 0;
+  auto task_place = [&](int t) { return !one_pass ? tbase + t : t < tbase ? t : a.task_cap - 1 - (t - tbase); };
   int* const counter = &a.task_counter[KIND == 1 ? 1 : redo ? 2 : 0];
   const bool fast = exact_f64(a);
   if (kLook && tid == 0) {
@@ -1499,7 +1503,7 @@ __global__ __launch_bounds__(BLOCK) void k_owner_block(EngineArgs a) {
       hi0 = s_hdr[5];
       npieces = kQ ? s_hdr[6] : 1;  // bitmap tasks are one piece
     } else {
-      const int2 tk = a.tasks[tbase + (redo ? a.redo[t] : t)];
+      const int2 tk = a.tasks[KIND == 1 ? task_place(t) : redo ? a.redo[t] : t];
       u = tk.x;
       ou = a.off[u];
       du = a.off[u + 1] - ou;
@@ -1637,7 +1641,7 @@ __global__ __launch_bounds__(BLOCK) void k_owner_block(EngineArgs a) {
           if (lane == 0) tn = atomicAdd(counter, 1);
           tn = __shfl(tn, 0);
           if (tn < ntasks) {
-            const int2 tk2 = a.tasks[tbase + tn];
+            const int2 tk2 = a.tasks[task_place(tn)];
             const int ou2 = a.off[tk2.x];
             const int du2 = a.off[tk2.x + 1] - ou2;
             const int ka2 = ou2 + tk2.y * kTaskSpan;
@@ -2134,6 +2138,51 @@ __global__ __launch_bounds__(BLOCK) void k_sched_emit(int32_t rows, const int32_
   }
 }
 
+// The schedule in one launch, for graphs whose longer rows all take bitmaps
+// whatever their span: no table kind to count, so the small rows and two task
+// lists (rows above kLongRow entries from the front of the array, taken first;
+// the others from the back) are written as they are met, with one atomic per
+// list and workgroup. (The four launches of the counted schedule are 10 us.)
+constexpr int kLongRow = 512;
+
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_sched_one(int32_t rows, const int32_t* __restrict__ off, Sched* sc,
+                                                     int2* tasks, int32_t task_cap, int32_t* small_rows, int small_max,
+                                                     const int2* segs, int nseg, const int* skip) {
+  if (skip && *skip) return;
+  __shared__ int s_cnt[3], s_base[3];
+  for (int64_t b = (int64_t)blockIdx.x * BLOCK; b < rows; b += (int64_t)gridDim.x * BLOCK) {
+    if (threadIdx.x < 3) s_cnt[threadIdx.x] = 0;
+    __syncthreads();
+    const int64_t v = b + threadIdx.x;
+    int32_t u = 0;
+    int k = -1, c = 0, at = 0;
+    if (v < rows) {
+      u = seg_row(segs, nseg, (int32_t)v);
+      const int d = off[u + 1] - off[u];
+      if (d > 0) {
+        k = d <= small_max ? 2 : d > kLongRow ? 0 : 1;
+        c = k == 2 ? 1 : (d + kTaskSpan - 1) / kTaskSpan;
+        at = atomicAdd(&s_cnt[k], c);
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x < 3 && s_cnt[threadIdx.x])
+      s_base[threadIdx.x] =
+          atomicAdd(threadIdx.x == 2 ? &sc->num_small : &sc->num_tasks[threadIdx.x], s_cnt[threadIdx.x]);
+    __syncthreads();
+    if (k >= 0) {
+      at += s_base[k];
+      if (k == 2) {
+        small_rows[at] = u;
+      } else {
+        for (int p = 0; p < c; ++p) tasks[k == 0 ? at + p : task_cap - 1 - (at + p)] = make_int2(u, p);
+      }
+    }
+    __syncthreads();
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Host side.
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
@@ -2153,7 +2202,11 @@ hipError_t run_engine_t(const EngineArgs& base, void* ws, bool fixup, hipStream_
   if (a.nseg > 0 && fixup) return hipErrorInvalidValue;  // segments need a symmetric graph
   const int32_t rows = a.nseg > 0 ? a.seg_rows : a.n;
   const int64_t edges = a.nseg > 0 ? a.seg_edges : a.m;
-  if (a.small_max < 1 || a.small_max > kSmallMax) a.small_max = kSmallMax;
+  // one wave per row up to 128 entries where there are rows enough to fill the
+  // chip; small graphs end sooner with a workgroup per row above 32 (700
+  // vertices 57 -> 39 us, 9001 vertices 86 -> 71; RMAT-16, 1.8M entries, 262
+  // -> 297 the other way)
+  if (a.small_max < 1 || a.small_max > kSmallMax) a.small_max = edges <= (1 << 19) ? 32 : kSmallMax;
   if (a.small_blocks_per_cu < 1) a.small_blocks_per_cu = 16;
   // buffer-load offsets reach 4 * (m + 256) bytes
   if (a.m * 4 + 8192 > (int64_t)UINT32_MAX) a.wide_index = 1;
@@ -2178,8 +2231,10 @@ hipError_t run_engine_t(const EngineArgs& base, void* ws, bool fixup, hipStream_
 
   const int cus = device_cu_count();
   hipError_t err;
-  hipLaunchKernelGGL(k_sched_init, dim3(1), dim3(128), 0, stream, sc);
-  if ((err = hipGetLastError()) != hipSuccess) return err;
+  if (!a.counters_ready) {
+    hipLaunchKernelGGL(k_sched_init, dim3(1), dim3(128), 0, stream, sc);
+    if ((err = hipGetLastError()) != hipSuccess) return err;
+  }
   if (rows > 0) {
     const int g = std::min<int64_t>((rows + PB - 1) / PB, (int64_t)cus * 8);
     using Cfg = BlockCfg<W>;
@@ -2192,7 +2247,17 @@ hipError_t run_engine_t(const EngineArgs& base, void* ws, bool fixup, hipStream_
     a.bm_budget = (uint32_t)bm_budget;
     // hash-table rows up to one chunk of keys are whole-row tasks
     const int whole_max = quot ? Cfg::QCH : Cfg::CH;
-    {
+    // a row over all ids, as long as there are ids, still fits: no hash tasks,
+    // so neither their launches (5 us each, empty) nor the counted schedule
+    const bool bitmap_only = bitmap_fits<W>(0, a.n - 1, a.n, bm_budget) && max_tasks(rows, edges) <= INT32_MAX;
+    a.task_cap = bitmap_only ? (int32_t)max_tasks(rows, edges) : 0;
+    if (bitmap_only) {
+      ProfScope ps("sched", stream);
+      const int g1 = (int)std::min<int64_t>((rows + PB - 1) / PB, (int64_t)cus * 8);
+      hipLaunchKernelGGL((k_sched_one<PB>), dim3(g1), dim3(PB), 0, stream, rows, a.off, sc, tasks, a.task_cap, small,
+                         a.small_max, a.segs, a.nseg, a.skip);
+      if ((err = hipGetLastError()) != hipSuccess) return err;
+    } else {
       ProfScope ps("sched", stream);
       hipLaunchKernelGGL((k_sched_count<W, PB>), dim3(g), dim3(PB), 0, stream, rows, a.off, a.ind, sc, a.small_max,
                          bm_budget, whole_max, a.segs, a.nseg, a.skip);
@@ -2207,17 +2272,21 @@ hipError_t run_engine_t(const EngineArgs& base, void* ws, bool fixup, hipStream_
     // (quotient-table kernel first when n allows it, then the 32-bit kernel
     // over the tasks it could not hold, usually none)
     int occ0 = 0, occ1 = 0, occ2 = 0;
-    err = hipFuncSetAttribute(reinterpret_cast<const void*>(k_owner_block<MODE, W, BB, 0>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)Cfg::lds_bytes);
-    if (err != hipSuccess) return err;
+    if (!bitmap_only) {
+      err = hipFuncSetAttribute(reinterpret_cast<const void*>(k_owner_block<MODE, W, BB, 0>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)Cfg::lds_bytes);
+      if (err != hipSuccess) return err;
+    }
     err = hipFuncSetAttribute(reinterpret_cast<const void*>(k_owner_block<MODE, W, BB, 1>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds1);
     if (err != hipSuccess) return err;
-    err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ0, k_owner_block<MODE, W, BB, 0>, BB, Cfg::lds_bytes);
-    if (err != hipSuccess) return err;
+    if (!bitmap_only) {
+      err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ0, k_owner_block<MODE, W, BB, 0>, BB, Cfg::lds_bytes);
+      if (err != hipSuccess) return err;
+    }
     err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ1, k_owner_block<MODE, W, BB, 1>, BB, lds1);
     if (err != hipSuccess) return err;
-    if (quot) {
+    if (quot && !bitmap_only) {
       err = hipFuncSetAttribute(reinterpret_cast<const void*>(k_owner_block<MODE, W, BB, 2>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)Cfg::q_lds_bytes);
       if (err != hipSuccess) return err;
@@ -2226,11 +2295,12 @@ hipError_t run_engine_t(const EngineArgs& base, void* ws, bool fixup, hipStream_
       if (err != hipSuccess) return err;
       if (occ2 < 1) return hipErrorInvalidConfiguration;
     }
-    if (occ0 < 1 || occ1 < 1) return hipErrorInvalidConfiguration;
+    if ((!bitmap_only && occ0 < 1) || occ1 < 1) return hipErrorInvalidConfiguration;
     occ1 = std::min(occ1, bm_per_cu);
     {
       ProfScope ps("owner_block", stream);
-      if (quot) {
+      if (bitmap_only) {
+      } else if (quot) {
         hipLaunchKernelGGL((k_owner_block<MODE, W, BB, 2>), dim3(cus * occ2), dim3(BB), Cfg::q_lds_bytes, stream,
                            a);
         EngineArgs ar = a;

@@ -100,7 +100,15 @@ struct EngineArgs {
   // (the oriented engine delivered them) and the pass does nothing.
   const int* skip;
   int members;  // the graph is a union of many small graphs (oriented engine)
+  // The schedule counters at the head of the workspace are zero already
+  // (launch_prepare over engine_counter_words() words of it).
+  int counters_ready;
+  // Capacity of the task array when every task is a bitmap task and the list
+  // was written in one pass, longer rows from the front, the others from the
+  // back (set by the launcher; 0: two counted lists).
+  int32_t task_cap;
 };
+int engine_counter_words();
 
 // Oriented engine (jc_tri.hip): kModeEcU / kModeEcW (out32 the result) and
 // kModeIsF32. It delivers only where its conditions hold, which the device
@@ -144,12 +152,24 @@ hipError_t launch_fill_u64(uint64_t* x, int64_t n, uint64_t v, hipStream_t s, co
 // Row sums take a scratch area of rowsum_scratch_bytes(n) (long-row list),
 // or nullptr to allocate one on the stream for the call.
 size_t rowsum_scratch_bytes(int32_t n);
-hipError_t launch_rowsum_f32(int32_t n, const int32_t* off, const int32_t* ind, const float* v,
+hipError_t launch_rowsum_f32(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* v,
                              float* work, void* scratch, hipStream_t s);
-hipError_t launch_rowsum_f64(int32_t n, const int32_t* off, const int32_t* ind, const float* v,
+hipError_t launch_rowsum_f64(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* v,
                              double* S, void* scratch, hipStream_t s, const int* skip = nullptr);
-hipError_t launch_vertex_weights(int32_t n, const int32_t* off, const float* edge_w, float* W,
+hipError_t launch_vertex_weights(int32_t n, int64_t m, const int32_t* off, const float* edge_w, float* W,
                                  void* scratch, hipStream_t s);
+// Row sums of graphs of up to m stored edges are one launch, which can also
+// fill *info (as launch_exact_info, into a started ExactInfo: launch_prepare).
+bool rowsum_one_launch(int64_t m);
+hipError_t launch_rowsum_exact(int32_t n, const int32_t* off, const int32_t* ind, const float* v, double* S,
+                               ExactInfo* info, hipStream_t s);
+// x[0, n) = v (x may be nullptr), zero[0, nzero) = 0, *info (may be nullptr) started.
+hipError_t launch_prepare(uint32_t* x, int64_t n, uint32_t v, int* zero, int nzero, ExactInfo* info, hipStream_t s);
+// Everything in one launch for graphs whose CSR fits the LDS (jc_tiny.hip):
+// out as kModeEcU / kModeEcW. Any CSR, symmetric or not.
+bool tiny_fits(int32_t n, int64_t m, bool weighted);
+hipError_t run_tiny(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* vw, float* out,
+                    hipStream_t s);
 hipError_t launch_jw_f32(int64_t m, const float* wi, const float* ws, float* out, hipStream_t s);
 hipError_t launch_jw_f64(int64_t m, const double* wi, const double* ws, float* out, hipStream_t s);
 hipError_t launch_ec_scan(int32_t n, const int32_t* off, int32_t* dest, float* wj, hipStream_t s);

@@ -366,7 +366,7 @@ int jc_server_create(int32_t num_graphs, const jc_csr* graphs, const float* cons
     }
   }
   if (s->weighted && N > 0 &&
-      (e = jc::launch_rowsum_f64(s->N, s->off, s->ind, s->W, s->S64, nullptr, st)) != hipSuccess)
+      (e = jc::launch_rowsum_f64(s->N, s->M, s->off, s->ind, s->W, s->S64, nullptr, st)) != hipSuccess)
     return fail(e);
   if (s->weighted && (e = jc::launch_exact_info(s->N, s->W, s->S64, s->exact, st)) != hipSuccess) return fail(e);
   if ((e = hipStreamSynchronize(st)) != hipSuccess) return fail(e);
