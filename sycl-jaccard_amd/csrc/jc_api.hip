@@ -74,12 +74,15 @@ Layout layout(int32_t n, int32_t m, bool weighted, bool ec) {
   return L;
 }
 
-// Oriented engine (jc_tri.hip) before the owner engine: from kTriMinEdges
-// stored edges on, where no tuning is given or it names a batch. Measured:
-// RMAT-16 (1.8M entries) 0.27 ms by the owner engine, 0.40 by this one, whose
-// two dozen dependent launches are then most of it; RMAT of 200003 vertices
-// (5.7M) 1.58 and 0.90, the kernel-level sequence on 150001 (4.3M) 1.26 and 0.77.
-constexpr int32_t kTriMinEdges = 1 << 22;
+// Oriented engine (jc_tri.hip) before the owner engine: from tri_min_edges
+// stored entries on, where no tuning is given or it names a batch (and then
+// only if the device finds the rows skewed enough, see k_tri_scan). Below,
+// its two dozen dependent launches are most of its time. Owner and oriented
+// engine, ms: weighted RMAT 2.8M entries 0.54 / 0.55, 4.0M 0.96 / 0.69, 6.0M
+// 1.30 / 0.85, Chung-Lu 3.2M 0.47 / 0.66, 4.5M 1.07 / 0.76; unweighted RMAT
+// 5.8M 0.78 / 0.73, 9.2M 1.18 / 1.09, 11.7M 1.63 / 1.28, Chung-Lu 9.6M
+// 1.04 / 1.25, 12.8M 1.35 / 1.30, 25.6M 2.88 / 2.37.
+constexpr int32_t tri_min_edges(bool weighted) { return weighted ? 1 << 22 : 10 << 20; }
 
 // The one-launch kernel for graphs that fit the LDS, where the caller names
 // nothing of the owner engine.
@@ -87,10 +90,13 @@ bool tiny_wanted(const jc_csr* g, bool weighted, const jc_tuning* t) {
   return !t && jc::tiny_fits(g->n, g->m, weighted);
 }
 
-bool tri_wanted(const jc_csr* g, const jc_tuning* t) {
+bool tri_wanted(const jc_csr* g, bool weighted, const jc_tuning* t) {
   if (t && (t->engine == JC_ENGINE_OWNER || t->wide_index || t->hash_table == 1 || t->quot_max_disp > 0)) return false;
-  if (g->n > jc::kTriMaxN) return false;
-  return (t && t->engine == JC_ENGINE_ORIENTED) || ((!t || t->members) && g->m >= kTriMinEdges);
+  // (sum |R|^2 / 64 words of bit matrix are at least (m / 2)^2 / n / 64, above
+  // the engine's 4 m words from a mean row of 1024 entries on; a uniform
+  // random graph reaches them at 768)
+  if (g->n > jc::kTriMaxN || g->m > 768ll * g->n) return false;
+  return (t && t->engine == JC_ENGINE_ORIENTED) || ((!t || t->members) && g->m >= tri_min_edges(weighted));
 }
 
 // RAII for a stream-ordered allocation.
@@ -127,7 +133,7 @@ int run_jaccard(const jc_csr* g, const float* vw, float* result, bool ec, unsign
     jc::EngineArgs t = a;
     t.out32 = result;
     t.members = tuning ? tuning->members != 0 : 0;
-    JC_TRY(jc::run_tri(weighted ? jc::kModeEcW : jc::kModeEcU, t, tri_ws, &a.skip, s));
+    JC_TRY(jc::run_tri(weighted ? jc::kModeEcW : jc::kModeEcU, t, tuning && tuning->engine == JC_ENGINE_ORIENTED, tri_ws, &a.skip, s));
   }
   double* S64 = weighted ? reinterpret_cast<double*>(ws + L.s64) : nullptr;
   if (ec && !tri_ws) {
@@ -224,7 +230,7 @@ extern "C" {
 size_t jc_jaccard_workspace_size(int32_t n, int32_t m, int weighted, int edge_centric) {
   if (n < 0 || m < 0) return 0;
   size_t b = layout(n, m, weighted != 0, edge_centric != 0).total;
-  if (m >= kTriMinEdges) b += al(jc::tri_workspace_bytes(n, m, weighted != 0));
+  if (m >= tri_min_edges(weighted != 0)) b += al(jc::tri_workspace_bytes(n, m, weighted != 0));
   return b;
 }
 
@@ -243,7 +249,7 @@ int jc_jaccard_tuned(const jc_csr* g, const float* vertex_weights, float* result
     JC_TRY(jc::run_tiny(g->n, g->m, g->offsets, g->indices, vertex_weights, result, s));
     return JC_OK;
   }
-  bool tri = tri_wanted(g, tuning);
+  bool tri = tri_wanted(g, weighted, tuning);
   if (workspace) {
     unsigned char* ws = static_cast<unsigned char*>(workspace);
     return run_jaccard(g, vertex_weights, result, ec, flags, ws,
@@ -367,7 +373,7 @@ int jc_intersect(int32_t n, int32_t m, const int32_t* offsets, const int32_t* in
   const size_t need = al(jc::engine_workspace_bytes(n, m));
   AsyncBuf buf;
   buf.s = s;
-  bool tri = tri_wanted(&g, nullptr);
+  bool tri = tri_wanted(&g, v != nullptr, nullptr);
   if (tri && hipMallocAsync(&buf.p, need + jc::tri_workspace_bytes(n, m, v != nullptr), s) != hipSuccess) {
     (void)hipGetLastError();
     buf.p = nullptr;
@@ -387,7 +393,7 @@ int jc_intersect(int32_t n, int32_t m, const int32_t* offsets, const int32_t* in
   a.small_max = 0;
   a.small_blocks_per_cu = 0;
   if (tri)
-    JC_TRY(jc::run_tri(jc::kModeIsF32, a, static_cast<unsigned char*>(buf.p) + need, &a.skip, s));
+    JC_TRY(jc::run_tri(jc::kModeIsF32, a, false, static_cast<unsigned char*>(buf.p) + need, &a.skip, s));
   JC_TRY(jc::launch_fill_u32(reinterpret_cast<uint32_t*>(weight_s), m, jc::kSentinel32, s, a.skip));
   JC_TRY(jc::run_engine(jc::kModeIsF32, v != nullptr, a, buf.p, true, s));
   return JC_OK;

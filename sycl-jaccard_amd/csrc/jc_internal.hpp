@@ -114,10 +114,11 @@ int engine_counter_words();
 // kModeIsF32. It delivers only where its conditions hold, which the device
 // decides; *done then receives the address (in ws) of a flag that is set when
 // the results were written, for EngineArgs::skip of the owner engine that
-// must follow. ws holds tri_workspace_bytes(n, m, weighted) bytes.
+// must follow. ws holds tri_workspace_bytes(n, m, weighted) bytes. always: not
+// only where the rows say that it is the faster engine.
 constexpr int32_t kTriMaxN = 1 << 26;  // its hash keys hold 26-bit ranks
 size_t tri_workspace_bytes(int32_t n, int64_t m, bool weighted);
-hipError_t run_tri(int mode, const EngineArgs& base, void* ws, const int** done, hipStream_t s);
+hipError_t run_tri(int mode, const EngineArgs& base, bool always, void* ws, const int** done, hipStream_t s);
 
 // Workspace needed by an owner-engine pass over a graph with n vertices and m
 // stored edges (task list, small-row list, counters). With row segments, n and

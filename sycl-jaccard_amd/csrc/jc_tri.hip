@@ -54,6 +54,8 @@ namespace jc {
 namespace {
 
 constexpr int kTriBuckets = 1024;
+constexpr int kSamples = 1024;     // entries looked at before the engine is chosen
+constexpr int kSampleCap = 512;
 constexpr int kTriParts = 1024;    // vertex ranges of the rank kernels, at most
 constexpr int kPartMax = 65536;    // vertices of a disjoint part
 constexpr int kTriMaxOut = 4096;   // largest |R(u)|: the sort and reduce buffers in LDS
@@ -111,6 +113,8 @@ struct TriCtl {
   int bad;
   int done;
   int lsb, maxexp;               // exactness of the weights (see ExactInfo)
+  int wexp;                      // every weight is below 2^wexp
+  unsigned long long sampled;    // min(d_u, d_x, kSampleCap) over kSamples entries (u, x)
   unsigned long long out_total;  // sum of |R(u)|
   unsigned long long bits;       // words of the bit matrix handed out
   int num_big;                   // rows oriented by a workgroup
@@ -144,6 +148,7 @@ struct TriArgs {
   int32_t* dr;      // per rank: degree
   int32_t* ord;     // vertices and their degrees by descending degree bucket: vtx
   int32_t* dord;    // and dr, but for disjoint parts, whose ranks are in id order
+  int always;       // whatever the rows' lengths
   int members;      // rank disjoint parts by themselves
   int32_t grp_from; // place in ord from which longer rows than kWgMinDeg are taken in groups too
   int32_t* starts;  // first vertices of the parts: per vertex range, then
@@ -191,19 +196,44 @@ __global__ void k_tri_init(TriCtl* c) {
   if (threadIdx.x == 0) {
     c->lsb = INT32_MAX;
     c->maxexp = INT32_MIN;
+    c->wexp = INT32_MIN;
   }
 }
 
 // Degree histogram over each workgroup's contiguous range of vertices, and
-// the finest set bit of the weights.
+// the finest and the highest bit of the weights. The first kSamples / BLOCK
+// workgroups look at one entry (u, x) per thread instead: for its mirror, so
+// that most graphs that are not symmetric are refused before the work of
+// orient, and at the shorter row's length, what the owner engine streams.
 template <bool W, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_tri_hist(TriArgs a) {
   __shared__ int h[kTriBuckets];
+  constexpr int kLook = kSamples / BLOCK;
+  if (blockIdx.x < kLook) {
+    const int32_t t = blockIdx.x * BLOCK + threadIdx.x;
+    // one in each of kSamples equal runs of entries
+    const int64_t k = min(a.m - 1, (t * a.m + (int64_t)((t * 0x9E3779B1u) >> 22) * a.m / 1024) / kSamples);
+    int lo = 0, hi = a.n;  // off[lo] <= k < off[hi]
+    while (hi - lo > 1) {
+      const int mid = (int)(((uint32_t)lo + (uint32_t)hi) >> 1);
+      if (a.off[mid] <= k) lo = mid;
+      else hi = mid;
+    }
+    const int32_t x = a.ind[k];
+    const int b = a.off[x], e = a.off[x + 1], at = lane_lower_bound(a.ind, b, e, lo);
+    if (at >= e || a.ind[at] != lo) a.ctl->bad = 1;
+    int len = min(min(a.off[lo + 1] - a.off[lo], e - b), kSampleCap);
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) len += __shfl_xor(len, o);
+    if (lane_id() == 0) atomicAdd(&a.ctl->sampled, (unsigned long long)len);
+    return;
+  }
+  const int ranges = gridDim.x - kLook, range = blockIdx.x - kLook;
   for (int i = threadIdx.x; i < kTriBuckets; i += BLOCK) h[i] = 0;
   __syncthreads();
-  const int64_t per = ((int64_t)a.n + gridDim.x - 1) / gridDim.x;
-  const int32_t r0 = (int32_t)min(per * blockIdx.x, (int64_t)a.n), r1 = (int32_t)min(per * (blockIdx.x + 1), (int64_t)a.n);
-  int lsb = INT32_MAX;
+  const int64_t per = ((int64_t)a.n + ranges - 1) / ranges;
+  const int32_t r0 = (int32_t)min(per * range, (int64_t)a.n), r1 = (int32_t)min(per * (range + 1), (int64_t)a.n);
+  int lsb = INT32_MAX, top = INT32_MIN;
   bool bad = false;
   for (int32_t u = r0 + threadIdx.x; u < r1; u += BLOCK) {
     const int d = a.off[u + 1] - a.off[u];
@@ -212,14 +242,21 @@ __global__ __launch_bounds__(BLOCK) void k_tri_hist(TriArgs a) {
       const uint32_t b = __float_as_uint(a.vw[u]);
       const uint32_t ex = (b >> 23) & 0xFFu, man = b & 0x7FFFFFu;
       if (((b >> 31) && (b << 1)) || ex == 0xFFu) bad = true;  // negative or not finite (-0 is harmless)
-      else if (ex != 0 || man != 0) lsb = min(lsb, (ex ? (int)ex - 150 : -149) + (int)__builtin_ctz(ex ? (man | 0x800000u) : man));
+      else if (ex != 0 || man != 0) {
+        lsb = min(lsb, (ex ? (int)ex - 150 : -149) + (int)__builtin_ctz(ex ? (man | 0x800000u) : man));
+        top = max(top, max((int)ex, 1) - 126);
+      }
     }
   }
   if constexpr (W) {
 #pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) lsb = min(lsb, __shfl_xor(lsb, o));
+    for (int o = 1; o < kWave; o <<= 1) {
+      lsb = min(lsb, __shfl_xor(lsb, o));
+      top = max(top, __shfl_xor(top, o));
+    }
     if (ballot(bad) && lane_id() == 0) atomicOr(&a.ctl->bad, 1);
     if (lane_id() == 0 && lsb < *(volatile int*)&a.ctl->lsb) atomicMin(&a.ctl->lsb, lsb);
+    if (lane_id() == 0 && top > *(volatile int*)&a.ctl->wexp) atomicMax(&a.ctl->wexp, top);
   }
   __syncthreads();
   for (int i = threadIdx.x; i < kTriBuckets; i += BLOCK)
@@ -229,10 +266,24 @@ __global__ __launch_bounds__(BLOCK) void k_tri_hist(TriArgs a) {
 // Vertices of degree d in a group task of wedge.
 __device__ __forceinline__ int group_rows(int d) { return min(kGroupRows, kWedgeB / d); }
 
-// First rank of every bucket, largest degrees first.
-__global__ __launch_bounds__(kTriBuckets) void k_tri_scan(TriCtl* c, int grp_from) {
+// First rank of every bucket, largest degrees first; and whether to go on.
+// With len the mean of min(d_u, d_x, 512) over the entries and d the mean
+// degree, the engine is the faster one where len is well above d (few hubs on
+// most edges), or rows are long in any case. Owner / oriented engine, ms,
+// weighted: RMAT len 85..230, d 6..54: 1.3 to 2.2 times as fast; Chung-Lu len
+// 53..206, d 6..64: 1.4 to 2.2 times; uniform random graphs d = len = 16 1.44
+// / 1.99, 37 0.99 / 1.39, 63 0.99 / 1.21, 76 1.77 / 1.78, 154 3.88 / 2.06;
+// neighbours on a ring 24 1.56 / 2.50, 72 3.68 / 3.54, 196 3.62 / 2.15.
+// Giving up here costs 0.05 ms.
+__global__ __launch_bounds__(kTriBuckets) void k_tri_scan(TriCtl* c, int32_t n, int64_t m, int always, int grp_from) {
   __shared__ int part[kTriBuckets / kWave];
   const int b = kTriBuckets - 1 - threadIdx.x;
+  // a weight that alone is wider than fp64 sums can hold
+  if (b == 0 && c->lsb != INT32_MAX && c->wexp - c->lsb > 53) c->bad = 1;
+  if (b == 0 && !always) {
+    const float len = (float)c->sampled / kSamples, d = (float)m / (float)n;
+    if (len < 48.f || (len < 96.f && len < 1.5f * d)) c->bad = 1;
+  }
   const int v = c->hist[b];
   int incl = v;
 #pragma unroll
@@ -550,8 +601,9 @@ __device__ __forceinline__ void orient_group(const TriArgs& a, bool valid, int32
   if (in_row) {
     x = a.ind[o + gl];
     rw = a.rw[x];
-    if (x == u || (gl > 0 && a.ind[o + gl - 1] >= x)) a.ctl->bad = 1;  // a self loop; a row out of order
   }
+  const int32_t before = __shfl_up(x, 1);
+  if (in_row && (x == u || (gl > 0 && before >= x))) a.ctl->bad = 1;  // a self loop; a row out of order
   const bool keep = in_row && rw.x < ru;
   const uint64_t km = ballot(keep);
   // kept ranks below mine: a lane that keeps nothing offers no rank
@@ -1828,8 +1880,8 @@ hipError_t tri_launch(const TriArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(k_tri_init, dim3(1), dim3(1024), 0, s, a.ctl);
     const dim3 g = grid(a.n, PB * 4, kTriParts / 256);
     static_assert(kTriParts % 256 == 0, "ranges");
-    hipLaunchKernelGGL((k_tri_hist<W, PB>), g, dim3(PB), 0, s, a);
-    hipLaunchKernelGGL(k_tri_scan, dim3(1), dim3(kTriBuckets), 0, s, a.ctl, a.grp_from);
+    hipLaunchKernelGGL((k_tri_hist<W, PB>), dim3(g.x + kSamples / PB), dim3(PB), 0, s, a);
+    hipLaunchKernelGGL(k_tri_scan, dim3(1), dim3(kTriBuckets), 0, s, a.ctl, a.n, a.m, a.always, a.grp_from);
     hipLaunchKernelGGL((k_tri_rank<W, PB>), g, dim3(PB), 0, s, a);
     if (a.members) {
       const dim3 gp((unsigned)std::min<int64_t>(g.x, kTriParts));
@@ -1878,7 +1930,7 @@ size_t tri_workspace_bytes(int32_t n, int64_t m, bool weighted) {
   return carve(a, nullptr, n, m, weighted);
 }
 
-hipError_t run_tri(int mode, const EngineArgs& e, void* ws, const int** done, hipStream_t s) {
+hipError_t run_tri(int mode, const EngineArgs& e, bool always, void* ws, const int** done, hipStream_t s) {
   TriArgs a{};
   const bool weighted = e.vw != nullptr;
   carve(a, static_cast<unsigned char*>(ws), e.n, e.m, weighted);
@@ -1893,6 +1945,7 @@ hipError_t run_tri(int mode, const EngineArgs& e, void* ws, const int** done, hi
   a.ws32 = e.ws32;
   a.accumulate = e.accumulate;
   a.members = e.members;
+  a.always = always;
   if (!a.members) {
     a.ord = a.vtx;
     a.dord = a.dr;
