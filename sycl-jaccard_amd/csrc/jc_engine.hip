@@ -1,5 +1,4 @@
-// Owner engine: dispatch over the result modes, workspace size and the pair
-// path. The kernels and the launch sequence are in jc_engine.hpp; each
+// Owner engine: dispatch over the result modes and workspace size. The kernels and the launch sequence are in jc_engine.hpp; each
 // result mode is instantiated in a translation unit of its own
 // (jc_engine_<mode>.hip), so the instantiations compile in parallel.
 #include "jc_engine.hpp"
@@ -87,79 +86,6 @@ hipError_t launch_degree_stats(int32_t n, const int32_t* off, const int32_t* ind
   const size_t bud_u = BlockCfg<false>::bm_budget1, bud_w = BlockCfg<true>::bm_budget1;
   const int g = (int)std::min<int64_t>((n + B - 1) / B, (int64_t)device_cu_count() * 8);
   hipLaunchKernelGGL((k_degree_stats<B>), dim3(g), dim3(B), 0, stream, n, off, ind, bud_u, bud_w, out);
-  return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// Pair list: one wave per pair.
-template <int MODE, bool W, int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_pairs(int32_t n, const int32_t* __restrict__ off,
-                                                 const int32_t* __restrict__ ind,
-                                                 const float* __restrict__ vw,
-                                                 const float* __restrict__ work32, int64_t np,
-                                                 const int32_t* __restrict__ first,
-                                                 const int32_t* __restrict__ second, float* out32,
-                                                 float* ws32, int accumulate) {
-  const int64_t nwaves = (int64_t)gridDim.x * (BLOCK / kWave);
-  for (int64_t i = (int64_t)blockIdx.x * (BLOCK / kWave) + threadIdx.x / kWave; i < np; i += nwaves) {
-    const int32_t pa = first[i], pb = second[i];
-    if (pa < 0 || pa >= n || pb < 0 || pb >= n) {
-      if (lane_id() == 0) {
-        out32[i] = __int_as_float(0x7fc00000);
-        if (MODE == kModeIsF32) ws32[i] = __int_as_float(0x7fc00000);
-      }
-      continue;
-    }
-    uint32_t cnt;
-    DD acc;
-    wave_pair<W>(off, ind, vw, pa, pb, cnt, acc);
-    if constexpr (MODE == kModeEcU) {
-      if (lane_id() == 0) {
-        const int da = off[pa + 1] - off[pa], db = off[pb + 1] - off[pb];
-        const float fI = (float)cnt;
-        out32[i] = fI / ((float)(da + db) - fI);
-      }
-    } else if constexpr (MODE == kModeEcW) {
-      const double sa = wave_row_wsum(off, ind, vw, pa);
-      const double sb = wave_row_wsum(off, ind, vw, pb);
-      if (lane_id() == 0) out32[i] = (float)(acc.hi / ((sa + sb) - acc.hi));
-    } else {
-      if (lane_id() == 0) {
-        const float add = W ? (float)acc.hi : (float)cnt;
-        out32[i] = (accumulate ? out32[i] : 0.0f) + add;
-        ws32[i] = work32[pa] + work32[pb];
-      }
-    }
-  }
-}
-
-hipError_t run_pairs(int mode, bool weighted, int32_t n, const int32_t* off, const int32_t* ind,
-                     const float* vw, const float* work32, int64_t np, const int32_t* first,
-                     const int32_t* second, float* out32, float* ws32, int accumulate,
-                     hipStream_t stream) {
-  if (np <= 0) return hipSuccess;
-  constexpr int B = 256;
-  const int g = (int)std::min<int64_t>((np + (B / kWave) - 1) / (B / kWave), (int64_t)device_cu_count() * 16);
-  ProfScope ps("pairs", stream);
-  switch (mode) {
-    case kModeEcU:
-      hipLaunchKernelGGL((k_pairs<kModeEcU, false, B>), dim3(g), dim3(B), 0, stream, n, off, ind, vw,
-                         work32, np, first, second, out32, ws32, accumulate);
-      break;
-    case kModeEcW:
-      hipLaunchKernelGGL((k_pairs<kModeEcW, true, B>), dim3(g), dim3(B), 0, stream, n, off, ind, vw,
-                         work32, np, first, second, out32, ws32, accumulate);
-      break;
-    case kModeIsF32:
-      if (weighted)
-        hipLaunchKernelGGL((k_pairs<kModeIsF32, true, B>), dim3(g), dim3(B), 0, stream, n, off, ind,
-                           vw, work32, np, first, second, out32, ws32, accumulate);
-      else
-        hipLaunchKernelGGL((k_pairs<kModeIsF32, false, B>), dim3(g), dim3(B), 0, stream, n, off, ind,
-                           vw, work32, np, first, second, out32, ws32, accumulate);
-      break;
-    default: return hipErrorInvalidValue;
-  }
   return hipGetLastError();
 }
 

@@ -1869,7 +1869,7 @@ __global__ __launch_bounds__(BLOCK) void k_owner_block(EngineArgs a) {
 // ---------------------------------------------------------------------------
 // Generic pair routine (one wave): intersection of N(a) and N(b) by per-lane
 // binary search of the shorter row's elements in the longer row. Used by the
-// fix-up pass and the pair-list path.
+// fix-up pass.
 template <bool W>
 __device__ __forceinline__ void wave_pair(const int32_t* __restrict__ off, const int32_t* __restrict__ ind,
                                           const float* __restrict__ vw, int32_t pa, int32_t pb,
@@ -1900,19 +1900,6 @@ __device__ __forceinline__ void wave_pair(const int32_t* __restrict__ off, const
     }
   }
   if constexpr (W) acc = wave_sum_dd(acc);
-}
-
-// Exact row sum of vw over N(r), one wave.
-__device__ __forceinline__ double wave_row_wsum(const int32_t* __restrict__ off,
-                                                const int32_t* __restrict__ ind,
-                                                const float* __restrict__ vw, int32_t r) {
-  DD acc{0.0, 0.0};
-  const int o = off[r], d = off[r + 1] - o;
-  for (int p0 = o; p0 < o + d; p0 += kWave) {
-    const int p = p0 + lane_id();
-    if (p < o + d) acc = dd_add1(acc, (double)vw[ind[p]]);
-  }
-  return wave_sum_dd(acc).hi;
 }
 
 template <bool W64>

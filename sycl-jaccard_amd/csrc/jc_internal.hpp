@@ -132,9 +132,10 @@ size_t engine_workspace_bytes(int32_t n, int64_t m);
 hipError_t run_engine(int mode, bool weighted, const EngineArgs& base, void* ws, bool fixup,
                       hipStream_t stream);
 
-// Pair path: out per (first[i], second[i]); invalid ids give NaN.
+// Pair path: out per (first[i], second[i]); invalid ids give NaN. S: the row
+// sums of vw, or nullptr (kModeEcW then sums the rows of each pair).
 hipError_t run_pairs(int mode, bool weighted, int32_t n, const int32_t* off, const int32_t* ind,
-                     const float* vw, const float* work32, int64_t np, const int32_t* first,
+                     const float* vw, const float* work32, const double* S, int64_t np, const int32_t* first,
                      const int32_t* second, float* out32, float* ws32, int accumulate,
                      hipStream_t stream);
 

@@ -550,7 +550,7 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
       e = jc::run_engine(mode, s->weighted, a, dev + L.ws, false, st);
     }
     if (e == hipSuccess && K > 0)
-      e = jc::run_pairs(mode, s->weighted, s->N, s->off, s->ind, s->W, nullptr, K,
+      e = jc::run_pairs(mode, s->weighted, s->N, s->off, s->ind, s->W, nullptr, s->S64, K,
                         reinterpret_cast<const int32_t*>(dev + L.first), reinterpret_cast<const int32_t*>(dev + L.second),
                         reinterpret_cast<float*>(dev + L.pout), nullptr, 0, st);
     if (e == hipSuccess && maxcount > 0) {
