@@ -84,3 +84,27 @@ def test_empty_and_errors(cuda):
     with pytest.raises(api.JaccardError) as ex:
         api.csr_from_edges(10, bad, ok)
     assert ex.value.code == api.ERR_INVALID_ARG
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 255, 256, 257, 65535, 65536, 65537, 1 << 20, (1 << 20) + 1])
+@pytest.mark.parametrize("e", [1, 4095, 4096, 4097, 8192, 30001])
+def test_key_widths_and_tiles(n, e, cuda):
+    """32- and 64-bit keys around powers of two of n, whole and ragged tiles of
+    the compaction, edges of the first and last vertices, repeats across tiles."""
+    rng = np.random.default_rng(n + e)
+    s = rng.integers(0, n, e).astype(np.int32)
+    d = rng.integers(0, n, e).astype(np.int32)
+    s[: e // 4], d[: e // 4] = n - 1, max(n - 2, 0)  # one edge, many times
+    d[e // 4: e // 3] = s[e // 4: e // 3]            # self loops
+    s[-1], d[-1] = 0, n - 1
+    w = rng.random(e).astype(np.float32)
+    print(f"[gpu] ingest n={n} e={e}", flush=True)
+    for sym in (False, True):
+        g = api.csr_from_edges(n, dev(s, cuda), dev(d, cuda), dev(w, cuda), symmetrize=sym)
+        want = graphs.from_edges(n, s, d, symmetrize=sym)
+        assert np.array_equal(g.offsets.cpu().numpy(), want.offsets)
+        assert np.array_equal(g.indices.cpu().numpy(), want.indices)
+        ss, dd, ww = (np.r_[s, d], np.r_[d, s], np.r_[w, w]) if sym else (s, d, w)
+        keep = ss != dd
+        _, first = np.unique(ss[keep].astype(np.int64) * n + dd[keep], return_index=True)
+        assert np.array_equal(g.edge_w.cpu().numpy(), ww[keep][first])
