@@ -151,19 +151,19 @@ int run_jaccard(const jc_csr* g, const float* vw, float* result, bool ec, unsign
     JC_TRY(jc::run_tri(weighted ? jc::kModeEcW : jc::kModeEcU, t, tuning && tuning->engine == JC_ENGINE_ORIENTED, tri_ws, &a.skip, s));
   }
   double* S64 = weighted ? reinterpret_cast<double*>(ws + L.s64) : nullptr;
-  if (ec && !tri_ws) {
+  if (ec || tri_ws) {
     // one launch: the sentinels, the schedule's counters, the range facts
     const bool ex = weighted && jc::rowsum_one_launch(g->m);
     JC_TRY(jc::launch_prepare(fixup ? reinterpret_cast<uint32_t*>(result) : nullptr, g->m, jc::kSentinel32,
                               reinterpret_cast<int*>(ws + L.engine), jc::engine_counter_words(),
-                              ex ? reinterpret_cast<jc::ExactInfo*>(ws + L.exact) : nullptr, s));
+                              ex ? reinterpret_cast<jc::ExactInfo*>(ws + L.exact) : nullptr, s, a.skip));
     a.counters_ready = 1;
   }
   if (weighted) {
     jc::ExactInfo* ex = reinterpret_cast<jc::ExactInfo*>(ws + L.exact);
-    if (!tri_ws && jc::rowsum_one_launch(g->m)) {
-      if (!ec) JC_TRY(jc::launch_prepare(nullptr, 0, 0u, nullptr, 0, ex, s));
-      JC_TRY(jc::launch_rowsum_exact(g->n, g->offsets, g->indices, vw, S64, ex, s));
+    if (jc::rowsum_one_launch(g->m)) {
+      if (!ec && !tri_ws) JC_TRY(jc::launch_prepare(nullptr, 0, 0u, nullptr, 0, ex, s));
+      JC_TRY(jc::launch_rowsum_exact(g->n, g->offsets, g->indices, vw, S64, ex, s, a.skip));
     } else {
       JC_TRY(jc::launch_rowsum_f64(g->n, g->m, g->offsets, g->indices, vw, S64, ws + L.rows, s, a.skip));
       JC_TRY(jc::launch_exact_info(g->n, vw, S64, ex, s, a.skip));
@@ -175,8 +175,6 @@ int run_jaccard(const jc_csr* g, const float* vw, float* result, bool ec, unsign
     // (vertex-centric after the oriented engine: what that left is computed
     // by the fused pass, with the same bits)
     a.out32 = result;
-    if (fixup && tri_ws)
-      JC_TRY(jc::launch_fill_u32(reinterpret_cast<uint32_t*>(result), g->m, jc::kSentinel32, s, a.skip));
     JC_TRY(jc::run_engine(weighted ? jc::kModeEcW : jc::kModeEcU, weighted, a, ws + L.engine, fixup, s));
     return JC_OK;
   }
@@ -423,7 +421,9 @@ int jc_intersect(int32_t n, int32_t m, const int32_t* offsets, const int32_t* in
   a.small_blocks_per_cu = 0;
   if (tri)
     JC_TRY(jc::run_tri(jc::kModeIsF32, a, false, static_cast<unsigned char*>(buf.p) + need, &a.skip, s));
-  JC_TRY(jc::launch_fill_u32(reinterpret_cast<uint32_t*>(weight_s), m, jc::kSentinel32, s, a.skip));
+  JC_TRY(jc::launch_prepare(reinterpret_cast<uint32_t*>(weight_s), m, jc::kSentinel32, static_cast<int*>(buf.p),
+                            jc::engine_counter_words(), nullptr, s, a.skip));
+  a.counters_ready = 1;
   JC_TRY(jc::run_engine(jc::kModeIsF32, v != nullptr, a, buf.p, true, s));
   return JC_OK;
 }

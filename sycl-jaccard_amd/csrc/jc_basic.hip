@@ -11,6 +11,9 @@
 // and reduced with an xor butterfly (double-double, exact for fp32 addends of
 // moderate dynamic range) instead of the reference's LDS-emulated 32-lane
 // shuffle scan with two barriers per step.
+#include <algorithm>
+#include <numeric>
+
 #include "jc_device.hpp"
 #include "jc_internal.hpp"
 #include "jc_profile.hpp"
@@ -311,15 +314,21 @@ __global__ __launch_bounds__(BLOCK) void k_rowsum_w_long(const int32_t* __restri
   }
 }
 
-// Row sums of a small graph in one launch: the five launches of the way above
-// take 40 us however small the graph, this 6 to 8 (9001 vertices, 2.4e5
-// entries). Workgroup b takes the rows b, b + G, ... (consecutive rows would
-// put the hubs of RMAT-like graphs, ids with many trailing zeros, into one
-// workgroup), 64 at a time: rows up to kRowShort entries by 4 lanes each, up to
-// kOneWave by a wave, longer ones by the workgroup. EX: also the range facts
-// of v and the sums (k_exact_scan).
+// Row sums of all but the largest graphs in one launch: the five launches of
+// the way above take 40 us however small the graph, this 6 to 8 (9001 vertices,
+// 2.4e5 entries). A workgroup takes 64 rows: rows up to kRowShort entries by 4
+// lanes each, up to kOneWave by a wave, longer ones by the workgroup. EX: also
+// the range facts of v and the sums (k_exact_scan). The rows come in an order
+// that scatters them (step): with consecutive ids, or ids a fixed stride apart,
+// the hubs of RMAT-like graphs, whose ids have many trailing zeros, met in a few
+// workgroups (RMAT-18 gathered sums 86 us with a stride, 48 so).
 constexpr int kOneWave = 1024;
-constexpr int64_t kOneMaxEdges = 1 << 21;  // above, hub rows outlast one workgroup
+constexpr int kOneU = 8;  // loads in flight per thread in those
+// Above, hub rows outlast one workgroup. Vertex weights / gathered sums, one
+// launch and five, us: RMAT of 5.8M entries 22 / 32 and 45 / 60, 11.7M 37 / 61
+// and 66 / 92, 17.8M 54 / 92 and 91 / 127, 31M 104 / 232 and 131 / 197; Chung-Lu
+// 8.4M 27 / 41 and 48 / 62, 19.2M 55 / 102 and 68 / 107.
+constexpr int64_t kOneMaxEdges = 20 << 20;
 
 __device__ __forceinline__ void exact_fact(float w, int& lsb, int& bad) {
   const uint32_t b = __float_as_uint(w);
@@ -343,7 +352,8 @@ __device__ __forceinline__ void exact_sum_fact(double sv, int& mx, int& bad) {
 template <typename OutT, bool IDX, bool EX>
 __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __restrict__ off,
                                                     const int32_t* __restrict__ ind, const float* __restrict__ v,
-                                                    OutT* __restrict__ out, ExactInfo* info, const int* skip) {
+                                                    OutT* __restrict__ out, ExactInfo* info, uint32_t step,
+                                                    const int* skip) {
   if (skip && *skip) return;
   constexpr int BLOCK = 256, NW = BLOCK / kWave, R = BLOCK / kRowGroup;
   __shared__ int s_long[R], s_nlong;
@@ -355,14 +365,13 @@ __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __
     out[u] = (OutT)sum;
     if constexpr (EX) exact_sum_fact(sum, mx, bad);
   };
-  const int64_t G = gridDim.x;
-  for (int64_t i0 = 0; i0 * G + blockIdx.x < n; i0 += R) {
+  for (int64_t i0 = (int64_t)blockIdx.x * R; i0 < n; i0 += (int64_t)gridDim.x * R) {
     if (tid == 0) s_nlong = 0;
     __syncthreads();
-    const int64_t ul = (i0 + tid / kRowGroup) * G + blockIdx.x;
-    const int32_t u = (int32_t)ul;
+    const int64_t k = i0 + tid / kRowGroup;
+    const int32_t u = (int32_t)((uint64_t)k * step % (uint32_t)n);
     int o = 0, d = 0;
-    const bool live = ul < n;
+    const bool live = k < n;
     if (live) {
       o = off[u];
       d = off[u + 1] - o;
@@ -406,11 +415,11 @@ __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __
       const int qo = off[q], qe = off[q + 1];
       if (qe - qo <= kOneWave) continue;  // uniform over the workgroup
       DD2 a2{0.0, 0.0};
-      for (int p0 = qo; p0 < qe; p0 += BLOCK * kRowU) {
-        float x[kRowU];
-        gather_step<IDX, kRowU>(ind, v, p0, BLOCK, tid, qe, x);
+      for (int p0 = qo; p0 < qe; p0 += BLOCK * kOneU) {
+        float x[kOneU];
+        gather_step<IDX, kOneU>(ind, v, p0, BLOCK, tid, qe, x);
 #pragma unroll
-        for (int t = 0; t < kRowU; ++t) a2 = add_d(a2, (double)x[t]);
+        for (int t = 0; t < kOneU; ++t) a2 = add_d(a2, (double)x[t]);
       }
 #pragma unroll
       for (int sh = 1; sh < kWave; sh <<= 1) a2 = add_dd(a2, DD2{__shfl_xor(a2.hi, sh), __shfl_xor(a2.lo, sh)});
@@ -454,21 +463,33 @@ __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __
   }
 }
 
-int grid_one(int32_t n) { return grid_rows((n + 63) / 64, 1, 4); }
+// A second round of rows would make the workgroups that met the long ones the
+// tail (11.7M entries, 4097 workgroups: 84 us and not 39).
+int grid_one(int32_t n) { return grid_rows((n + 63) / 64, 1, 256); }
+
+// Place k of the order holds row k * step_one(n) mod n: n / golden ratio, less
+// what it takes to share no factor with n.
+uint32_t step_one(int32_t n) {
+  uint32_t p = (uint32_t)(n * 0.6180339887498949);
+  while (p > 1 && std::gcd(p, (uint32_t)n) != 1) --p;
+  return std::max(p, 1u);
+}
 
 bool rowsum_one_launch(int64_t m) { return m <= kOneMaxEdges; }
 
 hipError_t launch_rowsum_exact(int32_t n, const int32_t* off, const int32_t* ind, const float* v, double* S,
-                               ExactInfo* info, hipStream_t s) {
+                               ExactInfo* info, hipStream_t s, const int* skip) {
   ProfScope ps_("rowsum", s);
   hipLaunchKernelGGL((k_rowsum_one<double, true, true>), dim3(grid_one(n)), dim3(256), 0, s, n, off, ind, v, S, info,
-                     (const int*)nullptr);
+                     step_one(n), skip);
   return hipGetLastError();
 }
 
 // Sentinel fill of the result (when x is not null) and the start values of a
 // pass's counters and range facts, in one launch.
-__global__ void k_prepare(uint32_t* __restrict__ x, int64_t n, uint32_t v, int* __restrict__ z, int nz, ExactInfo* info) {
+__global__ void k_prepare(uint32_t* __restrict__ x, int64_t n, uint32_t v, int* __restrict__ z, int nz, ExactInfo* info,
+                          const int* skip) {
+  if (skip && *skip) x = nullptr;  // (the counters are read all the same)
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (x)
     for (int64_t i = t; i < n; i += (int64_t)gridDim.x * blockDim.x) x[i] = v;
@@ -478,9 +499,10 @@ __global__ void k_prepare(uint32_t* __restrict__ x, int64_t n, uint32_t v, int* 
   }
 }
 
-hipError_t launch_prepare(uint32_t* x, int64_t n, uint32_t v, int* zero, int nzero, ExactInfo* info, hipStream_t s) {
+hipError_t launch_prepare(uint32_t* x, int64_t n, uint32_t v, int* zero, int nzero, ExactInfo* info, hipStream_t s,
+                          const int* skip) {
   ProfScope ps_("fill", s);
-  hipLaunchKernelGGL(k_prepare, dim3(x ? grid_for(n, 256 * 4, 32) : 1), dim3(256), 0, s, x, n, v, zero, nzero, info);
+  hipLaunchKernelGGL(k_prepare, dim3(x ? grid_for(n, 256 * 4, 32) : 1), dim3(256), 0, s, x, n, v, zero, nzero, info, skip);
   return hipGetLastError();
 }
 
@@ -494,10 +516,10 @@ static hipError_t rowsum_both(int32_t n, int64_t m, const int32_t* off, const in
   if (rowsum_one_launch(m)) {
     if (ind)
       hipLaunchKernelGGL((k_rowsum_one<OutT, true, false>), dim3(grid_one(n)), dim3(256), 0, s, n, off, ind, v, out,
-                         (ExactInfo*)nullptr, skip);
+                         (ExactInfo*)nullptr, step_one(n), skip);
     else
       hipLaunchKernelGGL((k_rowsum_one<OutT, false, false>), dim3(grid_one(n)), dim3(256), 0, s, n, off, ind, v, out,
-                         (ExactInfo*)nullptr, skip);
+                         (ExactInfo*)nullptr, step_one(n), skip);
     return hipGetLastError();
   }
   void* own = nullptr;

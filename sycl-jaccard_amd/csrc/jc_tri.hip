@@ -123,6 +123,7 @@ struct TriCtl {
   Own<int> lsb, maxexp;             // exactness of the weights (see ExactInfo)
   Own<int> wexp;                    // every weight is below 2^wexp
   Own<unsigned long long> sampled;  // min(d_u, d_x, kSampleCap) over kSamples entries (u, x)
+  Own<double> sampled_w;            // weights of the x
   Own<unsigned long long> out_total;  // sum of |R(u)|
   Own<unsigned long long> bits;     // words of the bit matrix handed out
   Own<int> num_big;                 // rows oriented by a workgroup
@@ -235,6 +236,12 @@ __global__ __launch_bounds__(BLOCK) void k_tri_hist(TriArgs a) {
 #pragma unroll
     for (int o = 1; o < kWave; o <<= 1) len += __shfl_xor(len, o);
     if (lane_id() == 0) atomicAdd(&a.ctl->sampled.v, (unsigned long long)len);
+    if constexpr (W) {
+      float w = a.vw[x];
+#pragma unroll
+      for (int o = 1; o < kWave; o <<= 1) w += __shfl_xor(w, o);
+      if (lane_id() == 0) unsafeAtomicAdd(&a.ctl->sampled_w.v, (double)w);
+    }
     return;
   }
   const int ranges = gridDim.x - kLook, range = blockIdx.x - kLook;
@@ -286,12 +293,22 @@ __device__ __forceinline__ int group_rows(int d) { return min(kGroupRows, kWedge
 // Giving up here costs 0.05 ms.
 __global__ __launch_bounds__(kTriBuckets) void k_tri_scan(TriCtl* c, int32_t n, int64_t m, int always, int grp_from) {
   __shared__ int part[kTriBuckets / kWave];
+  __shared__ int s_top;
   const int b = kTriBuckets - 1 - threadIdx.x;
+  if (b == 0) s_top = 0;
+  __syncthreads();
+  if (c->hist[b]) atomicMax(&s_top, b);
+  __syncthreads();
   // a weight that alone is wider than fp64 sums can hold
   if (b == 0 && c->lsb.v != INT32_MAX && c->wexp.v - c->lsb.v > 53) c->bad = 1;
   if (b == 0 && !always) {
     const float len = (float)c->sampled.v / kSamples, d = (float)m / (float)n;
     if (len < 48.f || (len < 96.f && len < 1.5f * d)) c->bad = 1;
+    // the longest row's weights, were they the sampled ones' mean: sums that
+    // surely round are not found out after orient only
+    const int top = s_top < 512 ? s_top : (16 + (s_top & 15)) << ((s_top - 512) / 16 + 5);
+    const double sum = (double)top * c->sampled_w.v / kSamples;
+    if (c->lsb.v != INT32_MAX && sum > 0.0 && ilogb(sum) - c->lsb.v > 53) c->bad = 1;
   }
   const int v = c->hist[b];
   int incl = v;
