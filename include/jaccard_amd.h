@@ -92,10 +92,10 @@ int jc_jaccard(const jc_csr *g, const float *vertex_weights, float *result, int 
 
 /* jc_jaccard with flags (JC_FLAG_*) and an optional caller workspace of at
  * least jc_jaccard_workspace_size() bytes (NULL: allocate per call). With a
- * workspace the call allocates nothing. From 2^22 stored edges on that size
- * includes the oriented engine's arrays (about 37 bytes per edge); a smaller
- * workspace that still holds the owner engine's is accepted, and the call
- * then uses that engine alone, with the same bits. No reference counterpart: the
+ * workspace the call allocates nothing. From 3 * 2^20 stored edges on
+ * (unweighted 6 * 2^20) that size includes the oriented engine's arrays (about
+ * 37 bytes per edge); a smaller workspace that still holds the owner engine's
+ * is accepted, and the call then uses that engine alone, with the same bits. No reference counterpart: the
  * reference allocates temporaries inside the call (jaccard.cpp:931-934). */
 int jc_jaccard_ex(const jc_csr *g, const float *vertex_weights, float *result, int edge_centric,
                   unsigned flags, void *workspace, size_t workspace_bytes, jc_stream_t stream);

@@ -78,11 +78,14 @@ Layout layout(int32_t n, int32_t m, bool weighted, bool ec) {
 // stored entries on, where no tuning is given or it names a batch (and then
 // only if the device finds the rows skewed enough, see k_tri_scan). Below,
 // its two dozen dependent launches are most of its time. Owner and oriented
-// engine, ms: weighted RMAT 2.8M entries 0.54 / 0.55, 4.0M 0.96 / 0.69, 6.0M
-// 1.30 / 0.85, Chung-Lu 3.2M 0.47 / 0.66, 4.5M 1.07 / 0.76; unweighted RMAT
-// 5.8M 0.78 / 0.73, 9.2M 1.18 / 1.09, 11.7M 1.63 / 1.28, Chung-Lu 9.6M
-// 1.04 / 1.25, 12.8M 1.35 / 1.30, 25.6M 2.88 / 2.37.
-constexpr int32_t tri_min_edges(bool weighted) { return weighted ? 1 << 22 : 10 << 20; }
+// engine, ms: weighted RMAT 1.5M entries 0.32 / 0.30, 2.8M 0.54 / 0.42, 4.0M
+// 0.98 / 0.53, Chung-Lu 1.6M 0.29 / 0.32, 3.2M 0.49 / 0.44, 4.5M 1.09 / 0.52;
+// unweighted RMAT 2.8M 0.37 / 0.36, 4.0M 0.53 / 0.47, 5.8M 0.78 / 0.61, 11.7M
+// 1.63 / 1.19, Chung-Lu 3.2M 0.35 / 0.37, 4.2M 0.45 / 0.44, 6.4M 0.68 / 0.58,
+// 12.8M 1.34 / 1.09, 25.6M 2.86 / 2.17. Above the crossing, for what a graph
+// that the device turns down pays: 0.06 ms (uniform random 9M unweighted 0.87 ->
+// 0.95, 4M weighted 0.56 -> 0.62).
+constexpr int32_t tri_min_edges(bool weighted) { return weighted ? 3 << 20 : 6 << 20; }
 
 // The one-launch kernel for graphs that fit the LDS, where the caller names
 // nothing of the owner engine.

@@ -318,16 +318,21 @@ __global__ __launch_bounds__(BLOCK) void k_rowsum_w_long(const int32_t* __restri
 // the way above take 40 us however small the graph, this 6 to 8 (9001 vertices,
 // 2.4e5 entries). A workgroup takes 64 rows: rows up to kRowShort entries by 4
 // lanes each, up to kOneWave by a wave, longer ones by the workgroup. EX: also
-// the range facts of v and the sums (k_exact_scan). The rows come in an order
-// that scatters them (step): with consecutive ids, or ids a fixed stride apart,
-// the hubs of RMAT-like graphs, whose ids have many trailing zeros, met in a few
-// workgroups (RMAT-18 gathered sums 86 us with a stride, 48 so).
+// the range facts of v and the sums (k_exact_scan). Pairs of rows come in an
+// order that scatters them (step): hubs are neighbours in graphs sorted by
+// degree, and in RMAT-like ones their ids have many trailing zeros, so with
+// consecutive rows or with a fixed stride they meet in a few workgroups
+// (RMAT-18 gathered sums 86 us with a stride, 56 so; Chung-Lu of 8.4M entries
+// 134 us in runs of 16 rows, 43 in pairs). Single rows measured
+// a little better still on those and a little worse on uniform random ones.
 constexpr int kOneWave = 1024;
+constexpr int kOneRun = 2;   // consecutive rows that stay together
 constexpr int kOneU = 8;  // loads in flight per thread in those
 // Above, hub rows outlast one workgroup. Vertex weights / gathered sums, one
-// launch and five, us: RMAT of 5.8M entries 22 / 32 and 45 / 60, 11.7M 37 / 61
-// and 66 / 92, 17.8M 54 / 92 and 91 / 127, 31M 104 / 232 and 131 / 197; Chung-Lu
-// 8.4M 27 / 41 and 48 / 62, 19.2M 55 / 102 and 68 / 107.
+// launch and five, us: RMAT of 5.8M entries 23 / 34 and 45 / 59, 11.7M 40 / 63
+// and 64 / 94, 17.8M 58 / 94 and 90 / 128, 31M 104 / 232 and 121 / 201; Chung-Lu
+// 8.4M 31 / 43 and 45 / 61, 19.2M 60 / 107 and 69 / 108; uniform random 16M 36 /
+// 104 and 52 / 112.
 constexpr int64_t kOneMaxEdges = 20 << 20;
 
 __device__ __forceinline__ void exact_fact(float w, int& lsb, int& bad) {
@@ -365,13 +370,21 @@ __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __
     out[u] = (OutT)sum;
     if constexpr (EX) exact_sum_fact(sum, mx, bad);
   };
+  // The facts as the workgroup began: most workgroups change nothing, and their
+  // atomics on one line were 0.3 ms of a graph of 1M vertices.
+  ExactInfo seen{INT32_MAX, INT32_MIN, 0, 0};
+  if constexpr (EX) {
+    if (tid == 0) seen = ExactInfo{*(volatile int*)&info->min_lsb, *(volatile int*)&info->max_exp, *(volatile int*)&info->bad, 0};
+  }
+  const uint32_t runs = ((uint32_t)n + kOneRun - 1) / kOneRun;
   for (int64_t i0 = (int64_t)blockIdx.x * R; i0 < n; i0 += (int64_t)gridDim.x * R) {
     if (tid == 0) s_nlong = 0;
     __syncthreads();
-    const int64_t k = i0 + tid / kRowGroup;
-    const int32_t u = (int32_t)((uint64_t)k * step % (uint32_t)n);
+    const uint32_t run = (uint32_t)(i0 / kOneRun) + tid / (kOneRun * kRowGroup);
+    const uint32_t at = (uint32_t)((uint64_t)run * step % runs) * kOneRun + tid / kRowGroup % kOneRun;
+    const int32_t u = (int32_t)at;
     int o = 0, d = 0;
-    const bool live = k < n;
+    const bool live = run < runs && at < (uint32_t)n;
     if (live) {
       o = off[u];
       d = off[u + 1] - o;
@@ -456,9 +469,9 @@ __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __
         mx = max(mx, s_r[1][k]);
         bad |= s_r[2][k];
       }
-      if (lsb != INT32_MAX) atomicMin(&info->min_lsb, lsb);
-      if (mx != INT32_MIN) atomicMax(&info->max_exp, mx);
-      if (bad) atomicOr(&info->bad, 1);
+      if (lsb < seen.min_lsb) atomicMin(&info->min_lsb, lsb);
+      if (mx > seen.max_exp) atomicMax(&info->max_exp, mx);
+      if (bad && !seen.bad) atomicOr(&info->bad, 1);
     }
   }
 }
@@ -467,11 +480,12 @@ __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __
 // tail (11.7M entries, 4097 workgroups: 84 us and not 39).
 int grid_one(int32_t n) { return grid_rows((n + 63) / 64, 1, 256); }
 
-// Place k of the order holds row k * step_one(n) mod n: n / golden ratio, less
-// what it takes to share no factor with n.
+// Run k of the order is run k * step_one(n) mod runs: runs / golden ratio, less
+// what it takes to share no factor with them.
 uint32_t step_one(int32_t n) {
-  uint32_t p = (uint32_t)(n * 0.6180339887498949);
-  while (p > 1 && std::gcd(p, (uint32_t)n) != 1) --p;
+  const uint32_t runs = ((uint32_t)n + kOneRun - 1) / kOneRun;
+  uint32_t p = (uint32_t)(runs * 0.6180339887498949);
+  while (p > 1 && std::gcd(p, runs) != 1) --p;
   return std::max(p, 1u);
 }
 

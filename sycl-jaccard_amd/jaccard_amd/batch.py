@@ -103,9 +103,9 @@ JcTuning = api.JcTuning
 def _tuned(dg, weights, out, ws, tuning, stream):
     lib = load_jaccard_lib()
     g = dg.c_struct()
-    # members: from 2^22 stored edges on the oriented engine ranks every graph by
-    # itself (128 graphs, 4.4e7 stored edges in two unions: 5.66 ms by the owner
-    # engine, 4.66 by this). tuning is None only before autotune or select.
+    # members: from 3 * 2^20 stored edges on (unweighted 6 * 2^20) the oriented
+    # engine ranks every graph by itself (128 graphs, 4.4e7 stored edges in two unions: 5.66 ms by the owner
+    # engine, 4.30 by this). tuning is None only before autotune or select.
     tuning = tuning or (0, 0, 0)
     t = ctypes.byref(
         JcTuning(small_max=tuning[0], small_blocks_per_cu=tuning[1], bitmap_blocks_per_cu=tuning[2], members=1))
