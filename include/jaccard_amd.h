@@ -152,6 +152,12 @@ typedef struct jc_tuning {
 int jc_jaccard_noalloc(const jc_csr *g, const float *vertex_weights, float *result, int edge_centric,
                        unsigned flags, jc_stream_t stream);
 
+/* Calls that take no workspace allocate theirs on their stream, from a pool of
+ * the library's own that keeps up to 2 GiB per device for the calls to come.
+ * This gives back to the system what no call is using (of every device). Safe
+ * at any time, from any thread. No reference counterpart. */
+int jc_release_workspaces(void);
+
 /* jc_jaccard_ex with launch tuning (NULL = defaults). */
 int jc_jaccard_tuned(const jc_csr *g, const float *vertex_weights, float *result, int edge_centric,
                      unsigned flags, void *workspace, size_t workspace_bytes, const jc_tuning *tuning,

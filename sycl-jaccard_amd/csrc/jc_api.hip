@@ -273,12 +273,12 @@ int jc_jaccard_tuned(const jc_csr* g, const float* vertex_weights, float* result
   }
   AsyncBuf buf;
   buf.s = s;
-  if (tri && hipMallocAsync(&buf.p, full, s) != hipSuccess) {
+  if (tri && jc::call_alloc(&buf.p, full, s) != hipSuccess) {
     (void)hipGetLastError();
     buf.p = nullptr;
     tri = false;  // the owner engine needs a small part of it
   }
-  if (!tri) JC_TRY(hipMallocAsync(&buf.p, need, s));
+  if (!tri) JC_TRY(jc::call_alloc(&buf.p, need, s));
   unsigned char* ws = static_cast<unsigned char*>(buf.p);
   return run_jaccard(g, vertex_weights, result, ec, flags, ws, tri ? ws + need : nullptr, tuning, s);
 }
@@ -325,7 +325,7 @@ int jc_jaccard_list(const jc_csr* g, const float* vertex_weights, int32_t num_pa
   double* S64 = nullptr;
   if (weighted && pairs_sum_all(g, num_pairs, s)) {
     const size_t rows_b = al(jc::rowsum_scratch_bytes(g->n));
-    if (hipMallocAsync(&buf.p, rows_b + al((size_t)g->n * sizeof(double)), s) == hipSuccess) {
+    if (jc::call_alloc(&buf.p, rows_b + al((size_t)g->n * sizeof(double)), s) == hipSuccess) {
       S64 = reinterpret_cast<double*>(static_cast<unsigned char*>(buf.p) + rows_b);
       JC_TRY(jc::launch_rowsum_f64(g->n, g->m, g->offsets, g->indices, vertex_weights, S64, buf.p, s));
     } else {
@@ -370,7 +370,7 @@ int jc_nonzero_count(int32_t m, const float* result, float thresh, int64_t* coun
   hipStream_t s = hs(stream);
   AsyncBuf buf;
   buf.s = s;
-  JC_TRY(hipMallocAsync(&buf.p, sizeof(unsigned long long), s));
+  JC_TRY(jc::call_alloc(&buf.p, sizeof(unsigned long long), s));
   auto* c = static_cast<unsigned long long*>(buf.p);
   JC_TRY(jc::launch_fill_u64(reinterpret_cast<uint64_t*>(c), 1, 0ull, s));
   JC_TRY(jc::launch_count_above(m, result, thresh, c, s));
@@ -404,12 +404,12 @@ int jc_intersect(int32_t n, int32_t m, const int32_t* offsets, const int32_t* in
   AsyncBuf buf;
   buf.s = s;
   bool tri = tri_wanted(&g, v != nullptr, nullptr);
-  if (tri && hipMallocAsync(&buf.p, need + jc::tri_workspace_bytes(n, m, v != nullptr), s) != hipSuccess) {
+  if (tri && jc::call_alloc(&buf.p, need + jc::tri_workspace_bytes(n, m, v != nullptr), s) != hipSuccess) {
     (void)hipGetLastError();
     buf.p = nullptr;
     tri = false;
   }
-  if (!tri) JC_TRY(hipMallocAsync(&buf.p, need, s));
+  if (!tri) JC_TRY(jc::call_alloc(&buf.p, need, s));
   jc::EngineArgs a{};
   a.n = n;
   a.m = m;
@@ -472,7 +472,7 @@ int jc_weighted_sum_mode(const jc_csr* g, const float* vertex_weights, int* mode
   const size_t s64_b = al((size_t)g->n * sizeof(double));
   AsyncBuf buf;
   buf.s = s;
-  JC_TRY(hipMallocAsync(&buf.p, rows_b + s64_b + al(sizeof(jc::ExactInfo)), s));
+  JC_TRY(jc::call_alloc(&buf.p, rows_b + s64_b + al(sizeof(jc::ExactInfo)), s));
   unsigned char* p = static_cast<unsigned char*>(buf.p);
   double* S64 = reinterpret_cast<double*>(p + rows_b);
   jc::ExactInfo* ex = reinterpret_cast<jc::ExactInfo*>(p + rows_b + s64_b);
@@ -494,7 +494,7 @@ int jc_degree_stats(const jc_csr* g, jc_graph_stats* stats, jc_stream_t stream) 
   constexpr int kWords = 69;  // see launch_degree_stats
   AsyncBuf buf;
   buf.s = s;
-  JC_TRY(hipMallocAsync(&buf.p, kWords * sizeof(unsigned long long), s));
+  JC_TRY(jc::call_alloc(&buf.p, kWords * sizeof(unsigned long long), s));
   auto* d = static_cast<unsigned long long*>(buf.p);
   JC_TRY(jc::launch_fill_u64(reinterpret_cast<uint64_t*>(d), kWords, 0ull, s));
   JC_TRY(jc::launch_degree_stats(g->n, g->offsets, g->indices, d, s));
@@ -541,7 +541,7 @@ int jc_validate_csr(const jc_csr* g, int* what, jc_stream_t stream) {
   hipStream_t s = hs(stream);
   AsyncBuf buf;
   buf.s = s;
-  JC_TRY(hipMallocAsync(&buf.p, 4 * sizeof(int), s));
+  JC_TRY(jc::call_alloc(&buf.p, 4 * sizeof(int), s));
   int* f = static_cast<int*>(buf.p);
   JC_TRY(jc::launch_fill_u32(reinterpret_cast<uint32_t*>(f), 4, 0u, s));
   JC_TRY(jc::launch_validate(g->n, g->m, g->offsets, g->indices, f, s));
@@ -565,7 +565,7 @@ int jc_csr_is_symmetric(const jc_csr* g, int* symmetric, jc_stream_t stream) {
   hipStream_t s = hs(stream);
   AsyncBuf buf;
   buf.s = s;
-  JC_TRY(hipMallocAsync(&buf.p, sizeof(int), s));
+  JC_TRY(jc::call_alloc(&buf.p, sizeof(int), s));
   int* f = static_cast<int*>(buf.p);
   JC_TRY(jc::launch_fill_u32(reinterpret_cast<uint32_t*>(f), 1, 0u, s));
   JC_TRY(jc::launch_symcheck(g->n, g->m, g->offsets, g->indices, f, s));

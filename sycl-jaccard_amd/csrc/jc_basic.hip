@@ -539,7 +539,7 @@ static hipError_t rowsum_both(int32_t n, int64_t m, const int32_t* off, const in
   void* own = nullptr;
   hipError_t err;
   if (!scratch) {
-    if ((err = hipMallocAsync(&own, rowsum_scratch_bytes(n), s)) != hipSuccess) return err;
+    if ((err = call_alloc(&own, rowsum_scratch_bytes(n), s)) != hipSuccess) return err;
     scratch = own;
   }
   int* counters = static_cast<int*>(scratch);

@@ -209,7 +209,7 @@ hipError_t ingest(int32_t n, int64_t num_edges, int64_t e2, const int32_t* src, 
   const size_t o_ct = o; o += al(2 * sizeof(int32_t));
   const size_t o_tmp = o; o += al(sort_bytes);
   unsigned char* ws = nullptr;
-  if ((err = hipMallocAsync(reinterpret_cast<void**>(&ws), o, s)) != hipSuccess) return err;
+  if ((err = call_alloc(reinterpret_cast<void**>(&ws), o, s)) != hipSuccess) return err;
   Key* k0 = reinterpret_cast<Key*>(ws + o_k0);
   Key* k1 = reinterpret_cast<Key*>(ws + o_k1);
   float* v0 = weighted ? reinterpret_cast<float*>(ws + o_v0) : nullptr;

@@ -146,6 +146,10 @@ hipError_t launch_exact_info(int32_t n, const float* vw, const double* S, ExactI
 // Records a failing HIP call for jc_last_hip_error(); returns the JC_ERR_* code.
 int note_hip_error(hipError_t e);
 
+// Workspace of one call, stream-ordered (jc_mem.hip): as hipMallocAsync, freed
+// with hipFreeAsync, from a pool that keeps some of what is freed.
+hipError_t call_alloc(void** p, size_t bytes, hipStream_t s);
+
 // Streaming kernels.
 hipError_t launch_fill_f32(float* x, int64_t n, float v, hipStream_t s);
 // (skip: as EngineArgs::skip)

@@ -208,6 +208,12 @@ def workspace_size(n: int, m: int, weighted: bool, edge_centric: bool) -> int:
     return int(load_jaccard_lib().jc_jaccard_workspace_size(n, m, int(weighted), int(edge_centric)))
 
 
+def release_workspaces() -> None:
+    """Give back the device memory that the library keeps between calls
+    (``jc_release_workspaces``; up to 2 GiB per device, and none in use)."""
+    _check(load_jaccard_lib().jc_release_workspaces(), "jc_release_workspaces")
+
+
 def jaccard_list(graph: DeviceCSR, first, second, result=None, weights=None, stream=None):
     """Jaccard coefficient of arbitrary vertex pairs (``sygraph::jaccard_list``)."""
     torch = _torch()
