@@ -10,9 +10,9 @@
 // in 32-bit words where these suffice. Flags, positions and source rows are
 // formed again from the sorted keys where they are needed, not stored.
 // Measured, 16M weighted draws symmetrized over 1000003 vertices: 5
-// digits instead of 7, 2.66 -> 1.94 ms, of which the sort takes 1.46 (0.27 a
-// digit, 768 MB each); keys 0.11, counting 0.08 and compacting 0.21, where
-// flags, their scan and the offsets' pass took 0.47.
+// digits instead of 7, 2.66 -> 1.86 ms, of which the sort takes 1.46 (0.27 a
+// digit, 768 MB each); keys 0.11, counting 0.08 and compacting 0.13 (8 keys per
+// thread; 16 took 0.21), where flags, their scan and the offsets took 0.47.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 #include <stdint.h>
@@ -27,7 +27,7 @@ namespace jc {
 namespace {
 
 constexpr int kTile = 4096;  // sorted keys of a workgroup of the compaction
-constexpr int kTileB = 256;
+constexpr int kTileB = 512;
 
 // Bits of an id in a key.
 int id_bits(int32_t n) {
