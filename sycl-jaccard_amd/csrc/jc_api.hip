@@ -74,19 +74,6 @@ Layout layout(int32_t n, int32_t m, bool weighted, bool ec) {
   return L;
 }
 
-// Oriented engine (jc_tri.hip) before the owner engine: from tri_min_edges
-// stored entries on, where no tuning is given or it names a batch (and then
-// only if the device finds the rows skewed enough, see k_tri_scan). Below,
-// its two dozen dependent launches are most of its time. Owner and oriented
-// engine, ms: weighted RMAT 1.5M entries 0.32 / 0.30, 2.8M 0.54 / 0.42, 4.0M
-// 0.98 / 0.53, Chung-Lu 1.6M 0.29 / 0.32, 3.2M 0.49 / 0.44, 4.5M 1.09 / 0.52;
-// unweighted RMAT 2.8M 0.37 / 0.36, 4.0M 0.53 / 0.47, 5.8M 0.78 / 0.61, 11.7M
-// 1.63 / 1.19, Chung-Lu 3.2M 0.35 / 0.37, 4.2M 0.45 / 0.44, 6.4M 0.68 / 0.58,
-// 12.8M 1.34 / 1.09, 25.6M 2.86 / 2.17. Above the crossing, for what a graph
-// that the device turns down pays: 0.06 ms (uniform random 9M unweighted 0.87 ->
-// 0.95, 4M weighted 0.56 -> 0.62).
-constexpr int32_t tri_min_edges(bool weighted) { return weighted ? 3 << 20 : 6 << 20; }
-
 // The one-launch kernel for graphs that fit the LDS, where the caller names
 // nothing of the owner engine.
 bool tiny_wanted(const jc_csr* g, bool weighted, const jc_tuning* t) {
@@ -95,11 +82,8 @@ bool tiny_wanted(const jc_csr* g, bool weighted, const jc_tuning* t) {
 
 bool tri_wanted(const jc_csr* g, bool weighted, const jc_tuning* t) {
   if (t && (t->engine == JC_ENGINE_OWNER || t->wide_index || t->hash_table == 1 || t->quot_max_disp > 0)) return false;
-  // (sum |R|^2 / 64 words of bit matrix are at least (m / 2)^2 / n / 64, above
-  // the engine's 4 m words from a mean row of 1024 entries on; a uniform
-  // random graph reaches them at 768)
-  if (g->n > jc::kTriMaxN || g->m > 768ll * g->n) return false;
-  return (t && t->engine == JC_ENGINE_ORIENTED) || ((!t || t->members) && g->m >= tri_min_edges(weighted));
+  if (!jc::tri_can(g->n, g->m)) return false;
+  return (t && t->engine == JC_ENGINE_ORIENTED) || ((!t || t->members) && g->m >= jc::tri_min_edges(weighted));
 }
 
 // Weighted pair lists: sum every row of the graph once before the pairs, or
@@ -246,7 +230,7 @@ extern "C" {
 size_t jc_jaccard_workspace_size(int32_t n, int32_t m, int weighted, int edge_centric) {
   if (n < 0 || m < 0) return 0;
   size_t b = layout(n, m, weighted != 0, edge_centric != 0).total;
-  if (m >= tri_min_edges(weighted != 0)) b += al(jc::tri_workspace_bytes(n, m, weighted != 0));
+  if (m >= jc::tri_min_edges(weighted != 0)) b += al(jc::tri_workspace_bytes(n, m, weighted != 0));
   return b;
 }
 

@@ -117,8 +117,29 @@ int engine_counter_words();
 // must follow. ws holds tri_workspace_bytes(n, m, weighted) bytes. always: not
 // only where the rows say that it is the faster engine.
 constexpr int32_t kTriMaxN = 1 << 26;  // its hash keys hold 26-bit ranks
-size_t tri_workspace_bytes(int32_t n, int64_t m, bool weighted);
-hipError_t run_tri(int mode, const EngineArgs& base, bool always, void* ws, const int** done, hipStream_t s);
+// Oriented engine (jc_tri.hip) before the owner engine: from tri_min_edges
+// stored entries on, where no tuning is given or it names a batch (and then
+// only if the device finds the rows skewed enough, see k_tri_scan). Below,
+// its two dozen dependent launches are most of its time. Owner and oriented
+// engine, ms: weighted RMAT 1.5M entries 0.32 / 0.30, 2.8M 0.54 / 0.42, 4.0M
+// 0.98 / 0.53, Chung-Lu 1.6M 0.29 / 0.32, 3.2M 0.49 / 0.44, 4.5M 1.09 / 0.52;
+// unweighted RMAT 2.8M 0.37 / 0.36, 4.0M 0.53 / 0.47, 5.8M 0.78 / 0.61, 11.7M
+// 1.63 / 1.19, Chung-Lu 3.2M 0.35 / 0.37, 4.2M 0.45 / 0.44, 6.4M 0.68 / 0.58,
+// 12.8M 1.34 / 1.09, 25.6M 2.86 / 2.17. Above the crossing, for what a graph
+// that the device turns down pays: 0.06 ms (uniform random 9M unweighted 0.87 ->
+// 0.95, 4M weighted 0.56 -> 0.62).
+constexpr int32_t tri_min_edges(bool weighted) { return weighted ? 3 << 20 : 6 << 20; }
+// (sum |R|^2 / 64 words of bit matrix are at least (m / 2)^2 / n / 64, above the
+// engine's 4 m words from a mean row of 1024 entries on; a uniform random graph
+// reaches them at 768)
+constexpr bool tri_can(int32_t n, int64_t m) { return n <= kTriMaxN && m <= 768ll * n; }
+constexpr int32_t kTriPart = 65536;  // vertices of a member (EngineArgs::members), at most
+// bits: quarter words of bit matrix per stored entry; a graph that needs more is
+// refused after orient. RMAT graphs need 1 (16 entries per vertex of 2^12) to 5.
+constexpr int kTriBits = 16;
+size_t tri_workspace_bytes(int32_t n, int64_t m, bool weighted, int bits = kTriBits);
+hipError_t run_tri(int mode, const EngineArgs& base, bool always, void* ws, const int** done, hipStream_t s,
+                   int bits = kTriBits);
 
 // Workspace needed by an owner-engine pass over a graph with n vertices and m
 // stored edges (task list, small-row list, counters). With row segments, n and

@@ -53,6 +53,30 @@ __global__ void k_scatter(const ScatterDesc* __restrict__ d) {
     e.dst[i] = e.src[i];
 }
 
+// The requested graphs by themselves, one behind the other: what the oriented
+// engine takes, which has no row segments.
+struct CopyDesc {
+  int32_t vbase, row0, n;    // rows [vbase, vbase + n) of the arena, from row0 of the copy
+  int64_t ebase, e0, m;      // their entries, and in the copy
+};
+
+__global__ void k_copy_graphs(const CopyDesc* __restrict__ d, int rows_end, int e_end, const int32_t* __restrict__ off,
+                              const int32_t* __restrict__ ind, const float* __restrict__ W,
+                              const double* __restrict__ S, int32_t* __restrict__ off2, int32_t* __restrict__ ind2,
+                              float* __restrict__ W2, double* __restrict__ S2) {
+  const CopyDesc c = d[blockIdx.y];
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, nt = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = t; i < c.m; i += nt) ind2[c.e0 + i] = ind[c.ebase + i] - c.vbase + c.row0;
+  for (int64_t i = t; i < c.n; i += nt) {
+    off2[c.row0 + i] = (int32_t)(off[c.vbase + i] - c.ebase + c.e0);
+    if (W) {
+      W2[c.row0 + i] = W[c.vbase + i];
+      S2[c.row0 + i] = S[c.vbase + i];
+    }
+  }
+  if (t == 0 && c.row0 + c.n == rows_end) off2[rows_end] = e_end;
+}
+
 size_t al(size_t v) { return (v + 255) / 256 * 256; }
 
 // First-fit allocator over the budget region (offsets, 256-byte granules).
@@ -123,6 +147,7 @@ struct Slot {
   size_t host_bytes = 0;
   bool busy = false;
   size_t off = 0, bytes = 0;      // budget chunk
+  size_t off2 = 0, bytes2 = 0;    // and that of the oriented engine, if any
   int batch = -1;
   std::vector<int> reqs;
   std::vector<int> graphs;
@@ -150,6 +175,33 @@ BatchLayout batch_layout(int nseg, int nd, int64_t K, int32_t R, int64_t E) {
   o += al(sizeof(float) * (size_t)K);
   L.ws = o;
   if (nseg > 0) o += al(engine_workspace_bytes(R, E));
+  L.total = o;
+  return L;
+}
+
+// Byte layout of the chunk in which a batch's whole graphs are copied together
+// for the oriented engine.
+struct CopyLayout {
+  size_t desc, off, ind, W, S, out, tri, total;
+};
+
+CopyLayout copy_layout(int nseg, int32_t R, int64_t E, bool weighted, int bits) {
+  CopyLayout L{};
+  size_t o = 0;
+  L.desc = o;
+  o += al(sizeof(CopyDesc) * (size_t)nseg);
+  L.off = o;
+  o += al(sizeof(int32_t) * ((size_t)R + 1));
+  L.ind = o;
+  o += al(sizeof(int32_t) * (size_t)E);
+  L.W = o;
+  o += weighted ? al(sizeof(float) * (size_t)R) : 0;
+  L.S = o;
+  o += weighted ? al(sizeof(double) * (size_t)R) : 0;
+  L.out = o;
+  o += al(sizeof(float) * (size_t)E);
+  L.tri = o;
+  o += al(tri_workspace_bytes(R, E, weighted, bits));
   L.total = o;
   return L;
 }
@@ -422,11 +474,20 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
   int next = 0, finished = 0, batches = 0, in_flight = 0;
   int err = JC_OK;
 
+  constexpr int kMinBits = 5;
   auto finish = [&](int i, int status) {
     stats[i].completed = jc::now_s(t0);
     stats[i].status = status;
     ++finished;
   };
+
+  // Whole graphs of so many rows and entries can go to the oriented engine, given
+  // so much memory in one piece.
+  auto copy_fits_in = [&](size_t room, int nseg, int32_t R, int64_t E) {
+    return E >= jc::tri_min_edges(s->weighted) && jc::tri_can(R, E) &&
+           jc::copy_layout(nseg, R, E, s->weighted, kMinBits).total + s->pool.cap() / 8 <= room;
+  };
+  auto copy_fits = [&](int nseg, int32_t R, int64_t E) { return copy_fits_in(s->pool.largest(), nseg, R, E); };
 
   // Forms and launches one batch on slot sl from the pending queue; false if
   // nothing could be admitted.
@@ -435,12 +496,25 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
     int nseg = 0;
     int32_t R = 0;
     int64_t E = 0, K = 0;
+    const bool copies = std::any_of(s->slots.begin(), s->slots.end(), [](const jc::Slot& o) { return o.busy && o.bytes2 > 0; });
     for (auto it = pending.begin(); it != pending.end() && (int)take.size() < cfg.max_batch_requests;) {
       const jc_request& q = reqs[*it];
       const jc::Member& m = s->g[q.graph];
       const bool full = q.kind == JC_REQ_FULL;
       if (full && (graph_busy[q.graph] || in_batch[q.graph])) { ++it; continue; }
       if (!take.empty() && full && E + m.m > cfg.max_batch_edges) { ++it; continue; }
+      // a graph that the oriented engine lacks the memory for waits where another
+      // batch's copy holds it; the owner engine would take twice as long
+      if (full && nseg == 0 && copies && !copy_fits(1, m.n, m.m) && copy_fits_in(s->pool.cap(), 1, m.n, m.m)) {
+        ++it;
+        continue;
+      }
+      // a batch that the oriented engine has memory for is not grown beyond that
+      if (full && nseg > 0 && !copy_fits(nseg + 1, R + m.n, E + m.m) &&
+          (copy_fits(nseg, R, E) || copy_fits(1, m.n, m.m))) {
+        ++it;
+        continue;
+      }
       if (!take.empty() && !full && K + q.num_pairs > cfg.max_batch_pairs) { ++it; continue; }
       const jc::BatchLayout L = jc::batch_layout(nseg + (full ? 1 : 0), (int)take.size() + 1, K + (full ? 0 : q.num_pairs),
                                                  R + (full ? m.n : 0), E + (full ? m.m : 0));
@@ -476,8 +550,26 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
       return false;
     }
     unsigned char* dev = s->pool_mem + off;
-    if (sl.host_bytes < L.staged) {
-      const size_t want = std::max(L.staged, sl.host_bytes * 2);
+    // The oriented engine where it is the faster one (as in a call on one graph)
+    // and its memory leaves a sixteenth of the budget to the next batch, with a
+    // smaller bit matrix if it must; else the owner engine over the rows where
+    // they are. Ten graphs of 2^12 to 2^16 vertices, 96 requests: 5.57 -> 5.43 ms;
+    // 64 graphs of 2^14 to 2^20, 512 requests: 906 -> 991 requests/s with a
+    // budget of 1 GiB, 1170 with 4 GiB.
+    jc::CopyLayout C{};
+    size_t off2 = 0;
+    bool tri = false;
+    int bits = jc::kTriBits;
+    if (nseg > 0 && E >= jc::tri_min_edges(s->weighted) && jc::tri_can(R, E)) {
+      for (; !tri && bits >= kMinBits; bits -= tri ? 0 : 1) {
+        C = jc::copy_layout(nseg, R, E, s->weighted, bits);
+        tri = s->pool.largest() >= C.total + s->pool.cap() / 16 && s->pool.alloc(C.total, &off2);
+      }
+    }
+    unsigned char* dev2 = tri ? s->pool_mem + off2 : nullptr;
+    const size_t staged = L.staged + (tri ? sizeof(jc::CopyDesc) * (size_t)nseg : 0);
+    if (sl.host_bytes < staged) {
+      const size_t want = std::max(staged, sl.host_bytes * 2);
       if (sl.host) (void)hipHostFree(sl.host);
       sl.host = nullptr;
       sl.host_bytes = 0;
@@ -485,6 +577,7 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
       if (e != hipSuccess) {
         err = note_hip_error(e);
         s->pool.release(off, L.total);
+        if (tri) s->pool.release(off2, C.total);
         for (int i : take) {
           if (reqs[i].kind == JC_REQ_FULL) in_batch[reqs[i].graph] = 0;
           stats[i].admitted = jc::now_s(t0);
@@ -499,17 +592,23 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
     int32_t* hfirst = reinterpret_cast<int32_t*>(sl.host + L.first);
     int32_t* hsecond = reinterpret_cast<int32_t*>(sl.host + L.second);
     const float* dpout = reinterpret_cast<const float*>(dev + L.pout);
+    jc::CopyDesc* hcopy = reinterpret_cast<jc::CopyDesc*>(sl.host + L.staged);
+    const float* dcopy = tri ? reinterpret_cast<const float*>(dev2 + C.out) : nullptr;
     int si = 0;
-    int32_t rows = 0;
-    int64_t k0 = 0, maxcount = 0;
+    int32_t rows = 0, largest_n = 0;
+    int64_t k0 = 0, e0 = 0, maxcount = 0, maxm = 0;
     sl.graphs.clear();
     for (int d = 0; d < nd; ++d) {
       const jc_request& q = reqs[take[d]];
       const jc::Member& m = s->g[q.graph];
       if (q.kind == JC_REQ_FULL) {
+        if (tri) hcopy[si] = jc::CopyDesc{m.vbase, rows, m.n, m.ebase, e0, m.m};
         hsegs[si++] = make_int2(m.vbase, rows);
         rows += m.n;
-        hdesc[d] = jc::ScatterDesc{s->out + m.ebase, q.result, m.m};
+        hdesc[d] = jc::ScatterDesc{tri ? dcopy + e0 : s->out + m.ebase, q.result, m.m};
+        e0 += m.m;
+        maxm = std::max(maxm, m.m);
+        largest_n = std::max(largest_n, m.n);
         maxcount = std::max(maxcount, m.m);
         graph_busy[q.graph] = 1;
         in_batch[q.graph] = 0;
@@ -543,11 +642,35 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
       a.S64 = s->S64;
       a.exact = s->exact;
       a.out32 = s->out;
-      a.segs = reinterpret_cast<const int2*>(dev + L.segs);
-      a.nseg = nseg;
-      a.seg_rows = R;
-      a.seg_edges = E;
-      e = jc::run_engine(mode, s->weighted, a, dev + L.ws, false, st);
+      if (tri) {
+        int32_t* off2d = reinterpret_cast<int32_t*>(dev2 + C.off);
+        int32_t* ind2d = reinterpret_cast<int32_t*>(dev2 + C.ind);
+        float* W2d = s->weighted ? reinterpret_cast<float*>(dev2 + C.W) : nullptr;
+        double* S2d = s->weighted ? reinterpret_cast<double*>(dev2 + C.S) : nullptr;
+        e = hipMemcpyAsync(dev2 + C.desc, hcopy, sizeof(jc::CopyDesc) * (size_t)nseg, hipMemcpyHostToDevice, st);
+        if (e == hipSuccess) {
+          const int gx = (int)std::max<int64_t>(1, std::min<int64_t>((maxm + 1023) / 1024, 2048));
+          hipLaunchKernelGGL(jc::k_copy_graphs, dim3(gx, nseg), dim3(256), 0, st,
+                             reinterpret_cast<const jc::CopyDesc*>(dev2 + C.desc), R, (int)E, s->off, s->ind, s->W,
+                             s->S64, off2d, ind2d, W2d, S2d);
+          e = hipGetLastError();
+        }
+        a.n = R;
+        a.m = E;
+        a.off = off2d;
+        a.ind = ind2d;
+        a.vw = W2d;
+        a.S64 = S2d;
+        a.out32 = reinterpret_cast<float*>(dev2 + C.out);
+        a.members = largest_n <= jc::kTriPart;
+        if (e == hipSuccess) e = jc::run_tri(mode, a, false, dev2 + C.tri, &a.skip, st, bits);
+      } else {
+        a.segs = reinterpret_cast<const int2*>(dev + L.segs);
+        a.nseg = nseg;
+        a.seg_rows = R;
+        a.seg_edges = E;
+      }
+      if (e == hipSuccess) e = jc::run_engine(mode, s->weighted, a, dev + L.ws, false, st);
     }
     if (e == hipSuccess && K > 0)
       e = jc::run_pairs(mode, s->weighted, s->N, s->off, s->ind, s->W, nullptr, s->S64, K,
@@ -563,6 +686,8 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
     sl.busy = true;
     sl.off = off;
     sl.bytes = L.total;
+    sl.off2 = off2;
+    sl.bytes2 = tri ? C.total : 0;
     sl.batch = batches++;
     sl.reqs = take;
     if (e != hipSuccess) err = note_hip_error(e);  // the loop below retires everything
@@ -576,6 +701,7 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
         (void)hipStreamSynchronize(sl.stream);
         for (int i : sl.reqs) finish(i, err);
         s->pool.release(sl.off, sl.bytes);
+        if (sl.bytes2) s->pool.release(sl.off2, sl.bytes2);
         sl.busy = false;
       }
       for (int i : pending) finish(i, err);
@@ -617,6 +743,7 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
       for (int i : sl.reqs) finish(i, status);
       for (int gi : sl.graphs) graph_busy[gi] = 0;
       s->pool.release(sl.off, sl.bytes);
+      if (sl.bytes2) s->pool.release(sl.off2, sl.bytes2);
       sl.busy = false;
       progress = true;
     }

@@ -57,7 +57,7 @@ constexpr int kTriBuckets = 1024;
 constexpr int kSamples = 1024;     // entries looked at before the engine is chosen
 constexpr int kSampleCap = 512;
 constexpr int kTriParts = 1024;    // vertex ranges of the rank kernels, at most
-constexpr int kPartMax = 65536;    // vertices of a disjoint part
+constexpr int kPartMax = kTriPart; // vertices of a disjoint part
 constexpr int kTriMaxOut = 4096;   // largest |R(u)|: the sort and reduce buffers in LDS
 constexpr int kTriRowWave = 1024;  // rows up to this many entries are oriented by one wave
 constexpr int kSat16 = 65535;      // 16-bit ranks saturate here
@@ -1847,14 +1847,12 @@ __global__ __launch_bounds__(256) void k_tri_deliver(TriArgs a) {
 
 size_t al256(size_t v) { return (v + 255) / 256 * 256; }
 
-constexpr uint64_t kBitsWordsPerEdge = 4;
-
-uint64_t bits_cap(int64_t m) { return std::min<uint64_t>(kBitsWordsPerEdge * (uint64_t)m, 0xFFFFFF00ull); }
+uint64_t bits_cap(int64_t m, int bits) { return std::min<uint64_t>((uint64_t)m * bits / 4, 0xFFFFFF00ull); }
 
 int64_t tri_tasks(int32_t n, int64_t m) { return m / kWedgeB + std::min<int64_t>(n, m / kWgMinDeg) + 1; }
 
 // Carves the workspace; with p == nullptr only measures it.
-size_t carve(TriArgs& a, unsigned char* p, int32_t n, int64_t m, bool weighted) {
+size_t carve(TriArgs& a, unsigned char* p, int32_t n, int64_t m, bool weighted, int bits) {
   size_t o = 0;
   auto take = [&](size_t bytes) {
     unsigned char* q = p ? p + o : nullptr;
@@ -1878,7 +1876,7 @@ size_t carve(TriArgs& a, unsigned char* p, int32_t n, int64_t m, bool weighted) 
   unsigned char* acc = take(mm * (weighted ? 8 : 4));
   a.accw = weighted ? reinterpret_cast<double*>(acc) : nullptr;
   a.accu = weighted ? nullptr : reinterpret_cast<uint32_t*>(acc);
-  a.bits_cap = bits_cap(m);
+  a.bits_cap = bits_cap(m, bits);
   a.bits = reinterpret_cast<uint32_t*>(take((size_t)a.bits_cap * 4));
   a.list_mid = reinterpret_cast<int32_t*>(take(nn * 4));
   a.list_big = reinterpret_cast<int32_t*>(take(nn * 4));
@@ -1957,15 +1955,15 @@ hipError_t tri_launch(const TriArgs& a, hipStream_t s) {
 
 }  // namespace
 
-size_t tri_workspace_bytes(int32_t n, int64_t m, bool weighted) {
+size_t tri_workspace_bytes(int32_t n, int64_t m, bool weighted, int bits) {
   TriArgs a{};
-  return carve(a, nullptr, n, m, weighted);
+  return carve(a, nullptr, n, m, weighted, bits);
 }
 
-hipError_t run_tri(int mode, const EngineArgs& e, bool always, void* ws, const int** done, hipStream_t s) {
+hipError_t run_tri(int mode, const EngineArgs& e, bool always, void* ws, const int** done, hipStream_t s, int bits) {
   TriArgs a{};
   const bool weighted = e.vw != nullptr;
-  carve(a, static_cast<unsigned char*>(ws), e.n, e.m, weighted);
+  carve(a, static_cast<unsigned char*>(ws), e.n, e.m, weighted, bits);
   a.n = e.n;
   a.m = e.m;
   a.off = e.off;
