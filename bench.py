@@ -42,16 +42,17 @@ WORKLOADS = {
 }
 
 
-# rocprofv3 summary of the dominant kernel's HBM traffic per workload: bytes
-# from the TCC read/write request counts by request size (see the file for
-# the commands and the copy-kernel check).
-TRAFFIC_PROFILES = {"rmat22_weighted": "profiles/owner_block_rmat22_weighted_pmc.md",
-                    "chunglu20": "profiles/owner_block_chunglu20_pmc.md"}
+# rocprofv3 summary of the engine's traffic per workload: bytes from the TCC
+# read/write request counts by request size (see the file for the commands).
+TRAFFIC_PROFILES = {("owner", "rmat22_weighted"): "profiles/owner_block_rmat22_weighted_pmc.md",
+                    ("owner", "chunglu20"): "profiles/owner_block_chunglu20_pmc.md",
+                    ("oriented", "rmat22_weighted"): "profiles/oriented_rmat22_weighted.md",
+                    ("oriented", "chunglu20"): "profiles/oriented_chunglu20.md"}
 
 
-def profile_value(workload, key, cast=float):
+def profile_value(engine, workload, key, cast=float):
     """A `key = value` line of the committed counter summary of the workload, or None."""
-    rel = TRAFFIC_PROFILES.get(workload)
+    rel = TRAFFIC_PROFILES.get((engine, workload))
     if rel is None or not os.path.exists(os.path.join(ROOT, rel)):
         return None
     for line in open(os.path.join(ROOT, rel)):
@@ -60,9 +61,9 @@ def profile_value(workload, key, cast=float):
     return None
 
 
-def measured_traffic(workload):
-    """HBM bytes per k_owner_block launch from the committed counter summary, or None."""
-    return profile_value(workload, "traffic_bytes_per_launch", int)
+def measured_traffic(engine, workload):
+    """Bytes beyond the L2 per call of the engine from the committed counter summary, or None."""
+    return profile_value(engine, workload, "traffic_bytes_per_launch", int)
 
 
 def make_graph(spec, weighted):
@@ -335,15 +336,16 @@ def run_served(args):
         fifo.run(reqs, res)
         api.profile_enable(False)
         _, ms = api.profile_query(None)
-        owner = sum(api.profile_query(k)[1] for k in ("owner_block", "owner_small"))
+        owner = sum(api.profile_query(k)[1] for k in api.profile_names()
+                    if k in ("owner_block", "owner_small") or k.startswith("tri_"))
         api.profile_reset()
         del res
         return ms, owner
 
     dev_ms, _ = plain_device_ms(burst)
-    # the burst's full-graph requests: the owner-engine passes no schedule can
-    # avoid (continuous batching merges them into fewer launches but still
-    # streams every requested row once) bound the continuous throughput
+    # the burst's full-graph requests: the engine passes no schedule can avoid
+    # (continuous batching merges them into fewer launches but still computes
+    # every requested graph) bound the continuous throughput
     full = [q for q in burst if q.kind == serve.REQ_FULL]
     full_ms, full_owner_ms = plain_device_ms(full)
     b = out["burst"]
@@ -354,7 +356,7 @@ def run_served(args):
     b["full_owner_kernel_ms"] = full_owner_ms
     b["owner_bound_throughput_ratio"] = b["plain"]["wall_s"] * 1e3 / full_owner_ms if full_owner_ms else None
     print(f"[bench] serving burst device work {dev_ms:.1f} ms (full-graph requests {full_ms:.1f} ms, of which "
-          f"owner kernels {full_owner_ms:.1f} ms): continuous/plain at most "
+          f"engine kernels {full_owner_ms:.1f} ms): continuous/plain at most "
           f"{b['owner_bound_throughput_ratio']:.2f}x", file=sys.stderr, flush=True)
     plain_cap = out["burst"]["plain"]["requests_per_s"]
     # below the plain path's capacity (latency at moderate load), then above it
@@ -569,8 +571,8 @@ def main():
         api.jaccard(dg, out, weights=W if weighted else None, edge_centric=ec, stream=stream, tuning=tuning)
         torch.cuda.synchronize()
         calls.append((time.perf_counter() - t1) * 1e3)
-    # the committed counter summaries describe the owner engine's default kernels
-    traffic = None if args.hash_table32 or engine == "oriented" else measured_traffic(args.workload)
+    # the committed counter summaries describe the default, edge-centric kernels
+    traffic = None if args.hash_table32 else measured_traffic(engine, args.workload)
     Bc = compulsory_bytes(g, weighted)
     extras = {"device_ms_per_step": dev_ms,
               "kernel_ms_per_step": {k: t / args.steps for k, (c, t) in kern.items()},
@@ -578,7 +580,7 @@ def main():
               "call_ms": sorted(calls)[1],
               "compulsory_bytes": Bc,
               "compulsory_frac": Bc / (dev_ms * 1e-3) / HBM_PEAK if dev_ms else None,
-              "tcc_hit_rate": profile_value(args.workload, "tcc_hit_rate"),
+              "tcc_hit_rate": profile_value(engine, args.workload, "tcc_hit_rate"),
               "sum_min_deg": st["sum_min_deg"], "max_deg": st["max_deg"]}
     if args.extras:
         for name, kw in (("vc", dict(edge_centric=False)), ("ec_unweighted", dict(edge_centric=True))):

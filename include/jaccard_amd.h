@@ -347,7 +347,8 @@ int jc_profile_names(char *buf, size_t len);
  * JC_SERVE_CONTINUOUS mode requests that arrive while others run are admitted
  * into the next batch as soon as a slot (a HIP stream) and memory from the
  * HBM budget are free: one batch runs the whole-graph requests of several
- * graphs in one owner-engine launch over their row ranges and all pair
+ * graphs in one engine pass (over their row ranges, or from 3 * 2^20 stored
+ * edges on and where the budget has the memory over a copy of them) and all pair
  * requests in one pair launch, and up to `slots` batches overlap on the
  * device. JC_SERVE_FIFO serves one request at a time in arrival order with
  * the plain entry points (jc_jaccard, jc_jaccard_list) on each graph's own
