@@ -83,7 +83,7 @@ bool tiny_wanted(const jc_csr* g, bool weighted, const jc_tuning* t) {
 bool tri_wanted(const jc_csr* g, bool weighted, const jc_tuning* t) {
   if (t && (t->engine == JC_ENGINE_OWNER || t->wide_index || t->hash_table == 1 || t->quot_max_disp > 0)) return false;
   if (!jc::tri_can(g->n, g->m)) return false;
-  return (t && t->engine == JC_ENGINE_ORIENTED) || ((!t || t->members) && g->m >= jc::tri_min_edges(weighted));
+  return (t && t->engine == JC_ENGINE_ORIENTED) || ((!t || t->members) && jc::tri_pays(g->n, g->m, weighted));
 }
 
 // Weighted pair lists: sum every row of the graph once before the pairs, or
@@ -140,7 +140,7 @@ int run_jaccard(const jc_csr* g, const float* vw, float* result, bool ec, unsign
   double* S64 = weighted ? reinterpret_cast<double*>(ws + L.s64) : nullptr;
   if (ec || tri_ws) {
     // one launch: the sentinels, the schedule's counters, the range facts
-    const bool ex = weighted && jc::rowsum_one_launch(g->m);
+    const bool ex = weighted && jc::rowsum_one_launch(g->n, g->m);
     JC_TRY(jc::launch_prepare(fixup ? reinterpret_cast<uint32_t*>(result) : nullptr, g->m, jc::kSentinel32,
                               reinterpret_cast<int*>(ws + L.engine), jc::engine_counter_words(),
                               ex ? reinterpret_cast<jc::ExactInfo*>(ws + L.exact) : nullptr, s, a.skip));
@@ -148,7 +148,7 @@ int run_jaccard(const jc_csr* g, const float* vw, float* result, bool ec, unsign
   }
   if (weighted) {
     jc::ExactInfo* ex = reinterpret_cast<jc::ExactInfo*>(ws + L.exact);
-    if (jc::rowsum_one_launch(g->m)) {
+    if (jc::rowsum_one_launch(g->n, g->m)) {
       if (!ec && !tri_ws) JC_TRY(jc::launch_prepare(nullptr, 0, 0u, nullptr, 0, ex, s));
       JC_TRY(jc::launch_rowsum_exact(g->n, g->offsets, g->indices, vw, S64, ex, s, a.skip));
     } else {
@@ -230,7 +230,7 @@ extern "C" {
 size_t jc_jaccard_workspace_size(int32_t n, int32_t m, int weighted, int edge_centric) {
   if (n < 0 || m < 0) return 0;
   size_t b = layout(n, m, weighted != 0, edge_centric != 0).total;
-  if (m >= jc::tri_min_edges(weighted != 0)) b += al(jc::tri_workspace_bytes(n, m, weighted != 0));
+  if (jc::tri_pays(n, m, weighted != 0)) b += al(jc::tri_workspace_bytes(n, m, weighted != 0));
   return b;
 }
 

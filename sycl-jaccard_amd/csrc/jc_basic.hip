@@ -334,6 +334,9 @@ constexpr int kOneU = 8;  // loads in flight per thread in those
 // 8.4M 31 / 43 and 45 / 61, 19.2M 60 / 107 and 69 / 108; uniform random 16M 36 /
 // 104 and 52 / 112.
 constexpr int64_t kOneMaxEdges = 20 << 20;
+// Above, the scattered order costs more than the launches: uniform random, 1M
+// vertices and 2M entries 29 / 41 us and 42 / 46, 4M and 8M 103 / 225 and 84 / 147.
+constexpr int32_t kOneMaxRows = 2 << 20;
 
 __device__ __forceinline__ void exact_fact(float w, int& lsb, int& bad) {
   const uint32_t b = __float_as_uint(w);
@@ -489,7 +492,7 @@ uint32_t step_one(int32_t n) {
   return std::max(p, 1u);
 }
 
-bool rowsum_one_launch(int64_t m) { return m <= kOneMaxEdges; }
+bool rowsum_one_launch(int32_t n, int64_t m) { return m <= kOneMaxEdges && n <= kOneMaxRows; }
 
 hipError_t launch_rowsum_exact(int32_t n, const int32_t* off, const int32_t* ind, const float* v, double* S,
                                ExactInfo* info, hipStream_t s, const int* skip) {
@@ -527,7 +530,7 @@ size_t rowsum_scratch_bytes(int32_t n) { return ((size_t)std::max(n, 1) + 4) * s
 template <typename OutT>
 static hipError_t rowsum_both(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* v, OutT* out,
                               void* scratch, hipStream_t s, const int* skip = nullptr) {
-  if (rowsum_one_launch(m)) {
+  if (rowsum_one_launch(n, m)) {
     if (ind)
       hipLaunchKernelGGL((k_rowsum_one<OutT, true, false>), dim3(grid_one(n)), dim3(256), 0, s, n, off, ind, v, out,
                          (ExactInfo*)nullptr, step_one(n), skip);

@@ -133,6 +133,11 @@ constexpr int32_t tri_min_edges(bool weighted) { return weighted ? 3 << 20 : 6 <
 // engine's 4 m words from a mean row of 1024 entries on; a uniform random graph
 // reaches them at 768)
 constexpr bool tri_can(int32_t n, int64_t m) { return n <= kTriMaxN && m <= 768ll * n; }
+// Where it is tried without being asked for. (Below a mean row of 2 entries its
+// arrays over the vertices, 100 bytes of each, would be the most of it.)
+constexpr bool tri_pays(int32_t n, int64_t m, bool weighted) {
+  return m >= tri_min_edges(weighted) && m >= 2ll * n && tri_can(n, m);
+}
 constexpr int32_t kTriPart = 65536;  // vertices of a member (EngineArgs::members), at most
 // bits: quarter words of bit matrix per stored entry; a graph that needs more is
 // refused after orient. RMAT graphs need 1 (16 entries per vertex of 2^12) to 5.
@@ -185,9 +190,9 @@ hipError_t launch_rowsum_f64(int32_t n, int64_t m, const int32_t* off, const int
                              double* S, void* scratch, hipStream_t s, const int* skip = nullptr);
 hipError_t launch_vertex_weights(int32_t n, int64_t m, const int32_t* off, const float* edge_w, float* W,
                                  void* scratch, hipStream_t s);
-// Row sums of graphs of up to m stored edges are one launch, which can also
+// Row sums of graphs of n vertices and m stored edges are one launch, which can also
 // fill *info (as launch_exact_info, into a started ExactInfo: launch_prepare).
-bool rowsum_one_launch(int64_t m);
+bool rowsum_one_launch(int32_t n, int64_t m);
 hipError_t launch_rowsum_exact(int32_t n, const int32_t* off, const int32_t* ind, const float* v, double* S,
                                ExactInfo* info, hipStream_t s, const int* skip = nullptr);
 // x[0, n) = v (x may be nullptr; skip: as EngineArgs::skip), zero[0, nzero) = 0, *info (may be nullptr) started.

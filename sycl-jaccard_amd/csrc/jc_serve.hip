@@ -484,7 +484,7 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
   // Whole graphs of so many rows and entries can go to the oriented engine, given
   // so much memory in one piece.
   auto copy_fits_in = [&](size_t room, int nseg, int32_t R, int64_t E) {
-    return E >= jc::tri_min_edges(s->weighted) && jc::tri_can(R, E) &&
+    return jc::tri_pays(R, E, s->weighted) &&
            jc::copy_layout(nseg, R, E, s->weighted, kMinBits).total + s->pool.cap() / 8 <= room;
   };
   auto copy_fits = [&](int nseg, int32_t R, int64_t E) { return copy_fits_in(s->pool.largest(), nseg, R, E); };
@@ -560,7 +560,7 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
     size_t off2 = 0;
     bool tri = false;
     int bits = jc::kTriBits;
-    if (nseg > 0 && E >= jc::tri_min_edges(s->weighted) && jc::tri_can(R, E)) {
+    if (nseg > 0 && jc::tri_pays(R, E, s->weighted)) {
       for (; !tri && bits >= kMinBits; bits -= tri ? 0 : 1) {
         C = jc::copy_layout(nseg, R, E, s->weighted, bits);
         tri = s->pool.largest() >= C.total + s->pool.cap() / 16 && s->pool.alloc(C.total, &off2);

@@ -89,3 +89,32 @@ def test_small_graphs(name, cuda):
         assert torch.equal(o.view(torch.int32), outs[0].view(torch.int32))
         o = o.cpu().numpy().astype(np.float64)
         assert np.all(np.abs(o - refw) <= 1e-6 * np.abs(refw))
+
+
+@pytest.mark.parametrize("n", [(2 << 20) - 1, 2 << 20, (2 << 20) + 1])
+def test_row_sums_of_many_rows(n, cuda):
+    """Both sides of the number of rows that row sums take in one launch: a
+    row of 70,000 entries, one of 1,500, short ones, empty ones at both ends."""
+    import torch
+    rng = np.random.default_rng(n)
+    deg = np.zeros(n, np.int64)
+    deg[rng.integers(10, n - 10, 50000)] = rng.integers(1, 40, 50000)
+    deg[n // 2], deg[n // 3] = 70000, 1500
+    off = np.concatenate([[0], np.cumsum(deg)])
+    ind = rng.integers(0, n, off[-1]).astype(np.int32)
+    w = rng.random(off[-1]).astype(np.float32)
+    v = rng.random(n).astype(np.float32)
+    print(f"[gpu] row sums n={n} m={off[-1]}", flush=True)
+    dg = api.DeviceCSR(n, torch.from_numpy(off.astype(np.int32)).to(cuda), torch.from_numpy(ind).to(cuda),
+                       torch.from_numpy(w).to(cuda))
+    live = np.flatnonzero(deg)
+
+    def sums(x):
+        s = np.zeros(n)
+        s[live] = np.add.reduceat(x.astype(np.float64), off[live])
+        return s
+
+    np.testing.assert_allclose(api.vertex_weights(dg).cpu().numpy(), sums(w), rtol=1e-6, atol=0)
+    out = torch.empty(n, device=cuda)
+    api.rowsum(dg, out, v=torch.from_numpy(v).to(cuda))
+    np.testing.assert_allclose(out.cpu().numpy(), sums(v[ind]), rtol=1e-6, atol=0)
