@@ -19,7 +19,7 @@
 // What bounds it then is the gathers of the search's last steps. Measured on
 // RMAT of 2^18 vertices (7.6M entries), half edges and half random pairs, one
 // wave per pair before: 64 pairs 48 -> 14 us unweighted, 102 -> 19 weighted;
-// 1000 pairs 121 -> 18 and 191 -> 32; 65536 pairs 286 -> 115 and 568 -> 216.
+// 1000 pairs 121 -> 18 and 191 -> 32; 65536 pairs 286 -> 115 and 568 -> 197.
 #include "jc_engine.hpp"
 
 namespace jc {
