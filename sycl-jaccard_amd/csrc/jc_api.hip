@@ -89,7 +89,8 @@ bool tri_wanted(const jc_csr* g, bool weighted, const jc_tuning* t) {
 // Weighted pair lists: sum every row of the graph once before the pairs, or
 // the two rows of each pair. Once / per pair, us, whole calls: 65536 pairs on
 // RMAT of 2^15 vertices (0.9M entries) 68 / 125, 2^18 (7.6M) 197 / 330, 2^20
-// (31M) 459 / 714; 8192 pairs 48 / 32, 85 / 63, and 330 / 163.
+// (31M) 459 / 714; 8192 pairs, with the row sums in five launches, 121 / 62 on the
+// second.
 // Under capture the call stays one kernel node without an allocation.
 bool pairs_sum_all(const jc_csr* g, int64_t np, hipStream_t s) {
   if (np < 16384 || g->m > 512 * np) return false;
