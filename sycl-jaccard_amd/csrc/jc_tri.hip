@@ -33,7 +33,7 @@
 // No part depends on the order of the sums: counts are integers, and weights
 // are added in fp64 only when ExactInfo shows that every sum is exact. What
 // the engine cannot do it refuses before anything is written to the result
-// (TriCtl::bad): a graph that is not symmetric, has self loops or rows out of
+// (refuse): a graph that is not symmetric, has self loops or rows out of
 // order, weights
 // whose fp64 sums may round, a bit matrix larger than its budget, an |R(u)|
 // above kTriMaxOut. The owner engine, launched after it, then runs; when the
@@ -117,9 +117,18 @@ struct alignas(256) Own {
   T v;
 };
 
+// Why the engine may refuse a graph is found out in three stages, each with a
+// word of its own: a kernel reads the words of the stages before its own, which
+// no kernel in flight writes, and writes only its own stage's. So all waves of a
+// workgroup see the same and end together or not at all; with one word for all,
+// waves that found it set while the launch was under way left the others at
+// barriers and on LDS that nobody had filled.
+enum TriStage { kStRank, kStOrient, kStWedge, kStReduce };
+
 struct TriCtl {
-  int bad;
+  int bad_rank;
   int done;
+  int bad_orient, bad_wedge;
   Own<int> lsb, maxexp;             // exactness of the weights (see ExactInfo)
   Own<int> wexp;                    // every weight is below 2^wexp
   Own<unsigned long long> sampled;  // min(d_u, d_x, kSampleCap) over kSamples entries (u, x)
@@ -188,13 +197,26 @@ struct TriArgs {
   int accumulate;
 };
 
-__device__ __forceinline__ bool tri_go(const TriArgs& a) { return a.ctl->bad == 0; }
+// By a kernel of stage S: not this graph.
+template <int S>
+__device__ __forceinline__ void refuse(const TriArgs& a) {
+  static_assert(S < kStReduce, "reduce refuses nothing");
+  (S == kStRank ? a.ctl->bad_rank : S == kStOrient ? a.ctl->bad_orient : a.ctl->bad_wedge) = 1;
+}
 
-// after orient: the facts that must hold before wedge starts
-template <bool W>
-__device__ __forceinline__ bool tri_ready(const TriArgs& a) {
+// Whether the stages before S left the graph to S.
+template <int S>
+__device__ __forceinline__ bool tri_go(const TriArgs& a) {
   const TriCtl* c = a.ctl;
-  if (c->bad != 0 || 2ull * c->out_total.v != (unsigned long long)a.m || c->bits.v > a.bits_cap) return false;
+  return c->bad_rank == 0 && (S <= kStOrient || c->bad_orient == 0) && (S <= kStWedge || c->bad_wedge == 0);
+}
+
+// The same from wedge on, with the facts that must hold before it starts.
+template <bool W, int S>
+__device__ __forceinline__ bool tri_ready(const TriArgs& a) {
+  static_assert(S >= kStWedge, "plan counts what this looks at");
+  const TriCtl* c = a.ctl;
+  if (!tri_go<S>(a) || 2ull * c->out_total.v != (unsigned long long)a.m || c->bits.v > a.bits_cap) return false;
   if constexpr (W) return exact_sums_fit_f64(ExactInfo{c->lsb.v, c->maxexp.v, 0, 0});
   return true;
 }
@@ -231,7 +253,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_hist(TriArgs a) {
     }
     const int32_t x = a.ind[k];
     const int b = a.off[x], e = a.off[x + 1], at = lane_lower_bound(a.ind, b, e, lo);
-    if (at >= e || a.ind[at] != lo) a.ctl->bad = 1;
+    if (at >= e || a.ind[at] != lo) refuse<kStRank>(a);
     int len = min(min(a.off[lo + 1] - a.off[lo], e - b), kSampleCap);
 #pragma unroll
     for (int o = 1; o < kWave; o <<= 1) len += __shfl_xor(len, o);
@@ -270,7 +292,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_hist(TriArgs a) {
       lsb = min(lsb, __shfl_xor(lsb, o));
       top = max(top, __shfl_xor(top, o));
     }
-    if (ballot(bad) && lane_id() == 0) atomicOr(&a.ctl->bad, 1);
+    if (ballot(bad) && lane_id() == 0) refuse<kStRank>(a);
     if (lane_id() == 0 && lsb < *(volatile int*)&a.ctl->lsb.v) atomicMin(&a.ctl->lsb.v, lsb);
     if (lane_id() == 0 && top > *(volatile int*)&a.ctl->wexp.v) atomicMax(&a.ctl->wexp.v, top);
   }
@@ -300,15 +322,15 @@ __global__ __launch_bounds__(kTriBuckets) void k_tri_scan(TriCtl* c, int32_t n, 
   if (c->hist[b]) atomicMax(&s_top, b);
   __syncthreads();
   // a weight that alone is wider than fp64 sums can hold
-  if (b == 0 && c->lsb.v != INT32_MAX && c->wexp.v - c->lsb.v > 53) c->bad = 1;
+  if (b == 0 && c->lsb.v != INT32_MAX && c->wexp.v - c->lsb.v > 53) c->bad_rank = 1;
   if (b == 0 && !always) {
     const float len = (float)c->sampled.v / kSamples, d = (float)m / (float)n;
-    if (len < 48.f || (len < 96.f && len < 1.5f * d)) c->bad = 1;
+    if (len < 48.f || (len < 96.f && len < 1.5f * d)) c->bad_rank = 1;
     // the longest row's weights, were they the sampled ones' mean: sums that
     // surely round are not found out after orient only
     const int top = s_top < 512 ? s_top : (16 + (s_top & 15)) << ((s_top - 512) / 16 + 5);
     const double sum = (double)top * c->sampled_w.v / kSamples;
-    if (c->lsb.v != INT32_MAX && sum > 0.0 && ilogb(sum) - c->lsb.v > 53) c->bad = 1;
+    if (c->lsb.v != INT32_MAX && sum > 0.0 && ilogb(sum) - c->lsb.v > 53) c->bad_rank = 1;
   }
   const int v = c->hist[b];
   int incl = v;
@@ -515,7 +537,7 @@ __global__ __launch_bounds__(kTriBuckets) void k_tri_rank_parts(TriArgs a) {
     if (i >= count) return;
     const int32_t b0 = a.parts[i], b1 = i + 1 < count ? a.parts[i + 1] : a.n;
     if (b1 - b0 > kPartMax) {
-      if (tid == 0) a.ctl->bad = 1;
+      if (tid == 0) refuse<kStRank>(a);
       return;
     }
     for (int32_t u0 = b0; u0 < b1; u0 += 4 * kTriBuckets) {
@@ -544,7 +566,7 @@ __global__ __launch_bounds__(kTriBuckets) void k_tri_rank_parts(TriArgs a) {
     for (int k = 0; k < tid / kWave; ++k) before += part[k];
     base[b] = b0 + before + incl - v;
     // 16-bit ranks: every vertex with neighbours below kSat16
-    if (b == 0 && before + incl - v > kSat16) a.ctl->bad = 1;
+    if (b == 0 && before + incl - v > kSat16) refuse<kStRank>(a);
     __syncthreads();
     for (int32_t u0 = b0; u0 < b1; u0 += 4 * kTriBuckets) {
       int o[4], d[4];
@@ -578,7 +600,7 @@ __device__ __forceinline__ void put_row_sum(const TriArgs& a, int32_t ru, double
   if constexpr (W) {
     a.sr[ru] = s;
     if (!(s >= 0.0) || isinf(s)) {
-      a.ctl->bad = 1;
+      refuse<kStOrient>(a);
     } else if (s > 0.0) {
       const int e = ilogb(s) + 1;
       if (e > *(volatile int*)&a.ctl->maxexp.v) atomicMax(&a.ctl->maxexp.v, e);
@@ -629,7 +651,7 @@ __device__ __forceinline__ void orient_group(const TriArgs& a, bool valid, int32
     rw = a.rw[x];
   }
   const int32_t before = __shfl_up(x, 1);
-  if (in_row && (x == u || (gl > 0 && before >= x))) a.ctl->bad = 1;  // a self loop; a row out of order
+  if (in_row && (x == u || (gl > 0 && before >= x))) refuse<kStOrient>(a);  // a self loop; a row out of order
   const bool keep = in_row && rw.x < ru;
   const uint64_t km = ballot(keep);
   // kept ranks below mine: a lane that keeps nothing offers no rank
@@ -658,7 +680,7 @@ __device__ __forceinline__ void orient_group(const TriArgs& a, bool valid, int32
 // (Eight waves per SIMD: RMAT-22 0.86 -> 0.76 ms.)
 template <bool W, int BLOCK>
 __global__ __launch_bounds__(BLOCK, 8) void k_tri_orient_small(TriArgs a, int rows) {
-  if (!tri_go(a)) return;
+  if (!tri_go<kStOrient>(a)) return;
   const int lane = lane_id();
   const int nw = gridDim.x * (BLOCK / kWave);
   for (int64_t base = (int64_t)(blockIdx.x * (BLOCK / kWave) + threadIdx.x / kWave) * rows; base < a.n;
@@ -732,7 +754,7 @@ __device__ __forceinline__ void orient_row(const TriArgs& a, int32_t u, int tid,
       const int i = b + t * T + tid;
       const bool in_row = i < d;
       const bool keep = in_row && rw[t].x < ru;
-      if (in_row && (x[t] == u || (i > 0 && a.ind[o + i - 1] >= x[t]))) a.ctl->bad = 1;
+      if (in_row && (x[t] == u || (i > 0 && a.ind[o + i - 1] >= x[t]))) refuse<kStOrient>(a);
       const uint64_t km = ballot(keep);
       int at = 0;
       if constexpr (T == kWave) {
@@ -771,7 +793,7 @@ __device__ __forceinline__ void orient_row(const TriArgs& a, int32_t u, int tid,
   if (tid == 0) {
     put_row_sum<W>(a, ru, sum);
     put_info(a, u, o, cnt, me.y, ru);
-    if (cnt > CAP) a.ctl->bad = 1;
+    if (cnt > CAP) refuse<kStOrient>(a);
   }
   const int c = min(cnt, CAP);
   if (tid < 8) a.R16[8 * ((size_t)row16(o, u) + kHead) + c + tid] = (uint16_t)kSat16;
@@ -809,7 +831,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_orient_mid(TriArgs a) {
   __shared__ __align__(16) uint32_t s_r[NW][kTriRowWave + 4];
   __shared__ uint16_t s_k[NW][kTriRowWave];
   __shared__ int s_n[NW];
-  if (!tri_go(a)) return;
+  if (!tri_go<kStOrient>(a)) return;
   const int w = threadIdx.x / kWave;
   const int count = a.ctl->num_mid.v;
   for (int i = blockIdx.x * NW + w; i < count; i += gridDim.x * NW)
@@ -825,7 +847,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_orient_big(TriArgs a) {
   __shared__ int32_t s_k[kTriMaxOut];
   __shared__ int s_n, s_i;
   __shared__ double s_s;
-  if (!tri_go(a)) return;
+  if (!tri_go<kStOrient>(a)) return;
   const int count = a.ctl->num_big.v;
   for (int i = blockIdx.x; i < count;) {
     int next = 0;
@@ -848,7 +870,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_plan(TriArgs a) {
   __shared__ unsigned long long s_bw[NW], s_ow[NW];
   __shared__ int s_base[NL];
   __shared__ unsigned long long s_bbase;
-  if (!tri_go(a)) return;
+  if (!tri_go<kStWedge>(a)) return;
   const int lane = lane_id(), wv = threadIdx.x / kWave;
   for (int64_t b0 = (int64_t)blockIdx.x * BLOCK; b0 < a.n; b0 += (int64_t)gridDim.x * BLOCK) {
     const int32_t at_ord = (int32_t)(b0 + threadIdx.x);
@@ -1081,7 +1103,7 @@ __global__ __launch_bounds__(kWedgeB, (TAB <= kTabA ? 8 : 2)) void k_tri_wedge(T
   __shared__ uint16_t s_map[kMapCap];  // item | word << 9
   __shared__ int s_wsum[NW];
   __shared__ int s_task;
-  if (!tri_ready<W>(a)) return;
+  if (!tri_ready<W, kStWedge>(a)) return;
   const int tid = threadIdx.x, lane = lane_id(), w = tid / kWave;
   const int ntask = a.ctl->num_task[KIND].v;
   const unsigned char* const tabp = reinterpret_cast<const unsigned char*>(tab);
@@ -1130,7 +1152,7 @@ __global__ __launch_bounds__(kWedgeB, (TAB <= kTabA ? 8 : 2)) void k_tri_wedge(T
         if constexpr (KIND == 0) p = find_rank16(row_at(q), xi.y, (uint32_t)r, hd[1]);
         else p = find_rank(row_at(q), xi.y, (uint32_t)r);
         if (p < 0) {
-          a.ctl->bad = 1;  // (v, x) is stored, (x, v) is not
+          refuse<kStWedge>(a);  // (v, x) is stored, (x, v) is not
           p = 0;
         } else {
           a.emap[k] = xi.x + p;
@@ -1229,7 +1251,7 @@ __global__ __launch_bounds__(kWedgeB, 8) void k_tri_wedge_group(TriArgs a) {
   __shared__ int s_wsum[NW];
   __shared__ int s_task, s_d;
   __shared__ int s_gt[kGroupMax], s_gr[kGroupMax], s_ge[kGroupMax];  // per length: first task, first and end rank
-  if (!tri_ready<W>(a)) return;
+  if (!tri_ready<W, kStWedge>(a)) return;
   const int tid = threadIdx.x, lane = lane_id(), w = tid / kWave;
   const int ntask = a.ctl->num_group.v;
   s_gt[tid] = a.ctl->grp_task[tid];
@@ -1295,7 +1317,7 @@ __global__ __launch_bounds__(kWedgeB, 8) void k_tri_wedge_group(TriArgs a) {
         if (use16) p = find_rank16(reinterpret_cast<const uint16_t*>(hd + kHead), xi.y, r, hd[1]);
         else p = find_rank(a.R32 + xi.x, xi.y, r);
         if (p < 0) {
-          a.ctl->bad = 1;  // (v, x) is stored, (x, v) is not
+          refuse<kStWedge>(a);  // (v, x) is stored, (x, v) is not
           p = 0;
         } else {
           a.emap[ov + me.i] = xi.x + p;
@@ -1413,7 +1435,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_wedge_wave(TriArgs a) {
   __shared__ AT s_acc[NW][kWaveTab];
   __shared__ int4 s_item[NW][kWave];
   __shared__ uint16_t s_map[NW][kWaveMap];  // item | word << 6
-  if (!tri_ready<W>(a)) return;
+  if (!tri_ready<W, kStWedge>(a)) return;
   const int lane = lane_id(), w = threadIdx.x / kWave;
   const int count = a.ctl->num_wave.v;
   AT* const gacc = W ? (AT*)a.accw : (AT*)a.accu;
@@ -1448,7 +1470,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_wedge_wave(TriArgs a) {
           else
             p = find_rank(a.R32 + xi.x, xi.y, (uint32_t)r);
           if (p < 0) {
-            a.ctl->bad = 1;
+            refuse<kStWedge>(a);
             p = 0;
           } else {
             a.emap[k] = xi.x + p;
@@ -1600,7 +1622,7 @@ __device__ __forceinline__ void reduce_16(const TriArgs& a, bool valid, int32_t 
 
 template <bool W, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_tri_reduce_16(TriArgs a) {
-  if (!tri_ready<W>(a)) return;
+  if (!tri_ready<W, kStReduce>(a)) return;
   const int gw = blockIdx.x * (BLOCK / kWave) + threadIdx.x / kWave, nw = gridDim.x * (BLOCK / kWave);
   const int n16 = a.ctl->num_s16.v;
   for (int i = gw * 4; i < n16; i += nw * 4) {
@@ -1788,7 +1810,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_reduce_wave(TriArgs a) {
   constexpr int NW = BLOCK / kWave;
   __shared__ __align__(16) unsigned char dig[W ? NW : 1][W ? kRedWave * kDigits : 16];
   __shared__ __align__(16) int stage[W ? NW : 1][W ? kDigits * kRedRow : 4];
-  if (!tri_ready<W>(a)) return;
+  if (!tri_ready<W, kStReduce>(a)) return;
   const int w = threadIdx.x / kWave;
   const int count = a.ctl->num_s64.v;
   for (int i = blockIdx.x * NW + w; i < count; i += gridDim.x * NW)
@@ -1802,7 +1824,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_reduce_wg(TriArgs a) {
   __shared__ __align__(16) unsigned char dig[W ? CAP * kDigits : 16];
   __shared__ __align__(16) int stage[W ? NW : 1][W ? kDigits * kRedRow : 4];
   __shared__ int s_i;
-  if (!tri_ready<W>(a)) return;
+  if (!tri_ready<W, kStReduce>(a)) return;
   const int count = a.ctl->num_red[L].v;
   for (int i = blockIdx.x; i < count;) {
     int next = 0;
@@ -1816,7 +1838,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_reduce_wg(TriArgs a) {
 
 template <bool W>
 __global__ __launch_bounds__(256) void k_tri_deliver(TriArgs a) {
-  if (!tri_ready<W>(a)) return;
+  if (!tri_ready<W, kStReduce>(a)) return;
   if (blockIdx.x == 0 && threadIdx.x == 0) a.ctl->done = 1;
   const int64_t nt = (int64_t)gridDim.x * blockDim.x;
   if (a.mode == kModeIsF32) {
