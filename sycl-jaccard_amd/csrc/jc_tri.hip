@@ -98,6 +98,10 @@ __device__ __forceinline__ uint32_t tri_words(int L) {
 __host__ __device__ __forceinline__ uint64_t row16_line(uint64_t o, uint64_t u) { return ((o + 24 * u) >> 6) + u; }
 __device__ __forceinline__ uint32_t row16(int o, int32_t u) { return 8u * (uint32_t)row16_line((uint64_t)o, (uint64_t)u); }
 constexpr int kHead = 2;
+// In place of row16 where a row is empty: such a row gets no header, so no
+// entry may lead to one. In a symmetric graph none does; orient refuses the
+// graph at the first that would.
+constexpr int kNoRow = -1;
 
 // A task of the bitmap wedge kernels.
 struct __attribute__((aligned(32))) TriTask {
@@ -160,7 +164,7 @@ struct TriArgs {
   const int32_t* ind;
   const float* vw;
   TriCtl* ctl;
-  int4* rw;         // per vertex: rank, weight bits, place of its 16-bit row, first rank of its part
+  int4* rw;         // per vertex: rank, weight bits, place of its 16-bit row (kNoRow: it has no entries), first rank of its part
   int32_t* vtx;     // per rank: vertex
   float* wr;        // per rank: weight
   double* sr;       // per rank: row sum of the weights (unweighted: unused)
@@ -407,7 +411,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_rank(TriArgs a) {
     a.dord[r] = d;
     if (!a.members) {
       const float w = W ? a.vw[u] : 0.0f;
-      a.rw[u] = make_int4(r, __float_as_int(w), (int)row16(o, u), 0);
+      a.rw[u] = make_int4(r, __float_as_int(w), d > 0 ? (int)row16(o, u) : kNoRow, 0);
       if constexpr (W) a.wr[r] = w;
     }
     if (d > kTriRowWave) a.list_big[s_base[1] + atomicAdd(&s_cnt[1], 1)] = u;
@@ -583,7 +587,7 @@ __global__ __launch_bounds__(kTriBuckets) void k_tri_rank_parts(TriArgs a) {
         const int32_t u = u0 + t * kTriBuckets + tid;
         if (u < b1) {
           const int r = atomicAdd(&base[deg_bucket(d[t])], 1);
-          a.rw[u] = make_int4(r, __float_as_int(w[t]), (int)row16(o[t], u), b0);
+          a.rw[u] = make_int4(r, __float_as_int(w[t]), d[t] > 0 ? (int)row16(o[t], u) : kNoRow, b0);
           a.vtx[r] = u;
           a.dr[r] = d[t];
           if constexpr (W) a.wr[r] = w[t];
@@ -651,7 +655,8 @@ __device__ __forceinline__ void orient_group(const TriArgs& a, bool valid, int32
     rw = a.rw[x];
   }
   const int32_t before = __shfl_up(x, 1);
-  if (in_row && (x == u || (gl > 0 && before >= x))) refuse<kStOrient>(a);  // a self loop; a row out of order
+  // a self loop; a row out of order; a neighbour without entries of its own
+  if (in_row && (x == u || (gl > 0 && before >= x) || rw.z == kNoRow)) refuse<kStOrient>(a);
   const bool keep = in_row && rw.x < ru;
   const uint64_t km = ballot(keep);
   // kept ranks below mine: a lane that keeps nothing offers no rank
@@ -754,7 +759,7 @@ __device__ __forceinline__ void orient_row(const TriArgs& a, int32_t u, int tid,
       const int i = b + t * T + tid;
       const bool in_row = i < d;
       const bool keep = in_row && rw[t].x < ru;
-      if (in_row && (x[t] == u || (i > 0 && a.ind[o + i - 1] >= x[t]))) refuse<kStOrient>(a);
+      if (in_row && (x[t] == u || (i > 0 && a.ind[o + i - 1] >= x[t]) || rw[t].z == kNoRow)) refuse<kStOrient>(a);
       const uint64_t km = ballot(keep);
       int at = 0;
       if constexpr (T == kWave) {

@@ -32,7 +32,8 @@ def without(g, entries):
 
 def balanced(g, degree):
     """g less (x, v), x of the given degree and v above it, and less (h, l), h
-    the vertex of most neighbours and l one of its lesser ones."""
+    the vertex of most neighbours and l one of its lesser ones. With degree 1
+    the row of x is then empty, and v still names it."""
     deg = np.diff(g.offsets)
     row = lambda u: g.indices[g.offsets[u]:g.offsets[u + 1]]
     h = int(np.argmax(deg))
@@ -87,7 +88,7 @@ def test_self_loops(shortest, cuda):
         assert not done and same(out, api.jaccard(dg, weights=W, tuning=dict(engine=api.ENGINE_OWNER)))
 
 
-@pytest.mark.parametrize("degree", [3])
+@pytest.mark.parametrize("degree", [1, 3])
 def test_missing_mirrors_that_balance(degree, cuda):
     import torch
     g = graphs.rmat(14, 16, seed=2)
@@ -107,3 +108,20 @@ def test_missing_mirrors_that_balance(degree, cuda):
         assert done
         out, done = call(dg, W, ws, cuda)
         assert not done and same(out, own)
+
+
+def test_default_route(cuda):
+    """The same from the size on at which the plain call tries the engine."""
+    import torch
+    g = graphs.rmat(18, 16, seed=9)
+    a = balanced(g, 1)
+    assert a.m >= 3 << 20
+    W = torch.from_numpy(grid_weights(g.n, 3)).to(cuda)
+    dg, whole = (api.DeviceCSR.from_host(x, cuda) for x in (a, g))
+    own = api.jaccard(dg, weights=W, tuning=dict(engine=api.ENGINE_OWNER))
+    ws = torch.full((api.workspace_size(g.n, g.m, True, True),), 0x5A, dtype=torch.uint8, device=cuda)
+    print(f"[gpu] asymmetric default n={a.n} m={a.m}", flush=True)
+    assert same(api.jaccard(dg, weights=W, workspace=ws), own)
+    api.jaccard(whole, weights=W, workspace=ws)
+    assert same(api.jaccard(dg, weights=W, workspace=ws), own)
+    assert same(api.jaccard(dg, weights=W), own)
