@@ -421,7 +421,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_rank(TriArgs a) {
 
 // Disjoint parts of a batch. A part begins at a vertex with neighbours that no
 // row before it reaches past; vertices without neighbours belong to the part
-// before them. Per contiguous range of vertices: the largest neighbour id ...
+// before them, or to the first one. Per contiguous range of vertices: the largest neighbour id ...
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_tri_reach(TriArgs a) {
   __shared__ int s_max;
@@ -539,8 +539,9 @@ __global__ __launch_bounds__(kTriBuckets) void k_tri_rank_parts(TriArgs a) {
     __syncthreads();
     const int i = s_i;
     if (i >= count) return;
-    const int32_t b0 = a.parts[i], b1 = i + 1 < count ? a.parts[i + 1] : a.n;
-    if (b1 - b0 > kPartMax) {
+    // (every vertex has to be in a part: entries may name any of them)
+    const int32_t first = a.parts[i], b0 = i > 0 ? first : 0, b1 = i + 1 < count ? a.parts[i + 1] : a.n;
+    if (b1 - first > kPartMax) {
       if (tid == 0) refuse<kStRank>(a);
       return;
     }

@@ -125,3 +125,31 @@ def test_default_route(cuda):
     api.jaccard(whole, weights=W, workspace=ws)
     assert same(api.jaccard(dg, weights=W, workspace=ws), own)
     assert same(api.jaccard(dg, weights=W), own)
+
+
+def test_entry_before_the_first_part(cuda):
+    """A batch that begins with vertices without neighbours, and an entry that
+    names one of them all the same; another is missing, so the counts agree."""
+    import torch
+    from jaccard_amd import batch
+    pad = 37
+    u = batch.rmat_batch([700, 9001, 4096], [9.0, 12.0, 16.0], [1, 2, 3], False).union
+    g = graphs.CSRGraph(u.n + pad, np.concatenate([np.zeros(pad, np.int32), u.offsets]).astype(np.int32),
+                        (u.indices + pad).astype(np.int32))
+    deg = np.diff(g.offsets)
+    h = int(np.argmax(deg))
+    a = without(g, [(h, next(int(l) for l in g.indices[g.offsets[h]:g.offsets[h + 1]] if 4 <= deg[l] < deg[h] // 4))])
+    v = int(np.flatnonzero(deg > 40)[0])  # in the first part: 3 ranks after it
+    off = a.offsets.copy()
+    off[v + 1:] += 1
+    a = graphs.CSRGraph(a.n, off, np.insert(a.indices, a.offsets[v], 3).astype(np.int32))
+    assert a.m == g.m
+    dg = api.DeviceCSR.from_host(a, cuda)
+    for weighted in (False, True):
+        W = torch.from_numpy(grid_weights(a.n, 7)).to(cuda) if weighted else None
+        need = api.workspace_size(a.n, a.m, weighted, True)
+        ws = torch.full((need + 64 * a.m + 256 * a.n + (1 << 20),), 0x5A, dtype=torch.uint8, device=cuda)
+        print(f"[gpu] asymmetric members weighted={weighted} n={a.n} m={a.m}", flush=True)
+        out = api.jaccard(dg, weights=W, workspace=ws, tuning=dict(engine=api.ENGINE_ORIENTED, members=1))
+        assert int(ws[need + 4:need + 8].view(torch.int32)) == 0
+        assert same(out, api.jaccard(dg, weights=W, tuning=dict(engine=api.ENGINE_OWNER)))
