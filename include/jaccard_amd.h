@@ -152,9 +152,11 @@ typedef struct jc_tuning {
 int jc_jaccard_noalloc(const jc_csr *g, const float *vertex_weights, float *result, int edge_centric,
                        unsigned flags, jc_stream_t stream);
 
-/* Calls that take no workspace allocate theirs on their stream, from a pool of
- * the library's own that keeps up to 2 GiB per device for the calls to come.
- * This gives back to the system what no call is using (of every device). Safe
+/* Calls that take no workspace use one that the library keeps, one per stream
+ * that has work under way, of the size of its largest call: together up to 8 GiB
+ * per device (one for RMAT-22 is 5.65 GB; jc_csr_from_edges leaves 2 GiB at most). Calls that need more, or find them all
+ * in use, allocate theirs on their stream, or use the owner engine, whose workspace is
+ * smaller. This gives back to the system what no call is using (of every device). Safe
  * at any time, from any thread. No reference counterpart. */
 int jc_release_workspaces(void);
 

@@ -102,15 +102,6 @@ bool pairs_sum_all(const jc_csr* g, int64_t np, hipStream_t s) {
   return st == hipStreamCaptureStatusNone;
 }
 
-// RAII for a stream-ordered allocation.
-struct AsyncBuf {
-  void* p = nullptr;
-  hipStream_t s = nullptr;
-  ~AsyncBuf() {
-    if (p) (void)hipFreeAsync(p, s);
-  }
-};
-
 // ws: layout(...).total bytes; tri_ws: tri_workspace_bytes(...) bytes, or
 // nullptr to run the owner engine alone.
 int run_jaccard(const jc_csr* g, const float* vw, float* result, bool ec, unsigned flags,
@@ -256,14 +247,12 @@ int jc_jaccard_tuned(const jc_csr* g, const float* vertex_weights, float* result
     return run_jaccard(g, vertex_weights, result, ec, flags, ws,
                        tri && workspace_bytes >= full ? ws + need : nullptr, tuning, s);
   }
-  AsyncBuf buf;
-  buf.s = s;
-  if (tri && jc::call_alloc(&buf.p, full, s) != hipSuccess) {
+  jc::CallBuf buf;
+  if (tri && buf.get(full, s, jc::CallBuf::kOptional) != hipSuccess) {
     (void)hipGetLastError();
-    buf.p = nullptr;
     tri = false;  // the owner engine needs a small part of it
   }
-  if (!tri) JC_TRY(jc::call_alloc(&buf.p, need, s));
+  if (!tri) JC_TRY(buf.get(need, s));
   unsigned char* ws = static_cast<unsigned char*>(buf.p);
   return run_jaccard(g, vertex_weights, result, ec, flags, ws, tri ? ws + need : nullptr, tuning, s);
 }
@@ -305,17 +294,15 @@ int jc_jaccard_list(const jc_csr* g, const float* vertex_weights, int32_t num_pa
   if (!first || !second || !result || g->n == 0) return JC_ERR_INVALID_ARG;
   const bool weighted = vertex_weights != nullptr;
   hipStream_t s = hs(stream);
-  AsyncBuf buf;
-  buf.s = s;
+  jc::CallBuf buf;
   double* S64 = nullptr;
   if (weighted && pairs_sum_all(g, num_pairs, s)) {
     const size_t rows_b = al(jc::rowsum_scratch_bytes(g->n));
-    if (jc::call_alloc(&buf.p, rows_b + al((size_t)g->n * sizeof(double)), s) == hipSuccess) {
+    if (buf.get(rows_b + al((size_t)g->n * sizeof(double)), s, jc::CallBuf::kOptional) == hipSuccess) {
       S64 = reinterpret_cast<double*>(static_cast<unsigned char*>(buf.p) + rows_b);
       JC_TRY(jc::launch_rowsum_f64(g->n, g->m, g->offsets, g->indices, vertex_weights, S64, buf.p, s));
     } else {
-      (void)hipGetLastError();
-      buf.p = nullptr;  // the pair kernel sums the rows
+      (void)hipGetLastError();  // the pair kernel sums the rows
     }
   }
   JC_TRY(jc::run_pairs(weighted ? jc::kModeEcW : jc::kModeEcU, weighted, g->n, g->offsets, g->indices,
@@ -353,9 +340,8 @@ int jc_nonzero_count(int32_t m, const float* result, float thresh, int64_t* coun
   *count = 0;
   if (m == 0) return JC_OK;
   hipStream_t s = hs(stream);
-  AsyncBuf buf;
-  buf.s = s;
-  JC_TRY(jc::call_alloc(&buf.p, sizeof(unsigned long long), s));
+  jc::CallBuf buf;
+  JC_TRY(buf.get(sizeof(unsigned long long), s));
   auto* c = static_cast<unsigned long long*>(buf.p);
   JC_TRY(jc::launch_fill_u64(reinterpret_cast<uint64_t*>(c), 1, 0ull, s));
   JC_TRY(jc::launch_count_above(m, result, thresh, c, s));
@@ -386,15 +372,13 @@ int jc_intersect(int32_t n, int32_t m, const int32_t* offsets, const int32_t* in
   if (n == 0 || m == 0) return JC_OK;
   hipStream_t s = hs(stream);
   const size_t need = al(jc::engine_workspace_bytes(n, m));
-  AsyncBuf buf;
-  buf.s = s;
+  jc::CallBuf buf;
   bool tri = tri_wanted(&g, v != nullptr, nullptr);
-  if (tri && jc::call_alloc(&buf.p, need + jc::tri_workspace_bytes(n, m, v != nullptr), s) != hipSuccess) {
+  if (tri && buf.get(need + jc::tri_workspace_bytes(n, m, v != nullptr), s, jc::CallBuf::kOptional) != hipSuccess) {
     (void)hipGetLastError();
-    buf.p = nullptr;
     tri = false;
   }
-  if (!tri) JC_TRY(jc::call_alloc(&buf.p, need, s));
+  if (!tri) JC_TRY(buf.get(need, s));
   jc::EngineArgs a{};
   a.n = n;
   a.m = m;
@@ -455,9 +439,8 @@ int jc_weighted_sum_mode(const jc_csr* g, const float* vertex_weights, int* mode
   // the row sums and range facts exactly as run_jaccard computes them
   const size_t rows_b = al(jc::rowsum_scratch_bytes(g->n));
   const size_t s64_b = al((size_t)g->n * sizeof(double));
-  AsyncBuf buf;
-  buf.s = s;
-  JC_TRY(jc::call_alloc(&buf.p, rows_b + s64_b + al(sizeof(jc::ExactInfo)), s));
+  jc::CallBuf buf;
+  JC_TRY(buf.get(rows_b + s64_b + al(sizeof(jc::ExactInfo)), s));
   unsigned char* p = static_cast<unsigned char*>(buf.p);
   double* S64 = reinterpret_cast<double*>(p + rows_b);
   jc::ExactInfo* ex = reinterpret_cast<jc::ExactInfo*>(p + rows_b + s64_b);
@@ -477,9 +460,8 @@ int jc_degree_stats(const jc_csr* g, jc_graph_stats* stats, jc_stream_t stream) 
   if (g->n == 0) return JC_OK;
   hipStream_t s = hs(stream);
   constexpr int kWords = 69;  // see launch_degree_stats
-  AsyncBuf buf;
-  buf.s = s;
-  JC_TRY(jc::call_alloc(&buf.p, kWords * sizeof(unsigned long long), s));
+  jc::CallBuf buf;
+  JC_TRY(buf.get(kWords * sizeof(unsigned long long), s));
   auto* d = static_cast<unsigned long long*>(buf.p);
   JC_TRY(jc::launch_fill_u64(reinterpret_cast<uint64_t*>(d), kWords, 0ull, s));
   JC_TRY(jc::launch_degree_stats(g->n, g->offsets, g->indices, d, s));
@@ -524,9 +506,8 @@ int jc_validate_csr(const jc_csr* g, int* what, jc_stream_t stream) {
   if (!csr_args_ok(g)) return JC_ERR_INVALID_ARG;
   if (g->n == 0) return g->m == 0 ? JC_OK : JC_ERR_INVALID_CSR;
   hipStream_t s = hs(stream);
-  AsyncBuf buf;
-  buf.s = s;
-  JC_TRY(jc::call_alloc(&buf.p, 4 * sizeof(int), s));
+  jc::CallBuf buf;
+  JC_TRY(buf.get(4 * sizeof(int), s));
   int* f = static_cast<int*>(buf.p);
   JC_TRY(jc::launch_fill_u32(reinterpret_cast<uint32_t*>(f), 4, 0u, s));
   JC_TRY(jc::launch_validate(g->n, g->m, g->offsets, g->indices, f, s));
@@ -548,9 +529,8 @@ int jc_csr_is_symmetric(const jc_csr* g, int* symmetric, jc_stream_t stream) {
   *symmetric = 1;
   if (g->n == 0 || g->m == 0) return JC_OK;
   hipStream_t s = hs(stream);
-  AsyncBuf buf;
-  buf.s = s;
-  JC_TRY(jc::call_alloc(&buf.p, sizeof(int), s));
+  jc::CallBuf buf;
+  JC_TRY(buf.get(sizeof(int), s));
   int* f = static_cast<int*>(buf.p);
   JC_TRY(jc::launch_fill_u32(reinterpret_cast<uint32_t*>(f), 1, 0u, s));
   JC_TRY(jc::launch_symcheck(g->n, g->m, g->offsets, g->indices, f, s));

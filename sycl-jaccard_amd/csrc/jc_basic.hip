@@ -539,11 +539,11 @@ static hipError_t rowsum_both(int32_t n, int64_t m, const int32_t* off, const in
                          (ExactInfo*)nullptr, step_one(n), skip);
     return hipGetLastError();
   }
-  void* own = nullptr;
-  hipError_t err;
+  CallBuf own;
   if (!scratch) {
-    if ((err = call_alloc(&own, rowsum_scratch_bytes(n), s)) != hipSuccess) return err;
-    scratch = own;
+    const hipError_t err = own.get(rowsum_scratch_bytes(n), s);
+    if (err != hipSuccess) return err;
+    scratch = own.p;
   }
   int* counters = static_cast<int*>(scratch);
   int* list = counters + 4;
@@ -567,12 +567,7 @@ static hipError_t rowsum_both(int32_t n, int64_t m, const int32_t* off, const in
     hipLaunchKernelGGL((k_rowsum_w_long<OutT, false, 1024>), dim3(cus * 2), dim3(1024), 0, s, off, ind, v, out,
                        list, counters);
   }
-  err = hipGetLastError();
-  if (own) {
-    hipError_t e2 = hipFreeAsync(own, s);
-    if (err == hipSuccess) err = e2;
-  }
-  return err;
+  return hipGetLastError();
 }
 
 hipError_t launch_rowsum_f32(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* v,

@@ -208,8 +208,9 @@ hipError_t ingest(int32_t n, int64_t num_edges, int64_t e2, const int32_t* src, 
   const size_t o_tl = o; o += al((size_t)tiles * 4);
   const size_t o_ct = o; o += al(2 * sizeof(int32_t));
   const size_t o_tmp = o; o += al(sort_bytes);
-  unsigned char* ws = nullptr;
-  if ((err = call_alloc(reinterpret_cast<void**>(&ws), o, s)) != hipSuccess) return err;
+  CallBuf buf;
+  if ((err = buf.get(o, s, CallBuf::kOnce)) != hipSuccess) return err;
+  unsigned char* ws = static_cast<unsigned char*>(buf.p);
   Key* k0 = reinterpret_cast<Key*>(ws + o_k0);
   Key* k1 = reinterpret_cast<Key*>(ws + o_k1);
   float* v0 = weighted ? reinterpret_cast<float*>(ws + o_v0) : nullptr;
@@ -233,7 +234,6 @@ hipError_t ingest(int32_t n, int64_t num_edges, int64_t e2, const int32_t* src, 
     if ((err = hipMemcpyAsync(host, ctr, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, s)) != hipSuccess) break;
     err = hipStreamSynchronize(s);
   } while (false);
-  (void)hipFreeAsync(ws, s);
   return err;
 }
 

@@ -172,9 +172,26 @@ hipError_t launch_exact_info(int32_t n, const float* vw, const double* S, ExactI
 // Records a failing HIP call for jc_last_hip_error(); returns the JC_ERR_* code.
 int note_hip_error(hipError_t e);
 
-// Workspace of one call, stream-ordered (jc_mem.hip): as hipMallocAsync, freed
-// with hipFreeAsync, from a pool that keeps some of what is freed.
-hipError_t call_alloc(void** p, size_t bytes, hipStream_t s);
+// Workspace of one call (jc_mem.hip), for work on stream s from get() to
+// release(), as if by hipMallocAsync and hipFreeAsync; most of it memory that the
+// library keeps. kOptional: the caller can do without, and get() fails where a
+// large one would have to be fresh memory. kOnce: a call that programs do not
+// make over and over, for which less is kept.
+struct CallBuf {
+  enum Use { kNeeded, kOptional, kOnce };
+  void* p = nullptr;
+  CallBuf() = default;
+  CallBuf(const CallBuf&) = delete;
+  CallBuf& operator=(const CallBuf&) = delete;
+  ~CallBuf() { release(); }
+  hipError_t get(size_t bytes, hipStream_t stream, Use use = kNeeded);
+  void release();
+
+ private:
+  hipStream_t s = nullptr;
+  void* block = nullptr;  // the kept block, or nullptr
+  int device = 0;
+};
 
 // Streaming kernels.
 hipError_t launch_fill_f32(float* x, int64_t n, float v, hipStream_t s);

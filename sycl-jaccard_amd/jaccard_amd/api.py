@@ -210,7 +210,7 @@ def workspace_size(n: int, m: int, weighted: bool, edge_centric: bool) -> int:
 
 def release_workspaces() -> None:
     """Give back the device memory that the library keeps between calls
-    (``jc_release_workspaces``; up to 2 GiB per device, and none in use)."""
+    (``jc_release_workspaces``; up to 8 GiB per device, and none in use)."""
     _check(load_jaccard_lib().jc_release_workspaces(), "jc_release_workspaces")
 
 
