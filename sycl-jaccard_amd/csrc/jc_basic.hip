@@ -317,8 +317,10 @@ __global__ __launch_bounds__(BLOCK) void k_rowsum_w_long(const int32_t* __restri
 // Row sums of all but the largest graphs in one launch: the five launches of
 // the way above take 40 us however small the graph, this 6 to 8 (9001 vertices,
 // 2.4e5 entries). A workgroup takes 64 rows: rows up to kRowShort entries by 4
-// lanes each, up to kOneWave by a wave, longer ones by the workgroup. EX: also
-// the range facts of v and the sums (k_exact_scan). Pairs of rows come in an
+// lanes each, up to kOneWave by a wave, longer ones by the workgroup (and those
+// above kHubRow by one of k_rowsum_hubs). Fewer rows, down to 8, where 64 would
+// leave less than four workgroups per CU (3000 rows of 780 entries 36 -> 10 us, 20000
+// of 100 27 -> 12). EX: also the range facts of v and the sums (k_exact_scan). Pairs of rows come in an
 // order that scatters them (step): hubs are neighbours in graphs sorted by
 // degree, and in RMAT-like ones their ids have many trailing zeros, so with
 // consecutive rows or with a fixed stride they meet in a few workgroups
@@ -327,6 +329,7 @@ __global__ __launch_bounds__(BLOCK) void k_rowsum_w_long(const int32_t* __restri
 // a little better still on those and a little worse on uniform random ones.
 constexpr int kOneWave = 1024;
 constexpr int kOneRun = 2;   // consecutive rows that stay together
+constexpr int kHubRow = 32768;
 constexpr int kOneU = 8;  // loads in flight per thread in those
 // Above, hub rows outlast one workgroup. Vertex weights / gathered sums, one
 // launch and five, us: RMAT of 5.8M entries 23 / 34 and 45 / 59, 11.7M 40 / 63
@@ -360,7 +363,7 @@ __device__ __forceinline__ void exact_sum_fact(double sv, int& mx, int& bad) {
 template <typename OutT, bool IDX, bool EX>
 __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __restrict__ off,
                                                     const int32_t* __restrict__ ind, const float* __restrict__ v,
-                                                    OutT* __restrict__ out, ExactInfo* info, uint32_t step,
+                                                    OutT* __restrict__ out, ExactInfo* info, uint32_t step, int rows,
                                                     const int* skip) {
   if (skip && *skip) return;
   constexpr int BLOCK = 256, NW = BLOCK / kWave, R = BLOCK / kRowGroup;
@@ -380,14 +383,14 @@ __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __
     if (tid == 0) seen = ExactInfo{*(volatile int*)&info->min_lsb, *(volatile int*)&info->max_exp, *(volatile int*)&info->bad, 0};
   }
   const uint32_t runs = ((uint32_t)n + kOneRun - 1) / kOneRun;
-  for (int64_t i0 = (int64_t)blockIdx.x * R; i0 < n; i0 += (int64_t)gridDim.x * R) {
+  for (int64_t i0 = (int64_t)blockIdx.x * rows; i0 < n; i0 += (int64_t)gridDim.x * rows) {
     if (tid == 0) s_nlong = 0;
     __syncthreads();
     const uint32_t run = (uint32_t)(i0 / kOneRun) + tid / (kOneRun * kRowGroup);
     const uint32_t at = (uint32_t)((uint64_t)run * step % runs) * kOneRun + tid / kRowGroup % kOneRun;
     const int32_t u = (int32_t)at;
     int o = 0, d = 0;
-    const bool live = run < runs && at < (uint32_t)n;
+    const bool live = tid / kRowGroup < rows && run < runs && at < (uint32_t)n;
     if (live) {
       o = off[u];
       d = off[u + 1] - o;
@@ -407,7 +410,7 @@ __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __
     for (int sh = 1; sh < kRowGroup; sh <<= 1) acc = add_dd(acc, DD2{__shfl_xor(acc.hi, sh), __shfl_xor(acc.lo, sh)});
     if (live && gl == 0) {
       if (d <= kRowShort) put(u, acc.hi);
-      else s_long[atomicAdd(&s_nlong, 1)] = u;
+      else if (d <= kHubRow) s_long[atomicAdd(&s_nlong, 1)] = u;
     }
     __syncthreads();
     const int nl = s_nlong;
@@ -479,9 +482,73 @@ __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __
   }
 }
 
+// Rows above kHubRow entries: a workgroup of 1024 threads has twice the loads in
+// flight, and 63 other rows do not wait for it. Such rows are told apart by the
+// stretch of kHubRow entries that they start in, and cover the end of it, so one
+// workgroup per stretch finds its row by searching the offsets, 64 at a time.
+// Gathered sums, us, five launches / in k_rowsum_one / here: one row of 1M
+// entries 244 / 391 / 204, of 2M 460 / 768 / 401, three of 300K 92 / 223 / 67,
+// eight of 500K 137 / 404 / 107; 3 us where there is none.
+template <typename OutT, bool IDX, bool EX>
+__global__ __launch_bounds__(1024) void k_rowsum_hubs(int32_t n, const int32_t* __restrict__ off,
+                                                      const int32_t* __restrict__ ind, const float* __restrict__ v,
+                                                      OutT* __restrict__ out, ExactInfo* info, const int* skip) {
+  if (skip && *skip) return;
+  constexpr int BLOCK = 1024;
+  __shared__ double part[2][BLOCK / kWave];
+  const int lane = lane_id(), w = threadIdx.x / kWave;
+  const int m = off[n];
+  for (int64_t s = blockIdx.x; (s + 1) * kHubRow < m; s += gridDim.x) {
+    const int at = (int)((s + 1) * kHubRow);
+    // the last row that starts at or before `at`; every wave for itself
+    int u = 0;
+    for (int len = n; len > 1;) {
+      const int stride = (len + kWave - 1) / kWave;
+      const int k = lane * stride;
+      u += stride * (popc64(ballot(k < len && off[u + min(k, len - 1)] <= at)) - 1);
+      len = min(stride, n - u);
+    }
+    const int o = off[u], e = off[u + 1];
+    if (e - o <= kHubRow || o < at - kHubRow || o >= at) continue;  // uniform
+    DD2 acc{0.0, 0.0};
+    for (int p0 = o; p0 < e; p0 += BLOCK * kOneU) {
+      float x[kOneU];
+      gather_step<IDX, kOneU>(ind, v, p0, BLOCK, threadIdx.x, e, x);
+#pragma unroll
+      for (int t = 0; t < kOneU; ++t) acc = add_d(acc, (double)x[t]);
+    }
+#pragma unroll
+    for (int t = 1; t < kWave; t <<= 1) acc = add_dd(acc, DD2{__shfl_xor(acc.hi, t), __shfl_xor(acc.lo, t)});
+    if (lane == 0) {
+      part[0][w] = acc.hi;
+      part[1][w] = acc.lo;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      DD2 t{0.0, 0.0};
+      for (int k = 0; k < BLOCK / kWave; ++k) t = add_dd(t, DD2{part[0][k], part[1][k]});
+      out[u] = (OutT)t.hi;
+      if constexpr (EX) {
+        int mx = INT32_MIN, bad = 0;
+        exact_sum_fact(t.hi, mx, bad);
+        if (mx > *(volatile int*)&info->max_exp) atomicMax(&info->max_exp, mx);
+        if (bad) atomicOr(&info->bad, 1);
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// Rows of a workgroup, see above.
+int rows_one(int32_t n) {
+  int rows = 64;
+  while (rows > 8 && n < (int64_t)device_cu_count() * 4 * rows) rows /= 2;
+  return rows;
+}
+
 // A second round of rows would make the workgroups that met the long ones the
 // tail (11.7M entries, 4097 workgroups: 84 us and not 39).
-int grid_one(int32_t n) { return grid_rows((n + 63) / 64, 1, 256); }
+int grid_one(int32_t n) { return grid_rows((n + rows_one(n) - 1) / rows_one(n), 1, 256); }
 
 // Run k of the order is run k * step_one(n) mod runs: runs / golden ratio, less
 // what it takes to share no factor with them.
@@ -494,12 +561,21 @@ uint32_t step_one(int32_t n) {
 
 bool rowsum_one_launch(int32_t n, int64_t m) { return m <= kOneMaxEdges && n <= kOneMaxRows; }
 
+template <typename OutT, bool IDX, bool EX>
+static hipError_t rowsum_one(int32_t n, const int32_t* off, const int32_t* ind, const float* v, OutT* out,
+                             ExactInfo* info, hipStream_t s, const int* skip) {
+  hipLaunchKernelGGL((k_rowsum_one<OutT, IDX, EX>), dim3(grid_one(n)), dim3(256), 0, s, n, off, ind, v, out, info,
+                     step_one(n), rows_one(n), skip);
+  if (n > kHubRow)  // a row has at most n entries
+    hipLaunchKernelGGL((k_rowsum_hubs<OutT, IDX, EX>), dim3(device_cu_count() * 3), dim3(1024), 0, s, n, off, ind, v, out,
+                       info, skip);
+  return hipGetLastError();
+}
+
 hipError_t launch_rowsum_exact(int32_t n, const int32_t* off, const int32_t* ind, const float* v, double* S,
                                ExactInfo* info, hipStream_t s, const int* skip) {
   ProfScope ps_("rowsum", s);
-  hipLaunchKernelGGL((k_rowsum_one<double, true, true>), dim3(grid_one(n)), dim3(256), 0, s, n, off, ind, v, S, info,
-                     step_one(n), skip);
-  return hipGetLastError();
+  return rowsum_one<double, true, true>(n, off, ind, v, S, info, s, skip);
 }
 
 // Sentinel fill of the result (when x is not null) and the start values of a
@@ -531,13 +607,8 @@ template <typename OutT>
 static hipError_t rowsum_both(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* v, OutT* out,
                               void* scratch, hipStream_t s, const int* skip = nullptr) {
   if (rowsum_one_launch(n, m)) {
-    if (ind)
-      hipLaunchKernelGGL((k_rowsum_one<OutT, true, false>), dim3(grid_one(n)), dim3(256), 0, s, n, off, ind, v, out,
-                         (ExactInfo*)nullptr, step_one(n), skip);
-    else
-      hipLaunchKernelGGL((k_rowsum_one<OutT, false, false>), dim3(grid_one(n)), dim3(256), 0, s, n, off, ind, v, out,
-                         (ExactInfo*)nullptr, step_one(n), skip);
-    return hipGetLastError();
+    return ind ? rowsum_one<OutT, true, false>(n, off, ind, v, out, nullptr, s, skip)
+               : rowsum_one<OutT, false, false>(n, off, ind, v, out, nullptr, s, skip);
   }
   CallBuf own;
   if (!scratch) {
