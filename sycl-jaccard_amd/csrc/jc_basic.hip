@@ -319,7 +319,7 @@ __global__ __launch_bounds__(BLOCK) void k_rowsum_w_long(const int32_t* __restri
 // 2.4e5 entries). A workgroup takes 64 rows: rows up to kRowShort entries by 4
 // lanes each, up to kOneWave by a wave, longer ones by the workgroup (and those
 // above kHubRow by one of k_rowsum_hubs). Fewer rows, down to 8, where 64 would
-// leave less than four workgroups per CU (3000 rows of 780 entries 36 -> 10 us, 20000
+// leave less than four workgroups per CU and have more than 2048 entries (3000 rows of 780 entries 36 -> 10 us, 20000
 // of 100 27 -> 12). EX: also the range facts of v and the sums (k_exact_scan). Pairs of rows come in an
 // order that scatters them (step): hubs are neighbours in graphs sorted by
 // degree, and in RMAT-like ones their ids have many trailing zeros, so with
@@ -376,8 +376,10 @@ __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __
     out[u] = (OutT)sum;
     if constexpr (EX) exact_sum_fact(sum, mx, bad);
   };
-  // The facts as the workgroup began: most workgroups change nothing, and their
-  // atomics on one line were 0.3 ms of a graph of 1M vertices.
+  // The facts as the workgroup began, and again before it adds to them: most
+  // workgroups change nothing, and their atomics on one line were 0.3 ms of a
+  // graph of 1M vertices. (Without the second look those of all workgroups that
+  // begin together remain: 150000 vertices, 0.9M entries 259 us a call, 204 with it.)
   ExactInfo seen{INT32_MAX, INT32_MIN, 0, 0};
   if constexpr (EX) {
     if (tid == 0) seen = ExactInfo{*(volatile int*)&info->min_lsb, *(volatile int*)&info->max_exp, *(volatile int*)&info->bad, 0};
@@ -475,8 +477,8 @@ __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __
         mx = max(mx, s_r[1][k]);
         bad |= s_r[2][k];
       }
-      if (lsb < seen.min_lsb) atomicMin(&info->min_lsb, lsb);
-      if (mx > seen.max_exp) atomicMax(&info->max_exp, mx);
+      if (lsb < seen.min_lsb && lsb < *(volatile int*)&info->min_lsb) atomicMin(&info->min_lsb, lsb);
+      if (mx > seen.max_exp && mx > *(volatile int*)&info->max_exp) atomicMax(&info->max_exp, mx);
       if (bad && !seen.bad) atomicOr(&info->bad, 1);
     }
   }
@@ -540,15 +542,15 @@ __global__ __launch_bounds__(1024) void k_rowsum_hubs(int32_t n, const int32_t* 
 }
 
 // Rows of a workgroup, see above.
-int rows_one(int32_t n) {
+int rows_one(int32_t n, int64_t m) {
   int rows = 64;
-  while (rows > 8 && n < (int64_t)device_cu_count() * 4 * rows) rows /= 2;
+  while (rows > 8 && n < (int64_t)device_cu_count() * 4 * rows && m * rows > 2048ll * n) rows /= 2;
   return rows;
 }
 
 // A second round of rows would make the workgroups that met the long ones the
 // tail (11.7M entries, 4097 workgroups: 84 us and not 39).
-int grid_one(int32_t n) { return grid_rows((n + rows_one(n) - 1) / rows_one(n), 1, 256); }
+int grid_one(int32_t n, int rows) { return grid_rows((n + rows - 1) / rows, 1, 256); }
 
 // Run k of the order is run k * step_one(n) mod runs: runs / golden ratio, less
 // what it takes to share no factor with them.
@@ -562,20 +564,21 @@ uint32_t step_one(int32_t n) {
 bool rowsum_one_launch(int32_t n, int64_t m) { return m <= kOneMaxEdges && n <= kOneMaxRows; }
 
 template <typename OutT, bool IDX, bool EX>
-static hipError_t rowsum_one(int32_t n, const int32_t* off, const int32_t* ind, const float* v, OutT* out,
+static hipError_t rowsum_one(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* v, OutT* out,
                              ExactInfo* info, hipStream_t s, const int* skip) {
-  hipLaunchKernelGGL((k_rowsum_one<OutT, IDX, EX>), dim3(grid_one(n)), dim3(256), 0, s, n, off, ind, v, out, info,
-                     step_one(n), rows_one(n), skip);
+  const int rows = rows_one(n, m);
+  hipLaunchKernelGGL((k_rowsum_one<OutT, IDX, EX>), dim3(grid_one(n, rows)), dim3(256), 0, s, n, off, ind, v, out,
+                     info, step_one(n), rows, skip);
   if (n > kHubRow)  // a row has at most n entries
     hipLaunchKernelGGL((k_rowsum_hubs<OutT, IDX, EX>), dim3(device_cu_count() * 3), dim3(1024), 0, s, n, off, ind, v, out,
                        info, skip);
   return hipGetLastError();
 }
 
-hipError_t launch_rowsum_exact(int32_t n, const int32_t* off, const int32_t* ind, const float* v, double* S,
+hipError_t launch_rowsum_exact(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* v, double* S,
                                ExactInfo* info, hipStream_t s, const int* skip) {
   ProfScope ps_("rowsum", s);
-  return rowsum_one<double, true, true>(n, off, ind, v, S, info, s, skip);
+  return rowsum_one<double, true, true>(n, m, off, ind, v, S, info, s, skip);
 }
 
 // Sentinel fill of the result (when x is not null) and the start values of a
@@ -607,8 +610,8 @@ template <typename OutT>
 static hipError_t rowsum_both(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* v, OutT* out,
                               void* scratch, hipStream_t s, const int* skip = nullptr) {
   if (rowsum_one_launch(n, m)) {
-    return ind ? rowsum_one<OutT, true, false>(n, off, ind, v, out, nullptr, s, skip)
-               : rowsum_one<OutT, false, false>(n, off, ind, v, out, nullptr, s, skip);
+    return ind ? rowsum_one<OutT, true, false>(n, m, off, ind, v, out, nullptr, s, skip)
+               : rowsum_one<OutT, false, false>(n, m, off, ind, v, out, nullptr, s, skip);
   }
   CallBuf own;
   if (!scratch) {

@@ -210,7 +210,7 @@ hipError_t launch_vertex_weights(int32_t n, int64_t m, const int32_t* off, const
 // Row sums of graphs of n vertices and m stored edges are one launch, which can also
 // fill *info (as launch_exact_info, into a started ExactInfo: launch_prepare).
 bool rowsum_one_launch(int32_t n, int64_t m);
-hipError_t launch_rowsum_exact(int32_t n, const int32_t* off, const int32_t* ind, const float* v, double* S,
+hipError_t launch_rowsum_exact(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* v, double* S,
                                ExactInfo* info, hipStream_t s, const int* skip = nullptr);
 // x[0, n) = v (x may be nullptr; skip: as EngineArgs::skip), zero[0, nzero) = 0, *info (may be nullptr) started.
 hipError_t launch_prepare(uint32_t* x, int64_t n, uint32_t v, int* zero, int nzero, ExactInfo* info, hipStream_t s,
