@@ -124,8 +124,9 @@ Block* take(Device& d, int dev, size_t bytes, hipStream_t s, bool grow) {
   Block* b = own && own->bytes >= bytes ? own : fit ? fit : own ? own : any;
   if (!b || (b->bytes < bytes && !grow)) return nullptr;
   // the work it was last used for, also where the handle of s was another
-  // stream's before
-  if (b->pending && hipStreamWaitEvent(s, b->done, 0) != hipSuccess) {
+  // stream's before (asked first: a wait for what is over still costs the stream
+  // a few us)
+  if (!idle(*b) && hipStreamWaitEvent(s, b->done, 0) != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
   }
