@@ -142,7 +142,8 @@ int run_jaccard(const jc_csr* g, const float* vw, float* result, bool ec, unsign
     jc::ExactInfo* ex = reinterpret_cast<jc::ExactInfo*>(ws + L.exact);
     if (jc::rowsum_one_launch(g->n, g->m)) {
       if (!ec && !tri_ws) JC_TRY(jc::launch_prepare(nullptr, 0, 0u, nullptr, 0, ex, s));
-      JC_TRY(jc::launch_rowsum_exact(g->n, g->m, g->offsets, g->indices, vw, S64, ex, s, a.skip));
+      JC_TRY(jc::launch_rowsum_exact(g->n, g->m, g->offsets, g->indices, vw, S64, ws + L.rows, &a.nfacts, ex, s, a.skip));
+      a.facts = reinterpret_cast<const jc::ExactInfo*>(ws + L.rows);
     } else {
       JC_TRY(jc::launch_rowsum_f64(g->n, g->m, g->offsets, g->indices, vw, S64, ws + L.rows, s, a.skip));
       JC_TRY(jc::launch_exact_info(g->n, vw, S64, ex, s, a.skip));

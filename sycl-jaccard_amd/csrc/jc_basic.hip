@@ -319,8 +319,10 @@ __global__ __launch_bounds__(BLOCK) void k_rowsum_w_long(const int32_t* __restri
 // 2.4e5 entries). A workgroup takes 64 rows: rows up to kRowShort entries by 4
 // lanes each, up to kOneWave by a wave, longer ones by the workgroup (and those
 // above kHubRow by one of k_rowsum_hubs). Fewer rows, down to 8, where 64 would
-// leave less than four workgroups per CU and have more than 2048 entries (3000 rows of 780 entries 36 -> 10 us, 20000
-// of 100 27 -> 12). EX: also the range facts of v and the sums (k_exact_scan). Pairs of rows come in an
+// leave less than four workgroups per CU and have more than 2048 entries (3000
+// rows of 780 entries 36 -> 10 us, 20000 of 100 27 -> 12). EX: facts[workgroup]
+// receives the range facts of v and of its sums (k_exact_scan); added up by
+// atomics on one line they took 60 us on 150000 vertices. Pairs of rows come in an
 // order that scatters them (step): hubs are neighbours in graphs sorted by
 // degree, and in RMAT-like ones their ids have many trailing zeros, so with
 // consecutive rows or with a fixed stride they meet in a few workgroups
@@ -363,7 +365,7 @@ __device__ __forceinline__ void exact_sum_fact(double sv, int& mx, int& bad) {
 template <typename OutT, bool IDX, bool EX>
 __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __restrict__ off,
                                                     const int32_t* __restrict__ ind, const float* __restrict__ v,
-                                                    OutT* __restrict__ out, ExactInfo* info, uint32_t step, int rows,
+                                                    OutT* __restrict__ out, ExactInfo* facts, uint32_t step, int rows,
                                                     const int* skip) {
   if (skip && *skip) return;
   constexpr int BLOCK = 256, NW = BLOCK / kWave, R = BLOCK / kRowGroup;
@@ -376,14 +378,6 @@ __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __
     out[u] = (OutT)sum;
     if constexpr (EX) exact_sum_fact(sum, mx, bad);
   };
-  // The facts as the workgroup began, and again before it adds to them: most
-  // workgroups change nothing, and their atomics on one line were 0.3 ms of a
-  // graph of 1M vertices. (Without the second look those of all workgroups that
-  // begin together remain: 150000 vertices, 0.9M entries 259 us a call, 204 with it.)
-  ExactInfo seen{INT32_MAX, INT32_MIN, 0, 0};
-  if constexpr (EX) {
-    if (tid == 0) seen = ExactInfo{*(volatile int*)&info->min_lsb, *(volatile int*)&info->max_exp, *(volatile int*)&info->bad, 0};
-  }
   const uint32_t runs = ((uint32_t)n + kOneRun - 1) / kOneRun;
   for (int64_t i0 = (int64_t)blockIdx.x * rows; i0 < n; i0 += (int64_t)gridDim.x * rows) {
     if (tid == 0) s_nlong = 0;
@@ -477,9 +471,7 @@ __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __
         mx = max(mx, s_r[1][k]);
         bad |= s_r[2][k];
       }
-      if (lsb < seen.min_lsb && lsb < *(volatile int*)&info->min_lsb) atomicMin(&info->min_lsb, lsb);
-      if (mx > seen.max_exp && mx > *(volatile int*)&info->max_exp) atomicMax(&info->max_exp, mx);
-      if (bad && !seen.bad) atomicOr(&info->bad, 1);
+      facts[blockIdx.x] = ExactInfo{lsb, mx, bad, 0};
     }
   }
 }
@@ -487,18 +479,23 @@ __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __
 // Rows above kHubRow entries: a workgroup of 1024 threads has twice the loads in
 // flight, and 63 other rows do not wait for it. Such rows are told apart by the
 // stretch of kHubRow entries that they start in, and cover the end of it, so one
-// workgroup per stretch finds its row by searching the offsets, 64 at a time.
+// workgroup per stretch finds its row by searching the offsets, 64 at a time. EX:
+// the first one also gathers the nfacts facts of k_rowsum_one's workgroups.
 // Gathered sums, us, five launches / in k_rowsum_one / here: one row of 1M
 // entries 244 / 391 / 204, of 2M 460 / 768 / 401, three of 300K 92 / 223 / 67,
 // eight of 500K 137 / 404 / 107; 3 us where there is none.
 template <typename OutT, bool IDX, bool EX>
 __global__ __launch_bounds__(1024) void k_rowsum_hubs(int32_t n, const int32_t* __restrict__ off,
                                                       const int32_t* __restrict__ ind, const float* __restrict__ v,
-                                                      OutT* __restrict__ out, ExactInfo* info, const int* skip) {
+                                                      OutT* __restrict__ out, const ExactInfo* facts, int nfacts,
+                                                      ExactInfo* info, const int* skip) {
   if (skip && *skip) return;
   constexpr int BLOCK = 1024;
   __shared__ double part[2][BLOCK / kWave];
   const int lane = lane_id(), w = threadIdx.x / kWave;
+  if constexpr (EX) {
+    if (blockIdx.x == 0) gather_facts(facts, nfacts, info);
+  }
   const int m = off[n];
   for (int64_t s = blockIdx.x; (s + 1) * kHubRow < m; s += gridDim.x) {
     const int at = (int)((s + 1) * kHubRow);
@@ -565,20 +562,22 @@ bool rowsum_one_launch(int32_t n, int64_t m) { return m <= kOneMaxEdges && n <= 
 
 template <typename OutT, bool IDX, bool EX>
 static hipError_t rowsum_one(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* v, OutT* out,
-                             ExactInfo* info, hipStream_t s, const int* skip) {
-  const int rows = rows_one(n, m);
-  hipLaunchKernelGGL((k_rowsum_one<OutT, IDX, EX>), dim3(grid_one(n, rows)), dim3(256), 0, s, n, off, ind, v, out,
-                     info, step_one(n), rows, skip);
+                             ExactInfo* facts, int* nfacts, ExactInfo* info, hipStream_t s, const int* skip) {
+  const int rows = rows_one(n, m), g = grid_one(n, rows);
+  hipLaunchKernelGGL((k_rowsum_one<OutT, IDX, EX>), dim3(g), dim3(256), 0, s, n, off, ind, v, out, facts, step_one(n),
+                     rows, skip);
+  if (EX) *nfacts = n > kHubRow ? 0 : g;
   if (n > kHubRow)  // a row has at most n entries
-    hipLaunchKernelGGL((k_rowsum_hubs<OutT, IDX, EX>), dim3(device_cu_count() * 3), dim3(1024), 0, s, n, off, ind, v, out,
-                       info, skip);
+    hipLaunchKernelGGL((k_rowsum_hubs<OutT, IDX, EX>), dim3(device_cu_count() * 3), dim3(1024), 0, s, n, off, ind, v,
+                       out, facts, g, info, skip);
   return hipGetLastError();
 }
 
 hipError_t launch_rowsum_exact(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* v, double* S,
-                               ExactInfo* info, hipStream_t s, const int* skip) {
+                               void* scratch, int* nfacts, ExactInfo* info, hipStream_t s, const int* skip) {
   ProfScope ps_("rowsum", s);
-  return rowsum_one<double, true, true>(n, m, off, ind, v, S, info, s, skip);
+  // (one per workgroup, of eight rows at least: a part of rowsum_scratch_bytes)
+  return rowsum_one<double, true, true>(n, m, off, ind, v, S, static_cast<ExactInfo*>(scratch), nfacts, info, s, skip);
 }
 
 // Sentinel fill of the result (when x is not null) and the start values of a
@@ -610,8 +609,8 @@ template <typename OutT>
 static hipError_t rowsum_both(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* v, OutT* out,
                               void* scratch, hipStream_t s, const int* skip = nullptr) {
   if (rowsum_one_launch(n, m)) {
-    return ind ? rowsum_one<OutT, true, false>(n, m, off, ind, v, out, nullptr, s, skip)
-               : rowsum_one<OutT, false, false>(n, m, off, ind, v, out, nullptr, s, skip);
+    return ind ? rowsum_one<OutT, true, false>(n, m, off, ind, v, out, nullptr, nullptr, nullptr, s, skip)
+               : rowsum_one<OutT, false, false>(n, m, off, ind, v, out, nullptr, nullptr, nullptr, s, skip);
   }
   CallBuf own;
   if (!scratch) {

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "jc_internal.hpp"
+
 namespace jc {
 
 constexpr int kWave = 64;
@@ -32,6 +34,29 @@ __device__ __forceinline__ int lane_id() { return (int)__lane_id(); }
 
 // Orders one wave's LDS accesses before and after it (LDS private to the wave).
 __device__ __forceinline__ void lds_fence_wave() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront"); }
+
+// The range facts that nfacts workgroups left at `facts`, into *info, by one
+// workgroup.
+__device__ __forceinline__ void gather_facts(const ExactInfo* __restrict__ facts, int nfacts, ExactInfo* info) {
+  int lsb = INT32_MAX, mx = INT32_MIN, bad = 0;
+  for (int i = threadIdx.x; i < nfacts; i += blockDim.x) {
+    const ExactInfo f = facts[i];
+    lsb = min(lsb, f.min_lsb);
+    mx = max(mx, f.max_exp);
+    bad |= f.bad;
+  }
+#pragma unroll
+  for (int t = 1; t < kWave; t <<= 1) {
+    lsb = min(lsb, __shfl_xor(lsb, t));
+    mx = max(mx, __shfl_xor(mx, t));
+    bad |= __shfl_xor(bad, t);
+  }
+  if (lane_id() == 0) {
+    if (lsb != INT32_MAX) atomicMin(&info->min_lsb, lsb);
+    if (mx != INT32_MIN) atomicMax(&info->max_exp, mx);
+    if (bad) atomicOr(&info->bad, 1);
+  }
+}
 
 __device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
 

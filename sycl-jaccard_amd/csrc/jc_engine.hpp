@@ -2017,8 +2017,10 @@ template <bool W, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_sched_count(int32_t rows, const int32_t* __restrict__ off,
                                                        const int32_t* __restrict__ ind, Sched* sc, int small_max,
                                                        size_t bm_budget, int whole_max, const int2* segs,
-                                                       int nseg, const int* skip) {
+                                                       int nseg, const ExactInfo* facts, int nfacts,
+                                                       ExactInfo* exact, const int* skip) {
   if (skip && *skip) return;  // empty task lists: the kernels over them end at once
+  if (blockIdx.x == 0 && nfacts > 0) gather_facts(facts, nfacts, exact);
   __shared__ int hist[2 * kBuckets + 1];
   for (int i = threadIdx.x; i < 2 * kBuckets + 1; i += BLOCK) hist[i] = 0;
   __syncthreads();
@@ -2135,8 +2137,10 @@ constexpr int kLongRow = 512;
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_sched_one(int32_t rows, const int32_t* __restrict__ off, Sched* sc,
                                                      int2* tasks, int32_t task_cap, int32_t* small_rows, int small_max,
-                                                     const int2* segs, int nseg, const int* skip) {
+                                                     const int2* segs, int nseg, const ExactInfo* facts, int nfacts,
+                                                     ExactInfo* exact, const int* skip) {
   if (skip && *skip) return;
+  if (blockIdx.x == 0 && nfacts > 0) gather_facts(facts, nfacts, exact);
   __shared__ int s_cnt[3], s_base[3];
   for (int64_t b = (int64_t)blockIdx.x * BLOCK; b < rows; b += (int64_t)gridDim.x * BLOCK) {
     if (threadIdx.x < 3) s_cnt[threadIdx.x] = 0;
@@ -2245,12 +2249,13 @@ hipError_t run_engine_t(const EngineArgs& base, void* ws, bool fixup, hipStream_
       ProfScope ps("sched", stream);
       const int g1 = (int)std::min<int64_t>((rows + PB - 1) / PB, (int64_t)cus * 8);
       hipLaunchKernelGGL((k_sched_one<PB>), dim3(g1), dim3(PB), 0, stream, rows, a.off, sc, tasks, a.task_cap, small,
-                         a.small_max, a.segs, a.nseg, a.skip);
+                         a.small_max, a.segs, a.nseg, a.facts, a.nfacts, a.exact, a.skip);
       if ((err = hipGetLastError()) != hipSuccess) return err;
     } else {
       ProfScope ps("sched", stream);
       hipLaunchKernelGGL((k_sched_count<W, PB>), dim3(g), dim3(PB), 0, stream, rows, a.off, a.ind, sc, a.small_max,
-                         bm_budget, whole_max, a.segs, a.nseg, a.skip);
+                         bm_budget, whole_max, a.segs, a.nseg, a.facts, a.nfacts, a.exact,
+                         a.skip);
       hipLaunchKernelGGL(k_sched_scan, dim3(1), dim3(64), 0, stream, sc);
       hipLaunchKernelGGL((k_sched_emit<W, PB>), dim3(g), dim3(PB), 0, stream, rows, a.off, a.ind, sc, tasks, small,
                          a.small_max, bm_budget, whole_max, a.segs, a.nseg, a.skip);

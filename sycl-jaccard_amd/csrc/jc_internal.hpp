@@ -90,7 +90,10 @@ struct EngineArgs {
   int64_t seg_edges;
   // Weighted modes: optional range facts of vw and S64 (device memory); when
   // they show all sums are exact in fp64 the kernels add in plain fp64.
-  const ExactInfo* exact;
+  ExactInfo* exact;
+  // Parts of *exact that the schedule has yet to put together, or nfacts = 0.
+  const ExactInfo* facts;
+  int nfacts;
   // Hash-table tasks the quotient-table kernel had to abandon (device memory,
   // set by the launcher), and whether a launch is the 32-bit redo of them.
   int* redo;
@@ -208,10 +211,12 @@ hipError_t launch_rowsum_f64(int32_t n, int64_t m, const int32_t* off, const int
 hipError_t launch_vertex_weights(int32_t n, int64_t m, const int32_t* off, const float* edge_w, float* W,
                                  void* scratch, hipStream_t s);
 // Row sums of graphs of n vertices and m stored edges are one launch, which can also
-// fill *info (as launch_exact_info, into a started ExactInfo: launch_prepare).
+// fill *info (as launch_exact_info, into a started ExactInfo: launch_prepare), or, where
+// *nfacts is not 0, leaves that many parts of it at scratch (EngineArgs::facts).
 bool rowsum_one_launch(int32_t n, int64_t m);
 hipError_t launch_rowsum_exact(int32_t n, int64_t m, const int32_t* off, const int32_t* ind, const float* v, double* S,
-                               ExactInfo* info, hipStream_t s, const int* skip = nullptr);
+                               void* scratch, int* nfacts, ExactInfo* info, hipStream_t s,
+                               const int* skip = nullptr);
 // x[0, n) = v (x may be nullptr; skip: as EngineArgs::skip), zero[0, nzero) = 0, *info (may be nullptr) started.
 hipError_t launch_prepare(uint32_t* x, int64_t n, uint32_t v, int* zero, int nzero, ExactInfo* info, hipStream_t s,
                           const int* skip = nullptr);
