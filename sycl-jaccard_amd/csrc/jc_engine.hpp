@@ -2193,14 +2193,11 @@ hipError_t run_engine_t(const EngineArgs& base, void* ws, bool fixup, hipStream_
   if (a.nseg > 0 && fixup) return hipErrorInvalidValue;  // segments need a symmetric graph
   const int32_t rows = a.nseg > 0 ? a.seg_rows : a.n;
   const int64_t edges = a.nseg > 0 ? a.seg_edges : a.m;
-  // one wave per row up to 128 entries where there are rows enough to fill the
-  // chip; smaller graphs end sooner with a workgroup per longer row. Up to 32 /
-  // 64 / 96 / 128 entries, us: RMAT 0.23M entries 72 / 70 / 83 / 83, 0.43M 93 / 80
-  // / 89 / 97, 0.9M 165 / 133 / 135 / 136, 1.8M 287 / 278 / 251 / 253, 3.7M 660 /
-  // 525 / 524 / 496; Chung-Lu 0.64M 103 / 96 / 105 / 108, weighted 2.1M 451 / 347
-  // / 326 / 335
-  if (a.small_max < 1 || a.small_max > kSmallMax)
-    a.small_max = edges <= (1 << 20) ? 64 : edges <= (5 << 19) ? 96 : kSmallMax;
+  // one wave per row up to 128 entries; the smallest graphs end sooner with a
+  // workgroup for rows from 64 on. Up to 64 / 128 entries, us: RMAT 0.23M entries 70 /
+  // 83, 0.43M 80 / 97, 0.9M 133 / 136, 1.8M 278 / 253; uniform random, 100 a row, 0.5M
+  // 163 / 169, 2.0M 328 / 251; a ring with 120, 2.4M 366 / 196
+  if (a.small_max < 1 || a.small_max > kSmallMax) a.small_max = edges <= (1 << 19) ? 64 : kSmallMax;
   if (a.small_blocks_per_cu < 1) a.small_blocks_per_cu = 16;
   // buffer-load offsets reach 4 * (m + 256) bytes
   if (a.m * 4 + 8192 > (int64_t)UINT32_MAX) a.wide_index = 1;
