@@ -86,20 +86,30 @@ bool tri_wanted(const jc_csr* g, bool weighted, const jc_tuning* t) {
   return (t && t->engine == JC_ENGINE_ORIENTED) || ((!t || t->members) && jc::tri_pays(g->n, g->m, weighted));
 }
 
-// Weighted pair lists: sum every row of the graph once before the pairs, or
-// the two rows of each pair. Once / per pair, us, whole calls: 65536 pairs on
-// RMAT of 2^15 vertices (0.9M entries) 68 / 125, 2^18 (7.6M) 197 / 330, 2^20
-// (31M) 459 / 714; 8192 pairs, with the row sums in five launches, 121 / 62 on the
-// second.
+// Weighted pair lists: sum every row of the graph once before the pairs (kAlways),
+// or the two rows of each pair (kNever), or as a sample of the pairs says (kAsk).
+// All rows take some 8 us, 5 per 1M entries and 25 per 1M vertices, and then the
+// pairs 0.25 ns each; the rows of each pair take 0.75 to 0.9 ns a pair where they are short,
+// and far more where pairs name hubs. All rows / each pair, us: 65536 pairs, half of them edges,
+// of RMAT with 0.8M entries 83 / 132, 7.6M 202 / 311, 31M 454 / 723; random
+// pairs, uniform random graphs of 1.4M entries 34 / 45, 10M 77 / 49, 3M over 1M vertices 70 / 48;
+// 16384 pairs of those 22 / 14, 70 / 15, 58 / 14. Asking takes 8 us and up to 14 per 1M
+// vertices where the answer is no, about what a list of 65536 gained with the pair
+// kernel on graphs of short rows.
 // Under capture the call stays one kernel node without an allocation.
-bool pairs_sum_all(const jc_csr* g, int64_t np, hipStream_t s) {
-  if (np < 16384 || g->m > 512 * np) return false;
+enum PairSums { kNever, kAlways, kAsk };
+PairSums pairs_sum_all(const jc_csr* g, int64_t np, hipStream_t s) {
+  const double all_us = 8.0 + 5e-6 * g->m + 25e-6 * g->n;
+  const bool always = np >= 16384 && all_us <= 0.6e-3 * np;
+  const bool ask = np >= 65536 && g->m <= 512 * np && 8.0 + 14e-6 * g->n <= 0.2e-3 * np;
+  if (!always && !ask) return kNever;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) != hipSuccess) {
     (void)hipGetLastError();
-    return false;
+    return kNever;
   }
-  return st == hipStreamCaptureStatusNone;
+  if (st != hipStreamCaptureStatusNone) return kNever;
+  return always ? kAlways : kAsk;
 }
 
 // ws: layout(...).total bytes; tri_ws: tri_workspace_bytes(...) bytes, or
@@ -297,17 +307,24 @@ int jc_jaccard_list(const jc_csr* g, const float* vertex_weights, int32_t num_pa
   hipStream_t s = hs(stream);
   jc::CallBuf buf;
   double* S64 = nullptr;
-  if (weighted && pairs_sum_all(g, num_pairs, s)) {
-    const size_t rows_b = al(jc::rowsum_scratch_bytes(g->n));
-    if (buf.get(rows_b + al((size_t)g->n * sizeof(double)), s, jc::CallBuf::kOptional) == hipSuccess) {
-      S64 = reinterpret_cast<double*>(static_cast<unsigned char*>(buf.p) + rows_b);
-      JC_TRY(jc::launch_rowsum_f64(g->n, g->m, g->offsets, g->indices, vertex_weights, S64, buf.p, s));
+  int* no_S = nullptr;
+  const PairSums sums = weighted ? pairs_sum_all(g, num_pairs, s) : kNever;
+  if (sums != kNever) {
+    const size_t rows_b = al(jc::rowsum_scratch_bytes(g->n)), s64_b = al((size_t)g->n * sizeof(double));
+    if (buf.get(rows_b + s64_b + al(sizeof(int)), s, jc::CallBuf::kOptional) == hipSuccess) {
+      unsigned char* p = static_cast<unsigned char*>(buf.p);
+      S64 = reinterpret_cast<double*>(p + rows_b);
+      if (sums == kAsk) {
+        no_S = reinterpret_cast<int*>(p + rows_b + s64_b);
+        JC_TRY(jc::launch_pairs_want(g->n, g->m, g->offsets, num_pairs, first, second, no_S, s));
+      }
+      JC_TRY(jc::launch_rowsum_f64(g->n, g->m, g->offsets, g->indices, vertex_weights, S64, p, s, no_S));
     } else {
       (void)hipGetLastError();  // the pair kernel sums the rows
     }
   }
   JC_TRY(jc::run_pairs(weighted ? jc::kModeEcW : jc::kModeEcU, weighted, g->n, g->offsets, g->indices,
-                       vertex_weights, nullptr, S64, num_pairs, first, second, result, nullptr, 0, hs(stream)));
+                       vertex_weights, nullptr, S64, num_pairs, first, second, result, nullptr, 0, s, no_S));
   return JC_OK;
 }
 

@@ -162,11 +162,16 @@ hipError_t run_engine(int mode, bool weighted, const EngineArgs& base, void* ws,
                       hipStream_t stream);
 
 // Pair path: out per (first[i], second[i]); invalid ids give NaN. S: the row
-// sums of vw, or nullptr (kModeEcW then sums the rows of each pair).
+// sums of vw, or nullptr (kModeEcW then sums the rows of each pair, as where *no_S,
+// in device memory, is not 0).
 hipError_t run_pairs(int mode, bool weighted, int32_t n, const int32_t* off, const int32_t* ind,
                      const float* vw, const float* work32, const double* S, int64_t np, const int32_t* first,
                      const int32_t* second, float* out32, float* ws32, int accumulate,
-                     hipStream_t stream);
+                     hipStream_t stream, const int* no_S = nullptr);
+// *no_S (device memory) = whether the row sums of all of the graph are more work
+// than those of the pairs' rows.
+hipError_t launch_pairs_want(int32_t n, int64_t m, const int32_t* off, int64_t np, const int32_t* first,
+                             const int32_t* second, int* no_S, hipStream_t stream);
 
 // Fills *info (device memory) for vertex weights vw[n] and their row sums S[n].
 hipError_t launch_exact_info(int32_t n, const float* vw, const double* S, ExactInfo* info, hipStream_t s,
