@@ -122,15 +122,14 @@ int engine_counter_words();
 constexpr int32_t kTriMaxN = 1 << 26;  // its hash keys hold 26-bit ranks
 // Oriented engine (jc_tri.hip) before the owner engine: from tri_min_edges
 // stored entries on, where no tuning is given or it names a batch (and then
-// only if the device finds the rows skewed enough, see k_tri_scan). Below,
+// only if the device finds the rows skewed enough, see k_tri_init). Below,
 // its two dozen dependent launches are most of its time. Owner and oriented
 // engine, ms: weighted RMAT 1.5M entries 0.32 / 0.30, 2.8M 0.54 / 0.42, 4.0M
 // 0.98 / 0.53, Chung-Lu 1.6M 0.29 / 0.32, 3.2M 0.49 / 0.44, 4.5M 1.09 / 0.52;
 // unweighted RMAT 2.8M 0.37 / 0.36, 4.0M 0.53 / 0.47, 5.8M 0.78 / 0.61, 11.7M
 // 1.63 / 1.19, Chung-Lu 3.2M 0.35 / 0.37, 4.2M 0.45 / 0.44, 6.4M 0.68 / 0.58,
 // 12.8M 1.34 / 1.09, 25.6M 2.86 / 2.17. Above the crossing, for what a graph
-// that the device turns down pays: 0.06 ms (uniform random 9M unweighted 0.87 ->
-// 0.95, 4M weighted 0.56 -> 0.62).
+// that the device turns down pays, 25 to 50 us (k_tri_init).
 constexpr int32_t tri_min_edges(bool weighted) { return weighted ? 3 << 20 : 6 << 20; }
 // (sum |R|^2 / 64 words of bit matrix are at least (m / 2)^2 / n / 64, above the
 // engine's 4 m words from a mean row of 1024 entries on; a uniform random graph

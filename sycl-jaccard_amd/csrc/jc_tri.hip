@@ -121,22 +121,21 @@ struct alignas(256) Own {
   T v;
 };
 
-// Why the engine may refuse a graph is found out in three stages, each with a
+// Why the engine may refuse a graph is found out in stages, each with a
 // word of its own: a kernel reads the words of the stages before its own, which
 // no kernel in flight writes, and writes only its own stage's. So all waves of a
 // workgroup see the same and end together or not at all; with one word for all,
 // waves that found it set while the launch was under way left the others at
 // barriers and on LDS that nobody had filled.
-enum TriStage { kStRank, kStOrient, kStWedge, kStReduce };
+enum TriStage { kStLook, kStCount, kStRank, kStOrient, kStWedge, kStReduce };
 
 struct TriCtl {
-  int bad_rank;
+  int pad;
   int done;
-  int bad_orient, bad_wedge;
+  int bad[kStReduce];
   Own<int> lsb, maxexp;             // exactness of the weights (see ExactInfo)
   Own<int> wexp;                    // every weight is below 2^wexp
-  Own<unsigned long long> sampled;  // min(d_u, d_x, kSampleCap) over kSamples entries (u, x)
-  Own<double> sampled_w;            // weights of the x
+  Own<double> sampled_w;            // weights of the sampled entries' vertices
   Own<unsigned long long> out_total;  // sum of |R(u)|
   Own<unsigned long long> bits;     // words of the bit matrix handed out
   Own<int> num_big;                 // rows oriented by a workgroup
@@ -205,14 +204,16 @@ struct TriArgs {
 template <int S>
 __device__ __forceinline__ void refuse(const TriArgs& a) {
   static_assert(S < kStReduce, "reduce refuses nothing");
-  (S == kStRank ? a.ctl->bad_rank : S == kStOrient ? a.ctl->bad_orient : a.ctl->bad_wedge) = 1;
+  a.ctl->bad[S] = 1;
 }
 
 // Whether the stages before S left the graph to S.
 template <int S>
 __device__ __forceinline__ bool tri_go(const TriArgs& a) {
-  const TriCtl* c = a.ctl;
-  return c->bad_rank == 0 && (S <= kStOrient || c->bad_orient == 0) && (S <= kStWedge || c->bad_wedge == 0);
+  int bad = 0;
+#pragma unroll
+  for (int i = 0; i < S; ++i) bad |= a.ctl->bad[i];
+  return bad == 0;
 }
 
 // The same from wedge on, with the facts that must hold before it starts.
@@ -225,45 +226,80 @@ __device__ __forceinline__ bool tri_ready(const TriArgs& a) {
   return true;
 }
 
-__global__ void k_tri_init(TriCtl* c) {
-  int* p = reinterpret_cast<int*>(c);
-  for (int i = threadIdx.x; i < (int)(sizeof(TriCtl) / sizeof(int)); i += blockDim.x) p[i] = 0;
+// An entry (x, y) of the graph, the t-th of kSamples spread over it; false for x
+// without entries (in a graph that is not symmetric). A neighbour's neighbour is as
+// random an entry as any in a symmetric graph, and needs no search for its row.
+__device__ __forceinline__ bool sample_entry(const TriArgs& a, int t, int32_t& x, int32_t& y, int& dx) {
+  // one in each of kSamples equal runs of entries
+  const int64_t k = min(a.m - 1, (t * a.m + (int64_t)((t * 0x9E3779B1u) >> 22) * a.m / 1024) / kSamples);
+  x = a.ind[k];
+  const int o = a.off[x];
+  dx = a.off[x + 1] - o;
+  if (dx <= 0) return false;
+  y = a.ind[o + (int)((uint32_t)t * 0x85EBCA6Bu % (uint32_t)dx)];
+  return true;
+}
+
+// Clears the control words and, before anything else is done for the graph, looks
+// whether the engine would be the faster one. With len the mean of min(d_x, d_y, 512) over
+// sampled entries and d the mean degree, it is where len is well above d (few hubs on
+// most edges), or rows are long in any case. Owner / oriented engine, ms,
+// weighted: RMAT len 85..230, d 6..54: 1.3 to 2.2 times as fast; Chung-Lu len
+// 53..206, d 6..64: 1.4 to 2.2 times; uniform random graphs d = len = 16 1.44
+// / 1.99, 37 0.99 / 1.39, 63 0.99 / 1.21, 76 1.77 / 1.78, 154 3.88 / 2.06;
+// neighbours on a ring 24 1.56 / 2.50, 72 3.68 / 3.54, 196 3.62 / 2.15. A graph that
+// is turned down here costs the launches that then do nothing, 25 to 50 us (uniform
+// random, 4M entries weighted 422 us without the engine, 445 with; 576 when the degrees
+// were counted and ranked first).
+__global__ __launch_bounds__(kSamples) void k_tri_init(TriArgs a) {
+  __shared__ int s_len[kSamples / kWave];
+  int* p = reinterpret_cast<int*>(a.ctl);
+  for (int i = threadIdx.x; i < (int)(sizeof(TriCtl) / sizeof(int)); i += kSamples) p[i] = 0;
+  int len = 0;
+  if (!a.always) {
+    int32_t x, y;
+    int dx;
+    if (sample_entry(a, threadIdx.x, x, y, dx)) len = min(min(dx, a.off[y + 1] - a.off[y]), kSampleCap);
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) len += __shfl_xor(len, o);
+    if (lane_id() == 0) s_len[threadIdx.x / kWave] = len;
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
-    c->lsb.v = INT32_MAX;
-    c->maxexp.v = INT32_MIN;
-    c->wexp.v = INT32_MIN;
+    a.ctl->lsb.v = INT32_MAX;
+    a.ctl->maxexp.v = INT32_MIN;
+    a.ctl->wexp.v = INT32_MIN;
+    if (!a.always) {
+      int sum = 0;
+      for (int i = 0; i < kSamples / kWave; ++i) sum += s_len[i];
+      const float l = (float)sum / kSamples, d = (float)a.m / (float)a.n;
+      if (l < 48.f || (l < 96.f && l < 1.5f * d)) refuse<kStLook>(a);
+    }
   }
 }
 
 // Degree histogram over each workgroup's contiguous range of vertices, and
 // the finest and the highest bit of the weights. The first kSamples / BLOCK
-// workgroups look at one entry (u, x) per thread instead: for its mirror, so
+// workgroups look at one entry per thread instead, for its mirror, so
 // that most graphs that are not symmetric are refused before the work of
-// orient, and at the shorter row's length, what the owner engine streams.
+// orient.
 template <bool W, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_tri_hist(TriArgs a) {
   __shared__ int h[kTriBuckets];
   constexpr int kLook = kSamples / BLOCK;
+  if (!tri_go<kStCount>(a)) return;
   if (blockIdx.x < kLook) {
-    const int32_t t = blockIdx.x * BLOCK + threadIdx.x;
-    // one in each of kSamples equal runs of entries
-    const int64_t k = min(a.m - 1, (t * a.m + (int64_t)((t * 0x9E3779B1u) >> 22) * a.m / 1024) / kSamples);
-    int lo = 0, hi = a.n;  // off[lo] <= k < off[hi]
-    while (hi - lo > 1) {
-      const int mid = (int)(((uint32_t)lo + (uint32_t)hi) >> 1);
-      if (a.off[mid] <= k) lo = mid;
-      else hi = mid;
+    int32_t x = 0, y = 0;
+    int dx;
+    const bool any = sample_entry(a, blockIdx.x * BLOCK + threadIdx.x, x, y, dx);
+    if (any) {
+      const int e = a.off[y + 1], at = lane_lower_bound(a.ind, a.off[y], e, x);
+      if (at >= e || a.ind[at] != x) refuse<kStCount>(a);
+    } else {
+      refuse<kStCount>(a);
     }
-    const int32_t x = a.ind[k];
-    const int b = a.off[x], e = a.off[x + 1], at = lane_lower_bound(a.ind, b, e, lo);
-    if (at >= e || a.ind[at] != lo) refuse<kStRank>(a);
-    int len = min(min(a.off[lo + 1] - a.off[lo], e - b), kSampleCap);
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) len += __shfl_xor(len, o);
-    if (lane_id() == 0) atomicAdd(&a.ctl->sampled.v, (unsigned long long)len);
     if constexpr (W) {
-      float w = a.vw[x];
+      float w = any ? a.vw[y] : 0.0f;
 #pragma unroll
       for (int o = 1; o < kWave; o <<= 1) w += __shfl_xor(w, o);
       if (lane_id() == 0) unsafeAtomicAdd(&a.ctl->sampled_w.v, (double)w);
@@ -296,7 +332,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_hist(TriArgs a) {
       lsb = min(lsb, __shfl_xor(lsb, o));
       top = max(top, __shfl_xor(top, o));
     }
-    if (ballot(bad) && lane_id() == 0) refuse<kStRank>(a);
+    if (ballot(bad) && lane_id() == 0) refuse<kStCount>(a);
     if (lane_id() == 0 && lsb < *(volatile int*)&a.ctl->lsb.v) atomicMin(&a.ctl->lsb.v, lsb);
     if (lane_id() == 0 && top > *(volatile int*)&a.ctl->wexp.v) atomicMax(&a.ctl->wexp.v, top);
   }
@@ -308,33 +344,26 @@ __global__ __launch_bounds__(BLOCK) void k_tri_hist(TriArgs a) {
 // Vertices of degree d in a group task of wedge.
 __device__ __forceinline__ int group_rows(int d) { return min(kGroupRows, kWedgeB / d); }
 
-// First rank of every bucket, largest degrees first; and whether to go on.
-// With len the mean of min(d_u, d_x, 512) over the entries and d the mean
-// degree, the engine is the faster one where len is well above d (few hubs on
-// most edges), or rows are long in any case. Owner / oriented engine, ms,
-// weighted: RMAT len 85..230, d 6..54: 1.3 to 2.2 times as fast; Chung-Lu len
-// 53..206, d 6..64: 1.4 to 2.2 times; uniform random graphs d = len = 16 1.44
-// / 1.99, 37 0.99 / 1.39, 63 0.99 / 1.21, 76 1.77 / 1.78, 154 3.88 / 2.06;
-// neighbours on a ring 24 1.56 / 2.50, 72 3.68 / 3.54, 196 3.62 / 2.15.
-// Giving up here costs 0.06 ms, the launches that then do nothing.
-__global__ __launch_bounds__(kTriBuckets) void k_tri_scan(TriCtl* c, int32_t n, int64_t m, int always, int grp_from) {
+// First rank of every bucket, largest degrees first; and whether the weights'
+// sums may be exact.
+__global__ __launch_bounds__(kTriBuckets) void k_tri_scan(TriArgs a) {
   __shared__ int part[kTriBuckets / kWave];
   __shared__ int s_top;
+  if (!tri_go<kStCount>(a)) return;
+  TriCtl* const c = a.ctl;
   const int b = kTriBuckets - 1 - threadIdx.x;
   if (b == 0) s_top = 0;
   __syncthreads();
   if (c->hist[b]) atomicMax(&s_top, b);
   __syncthreads();
   // a weight that alone is wider than fp64 sums can hold
-  if (b == 0 && c->lsb.v != INT32_MAX && c->wexp.v - c->lsb.v > 53) c->bad_rank = 1;
-  if (b == 0 && !always) {
-    const float len = (float)c->sampled.v / kSamples, d = (float)m / (float)n;
-    if (len < 48.f || (len < 96.f && len < 1.5f * d)) c->bad_rank = 1;
+  if (b == 0 && c->lsb.v != INT32_MAX && c->wexp.v - c->lsb.v > 53) refuse<kStCount>(a);
+  if (b == 0 && !a.always) {
     // the longest row's weights, were they the sampled ones' mean: sums that
     // surely round are not found out after orient only
     const int top = s_top < 512 ? s_top : (16 + (s_top & 15)) << ((s_top - 512) / 16 + 5);
     const double sum = (double)top * c->sampled_w.v / kSamples;
-    if (c->lsb.v != INT32_MAX && sum > 0.0 && ilogb(sum) - c->lsb.v > 53) c->bad_rank = 1;
+    if (c->lsb.v != INT32_MAX && sum > 0.0 && !isinf(sum) && ilogb(sum) - c->lsb.v > 53) refuse<kStCount>(a);
   }
   const int v = c->hist[b];
   int incl = v;
@@ -353,7 +382,7 @@ __global__ __launch_bounds__(kTriBuckets) void k_tri_scan(TriCtl* c, int32_t n, 
   // long rows of low rank go to the bitmap kernel instead.
   int ng = 0;
   if (b > 0 && b < kGroupMax) {
-    const int first = b >= kWgMinDeg ? max(base + incl - v, grp_from) : base + incl - v;
+    const int first = b >= kWgMinDeg ? max(base + incl - v, a.grp_from) : base + incl - v;
     const int cnt = max(0, base + incl - first);
     c->grp_rank[b] = first;
     ng = (cnt + group_rows(b) - 1) / group_rows(b);
@@ -381,6 +410,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_rank(TriArgs a) {
   __shared__ int h[kTriBuckets];
   __shared__ int base[kTriBuckets];
   __shared__ int s_cnt[2], s_base[2];
+  if (!tri_go<kStRank>(a)) return;
   for (int i = threadIdx.x; i < kTriBuckets; i += BLOCK) h[i] = 0;
   if (threadIdx.x < 2) s_cnt[threadIdx.x] = 0;
   __syncthreads();
@@ -425,6 +455,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_rank(TriArgs a) {
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_tri_reach(TriArgs a) {
   __shared__ int s_max;
+  if (!tri_go<kStRank>(a)) return;
   if (threadIdx.x == 0) s_max = -1;
   __syncthreads();
   const int64_t per = ((int64_t)a.n + gridDim.x - 1) / gridDim.x;
@@ -440,8 +471,10 @@ __global__ __launch_bounds__(BLOCK) void k_tri_reach(TriArgs a) {
 }
 
 // ... then of all ranges before ...
-__global__ __launch_bounds__(kTriParts) void k_tri_reach_scan(TriCtl* c, int ranges) {
+__global__ __launch_bounds__(kTriParts) void k_tri_reach_scan(TriArgs a, int ranges) {
   __shared__ int s[2][kTriParts];
+  if (!tri_go<kStRank>(a)) return;
+  TriCtl* const c = a.ctl;
   const int t = threadIdx.x;
   s[0][t] = t < ranges ? c->reach[t] : -1;
   int b = 0;
@@ -459,6 +492,7 @@ template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_tri_starts(TriArgs a) {
   constexpr int NW = BLOCK / kWave;
   __shared__ int s_m[NW], s_c[NW];
+  if (!tri_go<kStRank>(a)) return;
   const int lane = lane_id(), w = threadIdx.x / kWave;
   const int64_t per = ((int64_t)a.n + gridDim.x - 1) / gridDim.x;
   const int32_t r0 = (int32_t)min(per * blockIdx.x, (int64_t)a.n), r1 = (int32_t)min(per * (blockIdx.x + 1), (int64_t)a.n);
@@ -507,6 +541,7 @@ __global__ __launch_bounds__(BLOCK) void k_tri_starts(TriArgs a) {
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_tri_parts(TriArgs a) {
   __shared__ int s_at, s_all;
+  if (!tri_go<kStRank>(a)) return;
   if (threadIdx.x == 0) s_at = s_all = 0;
   __syncthreads();
   int at = 0, all = 0;
@@ -531,6 +566,7 @@ __global__ __launch_bounds__(kTriBuckets) void k_tri_rank_parts(TriArgs a) {
   __shared__ int h[kTriBuckets], base[kTriBuckets];
   __shared__ int part[kTriBuckets / kWave];
   __shared__ int s_i;
+  if (!tri_go<kStRank>(a)) return;
   const int tid = threadIdx.x, lane = lane_id();
   const int count = a.ctl->num_part.v;
   for (;;) {
@@ -1930,16 +1966,16 @@ hipError_t tri_launch(const TriArgs& a, hipStream_t s) {
   };
   {
     ProfScope ps("tri_rank", s);
-    hipLaunchKernelGGL(k_tri_init, dim3(1), dim3(1024), 0, s, a.ctl);
+    hipLaunchKernelGGL(k_tri_init, dim3(1), dim3(kSamples), 0, s, a);
     const dim3 g = grid(a.n, PB * 4, kTriParts / 256);
     static_assert(kTriParts % 256 == 0, "ranges");
     hipLaunchKernelGGL((k_tri_hist<W, PB>), dim3(g.x + kSamples / PB), dim3(PB), 0, s, a);
-    hipLaunchKernelGGL(k_tri_scan, dim3(1), dim3(kTriBuckets), 0, s, a.ctl, a.n, a.m, a.always, a.grp_from);
+    hipLaunchKernelGGL(k_tri_scan, dim3(1), dim3(kTriBuckets), 0, s, a);
     hipLaunchKernelGGL((k_tri_rank<W, PB>), g, dim3(PB), 0, s, a);
     if (a.members) {
       const dim3 gp((unsigned)std::min<int64_t>(g.x, kTriParts));
       hipLaunchKernelGGL((k_tri_reach<PB>), gp, dim3(PB), 0, s, a);
-      hipLaunchKernelGGL(k_tri_reach_scan, dim3(1), dim3(kTriParts), 0, s, a.ctl, (int)gp.x);
+      hipLaunchKernelGGL(k_tri_reach_scan, dim3(1), dim3(kTriParts), 0, s, a, (int)gp.x);
       hipLaunchKernelGGL((k_tri_starts<PB>), gp, dim3(PB), 0, s, a);
       hipLaunchKernelGGL((k_tri_parts<PB>), gp, dim3(PB), 0, s, a);
       hipLaunchKernelGGL((k_tri_rank_parts<W>), dim3(cus * 2), dim3(kTriBuckets), 0, s, a);
@@ -1965,7 +2001,10 @@ hipError_t tri_launch(const TriArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((k_tri_wedge<W, uint16_t, kTabA, kAccA>), dim3(cus * 4), dim3(kWedgeB), 0, s, a);
     hipLaunchKernelGGL((k_tri_wedge<W, uint32_t, kTabB, kAccB>), dim3(cus), dim3(kWedgeB), 0, s, a);
     hipLaunchKernelGGL((k_tri_wedge_group<W>), dim3(cus * 4), dim3(kWedgeB), 0, s, a);
-    hipLaunchKernelGGL((k_tri_wedge_wave<W, PB>), grid(std::min<int64_t>(a.n, a.m / kGroupMax), PB / kWave, 16), dim3(PB), 0, s, a);
+    // (rows of kGroupMax entries and more at ranks past kSat16: not in smaller graphs,
+    // but a batch's large |R| may be there by their ranks in the whole)
+    if (a.members || a.m >= (int64_t)kGroupMax * kSat16)
+      hipLaunchKernelGGL((k_tri_wedge_wave<W, PB>), grid(std::min<int64_t>(a.n, a.m / kGroupMax), PB / kWave, 16), dim3(PB), 0, s, a);
   }
   {
     ProfScope ps("tri_reduce", s);
