@@ -470,6 +470,7 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
   const int mode = s->weighted ? jc::kModeEcW : jc::kModeEcU;
   s->pool.reset_peak();
   std::vector<char> graph_busy(s->g.size(), 0), in_batch(s->g.size(), 0);
+  std::vector<int> passed(count, -1);  // batches launched when a request was first passed over
   std::deque<int> pending;
   int next = 0, finished = 0, batches = 0, in_flight = 0;
   int err = JC_OK;
@@ -504,10 +505,16 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
       if (full && (graph_busy[q.graph] || in_batch[q.graph])) { ++it; continue; }
       if (!take.empty() && full && E + m.m > cfg.max_batch_edges) { ++it; continue; }
       // a graph that the oriented engine lacks the memory for waits where another
-      // batch's copy holds it; the owner engine would take twice as long
+      // batch's copy holds it; the owner engine would take twice as long. It waits for
+      // as many batches as there are slots, though, and no longer: in a steady
+      // stream some batch always holds a copy
       if (full && nseg == 0 && copies && !copy_fits(1, m.n, m.m) && copy_fits_in(s->pool.cap(), 1, m.n, m.m)) {
-        ++it;
-        continue;
+        int& since = passed[*it];
+        if (since < 0) since = batches;
+        if (batches - since < (int)s->slots.size()) {
+          ++it;
+          continue;
+        }
       }
       // a batch that the oriented engine has memory for is not grown beyond that
       if (full && nseg > 0 && !copy_fits(nseg + 1, R + m.n, E + m.m) &&
