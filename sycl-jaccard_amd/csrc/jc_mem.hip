@@ -18,6 +18,11 @@
 // hold kKeepBytes at most (the 5.65 GB of RMAT-22 and room for a second stream's),
 // until jc_release_workspaces or the end of the process. Beyond that and while a
 // stream is captured the allocation is the runtime's, stream-ordered.
+//
+// All of it comes from the device's default pool. Memory that a thread took from
+// a pool of the library's own while another thread captured a call (with its
+// allocation as a node of the graph) left that graph without effect from its second replay
+// on; with the default pool every replay is right.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -51,8 +56,6 @@ struct Block {
 
 struct Device {
   std::mutex mu;
-  hipMemPool_t pool = nullptr;
-  bool no_pool = false;           // none could be made: the default one serves
   hipStream_t stream = nullptr;   // jc_release_workspaces frees on it
   Block block[kBlocks];
 };
@@ -79,22 +82,6 @@ bool idle(Block& b) {
   return true;
 }
 
-hipError_t map(Device& d, int dev, void** p, size_t bytes, hipStream_t s) {
-  if (!d.pool && !d.no_pool) {
-    hipMemPoolProps props{};
-    props.allocType = hipMemAllocationTypePinned;
-    props.handleTypes = hipMemHandleTypeNone;
-    props.location.type = hipMemLocationTypeDevice;
-    props.location.id = dev;
-    if (hipMemPoolCreate(&d.pool, &props) != hipSuccess) {
-      (void)hipGetLastError();
-      d.pool = nullptr;
-      d.no_pool = true;
-    }
-  }
-  return d.pool ? hipMallocFromPoolAsync(p, bytes, d.pool, s) : hipMallocAsync(p, bytes, s);
-}
-
 // Gives an idle block's memory back, behind what is on s.
 void drop(Block& b, hipStream_t s) {
   if (b.p) (void)hipFreeAsync(b.p, s);
@@ -104,7 +91,7 @@ void drop(Block& b, hipStream_t s) {
 
 // A block of at least `bytes` for work on s, or nullptr. grow: also one that has
 // to be mapped anew.
-Block* take(Device& d, int dev, size_t bytes, hipStream_t s, bool grow) {
+Block* take(Device& d, size_t bytes, hipStream_t s, bool grow) {
   std::lock_guard<std::mutex> lock(d.mu);
   // usable now: this stream's own, whose work comes before what is added, and idle ones
   Block* own = nullptr;
@@ -150,7 +137,7 @@ Block* take(Device& d, int dev, size_t bytes, hipStream_t s, bool grow) {
     want = std::min((want + kGrain - 1) / kGrain * kGrain, std::max(bytes, (kKeepBytes - rest) / kGrain * kGrain));
     drop(*b, s);
     b->pending = false;
-    if (map(d, dev, &b->p, want, s) != hipSuccess) {
+    if (hipMallocAsync(&b->p, want, s) != hipSuccess) {
       (void)hipGetLastError();
       b->p = nullptr;
       return nullptr;
@@ -164,7 +151,7 @@ Block* take(Device& d, int dev, size_t bytes, hipStream_t s, bool grow) {
 // Gives back to the system what no call of the device is using.
 hipError_t release_idle(Device& d, int dev) {
   std::lock_guard<std::mutex> lock(d.mu);
-  if (!d.pool && !d.no_pool) return hipSuccess;
+  if (std::none_of(d.block, d.block + kBlocks, [](const Block& b) { return b.p != nullptr; })) return hipSuccess;
   int before = 0;
   hipError_t e = hipGetDevice(&before);
   if (e != hipSuccess) return e;
@@ -173,9 +160,9 @@ hipError_t release_idle(Device& d, int dev) {
   if (e == hipSuccess) {
     for (Block& b : d.block)
       if (b.p && idle(b)) drop(b, d.stream);
+    // (the default pool gives back what is free when a stream is waited for)
     e = hipStreamSynchronize(d.stream);
   }
-  if (e == hipSuccess && d.pool) e = hipMemPoolTrimTo(d.pool, 0);
   (void)hipSetDevice(before);
   return e;
 }
@@ -195,7 +182,7 @@ hipError_t CallBuf::get(size_t bytes, hipStream_t stream, Use use) {
   Relaxed relaxed;
   Device& d = g_dev[dev];
   if (bytes <= kKeepBytes) {
-    if (Block* b = take(d, dev, bytes, s, use != kOnce || bytes <= kOnceBytes)) {
+    if (Block* b = take(d, bytes, s, use != kOnce || bytes <= kOnceBytes)) {
       block = b;
       device = dev;
       p = b->p;

@@ -84,35 +84,48 @@ def test_streams_that_overlap(cuda):
             assert torch.equal(out.view(torch.int32), want.view(torch.int32))
 
 
-def test_call_while_another_thread_captures(cuda):
+@pytest.mark.parametrize("capture_first", [True, False])
+def test_calls_while_another_thread_captures(capture_first, cuda):
+    """Calls that take memory beside a capture, larger ones each time: neither they
+    nor any replay of the graph, with calls in between, may come out different."""
     import torch
     g = graphs.rmat(13, 16)
     dg = api.DeviceCSR.from_host(g, cuda)
     want = api.jaccard(dg)
     torch.cuda.synchronize()
-    a, b = torch.zeros(g.m, device=cuda), torch.zeros(g.m, device=cuda)
-    side, main = torch.cuda.Stream(device=cuda), torch.cuda.Stream(device=cuda)
-    torch.cuda.synchronize()
-    graph, errors = torch.cuda.CUDAGraph(), []
-
-    def work():
-        try:
-            for _ in range(4):
-                api.jaccard(dg, result=b, stream=side)
-        except Exception as e:  # noqa: BLE001
-            errors.append(e)
-
-    print("[gpu] call beside a capture", flush=True)
-    with torch.cuda.graph(graph, stream=main):
-        api.jaccard(dg, result=a, stream=main)
-        t = threading.Thread(target=work)
-        t.start()
-        t.join()
-    side.synchronize()
-    assert not errors
-    for _ in range(2):
-        a.zero_()
-        graph.replay()
+    for scale in (13, 14, 15, 16, 17, 18):
+        big = api.DeviceCSR.from_host(graphs.rmat(scale, 16), cuda)
+        a, b = torch.zeros(g.m, device=cuda), torch.zeros(big.m, device=cuda)
+        side, main = torch.cuda.Stream(device=cuda), torch.cuda.Stream(device=cuda)
         torch.cuda.synchronize()
-        assert torch.equal(a.view(torch.int32), want.view(torch.int32))
-    assert torch.equal(b.view(torch.int32), want.view(torch.int32))
+        graph, errors = torch.cuda.CUDAGraph(), []
+
+        def work():
+            try:
+                for _ in range(3):
+                    api.jaccard(big, result=b, stream=side)
+            except Exception as e:  # noqa: BLE001
+                errors.append(e)
+
+        print(f"[gpu] calls beside a capture, 2^{scale} vertices", flush=True)
+        with torch.cuda.graph(graph, stream=main):
+            if capture_first:
+                api.jaccard(dg, result=a, stream=main)
+            t = threading.Thread(target=work)
+            t.start()
+            t.join()
+            if not capture_first:
+                api.jaccard(dg, result=a, stream=main)
+        side.synchronize()
+        assert not errors
+        own = api.jaccard(big, tuning=dict(engine=api.ENGINE_OWNER))
+        assert torch.equal(b.view(torch.int32), own.view(torch.int32))
+        for _ in range(4):
+            a.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(a.view(torch.int32), want.view(torch.int32))
+            api.jaccard(big, result=b)
+            torch.cuda.synchronize()
+            assert torch.equal(b.view(torch.int32), own.view(torch.int32))
