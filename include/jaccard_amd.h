@@ -102,12 +102,14 @@ int jc_jaccard_ex(const jc_csr *g, const float *vertex_weights, float *result, i
 size_t jc_jaccard_workspace_size(int32_t n, int32_t m, int weighted, int edge_centric);
 
 /* Launch tuning for jc_jaccard_tuned. None of these change results; zero
- * fields take the defaults. No reference counterpart (the reference's launch
+ * fields take the defaults, and a struct of zeros is NULL: the library then also
+ * chooses the engine. A field of the owner engine's launches that is not zero
+ * names that engine (but for a batch, see members). No reference counterpart (the reference's launch
  * shapes are fixed, jaccard.cpp:264-276, 403-418, 745-753). */
 typedef struct jc_tuning {
   int32_t small_max;           /* degree bin threshold: rows up to this degree run one
                                   wave per row, longer rows one workgroup per task
-                                  (1..128, default 128) */
+                                  (1..128, default 128; 64 up to 2^19 stored edges) */
   int32_t small_blocks_per_cu; /* grid of the one-wave-per-row kernel (default 16) */
   int32_t wide_index;          /* nonzero: stream rows with 64-bit addresses even when
                                   the index array is small enough for 32-bit buffer
@@ -127,8 +129,9 @@ typedef struct jc_tuning {
                                   home bucket; a task whose table then does not build is
                                   redone with the 32-bit table (1 forces that for every
                                   chunk with a full bucket) */
-  int32_t engine;              /* 0 (default), JC_ENGINE_OWNER or JC_ENGINE_ORIENTED (then
-                                  the owner engine for what that one cannot do) */
+  int32_t engine;              /* 0 (default: the library's choice), JC_ENGINE_OWNER or
+                                  JC_ENGINE_ORIENTED (then the owner engine for what that
+                                  one cannot do) */
   int32_t members;             /* nonzero: the graph is a disjoint union of many graphs of at
                                   most 65536 vertices, with consecutive ids (a batch); the
                                   oriented engine then ranks each by itself */

@@ -74,16 +74,22 @@ Layout layout(int32_t n, int32_t m, bool weighted, bool ec) {
   return L;
 }
 
-// The one-launch kernel for graphs that fit the LDS, where the caller names
-// nothing of the owner engine.
+// Whether a tuning leaves the way to the result to the library: it names no engine
+// and nothing of the owner engine's launches.
+bool automatic(const jc_tuning* t) {
+  return !t || (t->small_max == 0 && t->small_blocks_per_cu == 0 && t->wide_index == 0 &&
+                t->bitmap_blocks_per_cu == 0 && t->hash_table == 0 && t->quot_max_disp == 0 && t->engine == 0);
+}
+
+// The one-launch kernel for graphs that fit the LDS.
 bool tiny_wanted(const jc_csr* g, bool weighted, const jc_tuning* t) {
-  return !t && jc::tiny_fits(g->n, g->m, weighted);
+  return automatic(t) && jc::tiny_fits(g->n, g->m, weighted);
 }
 
 bool tri_wanted(const jc_csr* g, bool weighted, const jc_tuning* t) {
   if (t && (t->engine == JC_ENGINE_OWNER || t->wide_index || t->hash_table == 1 || t->quot_max_disp > 0)) return false;
   if (!jc::tri_can(g->n, g->m)) return false;
-  return (t && t->engine == JC_ENGINE_ORIENTED) || ((!t || t->members) && jc::tri_pays(g->n, g->m, weighted));
+  return (t && t->engine == JC_ENGINE_ORIENTED) || ((automatic(t) || t->members) && jc::tri_pays(g->n, g->m, weighted));
 }
 
 // Weighted pair lists: sum every row of the graph once before the pairs (kAlways),
