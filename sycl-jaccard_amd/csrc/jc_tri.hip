@@ -42,6 +42,8 @@
 // Measured against the owner engine (whole calls): RMAT-22 weighted 58.2 ->
 // 15.9 ms, RMAT of 200003 vertices weighted vertex-centric 1.58 -> 0.72 ms,
 // Chung-Lu 2^20 4.00 -> 2.86 ms.
+#include <stddef.h>
+
 #include <type_traits>
 
 #include "jc_device.hpp"
@@ -153,6 +155,10 @@ struct TriCtl {
   int cur[kTriBuckets];
   int reach[kTriParts], nstart[kTriParts];  // per vertex range: largest neighbour id (then of all ranges before), parts begun
 };
+// (where the tests look to see what ran)
+static_assert(offsetof(TriCtl, done) == 4 && offsetof(TriCtl, num_task) == 9 * 256 &&
+                  offsetof(TriCtl, num_wave) == 11 * 256 && offsetof(TriCtl, num_red) == 14 * 256,
+              "places of the counters");
 
 namespace {
 
