@@ -62,6 +62,13 @@ struct PairJob {
   int o_l, d_l;    // the longer row
 };
 
+// A pair that is cut into units: its place in the workgroup, ids, rows.
+struct PairLong {
+  int q;
+  int32_t pa, pb;
+  int oa, da, ob, db;
+};
+
 template <bool W>
 struct PairSum;
 template <>
@@ -174,13 +181,12 @@ __global__ __launch_bounds__(kPairB) void k_pairs(PairArgs a) {
   __shared__ PairJob job[kWave];
   __shared__ int begin[kWave + 1];  // first unit of every job
   __shared__ PairSum<W> sum;
-  __shared__ int4 s_long[kList];    // pair (in the workgroup), its rows' ids
+  __shared__ PairLong s_long[kList];
   __shared__ int s_nl;
   const int lane = lane_id(), wave = threadIdx.x / kWave;
   const int64_t base_i = (int64_t)blockIdx.x * a.per;
   const bool sums = DIRECT && (!a.no_S || *a.no_S != 0);
   if (threadIdx.x == 0) s_nl = 0;
-  __syncthreads();
   {
     // a wave's pairs, one per lane up to here
     const int chunk = (a.per + kPairNW - 1) / kPairNW;
@@ -199,8 +205,9 @@ __global__ __launch_bounds__(kPairB) void k_pairs(PairArgs a) {
       ob = a.off[pb];
       db = a.off[pb + 1] - ob;
     }
+    __syncthreads();  // s_nl is 0
     const bool single = max(da, db) <= kPairShort || (!sums && min(da, db) <= kPairUnit);
-    if (valid && !single) s_long[atomicAdd(&s_nl, 1)] = make_int4(wave * chunk + lane, pa, pb, 0);
+    if (valid && !single) s_long[atomicAdd(&s_nl, 1)] = PairLong{wave * chunk + lane, pa, pb, oa, da, ob, db};
     uint32_t cnt = 0;
     double sum = 0.0, sa = 0.0, sb = 0.0;
     for (uint64_t todo = ballot(valid && single); todo; todo &= todo - 1) {
@@ -255,13 +262,13 @@ __global__ __launch_bounds__(kPairB) void k_pairs(PairArgs a) {
     PairJob j{0, 0, 0, -1};
     int units = 0;
     if (lane < jobs) {
-      const int4 l = s_long[lane % nl];
-      i = base_i + l.x;
-      pa = l.y;
-      pb = l.z;
-      const int oa = a.off[pa], ob = a.off[pb];
-      da = a.off[pa + 1] - oa;
-      db = a.off[pb + 1] - ob;
+      const PairLong l = s_long[lane % nl];
+      i = base_i + l.q;
+      pa = l.pa;
+      pb = l.pb;
+      da = l.da;
+      db = l.db;
+      const int oa = l.oa, ob = l.ob;
       const int kind = lane / nl;
       if (kind == 0) {
         const bool a_long = da > db || (da == db && pa >= pb);
