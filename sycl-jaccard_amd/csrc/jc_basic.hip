@@ -480,7 +480,7 @@ __global__ __launch_bounds__(256) void k_rowsum_one(int32_t n, const int32_t* __
 // flight, and 63 other rows do not wait for it. Such rows are told apart by the
 // stretch of kHubRow entries that they start in, and cover the end of it, so one
 // workgroup per stretch finds its row by searching the offsets, 64 at a time. EX:
-// the first one also gathers the nfacts facts of k_rowsum_one's workgroups.
+// the last one also gathers the nfacts facts of k_rowsum_one's workgroups.
 // Gathered sums, us, five launches / in k_rowsum_one / here: one row of 1M
 // entries 244 / 391 / 204, of 2M 460 / 768 / 401, three of 300K 92 / 223 / 67,
 // eight of 500K 137 / 404 / 107; 3 us where there is none.
@@ -494,7 +494,7 @@ __global__ __launch_bounds__(1024) void k_rowsum_hubs(int32_t n, const int32_t* 
   __shared__ double part[2][BLOCK / kWave];
   const int lane = lane_id(), w = threadIdx.x / kWave;
   if constexpr (EX) {
-    if (blockIdx.x == 0) gather_facts(facts, nfacts, info);
+    if (blockIdx.x == gridDim.x - 1) gather_facts(facts, nfacts, info);
   }
   const int m = off[n];
   for (int64_t s = blockIdx.x; (s + 1) * kHubRow < m; s += gridDim.x) {

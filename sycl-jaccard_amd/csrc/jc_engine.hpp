@@ -2020,11 +2020,15 @@ __global__ __launch_bounds__(BLOCK) void k_sched_count(int32_t rows, const int32
                                                        int nseg, const ExactInfo* facts, int nfacts,
                                                        ExactInfo* exact, const int* skip) {
   if (skip && *skip) return;  // empty task lists: the kernels over them end at once
-  if (blockIdx.x == 0 && nfacts > 0) gather_facts(facts, nfacts, exact);
+  const int blocks = gridDim.x - (nfacts > 0 ? 1 : 0);  // (and one for the facts)
+  if ((int)blockIdx.x == blocks) {
+    gather_facts(facts, nfacts, exact);
+    return;
+  }
   __shared__ int hist[2 * kBuckets + 1];
   for (int i = threadIdx.x; i < 2 * kBuckets + 1; i += BLOCK) hist[i] = 0;
   __syncthreads();
-  for (int32_t v = blockIdx.x * BLOCK + threadIdx.x; v < rows; v += gridDim.x * BLOCK) {
+  for (int32_t v = blockIdx.x * BLOCK + threadIdx.x; v < rows; v += blocks * BLOCK) {
     const int32_t u = seg_row(segs, nseg, v);
     const int o = off[u], d = off[u + 1] - o;
     if (d <= 0) continue;
@@ -2140,9 +2144,13 @@ __global__ __launch_bounds__(BLOCK) void k_sched_one(int32_t rows, const int32_t
                                                      const int2* segs, int nseg, const ExactInfo* facts, int nfacts,
                                                      ExactInfo* exact, const int* skip) {
   if (skip && *skip) return;
-  if (blockIdx.x == 0 && nfacts > 0) gather_facts(facts, nfacts, exact);
+  const int blocks = gridDim.x - (nfacts > 0 ? 1 : 0);  // (and one for the facts)
+  if ((int)blockIdx.x == blocks) {
+    gather_facts(facts, nfacts, exact);
+    return;
+  }
   __shared__ int s_cnt[3], s_base[3];
-  for (int64_t b = (int64_t)blockIdx.x * BLOCK; b < rows; b += (int64_t)gridDim.x * BLOCK) {
+  for (int64_t b = (int64_t)blockIdx.x * BLOCK; b < rows; b += (int64_t)blocks * BLOCK) {
     if (threadIdx.x < 3) s_cnt[threadIdx.x] = 0;
     __syncthreads();
     const int64_t v = b + threadIdx.x;
@@ -2245,12 +2253,12 @@ hipError_t run_engine_t(const EngineArgs& base, void* ws, bool fixup, hipStream_
     if (bitmap_only) {
       ProfScope ps("sched", stream);
       const int g1 = (int)std::min<int64_t>((rows + PB - 1) / PB, (int64_t)cus * 8);
-      hipLaunchKernelGGL((k_sched_one<PB>), dim3(g1), dim3(PB), 0, stream, rows, a.off, sc, tasks, a.task_cap, small,
+      hipLaunchKernelGGL((k_sched_one<PB>), dim3(g1 + (a.nfacts > 0 ? 1 : 0)), dim3(PB), 0, stream, rows, a.off, sc, tasks, a.task_cap, small,
                          a.small_max, a.segs, a.nseg, a.facts, a.nfacts, a.exact, a.skip);
       if ((err = hipGetLastError()) != hipSuccess) return err;
     } else {
       ProfScope ps("sched", stream);
-      hipLaunchKernelGGL((k_sched_count<W, PB>), dim3(g), dim3(PB), 0, stream, rows, a.off, a.ind, sc, a.small_max,
+      hipLaunchKernelGGL((k_sched_count<W, PB>), dim3(g + (a.nfacts > 0 ? 1 : 0)), dim3(PB), 0, stream, rows, a.off, a.ind, sc, a.small_max,
                          bm_budget, whole_max, a.segs, a.nseg, a.facts, a.nfacts, a.exact,
                          a.skip);
       hipLaunchKernelGGL(k_sched_scan, dim3(1), dim3(64), 0, stream, sc);
@@ -2292,6 +2300,7 @@ hipError_t run_engine_t(const EngineArgs& base, void* ws, bool fixup, hipStream_
     {
       ProfScope ps("owner_block", stream);
       if (bitmap_only) {
+        // no hash-table tasks
       } else if (quot) {
         hipLaunchKernelGGL((k_owner_block<MODE, W, BB, 2>), dim3(cus * occ2), dim3(BB), Cfg::q_lds_bytes, stream,
                            a);
