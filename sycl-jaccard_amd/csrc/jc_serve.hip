@@ -3,9 +3,10 @@
 //
 // No reference counterpart (the reference computes one graph per call,
 // jaccard.cpp:926-955). Arithmetic is that of jc_jaccard / jc_jaccard_list:
-// the owner engine accumulates exactly and every per-row reduction (row sums,
-// per-pair waves) depends only on the row, so a request's bits do not depend
-// on the batch it ran in.
+// the owner engine (over the rows where they lie) and the oriented one (over a
+// copy of the requested graphs, for large batches) accumulate exactly, and every
+// per-row reduction (row sums, per-pair waves) depends only on the row, so a
+// request's bits do not depend on the batch it ran in.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
