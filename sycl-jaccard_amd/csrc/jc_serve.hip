@@ -498,6 +498,7 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
     int nseg = 0;
     int32_t R = 0;
     int64_t E = 0, K = 0;
+    bool held = false;
     const bool copies = std::any_of(s->slots.begin(), s->slots.end(), [](const jc::Slot& o) { return o.busy && o.bytes2 > 0; });
     for (auto it = pending.begin(); it != pending.end() && (int)take.size() < cfg.max_batch_requests;) {
       const jc_request& q = reqs[*it];
@@ -506,16 +507,16 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
       if (full && (graph_busy[q.graph] || in_batch[q.graph])) { ++it; continue; }
       if (!take.empty() && full && E + m.m > cfg.max_batch_edges) { ++it; continue; }
       // a graph that the oriented engine lacks the memory for waits where another
-      // batch's copy holds it; the owner engine would take twice as long. It waits for
-      // as many batches as there are slots, though, and no longer: in a steady
-      // stream some batch always holds a copy
+      // batch's copy holds it; the owner engine would take twice as long. In a steady
+      // stream some batch always holds a copy, so when as many batches as there are
+      // slots have gone past it no later whole graph is taken until it is
+      if (full && held) { ++it; continue; }
       if (full && nseg == 0 && copies && !copy_fits(1, m.n, m.m) && copy_fits_in(s->pool.cap(), 1, m.n, m.m)) {
         int& since = passed[*it];
         if (since < 0) since = batches;
-        if (batches - since < (int)s->slots.size()) {
-          ++it;
-          continue;
-        }
+        held = batches - since >= (int)s->slots.size();
+        ++it;
+        continue;
       }
       // a batch that the oriented engine has memory for is not grown beyond that
       if (full && nseg > 0 && !copy_fits(nseg + 1, R + m.n, E + m.m) &&

@@ -1,6 +1,6 @@
 """A whole-graph request whose copy has to wait for memory is not held back by
-smaller ones that keep coming: it is served, by either engine, after at most as
-many batches as there are slots."""
+smaller ones that keep coming: it is served after at most as many batches as
+there are slots."""
 import numpy as np
 import pytest
 
