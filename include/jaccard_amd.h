@@ -211,7 +211,9 @@ int jc_degree_stats(const jc_csr *g, jc_graph_stats *stats, jc_stream_t stream);
  * These come from a sweep of every jc_tuning field over thirteen graph
  * families (RMAT 2^14 to 2^22, weighted and not, Chung-Lu 2^18 and 2^20, the
  * two halves of a 4096-graph batch), where the chosen configuration was the
- * fastest or within 1% of it on eleven; no field changes results. The
+ * fastest or within 1% of it on eleven; no field changes results. All of them
+ * are the owner engine's, and a call with the tuning takes that engine; no
+ * tuning, or one of zeros, leaves the engine to the library. The
  * table kind of each row (bitmap or hash) is decided per row from its
  * degree and column span by the scheduler, as jc_degree_stats reports. */
 int jc_config_from_stats(const jc_graph_stats *stats, int32_t n, int weighted, int *edge_centric,
@@ -368,8 +370,9 @@ typedef struct jc_server_config {
   int64_t max_batch_edges;    /* stored edges of whole-graph work per batch; a
                                  single larger graph still runs alone */
   int64_t max_batch_pairs;    /* pairs per batch; a single larger request runs alone */
-  size_t hbm_budget_bytes;    /* device memory for batch workspaces and pair staging;
-                                 a request is admitted only when its batch fits */
+  size_t hbm_budget_bytes;    /* device memory for batch workspaces, pair staging and
+                                 copies of large graphs; a request is admitted only
+                                 when its batch fits */
   int32_t mode;               /* JC_SERVE_CONTINUOUS or JC_SERVE_FIFO */
   int32_t reserved[5];
 } jc_server_config;

@@ -563,8 +563,8 @@ int jc_server_run(jc_server* s, const jc_request* reqs, int32_t count, jc_reques
     // and its memory leaves a sixteenth of the budget to the next batch, with a
     // smaller bit matrix if it must; else the owner engine over the rows where
     // they are. Ten graphs of 2^12 to 2^16 vertices, 96 requests: 5.57 -> 5.43 ms;
-    // 64 graphs of 2^14 to 2^20, 512 requests: 906 -> 991 requests/s with a
-    // budget of 1 GiB, 1170 with 4 GiB.
+    // 64 graphs of 2^14 to 2^20, 512 requests: 906 -> 1010 requests/s with a
+    // budget of 1 GiB, 1660 with 4 GiB.
     jc::CopyLayout C{};
     size_t off2 = 0;
     bool tri = false;
